@@ -1,0 +1,162 @@
+"""GPU: kernels at the sizes where their tiling can go wrong, against plain numpy / torch restatements."""
+import numpy as np
+import pytest
+import torch
+
+from libfusion_amd import capi
+from tests.helpers import triangles_in_hash_order
+
+pytestmark = pytest.mark.gpu
+
+FP32, MIXED = capi.PRECISION_FP32, capi.PRECISION_MIXED
+
+
+def dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def map_of_blocks(precision, pos, sdf, weight, rgb, voxel_size=0.005, buckets=1 << 12, size=(64, 64)):
+    """A map that holds the given blocks: pos int[n,3], sdf codes int16[n,512] (FP16 bits of a mixed map),
+    weight float32[n,512] or weight codes uint8 of a mixed map, rgb uint8[n,3,512]."""
+    n = len(pos)
+    p = capi.map_params(buckets, n + 5, voxel_size, 3 * voxel_size, precision=precision)
+    m = capi.Map(p, *size)
+    lib = capi.load()
+    keys = np.full(p.num_entries, -1, np.int64)
+    slot_block = np.full(p.num_entries, -1, np.int32)
+    block_pos = np.zeros((p.num_blocks, 4), np.int32)
+    cells, occ = [], np.zeros(capi.OCC_WORDS, np.uint32)
+    for b, (x, y, z) in enumerate(pos.tolist()):
+        slot = lib.lf_compute_hash(x, y, z, p.num_buckets)
+        while keys[slot] != -1:
+            slot = (slot + 1) % p.num_entries
+        keys[slot] = ((x & 0x1FFFFF) << 42) | ((y & 0x1FFFFF) << 21) | (z & 0x1FFFFF)
+        slot_block[slot] = b
+        block_pos[b] = (x, y, z, slot)
+        o = lib.lf_occupancy_bit(x, y, z)
+        occ[o >> 5] |= np.uint32(1 << (o & 31))
+        if lib.lf_dir_cell(x, y, z) >= 0:
+            cells.append((lib.lf_dir_cell(x, y, z), b))
+    m.t["keys"].copy_(dev(keys))
+    m.t["slot_block"].copy_(dev(slot_block))
+    m.t["block_pos"].copy_(dev(block_pos.reshape(-1)))
+    m.t["occupancy"].copy_(dev(occ.view(np.int32)))
+    if cells:
+        at, b = np.array(cells).T
+        m.t["block_dir"][dev(at)] = dev(b.astype(np.int32))
+    m.t["counters"][capi.CNT_ALLOCATED] = n
+    m.t["sdf"][: n * 512] = dev(sdf.reshape(-1))
+    if precision == MIXED:
+        w = weight.astype(np.uint32)
+        for k in range(3):
+            w |= rgb[:, k].astype(np.uint32) << (8 + 8 * k)
+        m.t["weight"][: n * 512] = dev(w.view(np.int32).reshape(-1))
+    else:
+        m.t["weight"][: n * 512] = dev(weight.reshape(-1))
+        m.t["rgb"][: n * 1536] = dev(rgb.reshape(-1))
+    return m
+
+
+def mesh_of_blocks(pos, val, ok, rgb, vs):
+    """Marching cubes of the blocks in float32 numpy: val float32[n,512], ok bool[n,512], rgb uint8[n,3,512]
+    -> (vertices[t,9], normals[t,9], colours[t,9])."""
+    edge, tri = capi.mc_tables()
+    where = {tuple(q): b for b, q in enumerate(pos.tolist())}
+    corner = np.array([(0, 0, 0), (1, 0, 0), (1, 1, 0), (0, 1, 0), (0, 0, 1), (1, 0, 1), (1, 1, 1), (0, 1, 1)])
+    ends = [(0, 1), (1, 2), (2, 3), (3, 0), (4, 5), (5, 6), (6, 7), (7, 4), (0, 4), (1, 5), (2, 6), (3, 7)]
+    one = np.float32(1)
+    out = []
+    for b, q in enumerate(pos.tolist()):
+        V, G, C = np.zeros((9, 9, 9), np.float32), np.zeros((9, 9, 9), bool), np.zeros((9, 9, 9, 3), np.uint8)  # z y x
+        for k in range(8):
+            d = (k & 1, k >> 1 & 1, k >> 2)
+            nb = where.get((q[0] + d[0], q[1] + d[1], q[2] + d[2]))
+            if nb is None:
+                continue
+            at = tuple(slice(8, 9) if e else slice(0, 8) for e in d[::-1])
+            src = tuple(slice(0, 1) if e else slice(0, 8) for e in d[::-1])
+            V[at] = val[nb].reshape(8, 8, 8)[src]
+            G[at] = ok[nb].reshape(8, 8, 8)[src]
+            C[at] = np.moveaxis(rgb[nb].reshape(3, 8, 8, 8), 0, -1)[src]
+        z, y, x = np.meshgrid(*[np.arange(8)] * 3, indexing="ij")
+        s = np.stack([V[z + c[2], y + c[1], x + c[0]] for c in corner], -1)
+        g = np.all([G[z + c[2], y + c[1], x + c[0]] for c in corner], 0)
+        ci = ((s < 0) << np.arange(8)).sum(-1) * g
+        for iz, iy, ix in np.argwhere(edge[ci] != 0):
+            c, sv = ci[iz, iy, ix], s[iz, iy, ix]
+            base = np.float32([q[0] * 8 + ix, q[1] * 8 + iy, q[2] * 8 + iz])
+            for t in range(0, 15, 3):
+                if tri[c, t] < 0:
+                    break
+                vtx, col = [], []
+                for e in tri[c, t:t + 3]:
+                    i, j = ends[e]
+                    a, d = sv[i], sv[j]
+                    f = (np.float32(0) if abs(float(a)) < 1e-6 else one if abs(float(d)) < 1e-6 else
+                         np.float32(0) if abs(float(a - d)) < 1e-6 else (np.float32(0) - a) / (d - a))
+                    off = corner[i].astype(np.float32)
+                    ax = int(np.flatnonzero(corner[i] != corner[j])[0])
+                    off[ax] = one - f if corner[i][ax] else f
+                    vtx.append((base + off) * np.float32(vs))
+                    k = corner[i]
+                    col.append(C[iz + k[2], iy + k[1], ix + k[0]])
+                u, w = vtx[1] - vtx[0], vtx[2] - vtx[0]
+                n = np.float32([u[1] * w[2] - u[2] * w[1], u[2] * w[0] - u[0] * w[2], u[0] * w[1] - u[1] * w[0]])
+                with np.errstate(invalid="ignore", divide="ignore"):
+                    n = n / np.sqrt((n[0] * n[0] + n[1] * n[1]) + n[2] * n[2])
+                out.append((np.concatenate(vtx), np.tile(n, 3), np.concatenate(col)))
+    v, n, c = (np.array(a) for a in zip(*out)) if out else (np.zeros((0, 9), np.float32),) * 3
+    return v, n, c
+
+
+# one block, a full row of neighbours, blocks on both sides of the block directory's end, a count that fills no
+# workgroup; dense random signs (up to 5 triangles a cube, layers that overflow the triangle list) and sparse ones
+@pytest.mark.parametrize("precision", [FP32, MIXED])
+@pytest.mark.parametrize("shape,origin,dense", [((1, 1, 1), (0, 0, 0), 1.0), ((3, 2, 2), (-1, -1, 3), 0.85),
+                                                ((2, 2, 2), (126, -129, 0), 0.5), ((3, 3, 1), (5, 0, -2), 0.02)])
+def test_mesh_of_random_blocks(precision, shape, origin, dense):
+    rng = np.random.default_rng(3)
+    pos = np.array([(x + origin[0], y + origin[1], z + origin[2]) for z in range(shape[2]) for y in range(shape[1])
+                    for x in range(shape[0])])
+    n = len(pos)
+    v = rng.uniform(-1, 1, (n, 512)) if dense > 0.1 else np.where(rng.random((n, 512)) < dense, -0.3, 0.7)
+    v[rng.random((n, 512)) < 0.02] = 0.0
+    seen = rng.random((n, 512)) < (dense if dense > 0.1 else 1.0)
+    if precision == MIXED:
+        codes = np.where(seen, v.astype(np.float16).view(np.int16), np.int16(-1)).astype(np.int16)
+        val = codes.view(np.float16).astype(np.float32)
+        weight = np.where(seen, rng.integers(1, 240, (n, 512)), 0).astype(np.uint8)
+        w = capi.weight_values()[weight]
+    else:
+        codes = np.where(seen, (v * 32767).astype(np.int16), np.int16(-32768)).astype(np.int16)
+        val = codes.astype(np.float32) / np.float32(32767)
+        weight = w = np.where(seen, rng.choice([5e-4, 0.1, 7.0], (n, 512)), 0).astype(np.float32)
+    rgb = rng.integers(0, 256, (n, 3, 512)).astype(np.uint8)
+    m = map_of_blocks(precision, pos, codes, weight, rgb)
+    vs = m.params.voxel_size
+    for mode in (0, 1, 2):
+        ok = w > 1e-3 if mode == 2 else w != 0
+        ov, on, oc = mesh_of_blocks(pos, np.where(ok, val, 0).astype(np.float32), ok, rgb, vs)
+        gv, gx, count = m.mesh(mode=mode, max_triangles=len(ov) + 64)
+        assert count == len(ov) and len(gv) == len(ov)
+        gv = gv.cpu().numpy().reshape(-1, 9)
+        if mode == 0:
+            assert np.array_equal(triangles_in_hash_order(gv.reshape(-1, 3, 3)), triangles_in_hash_order(ov.reshape(-1, 3, 3)))
+            continue
+        gx, ox = gx.cpu().numpy().reshape(-1, 9), on if mode == 1 else oc
+        # rows ordered by vertices, then by the normal / colour (equal triangles of neighbouring cubes)
+        rows = [np.concatenate([a, np.nan_to_num(b.astype(np.float32))], 1) + np.float32(0) for a, b in ((gv, gx), (ov, ox))]
+        g, o = (r[np.lexsort(r.T[::-1])] for r in rows)
+        assert np.array_equal(g[:, :9], o[:, :9])
+        # normals: one rounding apart per operation of the cross product and the normalisation
+        assert np.array_equal(g[:, 9:], o[:, 9:]) if mode == 2 else np.allclose(g[:, 9:], o[:, 9:], atol=1e-6)
+    # a capacity inside the output: the count goes on, nothing is written beyond it
+    cap = max(1, len(ov) - 70)
+    out = torch.full((len(ov) + 64, 9), 7.0, device="cuda")
+    import ctypes
+    got = ctypes.c_uint(0)
+    rc = capi.load().lf_create_mesh(ctypes.byref(m.params), ctypes.byref(m.storage), capi.ptr(out), None, None, cap,
+                                    ctypes.byref(got), capi.stream_ptr())
+    full = int(m.counters()[capi.CNT_TRIANGLES])
+    assert got.value == min(cap, full) and rc == (capi.LF_ERR_CAPACITY if full > cap else capi.LF_OK)
+    assert torch.all(out[got.value:] == 7.0) and not torch.any((out[: got.value] == 7.0).all(1))
