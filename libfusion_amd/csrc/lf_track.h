@@ -6,23 +6,29 @@
 
 #include "libfusion_amd.h"
 
-// One tracker's state in device memory.  Poses are 3x4 row-major doubles.
-struct LfTrackState {
-    double est[12];      // current estimate T (reference camera -> current camera)
-    double prev[12];     // Revertable<SE3d>::prev (revertable.h:7-45)
-    double init[12];     // initial estimate (identity in DenseOdometry)
-    float pose_f[12];    // float 3x4 of est, read by the next reduction
+// The Gauss-Newton state of a frame after one of its steps.
+struct LfGnState {
+    double est[12];        // current estimate T (reference camera -> current camera), 3x4 row-major
     float icp_error, rgb_error, stddev;
     float last_icp_error;  // icp error before the last step (last_icp_error of compute_transform(ctx))
     int icp_count, rgb_count;
-    int active;          // 0 once the current level broke out of its loop
-    int invalid;         // an error became NaN this frame
+    int active;            // 0 once the current level broke out of its loop
+    int invalid;           // an error became NaN this frame
+    int iterations;        // Gauss-Newton steps taken this frame
+    int pad;
+};
+
+// One tracker's state in device memory.  Poses are 3x4 row-major doubles.
+struct LfTrackState {
+    LfGnState gn;        // after the last step that was taken
+    LfGnState slot[2];   // after step k - 1, in slot k & 1: read by step k's launch while it writes the other
+    double prev[12];     // Revertable<SE3d>::prev (revertable.h:7-45)
+    double init[12];     // initial estimate (identity in DenseOdometry)
     int success;         // result of the last finished frame
-    int iterations;      // Gauss-Newton steps taken this frame
+    int pad;
     // odometry chain (DenseOdometry::trackFrame, rgbd_odometry.cpp:18-48)
     double pose[12];     // T_world_camera of the current frame
     float pose24[24];    // float T_world_camera and T_camera_world for the mapping kernels
-    int pad[3];
     // the last Gauss-Newton step's FP64 sums: A = w H_icp + H_rgb and b in
     // create_jtjjtr<6,7> order (0-26), ICP r^2 / count (27 / 28), RGB r^2 /
     // count (29 / 30)
@@ -38,26 +44,34 @@ struct LfTrackLevel {
     int half_maps;  // the maps hold FP16 (nmap 4 x FP16, intensity and gradients FP16; vmaps stay float4)
 };
 
-// Scratch floats needed by the reductions (partial rows of the workgroups).
+// Scratch floats needed by the stand-alone reductions and by a tracker's steps
+// (partial rows of the workgroups).
 size_t lf_reduce_partials(void);
+size_t lf_track_scratch_floats(void);
 
 // Schedule position of one Gauss-Newton step within a tracked frame.
 struct LfStepFlags {
-    int first_of_level;  // first iteration of a pyramid level (resets the error history)
-    int first_of_frame;  // the estimate starts at init (replaces lf_track_begin)
-    int last_level;      // a step of the finest level: breaking out of its loop ends the frame
-    int last_of_frame;   // the frame's last scheduled step: finish after it
-    int context_mode;    // compute_transform(ctx) (icp_tracker.cpp:210-314): NaN errors are not
-                         // flagged and the finish always succeeds with update = estimate^-1
-    double init[12];     // initial estimate, 3x4 row-major (first_of_frame)
+    int step;                 // index within the frame; 0 starts the estimate at init (replaces lf_track_begin)
+    int end;                  // the launch after the last step: no step of its own
+    int first_of_level;       // first iteration of a pyramid level (resets the error history)
+    // the step before
+    int prev_first_of_level;
+    int prev_ends;            // 1: a step of the finest level (breaking out of its loop ends the frame),
+                              // 2: the frame's last scheduled step; else 0
+    int prev_grid;            // its workgroups
+    int context_mode;         // compute_transform(ctx) (icp_tracker.cpp:210-314): NaN errors are not
+                              // flagged and the finish always succeeds with update = estimate^-1
+    double init[12];          // initial estimate, 3x4 row-major (step 0)
 };
 
 // One Gauss-Newton iteration of DenseTracking::compute_transform
-// (icp_tracker.cpp:50-140) in two launches: fused ICP + RGB reduction, FP64
-// solve, SE3 update, divergence checks and, when the frame ends at this step,
-// the finish of lf_track_finish — entirely on the device.
-int lf_track_iteration(const LfTrackLevel &lv, float *scratch, LfTrackState *st, const LfStepFlags &f,
-                       float icp_weight, hipStream_t stream);
+// (icp_tracker.cpp:50-140) in one launch, entirely on the device: the previous
+// step's sums, FP64 solve, SE3 update, divergence checks and, when the frame
+// ends there, the finish of lf_track_finish; then this step's fused ICP + RGB
+// reduction.  A frame is its steps in order and one launch with end set.
+// scratch: lf_track_scratch_floats().  *grid: the workgroups used.
+int lf_track_step(const LfTrackLevel &lv, float *scratch, LfTrackState *st, const LfStepFlags &f, float icp_weight,
+                  hipStream_t stream, int *grid);
 // Start a frame's estimate at T (3x4 doubles, host): est = prev = init = T.
 // Only needed when a frame schedules no step.
 int lf_track_begin(LfTrackState *st, const double *T12, hipStream_t stream);
@@ -67,15 +81,15 @@ int lf_track_finish(LfTrackState *st, hipStream_t stream);
 // Set the odometry pose directly (first frame / restart): T given as 3x4 doubles (host).
 int lf_track_set_pose(LfTrackState *st, const double *T12, hipStream_t stream);
 
-// Batched tracking: one step of several systems in one launch pair.  A job is
+// Batched tracking: one step of several systems in one launch.  A job is
 // the launch arguments of one system's step (lf_track_job_bytes each);
 // lf_track_job_make fills one and reports its grid, lf_track_job_skip marks a
-// system without a step at this index.  lf_track_batch_step runs step jobs[0..n)
+// system with nothing at this index.  lf_track_batch_step runs step jobs[0..n)
 // (device memory) with a grid of gmax workgroups per system (the largest job
-// grid).  A job made with share n takes 1/n of lf_track_iteration's
-// workgroups (at least one), so n systems together fill the resident grid
-// once; each lane then sums several pixels, and the system's sums equal
-// lf_track_iteration's up to FP32 summation order (exactly, for share 1).
+// grid).  A job made with share n takes 1/n of the resident workgroups (at
+// least one), so n systems together fill the grid once; each lane then sums
+// several pixels, and the system's sums equal lf_track_step's up to FP64
+// summation order (exactly, for share 1).
 // The jobs of one batch share one map format (half_maps as in their LfTrackLevel).
 size_t lf_track_job_bytes(void);
 // share: systems sharing the launch (the job's grid is 1/share of a lone

@@ -15,15 +15,15 @@
 //  * One lane per reference pixel, so a whole pyramid level is in flight at
 //    once (the pass is bound by memory latency, not bandwidth); each pixel's
 //    loads are issued in two rounds.
-//  * A tracking iteration is two launches: the partial rows, then one
-//    workgroup that sums them in a fixed order (deterministic), after which
-//    one lane builds A = 1e6 H_icp + H_rgb, solves it with an FP64 LDL^T,
-//    applies T <- exp(dx) T in FP64 and runs the reference's divergence /
-//    revert logic; the first step of a frame starts the estimate and the step
-//    that ends the frame runs the finish.  The next iteration reads the
-//    updated pose from device memory: a whole frame of tracking is a fixed
-//    sequence of launches with no host round trip (the reference downloads
-//    the sums and solves on the host twice per iteration).
+//  * A tracking iteration is one launch: every workgroup sums the previous
+//    iteration's partial rows in a fixed order (deterministic), one lane builds
+//    A = 1e6 H_icp + H_rgb, solves it with an FP64 LDL^T, applies T <- exp(dx) T
+//    in FP64 and runs the reference's divergence / revert logic; then the
+//    workgroup adds up its own partial row at the new pose.  The first launch of
+//    a frame starts the estimate and a last one, of one workgroup, ends it: a
+//    whole frame of tracking is a fixed sequence of launches with no host
+//    round trip (the reference downloads the sums and solves on the host twice
+//    per iteration).
 //  * The stand-alone reductions of the C-ABI (lf_icp_reduce, lf_rgb_step) are
 //    a partial-sum launch and a one-workgroup final-sum launch.
 #include <cfloat>
@@ -42,6 +42,7 @@ namespace {
 // count).  A larger level loops over pixels with the next pixel's loads in
 // flight, rather than waiting for a second round of workgroups.
 constexpr int kGrid = 512;
+constexpr int kStepGrid = 256;  // of a lone system's tracking step (step_grid)
 constexpr int kThreads = 512;  // lanes per workgroup (8 wavefronts)
 constexpr int kWaves = kThreads / 64;
 constexpr int kVals = 58;      // 29 ICP + 29 RGB sums
@@ -53,14 +54,17 @@ struct ReduceArgs {
     float angle, dthr;
     float *partials;       // kGrid * kVals floats
     float *out29;          // modes 1/2
-    LfTrackState *st;      // tracking step
+    // tracking step
+    LfTrackState *st;
+    int step;              // index within the frame; 0: the estimate starts at init
+    int end;               // no step of its own: only the previous one's solve (after the frame's last step)
     int first_iter;        // first iteration of a level
+    int prev_first_iter;   // the previous step's first_iter,
+    int prev_ends;         // whether the frame ends at it once its level breaks out (1) or in any case (2),
+    int prev_grid;         // and its workgroups (partial rows)
+    int context_mode;      // compute_transform(ctx) semantics
     float icp_weight;
-    int first_of_frame;    // tracking step: the estimate starts at init
-    int last_level;        // tracking step: the finest level
-    int last_of_frame;     // tracking step: the frame's last scheduled step
-    int context_mode;      // tracking step: compute_transform(ctx) semantics
-    double init[12];       // tracking step: initial estimate (first_of_frame)
+    double init[12];       // initial estimate (step 0)
     float init_f[12];      // the same in FP32 (the first step's pose, uniform across the grid)
 };
 
@@ -178,6 +182,7 @@ LF_DEV Own load_own(const LfTrackLevel &L, int i) {
 // kHalf (mixed precision) also takes one hardware reciprocal of the depth for
 // every projection and the hardware square root, where the FP32 path keeps
 // the reference's correctly rounded divisions and roots.
+LF_DEV float uniform_f(float x) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))); }
 LF_DEV float fast_sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 
 template <bool kIcp, bool kRgb, bool kHalf, class Sums>
@@ -431,33 +436,9 @@ LF_DEV void unpack27(const double *s, double *A, double *b) {
         }
 }
 
-// What a Gauss-Newton step reads of the tracker state.  k_track_final loads
-// it at entry, together with the flags that decide whether the step runs, so
-// the serial step starts from registers rather than from dependent loads.
-struct GnState {
-    double est[12];
-    float icp_error, rgb_error;
-    int icp_count, rgb_count, active, invalid, iterations;
-};
-
-LF_DEV GnState load_gn(const LfTrackState &st) {
-    GnState g;
-#pragma unroll
-    for (int k = 0; k < 12; ++k) g.est[k] = st.est[k];
-    g.icp_error = st.icp_error;
-    g.rgb_error = st.rgb_error;
-    g.icp_count = st.icp_count;
-    g.rgb_count = st.rgb_count;
-    g.active = st.active;
-    g.invalid = st.invalid;
-    g.iterations = st.iterations;
-    return g;
-}
-
 // One Gauss-Newton step of compute_transform (icp_tracker.cpp:50-139), run by
-// a single lane after the sums are final: reads g, updates g and writes the
-// step's results to st.
-LF_DEV void gn_step(LfTrackState &st, GnState &g, const double *sums, int first_iter, bool context_mode) {
+// a single lane after the sums are final: updates g.
+LF_DEV void gn_step(LfGnState &g, const double *sums, int first_iter, bool context_mode) {
     if (first_iter) {
         g.icp_error = FLT_MAX;
         g.rgb_error = FLT_MAX;
@@ -467,11 +448,11 @@ LF_DEV void gn_step(LfTrackState &st, GnState &g, const double *sums, int first_
     double last[12];
     for (int k = 0; k < 12; ++k) last[k] = g.est[k];
     const float last_icp = g.icp_error, last_rgb = g.rgb_error;
-    st.last_icp_error = last_icp;
+    g.last_icp_error = last_icp;
     // the residual terms in FP32, as the reference's (m_estimator.cu:470-480)
     const float icp_r2 = (float)sums[27], icp_n = (float)sums[28];
     const float rgb_r2 = (float)sums[29], rgb_n = (float)sums[30];
-    st.stddev = sqrtf(rgb_r2 / (rgb_n - 6.0f));
+    g.stddev = sqrtf(rgb_r2 / (rgb_n - 6.0f));
     double A[36], b[6], x[6];
     unpack27(sums, A, b);
     ldlt6(A, b, x);
@@ -516,18 +497,6 @@ LF_DEV void gn_step(LfTrackState &st, GnState &g, const double *sums, int first_
     if (revert)
         for (int k = 0; k < 12; ++k) g.est[k] = last[k];
     g.active = stop ? 0 : 1;
-    for (int k = 0; k < 12; ++k) {
-        st.prev[k] = last[k];
-        st.est[k] = g.est[k];
-        st.pose_f[k] = (float)g.est[k];
-    }
-    st.icp_error = g.icp_error;
-    st.rgb_error = g.rgb_error;
-    st.icp_count = g.icp_count;
-    st.rgb_count = g.rgb_count;
-    st.active = g.active;
-    st.invalid = g.invalid;
-    st.iterations = g.iterations;
 }
 
 // Wavefront sum of N values per lane (N a power of two, <= 64) as a
@@ -674,9 +643,11 @@ LF_DEV void final_sums_d_chunks(const double *partials, int G, double *s_sum) {
     const int v = wave + kWaves * (lane >> 4);
     if ((lane & 15) == 0 && v < kTrackVals) s_sum[v] = s;
 }
-// (a batch of 16 systems: 32 partials per value, one chunk)
+// (a batch of 16 systems: 32 partials per value, one chunk; a lone system's
+// levels: at most 256)
 LF_DEV void final_sums_d(const double *partials, int G, double *s_sum) {
     if (G <= 64) final_sums_d_chunks<1>(partials, G, s_sum);
+    else if (G <= 256) final_sums_d_chunks<4>(partials, G, s_sum);
     else final_sums_d_chunks<kGrid / 64>(partials, G, s_sum);
 }
 
@@ -736,33 +707,93 @@ LF_DEV void track_finish(LfTrackState &st, const double *est, int invalid, bool 
     }
 }
 
-// One Gauss-Newton iteration of compute_transform, first launch: every
-// workgroup sums the ICP and RGB rows of its pixels into one partial row.  The
-// pose-independent loads of the first pixel are issued together with the
-// tracker-state loads.
+// LDS of a tracking step's workgroup: the wavefronts' partial sums, and what
+// the previous step's solve leaves for this one.
+struct StepLds {
+    double wave[kWaves][32], sum[32];
+    float pose[12], stddev;
+    int run;
+};
+
+// The partial rows of step k: two halves of the scratch taken in turn, as a
+// step's workgroups read the previous step's rows while others write theirs.
+LF_DEV double *step_partials(const ReduceArgs &a, int k) {
+    return reinterpret_cast<double *>(a.partials) + (size_t)(k & 1) * (kGrid * kTrackVals);
+}
+
+// The previous step's end, at the head of every workgroup of this one: its
+// partial rows summed in a fixed order, then the FP64 solve on one lane, whose
+// pose is this step's.  Every workgroup computes the same; workgroup 0 stores
+// the state (the two slots in turn, for the same reason as the rows) and,
+// where the frame ends, runs the finish.
+LF_DEV void solve_previous(const ReduceArgs &a, int wg, StepLds &s) {
+    const int tid = threadIdx.x;
+    LfTrackState &st = *a.st;
+    LfGnState g = st.slot[(a.step - 1) & 1];
+    // a failed frame, or a level that broke out of its loop: no step was taken
+    const bool ran = !g.invalid && (a.prev_first_iter || g.active);
+    if (ran) {
+        final_sums_d(step_partials(a, a.step - 1), a.prev_grid, s.sum);
+        __syncthreads();
+        if (wg == 0 && tid < kTrackVals) st.sums[tid] = s.sum[tid];
+    }
+    if (tid == 0) {
+        if (ran) {
+            if (wg == 0)
+                for (int k = 0; k < 12; ++k) st.prev[k] = g.est[k];
+            gn_step(g, s.sum, a.prev_first_iter, a.context_mode != 0);
+        }
+#pragma unroll
+        for (int k = 0; k < 12; ++k) s.pose[k] = (float)g.est[k];
+        s.stddev = g.stddev;
+        s.run = !g.invalid && (a.first_iter || g.active);
+        if (wg == 0) {
+            st.slot[a.step & 1] = g;
+            if (ran) {
+                st.gn = g;
+                // the frame ends here when the estimate became invalid, when the
+                // finest level broke out of its loop, or after the frame's last step
+                if (g.invalid || (a.prev_ends && !g.active) || a.prev_ends == 2)
+                    track_finish(st, g.est, g.invalid, a.context_mode != 0);
+            }
+        }
+    }
+    __syncthreads();
+}
+
+// One Gauss-Newton iteration of compute_transform: the previous step's solve,
+// then every workgroup sums the ICP and RGB rows of its pixels into one partial
+// row.  The pose-independent loads of the first pixel are in flight during the
+// solve.  One launch per step: a step's own kernel boundary is the only wait
+// between the rows and their sum.  (The solve in a launch of its own, one
+// workgroup, cost 3.6-4.3 us a step beside 5.3-6.6 us of rows; a
+// last-workgroup ticket costs 11 ns per workgroup, as atomics on one address
+// are taken in turn, and more than the launch from 128 workgroups on.)
 // Workgroup wg of the nwg computing the step's partial rows.  kHalf: FP16 maps.
 template <bool kHalf>
-LF_DEV void track_step_wg(const ReduceArgs &a, int wg, int nwg, double (*s_wave)[32]) {
+LF_DEV void track_step_wg(const ReduceArgs &a, int wg, int nwg, StepLds &s) {
     const int tid = threadIdx.x;
-    const int n = a.lv.cols * a.lv.rows;
+    const int n = a.end ? 0 : a.lv.cols * a.lv.rows;
     const int stride = nwg * kThreads;
     int i = wg * kThreads + tid;
-    // the pixel's own loads and the state loads are in flight together
     Own o = {};
     if (i < n) o = load_own<true, true, kHalf>(a.lv, i);
     float P[12], stddev;
-    if (a.first_of_frame) {
+    if (a.step == 0) {
 #pragma unroll
         for (int k = 0; k < 12; ++k) P[k] = a.init_f[k];
         stddev = 0.0f;
+        if (wg == 0 && tid == 0) {
+            LfGnState g = {};
+            for (int k = 0; k < 12; ++k) a.st->init[k] = g.est[k] = a.init[k];
+            a.st->slot[0] = g;
+        }
     } else {
-        const LfTrackState &st = *a.st;
-        const bool run = !st.invalid && (a.first_iter || st.active);
+        solve_previous(a, wg, s);
+        if (a.end || !s.run) return;
 #pragma unroll
-        for (int k = 0; k < 12; ++k) P[k] = st.pose_f[k];
-        stddev = a.first_iter ? 0.0f : st.stddev;
-        // a failed frame, or a level that broke out of its loop: nothing to do
-        if (!run) return;
+        for (int k = 0; k < 12; ++k) P[k] = uniform_f(s.pose[k]);
+        stddev = a.first_iter ? 0.0f : uniform_f(s.stddev);
     }
     const float th = (float)(1.345 * (double)stddev);
     CombinedSums sums;
@@ -775,52 +806,15 @@ LF_DEV void track_step_wg(const ReduceArgs &a, int wg, int nwg, double (*s_wave)
         pixel_rows<true, true, kHalf>(a, cur, P, stddev, th, sums);
         i = next;
     }
-    const double t = block_sums_d(sums, s_wave);
-    if (tid < kTrackVals) reinterpret_cast<double *>(a.partials)[(size_t)tid * nwg + wg] = t;
+    const double t = block_sums_d(sums, s.wave);
+    if (tid < kTrackVals) step_partials(a, a.step)[(size_t)tid * nwg + wg] = t;
 }
 
 // Held to 128 VGPRs: 4 waves per SIMD, two 512-lane workgroups per CU.
 template <bool kHalf>
 __global__ __launch_bounds__(kThreads, 4) void k_track_step(ReduceArgs a) {
-    __shared__ double s_wave[kWaves][32];
-    track_step_wg<kHalf>(a, blockIdx.x, gridDim.x, s_wave);
-}
-
-// Second launch (one workgroup): the partial rows summed in a fixed order,
-// then the FP64 step; the first launch of a frame starts the estimate at init
-// and the launch that ends the frame runs the finish.  (A single launch with a
-// last-workgroup ticket needs an agent-scope release per workgroup, an L2
-// write-back on each of the 8 XCDs per workgroup; measured slower than the
-// kernel boundary.)
-LF_DEV void track_final_wg(const ReduceArgs &a, int G, double *s_sum) {
-    const int tid = threadIdx.x;
-    GnState g = load_gn(*a.st);
-    if (a.first_of_frame) {
-#pragma unroll
-        for (int k = 0; k < 12; ++k) g.est[k] = a.init[k];
-        g.invalid = 0;
-        g.iterations = 0;
-    } else if (!(!g.invalid && (a.first_iter || g.active))) {
-        return;
-    }
-    final_sums_d(reinterpret_cast<const double *>(a.partials), G, s_sum);
-    __syncthreads();
-    if (tid < kTrackVals) a.st->sums[tid] = s_sum[tid];
-    if (tid == 0) {
-        LfTrackState &st = *a.st;
-        if (a.first_of_frame)
-            for (int k = 0; k < 12; ++k) st.init[k] = a.init[k];
-        gn_step(st, g, s_sum, a.first_iter, a.context_mode != 0);
-        // the frame ends here when the estimate became invalid, when the
-        // finest level broke out of its loop, or after the frame's last step
-        if (g.invalid || (a.last_level && !g.active) || a.last_of_frame)
-            track_finish(st, g.est, g.invalid, a.context_mode != 0);
-    }
-}
-
-__global__ __launch_bounds__(kThreads) void k_track_final(ReduceArgs a, int G) {
-    __shared__ double s_sum[32];
-    track_final_wg(a, G, s_sum);
+    __shared__ StepLds s;
+    track_step_wg<kHalf>(a, blockIdx.x, gridDim.x, s);
 }
 
 // Launch arguments read from a descriptor table, their pointers asserted global.
@@ -837,7 +831,7 @@ LF_DEV ReduceArgs global_args(const ReduceArgs &d) {
 }
 
 // One system's step of a batch: its launch arguments and its grid (0: the
-// system has no step at this index).
+// system has nothing at this index).
 struct TrackJob {
     ReduceArgs a;
     int G;
@@ -848,40 +842,31 @@ struct TrackJob {
 // run exactly the single launch's code.
 template <bool kHalf>
 __global__ __launch_bounds__(kThreads, 4) void k_track_step_batch(const TrackJob *__restrict__ jobs) {
-    __shared__ double s_wave[kWaves][32];
+    __shared__ StepLds s;
     const TrackJob &j = jobs[blockIdx.y];
     if ((int)blockIdx.x >= j.G) return;
-    track_step_wg<kHalf>(global_args(j.a), blockIdx.x, j.G, s_wave);
-}
-
-// The final sums and Gauss-Newton step of each system: workgroup i, system i.
-__global__ __launch_bounds__(kThreads) void k_track_final_batch(const TrackJob *__restrict__ jobs) {
-    __shared__ double s_sum[32];
-    const TrackJob &j = jobs[blockIdx.x];
-    if (j.G <= 0) return;
-    track_final_wg(global_args(j.a), j.G, s_sum);
+    track_step_wg<kHalf>(global_args(j.a), blockIdx.x, j.G, s);
 }
 
 __global__ void k_track_finish(LfTrackState *st) {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
     LfTrackState &s = *st;
     double est[12];
-    for (int k = 0; k < 12; ++k) est[k] = s.est[k];
-    track_finish(s, est, s.invalid, false);
+    for (int k = 0; k < 12; ++k) est[k] = s.gn.est[k];
+    track_finish(s, est, s.gn.invalid, false);
 }
 
 __global__ void k_track_begin(LfTrackState *st, double t0, double t1, double t2, double t3, double t4, double t5,
                               double t6, double t7, double t8, double t9, double t10, double t11) {
     const double T[12] = {t0, t1, t2, t3, t4, t5, t6, t7, t8, t9, t10, t11};
     for (int k = 0; k < 12; ++k) {
-        st->est[k] = T[k];
+        st->gn.est[k] = T[k];
         st->prev[k] = T[k];
         st->init[k] = T[k];
-        st->pose_f[k] = (float)T[k];
     }
-    st->invalid = 0;
-    st->active = 1;
-    st->iterations = 0;
+    st->gn.invalid = 0;
+    st->gn.active = 1;
+    st->gn.iterations = 0;
 }
 
 __global__ void k_track_set_pose(LfTrackState *st, double t0, double t1, double t2, double t3, double t4, double t5,
@@ -912,11 +897,12 @@ int grid_for(const LfTrackLevel &lv) {
 
 }  // namespace
 
-// The stand-alone reductions' kGrid x kVals FP32 partials, or the tracking
-// step's kGrid x kTrackVals FP64 partials, whichever is larger.
+// The stand-alone reductions' kGrid x kVals FP32 partials.
 size_t lf_reduce_partials(void) {
     return std::max((size_t)kGrid * kVals, (size_t)kGrid * kTrackVals * 2) + 64;
 }
+// The tracking steps' two halves of kGrid x kTrackVals FP64 partials.
+size_t lf_track_scratch_floats(void) { return (size_t)kGrid * kTrackVals * 2 * 2; }
 
 extern "C" size_t lf_reduce_scratch_floats(void) { return lf_reduce_partials(); }
 
@@ -934,11 +920,13 @@ static ReduceArgs step_args(const LfTrackLevel &lv, float *scratch, LfTrackState
     a.dthr = 0.01f;
     a.partials = scratch;
     a.st = st;
+    a.step = f.step;
+    a.end = f.end;
     a.first_iter = f.first_of_level;
+    a.prev_first_iter = f.prev_first_of_level;
+    a.prev_ends = f.prev_ends;
+    a.prev_grid = f.prev_grid;
     a.icp_weight = icp_weight;
-    a.first_of_frame = f.first_of_frame;
-    a.last_level = f.last_level;
-    a.last_of_frame = f.last_of_frame;
     a.context_mode = f.context_mode;
     for (int k = 0; k < 12; ++k) {
         a.init[k] = f.init[k];
@@ -947,16 +935,24 @@ static ReduceArgs step_args(const LfTrackLevel &lv, float *scratch, LfTrackState
     return a;
 }
 
-int lf_track_iteration(const LfTrackLevel &lv, float *scratch, LfTrackState *st, const LfStepFlags &f,
-                       float icp_weight, hipStream_t stream) {
+// Workgroups of a tracking step of one of `share` systems (wgs > 0: given):
+// a lone system takes 256, one per CU.  Each of them sums all of the
+// previous step's rows, and a level-0 lane then sums two pixels with the
+// second one's loads in flight.
+static int step_grid(const LfTrackLevel &lv, int share, int wgs, int end) {
+    if (end) return 1;
+    return std::min(grid_for(lv), wgs > 0 ? std::min(wgs, kGrid) : std::max(1, std::min(kStepGrid, kGrid / std::max(1, share))));
+}
+
+int lf_track_step(const LfTrackLevel &lv, float *scratch, LfTrackState *st, const LfStepFlags &f, float icp_weight,
+                  hipStream_t stream, int *grid) {
     if (int rc = check_level(lv)) return rc;
     const ReduceArgs a = step_args(lv, scratch, st, f, icp_weight);
-    const int G = grid_for(lv);
+    const int G = step_grid(lv, 1, 0, f.end);
     if (lv.half_maps) k_track_step<true><<<G, kThreads, 0, stream>>>(a);
     else k_track_step<false><<<G, kThreads, 0, stream>>>(a);
     LF_LAUNCH_CHECK();
-    k_track_final<<<1, kThreads, 0, stream>>>(a, G);
-    LF_LAUNCH_CHECK();
+    if (grid) *grid = G;
     return LF_OK;
 }
 
@@ -973,7 +969,7 @@ int lf_track_job_make(const LfTrackLevel &lv, float *scratch, LfTrackState *st, 
     // flight, and do 1/16 of the block reductions): 4.1k -> 4.7k frames/s
     // aggregate in mixed precision.  16 and 64 workgroups each measured
     // slower than 32 (5.46k and 5.61k against 5.74k).
-    j.G = std::min(grid_for(lv), wgs > 0 ? std::min(wgs, kGrid) : std::max(1, kGrid / std::max(1, share)));
+    j.G = step_grid(lv, share, wgs, f.end);
     if (grid) *grid = j.G;
     return LF_OK;
 }
@@ -987,12 +983,9 @@ void lf_track_job_skip(void *job) {
 int lf_track_batch_step(const void *jobs, int n, int gmax, int half_maps, hipStream_t stream) {
     if (!jobs || n <= 0 || n > 65535) return lf_set_error(LF_ERR_ARG, "bad tracking batch of %d", n);
     const TrackJob *J = static_cast<const TrackJob *>(jobs);
-    if (gmax > 0) {
-        if (half_maps) k_track_step_batch<true><<<dim3(gmax, n), kThreads, 0, stream>>>(J);
-        else k_track_step_batch<false><<<dim3(gmax, n), kThreads, 0, stream>>>(J);
-        LF_LAUNCH_CHECK();
-    }
-    k_track_final_batch<<<n, kThreads, 0, stream>>>(J);
+    if (gmax <= 0) return LF_OK;
+    if (half_maps) k_track_step_batch<true><<<dim3(gmax, n), kThreads, 0, stream>>>(J);
+    else k_track_step_batch<false><<<dim3(gmax, n), kThreads, 0, stream>>>(J);
     LF_LAUNCH_CHECK();
     return LF_OK;
 }

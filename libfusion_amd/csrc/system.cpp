@@ -346,7 +346,7 @@ size_t DenseMapping::fetch_mesh_with_colour(float *vertex, unsigned char *colour
 
 DenseTracking::DenseTracking(hipStream_t stream) : stream_(stream) {
     if (hipMalloc(&state_, sizeof(LfTrackState)) != hipSuccess) throw std::bad_alloc();
-    if (hipMalloc(&scratch_, lf_reduce_partials() * sizeof(float)) != hipSuccess) throw std::bad_alloc();
+    if (hipMalloc(&scratch_, lf_track_scratch_floats() * sizeof(float)) != hipSuccess) throw std::bad_alloc();
     // every field defined before the first frame (errors 0, success 0, counts 0)
     if (hipMemsetAsync(state_, 0, sizeof(LfTrackState), stream_) != hipSuccess)
         throw std::runtime_error("hipMemsetAsync failed");
@@ -406,8 +406,10 @@ int DenseTracking::enqueue(DeviceImage &ref, DeviceImage &cur, const TrackingCon
         return lf_track_finish(state_, stream_);
     }
     const int finest = plan.back().level;
-    for (size_t s = 0; s < plan.size(); ++s) {
-        const int level = plan[s].level;
+    // a launch per step and one that ends the frame (the last step's level, of which it reads nothing)
+    for (size_t s = 0; s <= plan.size(); ++s) {
+        f.end = s == plan.size();
+        const int level = plan[s - (f.end ? 1 : 0)].level;
         LfTrackLevel lv;
         lv.curr_vmap = cur.get_vmap(level).ptr<float>();
         lv.curr_nmap = cur.get_nmap(level).ptr<float>();
@@ -422,20 +424,21 @@ int DenseTracking::enqueue(DeviceImage &ref, DeviceImage &cur, const TrackingCon
         lv.rows = K.height;
         lv.K = K;
         lv.half_maps = cur.half_maps() ? 1 : 0;
-        f.first_of_level = plan[s].it == 0;
-        f.first_of_frame = s == 0;
-        f.last_level = level == finest;
-        f.last_of_frame = s + 1 == plan.size();
+        f.step = (int)s;
+        f.first_of_level = !f.end && plan[s].it == 0;
+        int G = 0;
         if (jobs) {
             const size_t J = lf_track_job_bytes();
             jobs->resize(jobs->size() + J);
-            int G = 0;
-            LF_RC(lf_track_job_make(lv, scratch_, state_, f, icp_weight, batch_share_, batch_wgs_, jobs->data() + jobs->size() - J,
-                                    &G));
+            LF_RC(lf_track_job_make(lv, scratch_, state_, f, icp_weight, batch_share_, batch_wgs_,
+                                    jobs->data() + jobs->size() - J, &G));
             grids->push_back(G);
         } else {
-            LF_RC(lf_track_iteration(lv, scratch_, state_, f, icp_weight, stream_));
+            LF_RC(lf_track_step(lv, scratch_, state_, f, icp_weight, stream_, &G));
         }
+        f.prev_first_of_level = f.first_of_level;
+        f.prev_ends = s + 1 == plan.size() ? 2 : level == finest ? 1 : 0;
+        f.prev_grid = G;
     }
     return LF_OK;
 }
@@ -447,8 +450,8 @@ TrackingResult DenseTracking::result() {
     if (hipStreamSynchronize(stream_) != hipSuccess) return r;
     r.sucess = h.success != 0;
     // compute_transform(ctx) reports last_icp_error (icp_tracker.cpp:310)
-    r.icp_error = context_mode_ ? h.last_icp_error : h.icp_error;
-    r.update = r.sucess ? SE3d::from3x4(h.est).inverse() : SE3d();
+    r.icp_error = context_mode_ ? h.gn.last_icp_error : h.gn.icp_error;
+    r.update = r.sucess ? SE3d::from3x4(h.gn.est).inverse() : SE3d();
     return r;
 }
 
