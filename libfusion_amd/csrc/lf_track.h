@@ -52,12 +52,10 @@ size_t lf_track_scratch_floats(void);
 // Schedule position of one Gauss-Newton step within a tracked frame.
 struct LfStepFlags {
     int step;                 // index within the frame; 0 starts the estimate at init (replaces lf_track_begin)
-    int end;                  // the launch after the last step: no step of its own
+    int end;                  // the launch after the last step: its solve and lf_track_finish
     int first_of_level;       // first iteration of a pyramid level (resets the error history)
     // the step before
     int prev_first_of_level;
-    int prev_ends;            // 1: a step of the finest level (breaking out of its loop ends the frame),
-                              // 2: the frame's last scheduled step; else 0
     int prev_grid;            // its workgroups
     int context_mode;         // compute_transform(ctx) (icp_tracker.cpp:210-314): NaN errors are not
                               // flagged and the finish always succeeds with update = estimate^-1
@@ -66,9 +64,8 @@ struct LfStepFlags {
 
 // One Gauss-Newton iteration of DenseTracking::compute_transform
 // (icp_tracker.cpp:50-140) in one launch, entirely on the device: the previous
-// step's sums, FP64 solve, SE3 update, divergence checks and, when the frame
-// ends there, the finish of lf_track_finish; then this step's fused ICP + RGB
-// reduction.  A frame is its steps in order and one launch with end set.
+// step's sums, FP64 solve, SE3 update and divergence checks, then this step's
+// fused ICP + RGB reduction.  A frame is its steps in order and one launch with end set.
 // scratch: lf_track_scratch_floats().  *grid: the workgroups used.
 int lf_track_step(const LfTrackLevel &lv, float *scratch, LfTrackState *st, const LfStepFlags &f, float icp_weight,
                   hipStream_t stream, int *grid);
@@ -98,3 +95,5 @@ int lf_track_job_make(const LfTrackLevel &lv, float *scratch, LfTrackState *st, 
                       float icp_weight, int share, int wgs, void *job, int *grid);
 void lf_track_job_skip(void *job);
 int lf_track_batch_step(const void *jobs, int n, int gmax, int half_maps, hipStream_t stream);
+// The end jobs of n systems (made with end set), whatever their numbers of steps.
+int lf_track_batch_end(const void *jobs, int n, hipStream_t stream);

@@ -57,10 +57,8 @@ struct ReduceArgs {
     // tracking step
     LfTrackState *st;
     int step;              // index within the frame; 0: the estimate starts at init
-    int end;               // no step of its own: only the previous one's solve (after the frame's last step)
     int first_iter;        // first iteration of a level
     int prev_first_iter;   // the previous step's first_iter,
-    int prev_ends;         // whether the frame ends at it once its level breaks out (1) or in any case (2),
     int prev_grid;         // and its workgroups (partial rows)
     int context_mode;      // compute_transform(ctx) semantics
     float icp_weight;
@@ -499,33 +497,85 @@ LF_DEV void gn_step(LfGnState &g, const double *sums, int first_iter, bool conte
     g.active = stop ? 0 : 1;
 }
 
-// Wavefront sum of N values per lane (N a power of two, <= 64) as a
+// A value (float or double) as its 32-bit words, lane l receiving lane l ^ o's.
+// Within a row of 16 lanes by DPP; a ds_bpermute (__shfl_xor) goes through the
+// LDS pipe, which the 64 shuffles of a block reduction's 8 wavefronts filled
+// for 2.3 us of each tracking step.
+template <int o>
+LF_DEV int xor_word(int x) {
+    static_assert(o == 1 || o == 2 || o == 4 || o == 8, "inside a row");
+    if constexpr (o == 8) return __builtin_amdgcn_mov_dpp(x, 0x128, 0xF, 0xF, false);       // row_ror:8
+    else if constexpr (o == 2) return __builtin_amdgcn_mov_dpp(x, 0x4E, 0xF, 0xF, false);   // quad_perm 2,3,0,1
+    else if constexpr (o == 1) return __builtin_amdgcn_mov_dpp(x, 0xB1, 0xF, 0xF, false);   // quad_perm 1,0,3,2
+    else return __builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(x, 0x141, 0xF, 0xF, false), 0x1B, 0xF, 0xF,
+                                         false);  // row_half_mirror (l ^ 7), then quad_perm 3,2,1,0 (l ^ 3)
+}
+template <int o>
+LF_DEV float xor_lane(float v) { return __int_as_float(xor_word<o>(__float_as_int(v))); }
+template <int o>
+LF_DEV double xor_lane(double v) {
+    return __hiloint2double(xor_word<o>(__double2hiint(v)), xor_word<o>(__double2loint(v)));
+}
+// a and b exchanged between lanes 32 (16) apart: the upper half (odd row) of a
+// with the lower half (even row) of b.
+template <int o>
+LF_DEV void swap_word(unsigned int &a, unsigned int &b) {
+    static_assert(o == 32 || o == 16, "halves or rows");
+    const auto r = o == 32 ? __builtin_amdgcn_permlane32_swap(a, b, false, false)
+                           : __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+template <int o>
+LF_DEV float swap_sum(float a, float b) {
+    unsigned int x = __float_as_uint(a), y = __float_as_uint(b);
+    swap_word<o>(x, y);
+    return __uint_as_float(x) + __uint_as_float(y);
+}
+template <int o>
+LF_DEV double swap_sum(double a, double b) {
+    unsigned int xl = (unsigned int)__double2loint(a), xh = (unsigned int)__double2hiint(a),
+                 yl = (unsigned int)__double2loint(b), yh = (unsigned int)__double2hiint(b);
+    swap_word<o>(xl, yl);
+    swap_word<o>(xh, yh);
+    return __hiloint2double((int)xh, (int)xl) + __hiloint2double((int)yh, (int)yl);
+}
+
+// Wavefront sum of N values per lane (N a power of two, 4 to 64) as a
 // transpose butterfly: at each exchange a lane keeps half of its values and
 // sends the other half to its partner, so N values cost N - 1 + 6 - log2(N)
-// shuffles instead of 6 N.  Afterwards lane l holds the wavefront total of
+// exchanges instead of 6 N.  Afterwards lane l holds the wavefront total of
 // value l >> (6 - log2 N).  Fixed pairing: deterministic.
 // (Compile-time recursion keeps every index constant, so v stays in VGPRs.)
+template <int kOff, class T>
+LF_DEV T sum_lanes(T v) {
+    if constexpr (kOff >= 1) return sum_lanes<kOff / 2>(v + xor_lane<kOff>(v));
+    else return v;
+}
 template <int N, int kOff, class T>
 LF_DEV void transpose_halve(T *v, int lane) {
     if constexpr (N > 1) {
         constexpr int h = N / 2;
-        const bool hi = (lane & kOff) != 0;
 #pragma unroll
         for (int i = 0; i < h; ++i) {
-            const T keep = hi ? v[h + i] : v[i];
-            const T send = hi ? v[i] : v[h + i];
-            v[i] = keep + __shfl_xor(send, kOff);
+            if constexpr (kOff >= 16) {  // lanes with bit kOff clear keep v[i], the others v[h + i]
+                v[i] = swap_sum<kOff>(v[i], v[h + i]);
+            } else {
+                const bool hi = (lane & kOff) != 0;
+                const T keep = hi ? v[h + i] : v[i];
+                const T send = hi ? v[i] : v[h + i];
+                v[i] = keep + xor_lane<kOff>(send);
+            }
         }
         transpose_halve<h, kOff / 2>(v, lane);
     } else {
-#pragma unroll
-        for (int o = kOff; o >= 1; o >>= 1) v[0] += __shfl_xor(v[0], o);
+        v[0] = sum_lanes<kOff>(v[0]);
     }
 }
 
 template <int N, class T>
 LF_DEV T transpose_reduce(T (&v)[N]) {
-    static_assert(N >= 1 && N <= 64 && (N & (N - 1)) == 0, "N must be a power of two <= 64");
+    static_assert(N >= 4 && N <= 64 && (N & (N - 1)) == 0, "N must be a power of two, 4 to 64");
     transpose_halve<N, 32>(v, __lane_id());
     return v[0];
 }
@@ -611,11 +661,10 @@ LF_DEV double block_sums_d(CombinedSums &sums, double (*s_wave)[32]) {
     return t;
 }
 
-// final_sums of the G combined FP64 partial rows (value v of workgroup g at
-// v * G + g), in a fixed order; the kTrackVals totals land in s_sum.  kChunks
-// 64-lane chunks of partials per value, enough for G (the chunks past G hold
-// only masked zeros, which leave the sums unchanged: a sum started at +0 is
-// never -0).
+// final_sums of the G <= 64 kChunks combined FP64 partial rows (value v of
+// workgroup g at v * G + g), in a fixed order; the kTrackVals totals land in
+// s_sum.  Lane chunks past G hold only masked zeros, which leave the sums
+// unchanged: a sum started at +0 is never -0.
 template <int kChunks>
 LF_DEV void final_sums_d_chunks(const double *partials, int G, double *s_sum) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -643,8 +692,7 @@ LF_DEV void final_sums_d_chunks(const double *partials, int G, double *s_sum) {
     const int v = wave + kWaves * (lane >> 4);
     if ((lane & 15) == 0 && v < kTrackVals) s_sum[v] = s;
 }
-// (a batch of 16 systems: 32 partials per value, one chunk; a lone system's
-// levels: at most 256)
+// (a batch of 16 systems: 32 partials per value; a lone system's levels: at most 256)
 LF_DEV void final_sums_d(const double *partials, int G, double *s_sum) {
     if (G <= 64) final_sums_d_chunks<1>(partials, G, s_sum);
     else if (G <= 256) final_sums_d_chunks<4>(partials, G, s_sum);
@@ -724,25 +772,22 @@ LF_DEV double *step_partials(const ReduceArgs &a, int k) {
 // The previous step's end, at the head of every workgroup of this one: its
 // partial rows summed in a fixed order, then the FP64 solve on one lane, whose
 // pose is this step's.  Every workgroup computes the same; workgroup 0 stores
-// the state (the two slots in turn, for the same reason as the rows) and,
-// where the frame ends, runs the finish.
-LF_DEV void solve_previous(const ReduceArgs &a, int wg, StepLds &s) {
+// the state (the two slots in turn, for the same reason as the rows).  Lane 0
+// returns the state.  The rows are loaded beside the state, before it says
+// whether they are wanted: after a kernel boundary each dependent round of
+// loads costs about 1 us.
+LF_DEV LfGnState solve_previous(const ReduceArgs &a, int wg, StepLds &s) {
     const int tid = threadIdx.x;
     LfTrackState &st = *a.st;
     LfGnState g = st.slot[(a.step - 1) & 1];
+    final_sums_d(step_partials(a, a.step - 1), a.prev_grid, s.sum);
+    __syncthreads();
     // a failed frame, or a level that broke out of its loop: no step was taken
     const bool ran = !g.invalid && (a.prev_first_iter || g.active);
-    if (ran) {
-        final_sums_d(step_partials(a, a.step - 1), a.prev_grid, s.sum);
-        __syncthreads();
-        if (wg == 0 && tid < kTrackVals) st.sums[tid] = s.sum[tid];
-    }
     if (tid == 0) {
-        if (ran) {
-            if (wg == 0)
-                for (int k = 0; k < 12; ++k) st.prev[k] = g.est[k];
-            gn_step(g, s.sum, a.prev_first_iter, a.context_mode != 0);
-        }
+        double before[12];
+        for (int k = 0; k < 12; ++k) before[k] = g.est[k];
+        if (ran) gn_step(g, s.sum, a.prev_first_iter, a.context_mode != 0);
 #pragma unroll
         for (int k = 0; k < 12; ++k) s.pose[k] = (float)g.est[k];
         s.stddev = g.stddev;
@@ -751,14 +796,13 @@ LF_DEV void solve_previous(const ReduceArgs &a, int wg, StepLds &s) {
             st.slot[a.step & 1] = g;
             if (ran) {
                 st.gn = g;
-                // the frame ends here when the estimate became invalid, when the
-                // finest level broke out of its loop, or after the frame's last step
-                if (g.invalid || (a.prev_ends && !g.active) || a.prev_ends == 2)
-                    track_finish(st, g.est, g.invalid, a.context_mode != 0);
+                for (int k = 0; k < 12; ++k) st.prev[k] = before[k];
             }
         }
     }
     __syncthreads();
+    if (ran && wg == 0 && tid < kTrackVals) st.sums[tid] = s.sum[tid];
+    return g;
 }
 
 // One Gauss-Newton iteration of compute_transform: the previous step's solve,
@@ -769,11 +813,16 @@ LF_DEV void solve_previous(const ReduceArgs &a, int wg, StepLds &s) {
 // workgroup, cost 3.6-4.3 us a step beside 5.3-6.6 us of rows; a
 // last-workgroup ticket costs 11 ns per workgroup, as atomics on one address
 // are taken in turn, and more than the launch from 128 workgroups on.)
+// A coarse level's step is latency: of its 14.8k cycles (7.0-7.5 us with the
+// launch, 20.5k with ds_bpermute butterflies) 3.7k load the state and the
+// rows, 3.4k solve, 3.7k are two rounds of pixel loads and 2.6k the block's
+// sums; a 640x480 step (11.3 us) has 13k cycles of pixels, by their
+// instructions.  Re-tracking at 320x240: 246 -> 192 us a call.
 // Workgroup wg of the nwg computing the step's partial rows.  kHalf: FP16 maps.
 template <bool kHalf>
 LF_DEV void track_step_wg(const ReduceArgs &a, int wg, int nwg, StepLds &s) {
     const int tid = threadIdx.x;
-    const int n = a.end ? 0 : a.lv.cols * a.lv.rows;
+    const int n = a.lv.cols * a.lv.rows;
     const int stride = nwg * kThreads;
     int i = wg * kThreads + tid;
     Own o = {};
@@ -790,7 +839,7 @@ LF_DEV void track_step_wg(const ReduceArgs &a, int wg, int nwg, StepLds &s) {
         }
     } else {
         solve_previous(a, wg, s);
-        if (a.end || !s.run) return;
+        if (!s.run) return;
 #pragma unroll
         for (int k = 0; k < 12; ++k) P[k] = uniform_f(s.pose[k]);
         stddev = a.first_iter ? 0.0f : uniform_f(s.stddev);
@@ -815,6 +864,19 @@ template <bool kHalf>
 __global__ __launch_bounds__(kThreads, 4) void k_track_step(ReduceArgs a) {
     __shared__ StepLds s;
     track_step_wg<kHalf>(a, blockIdx.x, gridDim.x, s);
+}
+
+// After the frame's last step (one workgroup): its solve, then the finish.  A
+// frame that ended before (an error became NaN, the finest level broke out of
+// its loop) left the estimate as it was then.
+LF_DEV void track_end_wg(const ReduceArgs &a, StepLds &s) {
+    const LfGnState g = solve_previous(a, 0, s);
+    if (threadIdx.x == 0) track_finish(*a.st, g.est, g.invalid, a.context_mode != 0);
+}
+
+__global__ __launch_bounds__(kThreads) void k_track_end(ReduceArgs a) {
+    __shared__ StepLds s;
+    track_end_wg(a, s);
 }
 
 // Launch arguments read from a descriptor table, their pointers asserted global.
@@ -846,6 +908,14 @@ __global__ __launch_bounds__(kThreads, 4) void k_track_step_batch(const TrackJob
     const TrackJob &j = jobs[blockIdx.y];
     if ((int)blockIdx.x >= j.G) return;
     track_step_wg<kHalf>(global_args(j.a), blockIdx.x, j.G, s);
+}
+
+// The end of each system's frame: workgroup i, system i.
+__global__ __launch_bounds__(kThreads) void k_track_end_batch(const TrackJob *__restrict__ jobs) {
+    __shared__ StepLds s;
+    const TrackJob &j = jobs[blockIdx.x];
+    if (j.G <= 0) return;
+    track_end_wg(global_args(j.a), s);
 }
 
 __global__ void k_track_finish(LfTrackState *st) {
@@ -921,10 +991,8 @@ static ReduceArgs step_args(const LfTrackLevel &lv, float *scratch, LfTrackState
     a.partials = scratch;
     a.st = st;
     a.step = f.step;
-    a.end = f.end;
     a.first_iter = f.first_of_level;
     a.prev_first_iter = f.prev_first_of_level;
-    a.prev_ends = f.prev_ends;
     a.prev_grid = f.prev_grid;
     a.icp_weight = icp_weight;
     a.context_mode = f.context_mode;
@@ -938,7 +1006,8 @@ static ReduceArgs step_args(const LfTrackLevel &lv, float *scratch, LfTrackState
 // Workgroups of a tracking step of one of `share` systems (wgs > 0: given):
 // a lone system takes 256, one per CU.  Each of them sums all of the
 // previous step's rows, and a level-0 lane then sums two pixels with the
-// second one's loads in flight.
+// second one's loads in flight.  (A whole 640x480 frame on 128 or 512: 1.05x
+// and 1.04x the time; one at 320x240 on 128: 1.05x.)
 static int step_grid(const LfTrackLevel &lv, int share, int wgs, int end) {
     if (end) return 1;
     return std::min(grid_for(lv), wgs > 0 ? std::min(wgs, kGrid) : std::max(1, std::min(kStepGrid, kGrid / std::max(1, share))));
@@ -949,7 +1018,8 @@ int lf_track_step(const LfTrackLevel &lv, float *scratch, LfTrackState *st, cons
     if (int rc = check_level(lv)) return rc;
     const ReduceArgs a = step_args(lv, scratch, st, f, icp_weight);
     const int G = step_grid(lv, 1, 0, f.end);
-    if (lv.half_maps) k_track_step<true><<<G, kThreads, 0, stream>>>(a);
+    if (f.end) k_track_end<<<1, kThreads, 0, stream>>>(a);
+    else if (lv.half_maps) k_track_step<true><<<G, kThreads, 0, stream>>>(a);
     else k_track_step<false><<<G, kThreads, 0, stream>>>(a);
     LF_LAUNCH_CHECK();
     if (grid) *grid = G;
@@ -986,6 +1056,13 @@ int lf_track_batch_step(const void *jobs, int n, int gmax, int half_maps, hipStr
     if (gmax <= 0) return LF_OK;
     if (half_maps) k_track_step_batch<true><<<dim3(gmax, n), kThreads, 0, stream>>>(J);
     else k_track_step_batch<false><<<dim3(gmax, n), kThreads, 0, stream>>>(J);
+    LF_LAUNCH_CHECK();
+    return LF_OK;
+}
+
+int lf_track_batch_end(const void *jobs, int n, hipStream_t stream) {
+    if (!jobs || n <= 0 || n > 65535) return lf_set_error(LF_ERR_ARG, "bad tracking batch of %d", n);
+    k_track_end_batch<<<n, kThreads, 0, stream>>>(static_cast<const TrackJob *>(jobs));
     LF_LAUNCH_CHECK();
     return LF_OK;
 }

@@ -405,7 +405,6 @@ int DenseTracking::enqueue(DeviceImage &ref, DeviceImage &cur, const TrackingCon
         LF_RC(lf_track_begin(state_, f.init, stream_));
         return lf_track_finish(state_, stream_);
     }
-    const int finest = plan.back().level;
     // a launch per step and one that ends the frame (the last step's level, of which it reads nothing)
     for (size_t s = 0; s <= plan.size(); ++s) {
         f.end = s == plan.size();
@@ -437,7 +436,6 @@ int DenseTracking::enqueue(DeviceImage &ref, DeviceImage &cur, const TrackingCon
             LF_RC(lf_track_step(lv, scratch_, state_, f, icp_weight, stream_, &G));
         }
         f.prev_first_of_level = f.first_of_level;
-        f.prev_ends = s + 1 == plan.size() ? 2 : level == finest ? 1 : 0;
         f.prev_grid = G;
     }
     return LF_OK;
@@ -1013,7 +1011,7 @@ int Batch::step(const uint16_t *const *depth_in, const unsigned char *const *rgb
         const bool tracks = od.initialized() && !od.trackingLost;
         LF_RC(sys_[i]->plan_tracking(depth[i], rgb[i], jobs[i], grids[i], &up[i]));
         LF_RC(sys_[i]->plan_after_raycast(after[i]));
-        steps = std::max(steps, grids[i].size());
+        if (!grids[i].empty()) steps = std::max(steps, grids[i].size() - 1);  // the last job ends the frame
         n_up = std::max(n_up, up[i].size() / PB);
         n_after = std::max(n_after, after[i].size() / PB);
         // planning launches on the system's stream only to start a frame
@@ -1026,10 +1024,10 @@ int Batch::step(const uint16_t *const *depth_in, const unsigned char *const *rgb
         }
     }
     // One table per step, copied in one transfer: [pass p][system] (uploads,
-    // then re-pyramids), [step s][system] tracking jobs, [system] updates,
+    // then re-pyramids), [step s][system] tracking jobs and [system] their ends, [system] updates,
     // [system] raycasts.
     const size_t n_pass = n_up + n_after;
-    const size_t off_track = n_pass * n * PB, off_fuse = off_track + steps * n * J, off_ray = off_fuse + n * FJ,
+    const size_t off_track = n_pass * n * PB, off_fuse = off_track + (steps + 1) * n * J, off_ray = off_fuse + n * FJ,
                  bytes = off_ray + n * RJ;
     // the buffers of two steps ago must have been copied before they are rewritten
     const int k = parity_;
@@ -1050,12 +1048,13 @@ int Batch::step(const uint16_t *const *depth_in, const unsigned char *const *rgb
                 lf_pass_skip(dst);
             }
         }
-    for (size_t s = 0; s < steps; ++s)
+    for (size_t s = 0; s <= steps; ++s)  // row s < steps: step s of every system, row steps: their ends
         for (int i = 0; i < n; ++i) {
             unsigned char *dst = host + off_track + (s * n + i) * J;
-            if (s < grids[i].size()) {
-                std::memcpy(dst, jobs[i].data() + s * J, J);
-                gmax[s] = std::max(gmax[s], grids[i][s]);
+            const size_t last = grids[i].size() - (grids[i].empty() ? 0 : 1);  // the system's steps
+            if (s < steps ? s < last : last > 0) {
+                std::memcpy(dst, jobs[i].data() + std::min(s, last) * J, J);
+                if (s < steps) gmax[s] = std::max(gmax[s], grids[i][s]);
             } else {
                 lf_track_job_skip(dst);
             }
@@ -1097,6 +1096,7 @@ int Batch::step(const uint16_t *const *depth_in, const unsigned char *const *rgb
     auto enqueue_track = [&]() -> int {
         for (size_t s = 0; s < steps; ++s)
             LF_RC(lf_track_batch_step(dev + off_track + s * n * J, n, gmax[s], half_maps_, stream_));
+        if (steps) LF_RC(lf_track_batch_end(dev + off_track + steps * n * J, n, stream_));
         return LF_OK;
     };
     auto enqueue_fuse = [&](hipEvent_t i0, hipEvent_t i1, hipEvent_t f0, hipEvent_t f1, hipEvent_t r0,

@@ -1,4 +1,6 @@
 """GPU: kernels at the sizes where their tiling can go wrong, against plain numpy / torch restatements."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -153,10 +155,93 @@ def test_mesh_of_random_blocks(precision, shape, origin, dense):
     # a capacity inside the output: the count goes on, nothing is written beyond it
     cap = max(1, len(ov) - 70)
     out = torch.full((len(ov) + 64, 9), 7.0, device="cuda")
-    import ctypes
     got = ctypes.c_uint(0)
     rc = capi.load().lf_create_mesh(ctypes.byref(m.params), ctypes.byref(m.storage), capi.ptr(out), None, None, cap,
                                     ctypes.byref(got), capi.stream_ptr())
     full = int(m.counters()[capi.CNT_TRIANGLES])
     assert got.value == min(cap, full) and rc == (capi.LF_ERR_CAPACITY if full > cap else capi.LF_OK)
     assert torch.all(out[got.value:] == 7.0) and not torch.any((out[: got.value] == 7.0).all(1))
+
+
+def frame_pair(K, width, height):
+    """Two neighbouring views of the orbit scene: (reference vmap, rgb), (source vmap, rgb) on the device."""
+    from libfusion_amd.synth import Scene
+    sc = Scene(1, 7)
+    out = []
+    for i in (0, 1):
+        d, c = sc.render(sc.pose(i), width, height, K.fx, K.fy, K.cx, K.cy, frame_id=i)
+        z = d.astype(np.float32) * np.float32(sc.depth_scale)
+        u, v = np.meshgrid(np.arange(width, dtype=np.float32), np.arange(height, dtype=np.float32))
+        m = np.stack([z * (u - K.cx) / K.fx, z * (v - K.cy) / K.fy, z, np.ones_like(z)], -1)
+        m[~((z > 0.3) & (z < 5))] = (np.nan, np.nan, np.nan, -1)
+        out.append((dev(m), dev(c)))
+    return out
+
+
+# one workgroup, 66 partial rows (more than a wavefront's lanes), 263 pixel blocks on the 256 workgroups of a lone
+# tracker; the last with a coarser level below it
+@pytest.mark.parametrize("width,height,levels", [(24, 16, 1), (192, 176, 1), (400, 336, 1), (400, 336, 2)])
+def test_gauss_newton_steps_chain(width, height, levels):
+    """A schedule run at once is its steps run one call at a time, each started where the one before ended: the
+    solve that a launch finds at its head is the previous step's.  One step a level: a level's later steps take
+    the residual deviation of the step before them, which a call starts without."""
+    f = 525.0 * width / 640
+    K = capi.intrinsics(width, height, f, f, (width - 1) / 2, (height - 1) / 2)
+    ref, src = frame_pair(K, width, height)
+    t = capi.Tracker(K, levels)
+    for name, (v, c) in (("reference", ref), ("source", src)):
+        t.set("set_%s_vmap" % name, v)
+        t.set("set_%s_image" % name, c)
+    _, _, whole = t.compute_transform((1,) * levels, np.eye(4))
+    sums, est = t.sums(), np.eye(4)
+    for level in range(levels - 1, -1, -1):
+        _, _, upd = t.compute_transform(tuple(int(k == level) for k in range(levels)), est)
+        est = np.linalg.inv(upd)
+    # FP64 but for the pose that the rows are taken at, which an inversion may round to its other float
+    assert np.allclose(np.linalg.inv(est), whole, rtol=0, atol=1e-6)
+    assert np.allclose(t.sums(), sums, rtol=1e-3, atol=1e-5 * np.abs(sums[:27]).max())
+    if levels > 1:
+        return
+    # against the stand-alone reduction on the same maps and pose, which adds the same float32 rows up in
+    # float32: every correspondence counted, and r^2 within the rounding of a sum of at most 2^18 terms
+    lib = capi.load()
+
+    def plane(source, which):
+        out = ctypes.c_void_p()
+        capi.check(lib.lf_tracker_plane(t.h, source, 0, which, ctypes.byref(out)))
+        return out
+    pose = dev(np.eye(4, dtype=np.float32)[:3])
+    scratch, out = torch.empty(lib.lf_reduce_scratch_floats(), device="cuda"), torch.empty(29, device="cuda")
+    capi.check(lib.lf_icp_reduce(plane(1, capi.PLANE_VMAP), plane(1, capi.PLANE_NMAP), plane(0, capi.PLANE_VMAP),
+                                 plane(0, capi.PLANE_NMAP), width, height, capi.ptr(pose), ctypes.byref(K),
+                                 capi.ptr(scratch), capi.ptr(out), capi.stream_ptr()))
+    out = out.cpu().numpy()
+    assert sums[28] == out[28] > 0
+    assert np.isclose(sums[27], out[27], rtol=1e-4)
+
+
+@pytest.mark.parametrize("precision", [FP32, MIXED])
+def test_batch_tracking_workgroups(precision):
+    """A system's poses do not depend on the workgroups (1, 65, 300 or 512 partial rows) beyond the FP64 order of
+    its sums."""
+    from libfusion_amd.synth import Scene
+    sc = Scene(1, 7)
+    w, h = 640, 480
+    K = capi.intrinsics(w, h, sc.fx, sc.fy, sc.cx, sc.cy)
+    frames = [tuple(dev(a.view(np.int16) if a.dtype == np.uint16 else a) for a in sc.frame(i)) for i in range(3)]
+    p = capi.map_params(1 << 18, 1 << 15, 0.01, 0.03, precision=precision)
+    torch.cuda.synchronize()
+    poses = []
+    for wgs in (0, 1, 65, 300, 512):
+        b = capi.Batch([capi.system_config(K, p, 3, (4, 3, 3), sc.depth_scale)])
+        b.set_option(capi.BATCH_OPT_TRACK_WORKGROUPS, wgs)
+        for d, c in frames:
+            b.process([d], [c])
+        b.synchronize()
+        poses.append(b.pose(0))
+        assert b.tracking(0)[0]
+        b.close()
+    # sums in another order differ by 1e-13 of their terms; a pose that enters the next step rounded to float32
+    # another way moves it by up to 1e-7 of its 1.5 m
+    for q in poses[1:]:
+        assert np.allclose(q, poses[0], rtol=0, atol=3e-7)
