@@ -25,7 +25,8 @@
 //    round trip (the reference downloads the sums and solves on the host twice
 //    per iteration).
 //  * The stand-alone reductions of the C-ABI (lf_icp_reduce, lf_rgb_step) are
-//    a partial-sum launch and a one-workgroup final-sum launch.
+//    one launch, whose last workgroup sums the rows.
+#include <atomic>
 #include <cfloat>
 #include <climits>
 #include <mutex>
@@ -45,7 +46,6 @@ constexpr int kGrid = 512;
 constexpr int kStepGrid = 256;  // of a lone system's tracking step (step_grid)
 constexpr int kThreads = 512;  // lanes per workgroup (8 wavefronts)
 constexpr int kWaves = kThreads / 64;
-constexpr int kVals = 58;      // 29 ICP + 29 RGB sums
 
 struct ReduceArgs {
     LfTrackLevel lv;
@@ -53,7 +53,6 @@ struct ReduceArgs {
     float stddev;          // stand-alone RGB reduction
     float angle, dthr;
     float *partials;       // kGrid * kVals floats
-    float *out29;          // modes 1/2
     // tracking step
     LfTrackState *st;
     int step;              // index within the frame; 0: the estimate starts at init
@@ -77,14 +76,15 @@ LF_DEV void accumulate(float *s, const float *row) {
     s[28] += 1.0f;
 }
 
-struct FloatSums {  // the 29 ICP and 29 RGB sums of the stand-alone reductions
-    float si[29], sr[29];
+constexpr int kVals = 29;
+struct FloatSums {  // a stand-alone reduction's sums
+    float s[32];    // kVals, padded to a power of two for the wavefront transpose
     LF_DEV void clear() {
 #pragma unroll
-        for (int k = 0; k < 29; ++k) { si[k] = 0.0f; sr[k] = 0.0f; }
+        for (int k = 0; k < 32; ++k) s[k] = 0.0f;
     }
-    LF_DEV void icp(const float *row) { accumulate(si, row); }
-    LF_DEV void rgb(const float *row) { accumulate(sr, row); }
+    LF_DEV void icp(const float *row) { accumulate(s, row); }
+    LF_DEV void rgb(const float *row) { accumulate(s, row); }
 };
 
 // The tracking step's sums: the normal equations A = w H_icp + H_rgb,
@@ -580,23 +580,13 @@ LF_DEV T transpose_reduce(T (&v)[N]) {
     return v[0];
 }
 
-// Partial sums of one workgroup (ICP rows into si, RGB rows into sr) into
-// value order: transpose butterfly in each wavefront, then the wavefronts meet
-// in LDS.  Lanes with tid < kVals return value tid (the others return 0).
-template <bool kIcp, bool kRgb>
-LF_DEV float block_sums(const FloatSums &sums, float (*s_wave)[kVals]) {
-    const float *si = sums.si, *sr = sums.sr;
+// Partial sums of one workgroup in value order: transpose butterfly in each
+// wavefront, leaving value l >> 1 in lane l, then the wavefronts meet in LDS.
+// Lanes with tid < kVals return value tid (the others return 0).
+LF_DEV float block_sums(FloatSums &sums, float (*s_wave)[32]) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    float v[64];
-#pragma unroll
-    for (int k = 0; k < 29; ++k) {
-        v[k] = kIcp ? si[k] : 0.0f;
-        v[29 + k] = kRgb ? sr[k] : 0.0f;
-    }
-#pragma unroll
-    for (int k = kVals; k < 64; ++k) v[k] = 0.0f;
-    const float w = transpose_reduce<64>(v);
-    if (lane < kVals) s_wave[wave][lane] = w;
+    const float w = transpose_reduce<32>(sums.s);
+    if ((lane & 1) == 0) s_wave[wave][lane >> 1] = w;
     __syncthreads();
     float t = 0.0f;
     if (tid < kVals) {
@@ -606,41 +596,60 @@ LF_DEV float block_sums(const FloatSums &sums, float (*s_wave)[kVals]) {
     return t;
 }
 
-// Final sum of the G partial rows in a fixed order (deterministic): wavefront w
-// reduces values w, w+kWaves, ...; lane l adds partials l, l+64, ... of a value
-// (independent loads, in flight together), then a transpose butterfly over the
-// wavefront's values.  The kVals totals land in s_sum; the caller
-// synchronises before reading them.
-LF_DEV void final_sums(const float *partials, int G, float *s_sum) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    constexpr int kPer = 8;
-    static_assert(kPer * kWaves >= kVals, "values per wavefront");
-    constexpr int kChunks = kGrid / 64;
-    float acc[kPer];
+// The sums of G <= 64 kChunks partial rows of kN <= 32 values (value v of
+// workgroup g at v * G + g) in a fixed order: wavefront w takes values w, w +
+// kWaves, ..., a lane adds partials l, l + 64, ... of each, then a transpose
+// butterfly over the wavefront's values.  The totals land in s_sum; the caller
+// synchronises before reading them.  Every load of a value comes first, then
+// the sum: indices past G are clamped and their values masked to +0 with a
+// bitwise AND (a select of a loaded value becomes a branch around the load with
+// a wait inside it), which leaves the sum unchanged: started at +0 it is never
+// -0.
+LF_DEV float mask_word(float v, bool keep) { return __uint_as_float(__float_as_uint(v) & (keep ? ~0u : 0u)); }
+LF_DEV double mask_word(double v, bool keep) {
+    return __longlong_as_double((long long)((unsigned long long)__double_as_longlong(v) & (keep ? ~0ull : 0ull)));
+}
+// Stores and loads that every XCD's workgroups see (relaxed, agent scope).
+template <class T>
+LF_DEV void store_agent(T *p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+template <class T>
+LF_DEV T load_agent(const T *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+// This wavefront's stores have arrived where those loads look (a wait alone:
+// what it orders went out past the caches).
+LF_DEV void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// kAgent: rows written by this launch.
+template <int kChunks, int kN, bool kAgent, class T>
+LF_DEV void final_sums_chunks(const T *partials, int G, T *s_sum) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int kPer = 4;
+    static_assert(kPer * kWaves >= kN, "values per wavefront");
+    T acc[kPer];
 #pragma unroll
     for (int j = 0; j < kPer; ++j) {
         const int v = wave + kWaves * j;
-        const float *src = partials + (size_t)(v < kVals ? v : 0) * G;
-        // every load of the value first, then the fixed-order sum.  Indices
-        // past G are clamped and their values masked to +0 with a bitwise AND
-        // (a select of a loaded value becomes a branch around the load with a
-        // wait inside it), so all the loads are in flight together.
-        float x[kChunks];
+        const T *src = partials + (size_t)(v < kN ? v : 0) * G;
+        T x[kChunks];
 #pragma unroll
         for (int c = 0; c < kChunks; ++c) {
             const int g = c * 64 + lane;
-            const float t = src[g < G ? g : G - 1];
-            const unsigned keep = (v < kVals && g < G) ? 0xffffffffu : 0u;
-            x[c] = __uint_as_float(__float_as_uint(t) & keep);
+            const T *q = src + (g < G ? g : G - 1);
+            x[c] = mask_word(kAgent ? load_agent(q) : *q, v < kN && g < G);
         }
-        float s = 0.0f;
+        T s = 0;
 #pragma unroll
         for (int c = 0; c < kChunks; ++c) s += x[c];
         acc[j] = s;
     }
-    const float s = transpose_reduce<kPer>(acc);
-    const int v = wave + kWaves * (lane >> 3);
-    if ((lane & 7) == 0 && v < kVals) s_sum[v] = s;
+    const T s = transpose_reduce<kPer>(acc);
+    const int v = wave + kWaves * (lane >> 4);
+    if ((lane & 15) == 0 && v < kN) s_sum[v] = s;
+}
+// (a batch of 16 systems: 32 rows; a lone system's levels: at most 256)
+template <int kN, bool kAgent = false, class T>
+LF_DEV void final_sums(const T *partials, int G, T *s_sum) {
+    if (G <= 64) final_sums_chunks<1, kN, kAgent>(partials, G, s_sum);
+    else if (G <= 256) final_sums_chunks<4, kN, kAgent>(partials, G, s_sum);
+    else final_sums_chunks<kGrid / 64, kN, kAgent>(partials, G, s_sum);
 }
 
 // The combined FP64 sums of one workgroup: transpose butterfly over the 32
@@ -661,52 +670,27 @@ LF_DEV double block_sums_d(CombinedSums &sums, double (*s_wave)[32]) {
     return t;
 }
 
-// final_sums of the G <= 64 kChunks combined FP64 partial rows (value v of
-// workgroup g at v * G + g), in a fixed order; the kTrackVals totals land in
-// s_sum.  Lane chunks past G hold only masked zeros, which leave the sums
-// unchanged: a sum started at +0 is never -0.
-template <int kChunks>
-LF_DEV void final_sums_d_chunks(const double *partials, int G, double *s_sum) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    constexpr int kPer = 4;
-    static_assert(kPer * kWaves >= kTrackVals, "values per wavefront");
-    double acc[kPer];
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-        const int v = wave + kWaves * j;
-        const double *src = partials + (size_t)(v < kTrackVals ? v : 0) * G;
-        double x[kChunks];
-#pragma unroll
-        for (int c = 0; c < kChunks; ++c) {
-            const int g = c * 64 + lane;
-            const double t = src[g < G ? g : G - 1];
-            const unsigned long long keep = (v < kTrackVals && g < G) ? ~0ull : 0ull;
-            x[c] = __longlong_as_double((long long)((unsigned long long)__double_as_longlong(t) & keep));
-        }
-        double s = 0.0;
-#pragma unroll
-        for (int c = 0; c < kChunks; ++c) s += x[c];
-        acc[j] = s;
-    }
-    const double s = transpose_reduce<kPer>(acc);
-    const int v = wave + kWaves * (lane >> 4);
-    if ((lane & 15) == 0 && v < kTrackVals) s_sum[v] = s;
-}
-// (a batch of 16 systems: 32 partials per value; a lone system's levels: at most 256)
-LF_DEV void final_sums_d(const double *partials, int G, double *s_sum) {
-    if (G <= 64) final_sums_d_chunks<1>(partials, G, s_sum);
-    else if (G <= 256) final_sums_d_chunks<4>(partials, G, s_sum);
-    else final_sums_d_chunks<kGrid / 64>(partials, G, s_sum);
-}
-
-// Stand-alone reductions (lf_icp_reduce, lf_rgb_step).  kMode 1: ICP rows,
-// 2: RGB rows.  Each workgroup writes its kVals partials value-major (value v
-// of workgroup g at v * G + g).
+// Stand-alone reductions (lf_icp_reduce, lf_rgb_step) in one launch.  kMode 1:
+// ICP rows, 2: RGB rows.  Each workgroup writes its kVals partials value-major
+// (value v of workgroup g at v * G + g), then its flag, and reads every flag: the
+// workgroup that finds them all set sums the rows.  Nothing waits for another
+// workgroup, and the scratch needs no clearing first: a flag is set when it
+// holds the call's own tag, and the summing workgroup clears them all (a
+// captured call has the same tag at every replay).  Rows and flags pass through
+// the memory that all XCDs see (relaxed agent-scope atomics): each workgroup
+// waits for its rows' stores before its flag's, and for its flag's before it
+// reads the others, so the one whose flag arrives last sees them all.  Another
+// may too: both store the same sums.
+// A call's time is its launches on the host (19.6 us for an ICP and a
+// photometric reduction of 160x120 in two launches each): 5.0 + 2.8 us of
+// kernels became 6.3, and the call 13.8 us.
 template <int kMode>
-__global__ __launch_bounds__(kThreads) void k_reduce(ReduceArgs a) {
-    __shared__ float s_wave[kWaves][kVals];
+__global__ __launch_bounds__(kThreads) void k_reduce(ReduceArgs a, float *__restrict__ out29, unsigned long long *flags,
+                                                     unsigned long long tag) {
+    __shared__ float s_wave[kWaves][32], s_sum[32];
+    __shared__ int s_all;
     constexpr bool kIcp = kMode == 1, kRgb = kMode == 2;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, G = gridDim.x;
     float P[12];
 #pragma unroll
     for (int k = 0; k < 12; ++k) P[k] = a.pose12[k];
@@ -715,19 +699,25 @@ __global__ __launch_bounds__(kThreads) void k_reduce(ReduceArgs a) {
     FloatSums sums;
     sums.clear();
     const int n = a.lv.cols * a.lv.rows;
-    for (int i = blockIdx.x * kThreads + tid; i < n; i += gridDim.x * kThreads)
+    for (int i = blockIdx.x * kThreads + tid; i < n; i += G * kThreads)
         pixel_rows<kIcp, kRgb, false>(a, load_own<kIcp, kRgb>(a.lv, i), P, stddev, th, sums);
-    const float t = block_sums<kIcp, kRgb>(sums, s_wave);
-    if (tid < kVals) a.partials[(size_t)tid * gridDim.x + blockIdx.x] = t;
-}
-
-template <int kMode>
-__global__ __launch_bounds__(kThreads) void k_reduce_final(ReduceArgs a, int G) {
-    __shared__ float s_sum[kVals];
-    final_sums(a.partials, G, s_sum);
+    const float t = block_sums(sums, s_wave);
+    if (tid < 64) {
+        if (tid < kVals) store_agent(&a.partials[(size_t)tid * G + blockIdx.x], t);
+        wait_stores();
+        if (tid == 0) store_agent(&flags[blockIdx.x], tag);
+        wait_stores();
+        bool all = true;
+        for (int g = tid; g < G; g += 64) all = all && load_agent(&flags[g]) == tag;
+        if (__ballot(all) == ~0ull && tid == 0) s_all = 1;
+        else if (tid == 0) s_all = 0;
+    }
     __syncthreads();
-    if (threadIdx.x == 0)
-        for (int k = 0; k < 29; ++k) a.out29[k] = s_sum[(kMode == 2 ? 29 : 0) + k];
+    if (!s_all) return;
+    final_sums<kVals, true>(a.partials, G, s_sum);
+    __syncthreads();
+    if (tid < kVals) out29[tid] = s_sum[tid];
+    for (int g = tid; g < G; g += kThreads) store_agent(&flags[g], 0ull);
 }
 
 // End of DenseTracking::compute_transform (icp_tracker.cpp:143-155) and the
@@ -780,7 +770,7 @@ LF_DEV LfGnState solve_previous(const ReduceArgs &a, int wg, StepLds &s) {
     const int tid = threadIdx.x;
     LfTrackState &st = *a.st;
     LfGnState g = st.slot[(a.step - 1) & 1];
-    final_sums_d(step_partials(a, a.step - 1), a.prev_grid, s.sum);
+    final_sums<kTrackVals>(step_partials(a, a.step - 1), a.prev_grid, s.sum);
     __syncthreads();
     // a failed frame, or a level that broke out of its loop: no step was taken
     const bool ran = !g.invalid && (a.prev_first_iter || g.active);
@@ -887,7 +877,7 @@ LF_DEV ReduceArgs global_args(const ReduceArgs &d) {
     L.last_vmap = global_ptr(d.lv.last_vmap); L.last_nmap = global_ptr(d.lv.last_nmap);
     L.curr_I = global_ptr(d.lv.curr_I); L.last_I = global_ptr(d.lv.last_I);
     L.dIdx = global_ptr(d.lv.dIdx); L.dIdy = global_ptr(d.lv.dIdy);
-    a.pose12 = global_ptr(d.pose12); a.partials = global_ptr(d.partials); a.out29 = global_ptr(d.out29);
+    a.pose12 = global_ptr(d.pose12); a.partials = global_ptr(d.partials);
     a.st = global_ptr(d.st);
     return a;
 }
@@ -967,10 +957,9 @@ int grid_for(const LfTrackLevel &lv) {
 
 }  // namespace
 
-// The stand-alone reductions' kGrid x kVals FP32 partials.
-size_t lf_reduce_partials(void) {
-    return std::max((size_t)kGrid * kVals, (size_t)kGrid * kTrackVals * 2) + 64;
-}
+// The stand-alone reductions' kGrid x kVals FP32 partials (a caller's scratch
+// holds more than that: its size is part of the interface).
+size_t lf_reduce_partials(void) { return (size_t)kGrid * 62 + 64; }
 // The tracking steps' two halves of kGrid x kTrackVals FP64 partials.
 size_t lf_track_scratch_floats(void) { return (size_t)kGrid * kTrackVals * 2 * 2; }
 
@@ -1079,8 +1068,26 @@ int lf_track_set_pose(LfTrackState *st, const double *T, hipStream_t stream) {
     return LF_OK;
 }
 
-// icp_reduce of lf_icp_reduce and lf_icp_reduce_noalloc: the partial rows go
-// to `partials` (capacity floats), then the final kernel sums them.
+// The launch of a stand-alone reduction: rows and flags share the scratch of
+// `capacity` floats.
+template <int kMode>
+static int launch_reduce(ReduceArgs &a, float *scratch, size_t capacity, float *sum29, hipStream_t st) {
+    static std::atomic<unsigned long long> calls{0};
+    const int G = grid_for(a.lv);
+    a.partials = scratch;
+    // the flags behind the most rows, on an 8-byte boundary
+    const uintptr_t end = reinterpret_cast<uintptr_t>(scratch + (size_t)kGrid * kVals);
+    auto *flags = reinterpret_cast<unsigned long long *>((end + 7) & ~(uintptr_t)7);
+    if (reinterpret_cast<uintptr_t>(flags + G) > reinterpret_cast<uintptr_t>(scratch + capacity))
+        return lf_set_error(LF_ERR_CAPACITY, "a reduction of %d workgroups does not fit %zu scratch floats", G, capacity);
+    // a tag no other call has and no float pair is likely to hold
+    const unsigned long long tag = 0x9E3779B97F4A7C15ull * (calls.fetch_add(1, std::memory_order_relaxed) + 1);
+    k_reduce<kMode><<<G, kThreads, 0, st>>>(a, sum29, flags, tag);
+    LF_LAUNCH_CHECK();
+    return LF_OK;
+}
+
+// icp_reduce of lf_icp_reduce and lf_icp_reduce_noalloc.
 static int icp_reduce_into(const float *curr_vmap, const float *curr_nmap, const float *last_vmap,
                            const float *last_nmap, int cols, int rows, const float *pose12, const lf_intrinsics *K,
                            float *partials, size_t capacity, float *sum29, hipStream_t st) {
@@ -1093,17 +1100,7 @@ static int icp_reduce_into(const float *curr_vmap, const float *curr_nmap, const
     a.pose12 = pose12;
     a.angle = icp_angle();
     a.dthr = 0.01f;
-    a.partials = partials;
-    a.out29 = sum29;
-    const int G = grid_for(a.lv);
-    if ((size_t)G * kVals > capacity)
-        return lf_set_error(LF_ERR_CAPACITY, "icp_reduce: %d workgroups need %zu scratch floats, %zu available", G,
-                            (size_t)G * kVals, capacity);
-    k_reduce<1><<<G, kThreads, 0, st>>>(a);
-    LF_LAUNCH_CHECK();
-    k_reduce_final<1><<<1, kThreads, 0, st>>>(a, G);
-    LF_LAUNCH_CHECK();
-    return LF_OK;
+    return launch_reduce<1>(a, partials, capacity, sum29, st);
 }
 
 extern "C" int lf_icp_reduce(const float *curr_vmap, const float *curr_nmap, const float *last_vmap,
@@ -1116,12 +1113,12 @@ extern "C" int lf_icp_reduce(const float *curr_vmap, const float *curr_nmap, con
 }
 
 // Scratch of lf_icp_reduce_noalloc: the partial rows of at most kGrid
-// workgroups (kGrid * kVals floats, 116 KiB), one copy per GPU, held until the
+// workgroups (116 KiB, half of it used), one copy per GPU, held until the
 // process ends.  Host code never passes the array's name to a kernel or a
 // copy: on the host it is only a stand-in for the symbol, so its device
 // address is looked up per device (hipGetSymbolAddress, with that device
 // current) and that address is used everywhere.
-constexpr size_t kNoallocScratchFloats = (size_t)kGrid * kVals;
+constexpr size_t kNoallocScratchFloats = (size_t)kGrid * 58;
 static __device__ __align__(256) float scratch[kNoallocScratchFloats];
 
 namespace {
@@ -1156,8 +1153,8 @@ extern "C" int lf_icp_reduce_noalloc(const float *curr_vmap, const float *curr_n
         return lf_set_error(LF_ERR_ARG, "null argument to icp_reduce_noalloc");
     float *partials = nullptr;
     if (int rc = noalloc_scratch(&partials)) return rc;
-    // every partial the final kernel reads is written by this call's first
-    // kernel, so nothing in the scratch needs clearing
+    // every partial that is summed is written by the call itself, and a flag
+    // left from elsewhere is not its tag, so nothing in the scratch needs clearing
     return icp_reduce_into(curr_vmap, curr_nmap, last_vmap, last_nmap, cols, rows, pose12, K, partials,
                            kNoallocScratchFloats, sum29, lf_stream(stream));
 }
@@ -1176,14 +1173,7 @@ extern "C" int lf_rgb_step(const float *curr_intensity, const float *last_intens
     if (int rc = check_level(a.lv)) return rc;
     a.pose12 = pose12;
     a.stddev = stddev_estimate;
-    a.partials = scratch;
-    a.out29 = sum29;
-    const int G = grid_for(a.lv);
-    k_reduce<2><<<G, kThreads, 0, lf_stream(stream)>>>(a);
-    LF_LAUNCH_CHECK();
-    k_reduce_final<2><<<1, kThreads, 0, lf_stream(stream)>>>(a, G);
-    LF_LAUNCH_CHECK();
-    return LF_OK;
+    return launch_reduce<2>(a, scratch, lf_reduce_partials(), sum29, lf_stream(stream));
 }
 
 extern "C" void lf_unpack_jtjjtr(const float *sum29, float *jtj36, float *jtr6, float *residual2) {

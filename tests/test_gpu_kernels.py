@@ -245,3 +245,65 @@ def test_batch_tracking_workgroups(precision):
     # another way moves it by up to 1e-7 of its 1.5 m
     for q in poses[1:]:
         assert np.allclose(q, poses[0], rtol=0, atol=3e-7)
+
+
+# one workgroup, a partly filled one, 67 and 258 workgroups (past 64 and 256 rows), the capped grid on a ragged image
+@pytest.mark.parametrize("width,height", [(16, 16), (19, 27), (184, 184), (363, 363), (641, 479)])
+def test_reductions_in_one_launch(width, height):
+    """The stand-alone reductions on scratch that holds anything, called again and again and replayed from a graph."""
+    from oracle import oracle as O
+    f = 525.0 * width / 640
+    K = capi.intrinsics(width, height, f, f, (width - 1) / 2, (height - 1) / 2)
+    oK = O.make_intr(K.width, K.height, K.fx, K.fy, K.cx, K.cy)
+    maps = []
+    for v, c in frame_pair(K, width, height):
+        v = v.cpu().numpy()
+        I = O.grey(c.cpu().numpy())
+        maps.append((v, O.nmap(v), I) + tuple(O.derivative(I)))
+    (lv, ln, lI, _, _), (cv, cn, cI, cdx, cdy) = maps
+    t = [dev(a) for a in (cv, cn, lv, ln, cI, lI, cdx, cdy)]
+    P, lib = capi.ptr, capi.load()
+    n = lib.lf_reduce_scratch_floats()
+    scratch = torch.randint(-2 ** 31, 2 ** 31 - 1, (n,), dtype=torch.int32, device="cuda").view(torch.float32)
+    pose, icp, rgb = torch.empty(12, device="cuda"), torch.empty(29, device="cuda"), torch.empty(29, device="cuda")
+
+    def call():
+        st = capi.stream_ptr()
+        capi.check(lib.lf_icp_reduce(P(t[0]), P(t[1]), P(t[2]), P(t[3]), width, height, P(pose), ctypes.byref(K),
+                                     P(scratch), P(icp), st))
+        capi.check(lib.lf_rgb_step(P(t[4]), P(t[5]), P(t[2]), P(t[6]), P(t[7]), width, height, 5.0, P(pose),
+                                   ctypes.byref(K), P(scratch), P(rgb), st))
+
+    def check(p12):
+        # gates decided as by the float oracle; float32 sums of at most 2^19 terms against its FP64 ones
+        for got, o in ((icp, lambda dt: O.icp_reduce(cv, cn, lv, ln, p12, oK, dt)),
+                       (rgb, lambda dt: O.rgb_step(cI, lI, lv, cdx, cdy, np.float32(5.0), p12, oK, dt))):
+            g, o32, o64 = got.cpu().numpy().astype(np.float64), o(np.float32).astype(np.float64), o(np.float64)
+            assert g[28] == o32[28]
+            assert np.allclose(g, o32, rtol=1e-4, atol=1e-5 * np.abs(o32).max())
+            if o32[28] > 1000 and o32[28] == o64[28]:
+                assert np.allclose(g, o64, rtol=1e-3, atol=1e-4 * np.abs(o64).max())
+
+    poses = [np.eye(4)[:3].astype(np.float32).ravel() for _ in range(3)]
+    for k, p in enumerate(poses):
+        p[3] = 0.004 * k
+    side = torch.cuda.Stream()
+    for p in poses:
+        pose.copy_(dev(p))
+        call()
+        check(p)
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call()
+    torch.cuda.current_stream().wait_stream(side)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        call()
+    for p in poses:
+        pose.copy_(dev(p))
+        icp.fill_(-1)
+        rgb.fill_(-1)
+        g.replay()
+        check(p)
+        call()
+        check(p)
