@@ -774,6 +774,7 @@ static_assert(2 * kMaxRefuse < 64, "a wavefront tests every pose of a block; bit
 struct RefuseArgs {
     MapDev m;
     unsigned long long *slot_mask;  // per hash slot: bit k old pose k, bit n + k new pose k
+    unsigned long long *list_mask;  // per visible-list entry: the poses whose steps it takes, the same bits
     const float *depth[kMaxRefuse];
     const float4 *samples[kMaxRefuse];
     const float *old24[kMaxRefuse];
@@ -809,31 +810,49 @@ LF_DEV const float *refuse_pose(const RefuseArgs &a, int j) {
 }
 
 // The visible list becomes every allocated block that a keyframe's old or new
-// pose sees or whose slot the band walks marked (the slot flags, left set
-// for k_refuse to clear).
+// pose sees or whose slot the band walks marked (the slot flags are cleared),
+// each with the mask of the poses whose steps it takes.  One lane tests a
+// block against every pose, once: tested by each of a block's wavefronts in
+// k_refuse, the 2n poses' 8 corners were a quarter of that kernel's
+// instructions.
 template <bool kFast>
 __global__ __launch_bounds__(kVisThreads) void k_refuse_visible(RefuseArgs a) {
     __shared__ unsigned int s_cnt[kVisThreads / kWave];
     __shared__ unsigned int s_base;
+    __shared__ float s_pose[2 * kMaxRefuse][12];
     const MapDev &m = a.m;
+    for (int i = threadIdx.x; i < 2 * a.n * 12; i += kVisThreads)
+        s_pose[i / 12][i % 12] = refuse_pose(a, i / 12)[i % 12];
+    __syncthreads();
     const unsigned int nb = min(m.counters[LF_CNT_ALLOCATED], (unsigned int)m.num_blocks);
     const float scale = 8.0f * m.voxel_size;
     const unsigned int stride = gridDim.x * blockDim.x;
     const int lane = lane_id(), wave = threadIdx.x / kWave;
+    const unsigned long long all = (1ull << a.n) - 1ull;
     for (unsigned int b0 = blockIdx.x * blockDim.x; b0 < nb; b0 += stride) {
         const unsigned int b = b0 + threadIdx.x;
         bool vis = false;
         int4 p = make_int4(0, 0, 0, 0);
+        unsigned long long steps = 0ull;
         if (b < nb) {
             p = reinterpret_cast<const int4 *>(m.block_pos)[b];
-            vis = m.slot_flag[p.w] != 0 || a.slot_mask[p.w] != 0ull;
-            for (int j = 0; j < 2 * a.n && !vis; ++j) {
-                float Tcw[12];
-#pragma unroll
-                for (int i = 0; i < 12; ++i) Tcw[i] = refuse_pose(a, j)[i];
-                vis = block_visible<kFast>(p.x, p.y, p.z, Tcw, a.K, a.cols, a.rows, m.zmin_update, m.zmax_update,
-                                           scale);
+            const unsigned long long marks = a.slot_mask[p.w];
+            const bool flagged = m.slot_flag[p.w] != 0;
+            if (flagged) m.slot_flag[p.w] = 0;
+            unsigned long long seen = marks & ~kRefuseFresh;
+            for (int j = 0; j < 2 * a.n; ++j)
+                if (block_visible<kFast>(p.x, p.y, p.z, s_pose[j], a.K, a.cols, a.rows, m.zmin_update, m.zmax_update,
+                                         scale))
+                    seen |= 1ull << j;
+            vis = flagged || marks != 0ull || seen != 0ull;
+            unsigned long long old_mask = seen & all, new_mask = (seen >> a.n) & all;
+            if (marks & kRefuseFresh) {
+                // created here: by the first keyframe whose new-pose walk reached it
+                const unsigned long long walks = (marks >> a.n) & all;
+                old_mask = 0ull;
+                new_mask &= ~((walks & (0ull - walks)) - 1ull);
             }
+            steps = old_mask | new_mask << a.n;
         }
         const unsigned long long ballot = __ballot(vis);
         if (lane == 0) s_cnt[wave] = (unsigned int)__popcll(ballot);
@@ -852,155 +871,215 @@ __global__ __launch_bounds__(kVisThreads) void k_refuse_visible(RefuseArgs a) {
             const unsigned int slot = s_base + s_cnt[wave] + __popcll(ballot & ((1ull << lane) - 1ull));
             m.visible[slot] = (int)b;
             reinterpret_cast<int4 *>(m.visible_pos)[slot] = make_int4(p.x, p.y, p.z, (int)b);
+            a.list_mask[slot] = steps;
         }
         __syncthreads();
     }
 }
 
-// Keyframe k's observation of a voxel at world point (wx, wy, wz) under the
-// float 3x4 T_cw: the weighted update's selection (pixel in the image, depth
-// within the update range, sdf >= -truncation), its clamped sdf in truncation
-// units, its weight and colour.  kFast: the hardware reciprocal projection of
-// the mixed-precision update.
+// A keyframe's observation of a voxel before its sample has arrived: whether
+// it projects into the image, its depth in the camera, its pixel.
+struct RefuseProj {
+    float z;
+    unsigned int pix;
+    bool in;
+};
+// kFast: the hardware reciprocal projection of the mixed-precision update.
 template <bool kFast>
-LF_DEV bool refuse_observe(const RefuseArgs &a, int k, const float *Tcw, float wx, float wy, float wz, float &sdf,
-                           float &wt, unsigned int &rgb) {
-    const MapDev &m = a.m;
+LF_DEV RefuseProj refuse_project(const RefuseArgs &a, const float *Tcw, float wx, float wy, float wz) {
     const f3 pt = xform(Tcw, f3{wx, wy, wz});
-    int u, v;
+    float tu, tv;
     if (kFast) {
         const float iz = __builtin_amdgcn_rcpf(pt.z);
-        u = proj_floor(a.K.fx * pt.x * iz + a.K.cx + 0.5f);
-        v = proj_floor(a.K.fy * pt.y * iz + a.K.cy + 0.5f);
-    } else {
-        u = proj_floor(a.K.fx * pt.x / pt.z + a.K.cx + 0.5f);
-        v = proj_floor(a.K.fy * pt.y / pt.z + a.K.cy + 0.5f);
+        tu = a.K.fx * pt.x * iz + a.K.cx + 0.5f;
+        tv = a.K.fy * pt.y * iz + a.K.cy + 0.5f;
+    } else {  // a zero z projects nowhere either way
+        const Recip iz = recip(pt.z);
+        tu = quotient(a.K.fx * pt.x, iz) + a.K.cx + 0.5f;
+        tv = quotient(a.K.fy * pt.y, iz) + a.K.cy + 0.5f;
     }
-    if (u < 0 || v < 0 || u > a.cols - 1 || v > a.rows - 1) return false;
-    const float4 smp = a.samples[k][(size_t)v * a.cols + u];
-    const float d = smp.x;
-    if (isnan(d) || d > m.zmax_update || d < m.zmin_update) return false;
-    const float s = d - pt.z;
-    if (s < -m.truncation) return false;
-    sdf = fminf(1.0f, s * m.inv_truncation);
-    wt = smp.y;
-    rgb = __float_as_uint(smp.z);
-    return true;
+    // the pixel (floor(tu), floor(tv)), in the image exactly when 0 <= tu < cols
+    // and 0 <= tv < rows (NaN fails), where the floor is the truncating conversion
+    const bool in = tu >= 0.0f && tu < (float)a.cols && tv >= 0.0f && tv < (float)a.rows;
+    return {pt.z, in ? (unsigned int)(int)tv * (unsigned int)a.cols + (unsigned int)(int)tu : 0u, in};
+}
+
+// A voxel's running mean (sdf, colour) and weight.
+struct RefuseVoxel {
+    float w, sdf, col[3];
+    bool changed;
+};
+
+// The means' numerators over the new weight, each rounded as by a division; a
+// weight outside the range that recip() holds for takes divisions.
+template <int kN>
+LF_DEV void over_weight(float *n, float w) {
+    if (__builtin_expect(w >= 0x1p-60f && w <= 0x1p60f, 1)) {
+        const Recip d = recip(w);
+#pragma unroll
+        for (int k = 0; k < kN; ++k) n[k] = quotient(n[k], d);
+    } else {
+#pragma unroll 1
+        for (int k = 0; k < kN; ++k) n[k] /= w;
+    }
+}
+
+// k_deintegrate's step.
+template <bool kColour, bool kMixed>
+LF_DEV void refuse_take_out(RefuseVoxel &v, float s, float wt, unsigned int rgb) {
+    v.changed = true;
+    const float wr = v.w - wt;
+    const bool keep = kMixed ? wr > v.w * (1.0f / 16.0f) : wr > 0.0f;
+    if (!keep) {
+        v.w = 0.0f;
+        v.sdf = 0.0f;
+        if (kColour) v.col[0] = v.col[1] = v.col[2] = 0.0f;
+        return;
+    }
+    float n[4] = {v.sdf * v.w - s * wt, 0.0f, 0.0f, 0.0f};
+    if (kColour) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) n[1 + q] = v.col[q] * v.w - (float)((rgb >> (8 * q)) & 0xFFu) * wt;
+    }
+    over_weight<kColour ? 4 : 1>(n, wr);
+    v.sdf = fmaxf(-1.0f, fminf(1.0f, n[0]));
+    if (kColour) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) v.col[q] = fmaxf(0.0f, fminf(255.0f, n[1 + q]));
+    }
+    v.w = wr;
+}
+
+// The weighted update's step.
+template <bool kColour>
+LF_DEV void refuse_put_in(RefuseVoxel &v, float s, float wt, unsigned int rgb) {
+    v.changed = true;
+    if (v.w == 0.0f) {
+        v.sdf = s;
+        v.w = fminf(wt, 255.0f);
+        if (kColour) {
+#pragma unroll
+            for (int q = 0; q < 3; ++q) v.col[q] = (float)((rgb >> (8 * q)) & 0xFFu);
+        }
+        return;
+    }
+    const float wn = v.w + wt;
+    float n[4] = {v.sdf * v.w + s * wt, 0.0f, 0.0f, 0.0f};
+    if (kColour) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) n[1 + q] = v.col[q] * v.w + (float)((rgb >> (8 * q)) & 0xFFu) * wt;
+    }
+    over_weight<kColour ? 4 : 1>(n, wn);
+    v.sdf = n[0];
+    if (kColour) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) v.col[q] = n[1 + q];
+    }
+    v.w = fminf(wn, 255.0f);
 }
 
 // One lane per voxel (two voxels per lane, 256 lanes per block) of the visible
-// list.  kMixed: FP16 sdf and the packed weight-code / colour word, the
-// weights rounded stochastically once at the end (as the update stores them).
+// list: the steps of its mask in order, de-integrations (bits below n) first.
+// kMixed: FP16 sdf and the packed weight-code / colour word, the weights
+// rounded stochastically once at the end (as the update stores them).
+// Each step gathers 16 bytes per voxel: both voxels' samples of the next step
+// are loaded while the present one is applied, and the poses are in LDS.
+// 20 keyframes of 640x480 on 165k blocks (FP32, 4 mm): 1797 -> REFUSE_NOW us.
 template <bool kColour, bool kMixed>
 __global__ __launch_bounds__(256) void k_refuse(RefuseArgs a) {
+    __shared__ float s_pose[2 * kMaxRefuse][12];
     const MapDev &m = a.m;
+    const int t = threadIdx.x;
+    for (int i = t; i < 2 * a.n * 12; i += 256) s_pose[i / 12][i % 12] = refuse_pose(a, i / 12)[i % 12];
+    __syncthreads();
     const int nvis = (int)m.counters[LF_CNT_VISIBLE];
     const unsigned int pass = kMixed ? m.counters[LF_CNT_FUSE_PASSES] : 0u;
-    const float vs = m.voxel_size, scale = 8.0f * vs;
-    const int t = threadIdx.x, lane = lane_id();
+    const float vs = m.voxel_size, zmin = m.zmin_update, zmax = m.zmax_update;
     const int lx = t & 7, ly = (t >> 3) & 7, lz0 = t >> 6;
+    unsigned short *sdf16 = reinterpret_cast<unsigned short *>(m.sdf);
+    unsigned int *wd = reinterpret_cast<unsigned int *>(m.weight);
     for (int i = blockIdx.x; i < nvis; i += gridDim.x) {
         const int4 p = reinterpret_cast<const int4 *>(m.visible_pos)[i];
-        const int b = p.w;
-        // which poses see the block: lane j < 2n of each wavefront tests pose j
-        bool sees = false;
-        if (lane < 2 * a.n) {
-            float Tcw[12];
+        const unsigned long long mask = a.list_mask[i];
+        // the mask in scalar registers: the steps are the same for every lane
+        const unsigned int lo = (unsigned int)__builtin_amdgcn_readfirstlane((int)mask),
+                           hi = (unsigned int)__builtin_amdgcn_readfirstlane((int)(mask >> 32));
+        unsigned long long steps = lo | (unsigned long long)hi << 32;
+        if (!steps) continue;
+        const size_t b = (size_t)p.w;
+        const float wx = (float)(p.x * 8 + lx) * vs, wy = (float)(p.y * 8 + ly) * vs;
+        const float wz[2] = {(float)(p.z * 8 + lz0) * vs, (float)(p.z * 8 + lz0 + 4) * vs};
+        RefuseVoxel v[2];
+        unsigned int word[2] = {0u, 0u};
 #pragma unroll
-            for (int c = 0; c < 12; ++c) Tcw[c] = refuse_pose(a, lane)[c];
-            sees = block_visible<kMixed>(p.x, p.y, p.z, Tcw, a.K, a.cols, a.rows, m.zmin_update, m.zmax_update,
-                                         scale);
+        for (int h = 0; h < 2; ++h) {
+            const size_t vi = b * LF_BLOCK3 + (size_t)(t + 256 * h);
+            v[h].changed = false;
+            v[h].col[0] = v[h].col[1] = v[h].col[2] = 0.0f;
+            if constexpr (kMixed) {
+                word[h] = wd[vi];
+                v[h].w = weight_value(word_code(word[h]));
+                v[h].sdf = v[h].w > 0.0f ? half_bits_to_float(sdf16[vi]) : 0.0f;
+#pragma unroll
+                for (int k = 0; k < 3; ++k) v[h].col[k] = (float)word_channel(word[h], k);
+            } else {
+                v[h].w = m.weight[vi];
+                v[h].sdf = v[h].w > 0.0f ? unpack_sdf(m.sdf[vi]) : 0.0f;
+                if (kColour) {
+                    const unsigned char *c = m.rgb + b * (3 * LF_BLOCK3) + (size_t)(t + 256 * h);
+                    v[h].col[0] = c[0]; v[h].col[1] = c[LF_BLOCK3]; v[h].col[2] = c[2 * LF_BLOCK3];
+                }
+            }
         }
-        const int slot = reinterpret_cast<const int4 *>(m.block_pos)[b].w;
-        const bool flagged = m.slot_flag[slot] != 0;
-        const unsigned long long marks = a.slot_mask[slot], all = (1ull << a.n) - 1ull;
-        const unsigned long long seen = __ballot(sees) | (marks & ~kRefuseFresh);
-        unsigned long long old_mask = seen & all, new_mask = (seen >> a.n) & all;
-        if (marks & kRefuseFresh) {
-            // created here: by the first keyframe whose new-pose walk reached it
-            const unsigned long long walks = (marks >> a.n) & all;
-            old_mask = 0ull;
-            new_mask &= ~((walks & (0ull - walks)) - 1ull);
+        RefuseProj pr[2];
+        float4 smp[2];
+        // step j's projections and sample loads
+        auto look = [&](int j) {
+            float T[12];
+#pragma unroll
+            for (int c = 0; c < 12; ++c) T[c] = s_pose[j][c];
+            const float4 *samples = a.samples[j < a.n ? j : j - a.n];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                pr[h] = refuse_project<kMixed>(a, T, wx, wy, wz[h]);
+                smp[h] = samples[pr[h].pix];
+            }
+        };
+        int j = __builtin_ctzll(steps);
+        look(j);
+        while (true) {
+            const RefuseProj pc[2] = {pr[0], pr[1]};
+            const float4 sc[2] = {smp[0], smp[1]};
+            const bool put_in = j >= a.n;
+            steps &= steps - 1ull;
+            const bool more = steps != 0ull;
+            if (more) {
+                j = __builtin_ctzll(steps);
+                look(j);
+            }
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                // the update's selection: in the image, depth within the range, sdf >= -truncation
+                const float d = sc[h].x, s = d - pc[h].z;
+                if (!pc[h].in || isnan(d) || d > zmax || d < zmin || s < -m.truncation) continue;
+                const float sn = fminf(1.0f, s * m.inv_truncation);
+                const unsigned int rgb = __float_as_uint(sc[h].z);
+                if (put_in) refuse_put_in<kColour>(v[h], sn, sc[h].y, rgb);
+                else if (v[h].w != 0.0f) refuse_take_out<kColour, kMixed>(v[h], sn, sc[h].y, rgb);
+            }
+            if (!more) break;
         }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const int lz = lz0 + 4 * h;
-            const float wx = (float)(p.x * 8 + lx) * vs, wy = (float)(p.y * 8 + ly) * vs, wz = (float)(p.z * 8 + lz) * vs;
+            if (!v[h].changed) continue;
             const unsigned int o = (unsigned int)(t + 256 * h);
-            const size_t vi = (size_t)b * LF_BLOCK3 + o;
-            unsigned short *sdf16 = reinterpret_cast<unsigned short *>(m.sdf);
-            unsigned int *wd = reinterpret_cast<unsigned int *>(m.weight);
-            unsigned char *c = m.rgb + (size_t)b * (3 * LF_BLOCK3) + o;
-            // the voxel's running mean (sdf, colour) and weight
-            float w, sdf, col[3] = {0.0f, 0.0f, 0.0f};
-            unsigned int word = 0u;
+            const size_t vi = b * LF_BLOCK3 + o;
+            const float w = v[h].w, sdf = v[h].sdf;
             if constexpr (kMixed) {
-                word = wd[vi];
-                w = weight_value(word_code(word));
-                sdf = w > 0.0f ? half_bits_to_float(sdf16[vi]) : 0.0f;
-#pragma unroll
-                for (int k = 0; k < 3; ++k) col[k] = (float)word_channel(word, k);
-            } else {
-                w = m.weight[vi];
-                sdf = w > 0.0f ? unpack_sdf(m.sdf[vi]) : 0.0f;
-                if (kColour) {
-                    col[0] = c[0]; col[1] = c[LF_BLOCK3]; col[2] = c[2 * LF_BLOCK3];
-                }
-            }
-            bool changed = false;
-            // de-integration at the old poses (k_deintegrate's steps)
-            for (unsigned long long mk = old_mask; mk; mk &= mk - 1ull) {
-                const int k = __builtin_ctzll(mk);
-                float s, wt;
-                unsigned int rgb;
-                if (w == 0.0f || !refuse_observe<kMixed>(a, k, a.old24[k] + 12, wx, wy, wz, s, wt, rgb)) continue;
-                changed = true;
-                const float wr = w - wt;
-                const bool keep = kMixed ? wr > w * (1.0f / 16.0f) : wr > 0.0f;
-                if (!keep) {
-                    w = 0.0f;
-                    sdf = 0.0f;
-                    if (kColour) col[0] = col[1] = col[2] = 0.0f;
-                    continue;
-                }
-                sdf = fmaxf(-1.0f, fminf(1.0f, (sdf * w - s * wt) / wr));
-                if (kColour) {
-#pragma unroll
-                    for (int q = 0; q < 3; ++q)
-                        col[q] = fmaxf(0.0f, fminf(255.0f, (col[q] * w - (float)((rgb >> (8 * q)) & 0xFFu) * wt) / wr));
-                }
-                w = wr;
-            }
-            // the weighted update at the new poses
-            for (unsigned long long mk = new_mask; mk; mk &= mk - 1ull) {
-                const int k = __builtin_ctzll(mk);
-                float s, wt;
-                unsigned int rgb;
-                if (!refuse_observe<kMixed>(a, k, a.new24[k] + 12, wx, wy, wz, s, wt, rgb)) continue;
-                changed = true;
-                if (w == 0.0f) {
-                    sdf = s;
-                    w = fminf(wt, 255.0f);
-                    if (kColour) {
-#pragma unroll
-                        for (int q = 0; q < 3; ++q) col[q] = (float)((rgb >> (8 * q)) & 0xFFu);
-                    }
-                    continue;
-                }
-                const float wn = w + wt;
-                sdf = (sdf * w + s * wt) / wn;
-                if (kColour) {
-#pragma unroll
-                    for (int q = 0; q < 3; ++q) col[q] = (col[q] * w + (float)((rgb >> (8 * q)) & 0xFFu) * wt) / wn;
-                }
-                w = fminf(wn, 255.0f);
-            }
-            if (!changed) continue;
-            if constexpr (kMixed) {
-                unsigned int colour = word & ~0xFFu;
+                unsigned int colour = word[h] & ~0xFFu;
                 if (kColour)
-                    colour = word_colour_bits((unsigned int)(int)col[0], (unsigned int)(int)col[1],
-                                              (unsigned int)(int)col[2]);
+                    colour = word_colour_bits((unsigned int)(int)v[h].col[0], (unsigned int)(int)v[h].col[1],
+                                              (unsigned int)(int)v[h].col[2]);
                 // a voxel left with a positive weight stays seen (the smallest
                 // code stands for weights below it); none left: unseen
                 const unsigned int code =
@@ -1011,14 +1090,13 @@ __global__ __launch_bounds__(256) void k_refuse(RefuseArgs a) {
                 m.sdf[vi] = w > 0.0f ? pack_sdf(sdf) : kSdfUnseen;
                 m.weight[vi] = w;
                 if (kColour) {
-                    c[0] = (unsigned char)(int)col[0];
-                    c[LF_BLOCK3] = (unsigned char)(int)col[1];
-                    c[2 * LF_BLOCK3] = (unsigned char)(int)col[2];
+                    unsigned char *c = m.rgb + b * (3 * LF_BLOCK3) + o;
+                    c[0] = (unsigned char)(int)v[h].col[0];
+                    c[LF_BLOCK3] = (unsigned char)(int)v[h].col[1];
+                    c[2 * LF_BLOCK3] = (unsigned char)(int)v[h].col[2];
                 }
             }
         }
-        __syncthreads();  // every lane has read the slot flag
-        if (t == 0 && flagged) m.slot_flag[slot] = 0;
     }
 }
 
@@ -1225,11 +1303,12 @@ int lf_refuse_ev(const lf_map_params *p, const lf_map_storage *s, const float *c
     a.cols = cols;
     a.rows = rows;
     a.K = *K;
-    // the per-slot masks: stream-ordered device memory for the call's length
-    const size_t E = (size_t)p->num_entries;
+    // the masks per slot and per listed block: stream-ordered device memory for the call's length
+    const size_t E = (size_t)p->num_entries, B = (size_t)p->num_blocks;
     void *mask = nullptr;
-    LF_HIP_CHECK(hipMallocAsync(&mask, E * sizeof(unsigned long long), st));
+    LF_HIP_CHECK(hipMallocAsync(&mask, (E + B) * sizeof(unsigned long long), st));
     a.slot_mask = static_cast<unsigned long long *>(mask);
+    a.list_mask = a.slot_mask + E;
     k_fill_u64<<<(int)std::min<size_t>(4096, (E + 255) / 256), 256, 0, st>>>(a.slot_mask, E);
     const int rc = refuse_launch(p, a, colour, st);
     const hipError_t ef = hipFreeAsync(mask, st);
