@@ -78,6 +78,9 @@ LF_HD unsigned long long pack_key(int x, int y, int z) {
            (unsigned long long)(z & 0x1FFFFF);
 }
 
+// An axis of a packed key (its low 21 bits, two's complement).
+LF_HD int key_axis(unsigned long long k) { return (int)((unsigned int)k << 11) >> 11; }
+
 // sdf code of a voxel whose weight is 0 (never observed, or only with weight 0).
 // packFloat never produces it (|v| <= 1 maps into [-32767, 32767]), so the
 // raycast decides validity from the 2-byte sdf alone, without the weight.

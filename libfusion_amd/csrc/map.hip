@@ -136,9 +136,10 @@ LF_DEV void band_blocks(int x, int y, float z, const float *Twc, const lf_intrin
         const float iv = 1.0f / vs;
         vn = to_i3(mul(pn, iv));
         vf = to_i3(mul(pf, iv));
-    } else {
-        vn = to_i3(dvd(pn, vs));
-        vf = to_i3(dvd(pf, vs));
+    } else {  // the divisions' floats (an infinite coordinate is refused either way)
+        const Recip iv = recip(vs);
+        vn = to_i3(f3{quotient(pn.x, iv), quotient(pn.y, iv), quotient(pn.z, iv)});
+        vf = to_i3(f3{quotient(pf.x, iv), quotient(pf.y, iv), quotient(pf.z, iv)});
     }
     if (vn.x == kBad || vn.y == kBad || vn.z == kBad || vf.x == kBad || vf.y == kBad || vf.z == kBad) return;
     i3 a = {blk(vn.x), blk(vn.y), blk(vn.z)}, b = {blk(vf.x), blk(vf.y), blk(vf.z)};
@@ -188,11 +189,20 @@ LF_DEV unsigned int key_mix(unsigned long long k) {
 constexpr unsigned long long kRefuseFresh = 1ull << 63;
 
 LF_DEV int touch_block(const MapDev &m, int bx, int by, int bz) {
-    const int b = find_block(m.keys, m.slot_block, bx, by, bz, m.num_buckets, m.num_entries);
-    if (b < 0) return -1;
-    const int slot = reinterpret_cast<const int4 *>(m.block_pos)[b].w;
-    m.slot_flag[slot] = 1;
-    return slot;
+    const unsigned long long key = pack_key(bx, by, bz);
+    int slot = compute_hash(bx, by, bz, m.num_buckets);
+    for (int i = 0; i < m.num_entries; ++i) {  // find_block, for the slot
+        const unsigned long long k = m.keys[slot];
+        const int b = m.slot_block[slot];
+        if (k == key) {
+            if (b < 0) return -1;  // an entry whose block did not fit the pool
+            m.slot_flag[slot] = 1;
+            return slot;
+        }
+        if (k == kEmptyKey) return -1;
+        if (++slot == m.num_entries) slot = 0;
+    }
+    return -1;
 }
 
 // kInsert: create_blocks_kernel.  !kInsert (de-integration): the same band
@@ -201,17 +211,26 @@ LF_DEV int touch_block(const MapDev &m, int bx, int by, int bz) {
 // 16x16 pixel tile (tx, ty) of the frame.  slot_mask (keyframe re-fusion):
 // each block the walk marks also gets `bit` in its hash slot's mask, and
 // kRefuseFresh when the walk created it.
+// The walks only fill the LDS set and list its keys; then the listed blocks
+// go to the hash table side by side, one lane each.  A block's insertion is a
+// chain of global accesses, which inside the walks a lane waited for once per
+// block it was first to request.
+struct AllocLds {
+    unsigned long long set[kDedup];
+    unsigned short list[kDedup];  // positions in the set, in the order of insertion
+    unsigned int n;
+};
 template <bool kInsert, bool kFast = false>
 LF_DEV void alloc_wg(const MapDev &m, const float *__restrict__ depth, int cols, int rows,
-                     const float *__restrict__ pose24, const lf_intrinsics &K, int tx, int ty,
-                     unsigned long long *s_set, unsigned long long *slot_mask = nullptr,
-                     unsigned long long bit = 0ull) {
+                     const float *__restrict__ pose24, const lf_intrinsics &K, int tx, int ty, AllocLds &s,
+                     unsigned long long *slot_mask = nullptr, unsigned long long bit = 0ull) {
     const int tid = threadIdx.x;
     const int x = tx * 16 + (tid & 15), y = ty * 16 + (tid >> 4);
     const bool inside = x < cols && y < rows;
     // the pixel's depth is in flight while the request set is cleared
     const float z = inside ? depth[(size_t)y * cols + x] : 0.0f;
-    for (int i = tid; i < kDedup; i += 256) s_set[i] = kEmptyKey;
+    for (int i = tid; i < kDedup; i += 256) s.set[i] = kEmptyKey;
+    if (tid == 0) s.n = 0u;
     if (tx == 0 && ty == 0 && tid == 0) {
         m.counters[LF_CNT_VISIBLE] = 0u;
         // one more fusion pass: read by the integration / de-integration that
@@ -221,34 +240,39 @@ LF_DEV void alloc_wg(const MapDev &m, const float *__restrict__ depth, int cols,
     float Twc[12];
 #pragma unroll
     for (int i = 0; i < 12; ++i) Twc[i] = pose24[i];
-    __syncthreads();
-    if (!inside) return;
-    band_blocks<kFast>(x, y, z, Twc, K, m, [&](int bx, int by, int bz) {
-        const unsigned long long key = pack_key(bx, by, bz);
-        unsigned int h = key_mix(key) & (kDedup - 1);
-        for (int probe = 0; probe < kDedup; ++probe) {
-            unsigned long long old = atomicCAS(&s_set[h], kEmptyKey, key);
-            if (old == kEmptyKey) {
-                bool fresh = false;
-                const int slot = kInsert ? insert_block(m, bx, by, bz, &fresh) : touch_block(m, bx, by, bz);
-                if (slot_mask && slot >= 0) atomicOr(&slot_mask[slot], bit | (fresh ? kRefuseFresh : 0ull));
-                return;
-            }
-            if (old == key) return;  // another lane of this tile owns the request
-            h = (h + 1) & (kDedup - 1);
-        }
-        // LDS set full: go straight to the table
+    const auto request = [&](int bx, int by, int bz) {
         bool fresh = false;
         const int slot = kInsert ? insert_block(m, bx, by, bz, &fresh) : touch_block(m, bx, by, bz);
         if (slot_mask && slot >= 0) atomicOr(&slot_mask[slot], bit | (fresh ? kRefuseFresh : 0ull));
-    });
+    };
+    __syncthreads();
+    if (inside)
+        band_blocks<kFast>(x, y, z, Twc, K, m, [&](int bx, int by, int bz) {
+            const unsigned long long key = pack_key(bx, by, bz);
+            unsigned int h = key_mix(key) & (kDedup - 1);
+            for (int probe = 0; probe < kDedup; ++probe) {
+                const unsigned long long old = atomicCAS(&s.set[h], kEmptyKey, key);
+                if (old == kEmptyKey) {
+                    s.list[atomicAdd(&s.n, 1u)] = (unsigned short)h;
+                    return;
+                }
+                if (old == key) return;  // another lane of this tile owns the request
+                h = (h + 1) & (kDedup - 1);
+            }
+            request(bx, by, bz);  // LDS set full: go straight to the table
+        });
+    __syncthreads();
+    for (unsigned int i = tid; i < s.n; i += 256) {
+        const unsigned long long key = s.set[s.list[i]];
+        request(key_axis(key >> 42), key_axis(key >> 21), key_axis(key));
+    }
 }
 
 template <bool kInsert, bool kFast = false>
 __global__ __launch_bounds__(256) void k_alloc(MapDev m, const float *__restrict__ depth, int cols, int rows,
                                                const float *__restrict__ pose24, lf_intrinsics K) {
-    __shared__ unsigned long long s_set[kDedup];
-    alloc_wg<kInsert, kFast>(m, depth, cols, rows, pose24, K, blockIdx.x, blockIdx.y, s_set);
+    __shared__ AllocLds s;
+    alloc_wg<kInsert, kFast>(m, depth, cols, rows, pose24, K, blockIdx.x, blockIdx.y, s);
 }
 
 // is_block_visible (depth_fusion.cu:27-47): any of the 8 block corners inside
@@ -267,6 +291,10 @@ LF_DEV bool block_visible(int bx, int by, int bz, const float *Tcw, const lf_int
             const float iz = __builtin_amdgcn_rcpf(pt.z);
             u = K.fx * pt.x * iz + K.cx;
             v = K.fy * pt.y * iz + K.cy;
+        } else if (__builtin_expect(pt.z != 0.0f, 1)) {
+            const Recip iz = recip(pt.z);
+            u = quotient(K.fx * pt.x, iz) + K.cx;
+            v = quotient(K.fy * pt.y, iz) + K.cy;
         } else {
             u = K.fx * pt.x / pt.z + K.cx;
             v = K.fy * pt.y / pt.z + K.cy;
@@ -294,17 +322,20 @@ LF_DEV void visible_wg(const MapDev &m, const float *__restrict__ pose24, const 
     float Tcw[12];
 #pragma unroll
     for (int i = 0; i < 12; ++i) Tcw[i] = pose24[12 + i];
+    const unsigned int stride = nwg * blockDim.x;
+    // a lane's first block is loaded beside the number of blocks
+    const int4 *bpos = reinterpret_cast<const int4 *>(m.block_pos);
+    int4 pos = bpos[min(wg * blockDim.x + threadIdx.x, (unsigned int)m.num_blocks - 1)];
     const unsigned int n = min(m.counters[LF_CNT_ALLOCATED], (unsigned int)m.num_blocks);
     const float scale = 8.0f * m.voxel_size;
-    const unsigned int stride = nwg * blockDim.x;
     const int lane = lane_id(), wave = threadIdx.x / kWave;
     // the trip count is uniform over the workgroup (its barriers need every lane)
     for (unsigned int b0 = wg * blockDim.x; b0 < n; b0 += stride) {
         const unsigned int b = b0 + threadIdx.x;
         bool vis = false;
-        int4 p = make_int4(0, 0, 0, 0);
+        const int4 p = pos;
+        pos = bpos[min(b + stride, (unsigned int)m.num_blocks - 1)];
         if (b < n) {
-            p = reinterpret_cast<const int4 *>(m.block_pos)[b];
             if (!kGeometric && m.slot_flag[p.w]) {
                 vis = true;
                 m.slot_flag[p.w] = 0;
@@ -604,12 +635,12 @@ struct FuseJob {
 
 template <bool kFast>
 __global__ __launch_bounds__(256) void k_alloc_batch(const FuseJob *__restrict__ jobs) {
-    __shared__ unsigned long long s_set[kDedup];
+    __shared__ AllocLds s;
     const FuseJob &j = jobs[blockIdx.y];
     const int t = blockIdx.x;
     if (t >= j.tiles_x * j.tiles_y) return;
-    alloc_wg<true, kFast>(global_dev(j.m), global_ptr(j.depth), j.cols, j.rows, global_ptr(j.pose24), j.K, t % j.tiles_x,
-                   t / j.tiles_x, s_set);
+    alloc_wg<true, kFast>(global_dev(j.m), global_ptr(j.depth), j.cols, j.rows, global_ptr(j.pose24), j.K,
+                          t % j.tiles_x, t / j.tiles_x, s);
 }
 
 template <bool kFast>
@@ -792,15 +823,15 @@ __global__ void k_fill_u64(unsigned long long *p, size_t n) {
 // blocks only); row n + k: keyframe k's at its new pose, allocating.
 template <bool kFast>
 __global__ __launch_bounds__(256) void k_refuse_alloc(RefuseArgs a) {
-    __shared__ unsigned long long s_set[kDedup];
+    __shared__ AllocLds s;
     const int tiles_x = (a.cols + 15) / 16;
     const int y = blockIdx.y, t = blockIdx.x;
     if (y < a.n)
-        alloc_wg<false, kFast>(a.m, a.depth[y], a.cols, a.rows, a.old24[y], a.K, t % tiles_x, t / tiles_x, s_set,
+        alloc_wg<false, kFast>(a.m, a.depth[y], a.cols, a.rows, a.old24[y], a.K, t % tiles_x, t / tiles_x, s,
                                a.slot_mask, 1ull << y);
     else
         alloc_wg<true, kFast>(a.m, a.depth[y - a.n], a.cols, a.rows, a.new24[y - a.n], a.K, t % tiles_x,
-                              t / tiles_x, s_set, a.slot_mask, 1ull << y);
+                              t / tiles_x, s, a.slot_mask, 1ull << y);
 }
 
 // Pose j of the 2n (j < n: keyframe j's old pose, else keyframe j - n's new
@@ -809,12 +840,28 @@ LF_DEV const float *refuse_pose(const RefuseArgs &a, int j) {
     return (j < a.n ? a.old24[j] : a.new24[j - a.n]) + 12;
 }
 
+// Whether a pose surely sees no corner of the block around the camera point c
+// (every corner within r of it): behind or beyond the update range, or outside
+// one of the image's four planes.  Slack for the rounding of c and of the
+// projections of block_visible.
+LF_DEV bool surely_unseen(f3 c, float r, const lf_intrinsics &K, int cols, int rows, float zmin, float zmax) {
+    if (c.z + r < zmin || c.z - r > zmax) return true;
+    if (!(c.z - r > 0.0f)) return false;  // a corner may lie behind the camera: its projection flips
+    // u < 0 <=> fx x + cx z < 0; u > cols - 1 <=> fx x + (cx - cols + 1) z > 0
+    const float gu = K.fx * c.x + K.cx * c.z, hu = gu - (float)(cols - 1) * c.z;
+    const float gv = K.fy * c.y + K.cy * c.z, hv = gv - (float)(rows - 1) * c.z;
+    const float ru = r * (fabsf(K.fx) + fabsf(K.cx) + (float)cols), rv = r * (fabsf(K.fy) + fabsf(K.cy) + (float)rows);
+    return gu < -ru || hu > ru || gv < -rv || hv > rv;
+}
+
 // The visible list becomes every allocated block that a keyframe's old or new
 // pose sees or whose slot the band walks marked (the slot flags are cleared),
-// each with the mask of the poses whose steps it takes.  One lane tests a
-// block against every pose, once: tested by each of a block's wavefronts in
+// each with the mask of the poses whose steps it takes.  Four lanes test a
+// block, every fourth pose each, and only the poses that a bounding sphere
+// leaves open corner by corner.  (Tested by each of a block's wavefronts in
 // k_refuse, the 2n poses' 8 corners were a quarter of that kernel's
-// instructions.
+// instructions; one lane per block without the sphere took 104 us for 40
+// poses of 165k blocks, this 39 us.)
 template <bool kFast>
 __global__ __launch_bounds__(kVisThreads) void k_refuse_visible(RefuseArgs a) {
     __shared__ unsigned int s_cnt[kVisThreads / kWave];
@@ -825,25 +872,35 @@ __global__ __launch_bounds__(kVisThreads) void k_refuse_visible(RefuseArgs a) {
         s_pose[i / 12][i % 12] = refuse_pose(a, i / 12)[i % 12];
     __syncthreads();
     const unsigned int nb = min(m.counters[LF_CNT_ALLOCATED], (unsigned int)m.num_blocks);
-    const float scale = 8.0f * m.voxel_size;
-    const unsigned int stride = gridDim.x * blockDim.x;
-    const int lane = lane_id(), wave = threadIdx.x / kWave;
+    // the half diagonal of a block with a hundredth of it to spare (coordinates
+    // are rounded to 2^-24 of at most a few thousand blocks)
+    const float scale = 8.0f * m.voxel_size, radius = 0.875f * scale;
+    constexpr unsigned int kPerWg = kVisThreads / 4;
+    const unsigned int stride = gridDim.x * kPerWg;
+    const int lane = lane_id(), wave = threadIdx.x / kWave, sub = threadIdx.x & 3;
     const unsigned long long all = (1ull << a.n) - 1ull;
-    for (unsigned int b0 = blockIdx.x * blockDim.x; b0 < nb; b0 += stride) {
-        const unsigned int b = b0 + threadIdx.x;
+    for (unsigned int b0 = blockIdx.x * kPerWg; b0 < nb; b0 += stride) {
+        const unsigned int b = b0 + threadIdx.x / 4;
         bool vis = false;
         int4 p = make_int4(0, 0, 0, 0);
-        unsigned long long steps = 0ull;
+        unsigned long long steps = 0ull, seen = 0ull, marks = 0ull;
+        bool flagged = false;
         if (b < nb) {
             p = reinterpret_cast<const int4 *>(m.block_pos)[b];
-            const unsigned long long marks = a.slot_mask[p.w];
-            const bool flagged = m.slot_flag[p.w] != 0;
-            if (flagged) m.slot_flag[p.w] = 0;
-            unsigned long long seen = marks & ~kRefuseFresh;
-            for (int j = 0; j < 2 * a.n; ++j)
-                if (block_visible<kFast>(p.x, p.y, p.z, s_pose[j], a.K, a.cols, a.rows, m.zmin_update, m.zmax_update,
+            marks = a.slot_mask[p.w];
+            flagged = m.slot_flag[p.w] != 0;
+            const f3 centre = {((float)p.x + 0.5f) * scale, ((float)p.y + 0.5f) * scale, ((float)p.z + 0.5f) * scale};
+            for (int j = sub; j < 2 * a.n; j += 4)
+                if (!surely_unseen(xform(s_pose[j], centre), radius, a.K, a.cols, a.rows, m.zmin_update, m.zmax_update) &&
+                    block_visible<kFast>(p.x, p.y, p.z, s_pose[j], a.K, a.cols, a.rows, m.zmin_update, m.zmax_update,
                                          scale))
                     seen |= 1ull << j;
+        }
+        seen |= __shfl_xor(seen, 1);
+        seen |= __shfl_xor(seen, 2);
+        if (b < nb && sub == 0) {
+            if (flagged) m.slot_flag[p.w] = 0;
+            seen |= marks & ~kRefuseFresh;
             vis = flagged || marks != 0ull || seen != 0ull;
             unsigned long long old_mask = seen & all, new_mask = (seen >> a.n) & all;
             if (marks & kRefuseFresh) {
@@ -1263,8 +1320,9 @@ static int refuse_launch(const lf_map_params *p, const RefuseArgs &a, int colour
     if (mixed) k_refuse_alloc<true><<<g, 256, 0, st>>>(a);
     else k_refuse_alloc<false><<<g, 256, 0, st>>>(a);
     LF_LAUNCH_CHECK();
-    if (mixed) k_refuse_visible<true><<<visible_grid(p), kVisThreads, 0, st>>>(a);
-    else k_refuse_visible<false><<<visible_grid(p), kVisThreads, 0, st>>>(a);
+    const int V = std::min(4 * kVisGrid, std::max(1, (p->num_blocks + kVisThreads / 4 - 1) / (kVisThreads / 4)));
+    if (mixed) k_refuse_visible<true><<<V, kVisThreads, 0, st>>>(a);
+    else k_refuse_visible<false><<<V, kVisThreads, 0, st>>>(a);
     LF_LAUNCH_CHECK();
     const int G = integrate_grid();
     if (mixed) {

@@ -307,3 +307,41 @@ def test_reductions_in_one_launch(width, height):
         check(p)
         call()
         check(p)
+
+
+# random depths under a band of 8 and of 50 voxels: a 16x16 tile requests a few hundred blocks, and more than its
+# LDS set of 1024 holds; an image smaller than a tile and one with partial tiles
+@pytest.mark.parametrize("precision", [FP32, MIXED])
+@pytest.mark.parametrize("width,height,band", [(15, 9, 8), (72, 41, 8), (72, 41, 50)])
+def test_allocation_of_scattered_requests(precision, width, height, band):
+    """Allocated and visible blocks are the oracle's, and a de-integration lists the blocks the update did."""
+    from oracle import oracle as O
+    rng = np.random.default_rng(5)
+    f = 525.0 * width / 640
+    K = capi.intrinsics(width, height, f, f, (width - 1) / 2, (height - 1) / 2)
+    depth = rng.uniform(0.4, 4.8, (height, width)).astype(np.float32)
+    depth[rng.random(depth.shape) < 0.05] = 0.0
+    nmap = np.zeros((height, width, 4), np.float32)
+    nmap[..., 2] = 1.0
+    rgb = rng.integers(0, 256, (height, width, 3)).astype(np.uint8)
+    T = np.eye(4)
+    T[:3, 3] = (0.3, -0.2, 0.1)
+    p = capi.map_params(1 << 16, 1 << 16, 0.004, 0.004 * band, precision=precision)
+    m = capi.Map(p, max(width, 8), max(height, 8))
+    pose = dev(capi.pose24(T))
+    m.update_weighted(dev(depth), dev(nmap), dev(rgb), pose, K)
+    om = O.Map(O.Params(p.num_buckets, p.num_entries, p.num_blocks, p.max_triangles, p.zmin_raycast, p.zmax_raycast,
+                        p.zmin_update, p.zmax_update, p.voxel_size, p.truncation), np.float32)
+    om.update_weighted(depth, nmap, rgb, T, O.make_intr(K.width, K.height, K.fx, K.fy, K.cx, K.cy))
+    key = lambda b: set(map(tuple, b.tolist()))  # noqa: E731
+    got, want = key(m.blocks()), key(om.blocks())
+    if precision == FP32:
+        assert got == want
+    else:  # a product with the reciprocal voxel size moves band ends that lie on a block face
+        assert len(got ^ want) <= max(2, len(want) // 200)
+    seen = key(m.visible_blocks())
+    assert seen == got  # every requested block is listed
+    n = int(m.counters()[capi.CNT_ALLOCATED])
+    m.deintegrate_weighted(dev(depth), dev(nmap), dev(rgb), pose, K)
+    assert key(m.visible_blocks()) == seen and int(m.counters()[capi.CNT_ALLOCATED]) == n
+    assert not m.t["slot_flag"].any()
