@@ -377,15 +377,90 @@ int visible_grid(const lf_map_params *p) {
     return std::min(kVisGrid, std::max(1, (p->num_blocks + kVisThreads - 1) / kVisThreads));
 }
 
-// update_map_weighted_kernel (kWeighted, depth_fusion.cu:356-428) and
-// update_map_with_colour_kernel (!kWeighted, :288-354).  kPacked (weighted
-// only): the pixel's depth, weight and colour come from one 16-byte
-// integration sample (DeviceImage frames), whose weight is the same
-// expression evaluated when the sample was made; otherwise depth, normal and
-// colour are gathered separately.  kMixed: FP16 sdf and 8-bit weight codes,
-// and the projection and the weighted means use one reciprocal each instead
-// of correctly rounded divisions.
-// Workgroup wg of nwg (grid-stride over the visible list).
+// The means' numerators over the new weight, each rounded as by a division; a
+// weight outside the range that recip() holds for takes divisions.
+template <int kN>
+LF_DEV void over_weight(float *n, float w) {
+    if (__builtin_expect(w >= 0x1p-60f && w <= 0x1p60f, 1)) {
+        const Recip d = recip(w);
+#pragma unroll
+        for (int k = 0; k < kN; ++k) n[k] = quotient(n[k], d);
+    } else {
+#pragma unroll 1
+        for (int k = 0; k < kN; ++k) n[k] /= w;
+    }
+}
+
+// A pixel's normal (x, y, z of a float4 map whose rows need only be aligned to
+// floats) in one load.
+struct PackedNormal {
+    float x, y, z;
+};
+// Pixel pix of a packed 3-byte image as r | g << 8 | b << 16 in one load: the
+// four bytes that end with it, or for pixel 0 the first four.  (An image of one
+// pixel has three.)
+LF_DEV unsigned int rgb_at(const unsigned char *__restrict__ rgb, unsigned int pix, bool one_pixel) {
+    if (__builtin_expect(one_pixel, 0)) return rgb[0] | (unsigned int)rgb[1] << 8 | (unsigned int)rgb[2] << 16;
+    unsigned int w;
+    __builtin_memcpy(&w, rgb + (pix ? 3u * pix - 1u : 0u), 4);
+    return pix ? w >> 8 : w & 0xFFFFFFu;
+}
+
+// The de-integration of voxel o of a block: its weight w0 (kMixed: of its word),
+// sdf code and colours (FP32) as loaded, the frame's observation (sdf in
+// truncation units, weight, colour), the stochastic rounding's random bits.
+template <bool kColour, bool kMixed>
+LF_DEV void take_out_voxel(short *sdf_b, float *w_b, unsigned int *wd_b, unsigned char *c_b, unsigned int o, float w0,
+                           unsigned int word, short code, const unsigned char *cold, float sdf, float wt,
+                           const unsigned char *cin, unsigned int rnd) {
+    if (w0 == 0.0f) return;  // nothing fused here
+    const float wr = w0 - wt;
+    // mixed: the stored w0 is within one code step (at most 1/16 of it) of the
+    // exact sum, so a remainder below that is the rounding of the fused weights
+    // and the voxel returns to unseen; a larger one is rounded stochastically, as
+    // fusion stores it
+    const bool keep = kMixed ? wr > w0 * (1.0f / 16.0f) : wr > 0.0f;
+    if (!keep) {
+        if constexpr (kMixed) {
+            at_byte(sdf_b, 2u * o) = (short)kHalfUnseen;
+            at_byte(wd_b, 4u * o) = kColour ? 0u : word & ~0xFFu;  // weight 0; colour cleared with colour fusion
+        } else {
+            at_byte(sdf_b, 2u * o) = kSdfUnseen;
+            at_byte(w_b, 4u * o) = 0.0f;
+            if (kColour) {
+                at_byte(c_b, o) = 0; at_byte(c_b, o + LF_BLOCK3) = 0; at_byte(c_b, o + 2 * LF_BLOCK3) = 0;
+            }
+        }
+        return;
+    }
+    const float old = kMixed ? half_bits_to_float((unsigned short)code) : unpack_sdf(code);
+    float n[4] = {old * w0 - sdf * wt, 0.0f, 0.0f, 0.0f};
+    if (kColour) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+            n[1 + k] = (kMixed ? (float)word_channel(word, k) : (float)cold[k]) * w0 - (float)cin[k] * wt;
+    }
+    over_weight<kColour ? 4 : 1>(n, wr);
+    const float sr = fmaxf(-1.0f, fminf(1.0f, n[0]));
+    unsigned int ch[3] = {0u, 0u, 0u};
+    if (kColour) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) ch[k] = (unsigned int)(int)fmaxf(0.0f, fminf(255.0f, n[1 + k]));
+    }
+    if constexpr (kMixed) {
+        at_byte(sdf_b, 2u * o) = (short)float_to_half_bits(sr);
+        at_byte(wd_b, 4u * o) = max(1u, weight_code_sr(wr, rnd)) |
+                                (kColour ? word_colour_bits(ch[0], ch[1], ch[2]) : word & ~0xFFu);
+    } else {
+        at_byte(sdf_b, 2u * o) = pack_sdf(sr);
+        at_byte(w_b, 4u * o) = wr;
+        if (kColour) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) at_byte(c_b, o + k * LF_BLOCK3) = (unsigned char)ch[k];
+        }
+    }
+}
+
 // The 256 weight-code values (weight_value) in LDS: a mixed voxel's weight
 // is one LDS read instead of the decode's arithmetic.  Every thread of the
 // workgroup calls it.
@@ -394,14 +469,40 @@ LF_DEV void fill_weight_table(float *s) {
     __syncthreads();
 }
 
+// update_map_weighted_kernel (kWeighted, depth_fusion.cu:356-428) and
+// update_map_with_colour_kernel (!kWeighted, :288-354).  kPacked (weighted
+// only): the pixel's depth, weight and colour come from one 16-byte
+// integration sample (DeviceImage frames), whose weight is the same
+// expression evaluated when the sample was made; otherwise depth, normal and
+// colour are gathered separately.  kMixed: FP16 sdf and 8-bit weight codes,
+// and the projection and the weighted means use one reciprocal each instead
+// of correctly rounded divisions.
+// kTakeOut: de-integration, the inverse of the weighted update for one frame,
+// over the same voxels (the selection depends only on depth and pose; the
+// projection is correctly rounded in both precisions).  With w the voxel's
+// weight and w_f the frame's: w' = w - w_f, sdf' = (sdf w - sdf_f w_f) / w',
+// colour likewise; w' <= 0 returns the voxel to unseen.  Exact up to the int16
+// sdf and uint8 colour rounding (kMixed: that of the FP16 sdf and the weight
+// codes), except where the weight saturated at 255.  Not in the reference
+// (deleteBlock, map_struct.cu:327-363, has no callers).
 // kTable: the weight codes' values from wtab, an LDS array of 256 floats that
 // this function fills (every thread of the workgroup calls it).
-template <bool kWeighted, bool kColour, bool kPacked, bool kMixed, bool kTable = false>
+// Workgroup wg of nwg (grid-stride over the visible list).
+// Bound by the voxels' bytes with packed samples (a 640x480 frame, 5 mm, FP32:
+// 238 MB in 53 us; mixed at 848x480, 4 mm: 215 MB in 48 us).  With separate
+// planes by the gathers (three a voxel) and the arithmetic: the projection's two
+// quotients share one refined reciprocal, the update's four another, a colour and
+// a normal are one load each (645x483, 5 mm: 74.6 us with divisions and scalar
+// loads, 71.0 now; take-out, a voxel at a time with its loads in sequence before,
+// 89.8, now 71.5).
+template <bool kWeighted, bool kColour, bool kPacked, bool kMixed, bool kTable = false, bool kTakeOut = false>
 LF_DEV void integrate_wg(const MapDev &m, const float *__restrict__ depth, const float *__restrict__ nmap,
                          const unsigned char *__restrict__ rgb, int cols, int rows, const float *__restrict__ pose24,
                          const lf_intrinsics &K, const float4 *__restrict__ samples, int wg, int nwg,
                          float *wtab = nullptr) {
     static_assert(!kPacked || kWeighted, "packed samples carry the weighted update's weight");
+    static_assert(!kTakeOut || kWeighted, "only the weighted update is taken out");
+    constexpr bool kFast = kMixed && !kTakeOut;  // one hardware reciprocal a projection
     float Tcw[12];
 #pragma unroll
     for (int i = 0; i < 12; ++i) Tcw[i] = pose24[12 + i];
@@ -409,7 +510,7 @@ LF_DEV void integrate_wg(const MapDev &m, const float *__restrict__ depth, const
     const unsigned int pass = kMixed ? m.counters[LF_CNT_FUSE_PASSES] : 0u;
     // after the loads above: they stay scalar loads ahead of the barrier
     if constexpr (kTable) fill_weight_table(wtab);
-    if (wg == 0 && threadIdx.x == 0) {
+    if (!kTakeOut && wg == 0 && threadIdx.x == 0) {
         atomicAdd(&m.counters[LF_CNT_UPDATES], 1u);
         atomicAdd(reinterpret_cast<unsigned long long *>(&m.counters[LF_CNT_VIS_SUM_LO]), (unsigned long long)nvis);
     }
@@ -418,6 +519,7 @@ LF_DEV void integrate_wg(const MapDev &m, const float *__restrict__ depth, const
     const int t = threadIdx.x;
     const int lx = t & 7, ly = (t >> 3) & 7, lz0 = t >> 6;
     const float fcols = (float)cols, frows = (float)rows;
+    const bool one_pixel = cols * rows == 1;
     // A lane owns voxels t and t + 256 of the block.  Three phases, each
     // issuing both voxels' loads before anything waits on them: the
     // projections and input gathers, then (inside the truncation band) the
@@ -443,18 +545,19 @@ LF_DEV void integrate_wg(const MapDev &m, const float *__restrict__ depth, const
         float ptz[2], dist[2], nz[2], wpk[2];
         unsigned int cpk[2];
         f3 pt0 = {0.f, 0.f, 0.f};
-        if constexpr (kMixed) {
-            const float wx = (float)(p.x * 8 + lx) * vs, wy = (float)(p.y * 8 + ly) * vs, wz = (float)(p.z * 8 + lz0) * vs;
+        if constexpr (kFast) {
+            const float wx = (float)(p.x * 8 + lx) * vs, wy = (float)(p.y * 8 + ly) * vs,
+                        wz = (float)(p.z * 8 + lz0) * vs;
             pt0 = xform(Tcw, f3{wx, wy, wz});
         }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int lz = lz0 + 4 * h;
             f3 pt;
-            if constexpr (kMixed) {
+            if constexpr (kFast) {
                 // mixed: the second voxel, 4 voxels along z, is one step of the transform's z column
-                pt = h == 0 ? pt0
-                            : f3{pt0.x + Tcw[2] * (4.0f * vs), pt0.y + Tcw[6] * (4.0f * vs), pt0.z + Tcw[10] * (4.0f * vs)};
+                const float dz = 4.0f * vs;
+                pt = h == 0 ? pt0 : f3{pt0.x + Tcw[2] * dz, pt0.y + Tcw[6] * dz, pt0.z + Tcw[10] * dz};
             } else {
                 const float wx = (float)(p.x * 8 + lx) * vs, wy = (float)(p.y * 8 + ly) * vs,
                             wz = (float)(p.z * 8 + lz) * vs;
@@ -465,13 +568,14 @@ LF_DEV void integrate_wg(const MapDev &m, const float *__restrict__ depth, const
             // 0 <= tu < cols and 0 <= tv < rows (NaN fails), where the floor
             // is the truncating conversion.
             float tu, tv;
-            if constexpr (kMixed) {
+            if constexpr (kFast) {
                 const float iz = __builtin_amdgcn_rcpf(pt.z);
                 tu = K.fx * pt.x * iz + K.cx + 0.5f;
                 tv = K.fy * pt.y * iz + K.cy + 0.5f;
-            } else {
-                tu = K.fx * pt.x / pt.z + K.cx + 0.5f;
-                tv = K.fy * pt.y / pt.z + K.cy + 0.5f;
+            } else {  // the divisions' floats; a zero z projects nowhere either way
+                const Recip iz = recip(pt.z);
+                tu = quotient(K.fx * pt.x, iz) + K.cx + 0.5f;
+                tv = quotient(K.fy * pt.y, iz) + K.cy + 0.5f;
             }
             ok[h] = tu >= 0.0f && tu < fcols && tv >= 0.0f && tv < frows;
             pix[h] = ok[h] ? __umul24((unsigned int)tv, (unsigned int)cols) + (unsigned int)tu : 0u;
@@ -506,9 +610,11 @@ LF_DEV void integrate_wg(const MapDev &m, const float *__restrict__ depth, const
             } else {
                 dist[h] = at_byte(depth, 4u * pix[h]);
                 if (kWeighted) {
-                    nx[h] = at_byte(nmap, 16u * pix[h]);
-                    nz[h] = at_byte(nmap, 16u * pix[h] + 8u);
+                    const PackedNormal n = at_byte(reinterpret_cast<const PackedNormal *>(nmap), 16u * pix[h]);
+                    nx[h] = n.x;
+                    nz[h] = n.z;
                 }
+                if (kColour) cpk[h] = rgb_at(rgb, pix[h], one_pixel);
             }
         }
         float sdf[2], wraw[2];
@@ -548,8 +654,12 @@ LF_DEV void integrate_wg(const MapDev &m, const float *__restrict__ depth, const
             unsigned char cin[3];
             if (kColour) {
 #pragma unroll
-                for (int k = 0; k < 3; ++k)
-                    cin[k] = kPacked ? (unsigned char)(cpk[h] >> (8 * k)) : rgb[3 * pix[h] + k];
+                for (int k = 0; k < 3; ++k) cin[k] = (unsigned char)(cpk[h] >> (8 * k));
+            }
+            if constexpr (kTakeOut) {
+                take_out_voxel<kColour, kMixed>(sdf_b, w_b, wd_b, c_b, o, wp[h], word[h], sp[h], cold[h], sdf_h, wt,
+                                                cin, voxel_rand_mixed(p.x, p.y, p.z, rand_local[h], pass));
+                continue;
             }
             if constexpr (kMixed) {
                 unsigned short *sdf16 = reinterpret_cast<unsigned short *>(sdf_b);
@@ -594,16 +704,18 @@ LF_DEV void integrate_wg(const MapDev &m, const float *__restrict__ depth, const
                 continue;
             }
             const float spf = unpack_sdf(sp[h]);
-            const float fused = (spf * wp[h] + sdf_h * wt) / (wp[h] + wt);
-            at_byte(sdf_b, 2u * o) = pack_sdf(fused);
             const float wn = wp[h] + wt;
+            float n[4] = {spf * wp[h] + sdf_h * wt, 0.0f, 0.0f, 0.0f};
+            if (kColour) {
+#pragma unroll
+                for (int k = 0; k < 3; ++k) n[1 + k] = (float)cold[h][k] * wp[h] + (float)cin[k] * wt;
+            }
+            over_weight<kColour ? 4 : 1>(n, wn);
+            at_byte(sdf_b, 2u * o) = pack_sdf(n[0]);
             at_byte(w_b, 4u * o) = wn > 255.0f ? 255.0f : wn;
             if (kColour) {
 #pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    const float mixed = ((float)cold[h][k] * wp[h] + (float)cin[k] * wt) / (wp[h] + wt);
-                    at_byte(c_b, o + k * LF_BLOCK3) = (unsigned char)(int)mixed;
-                }
+                for (int k = 0; k < 3; ++k) at_byte(c_b, o + k * LF_BLOCK3) = (unsigned char)(int)n[1 + k];
             }
         }
     }
@@ -670,114 +782,15 @@ __global__ __launch_bounds__(256) void k_integrate_batch(const FuseJob *__restri
                                                         blockIdx.x, gridDim.x, s_wv);
 }
 
-// De-integration: the inverse of the weighted update for one frame, over the
-// same voxels (the selection depends only on depth and pose).  With w the
-// voxel's weight and w_f the frame's: w' = w - w_f, sdf' = (sdf w - sdf_f w_f) / w',
-// colour likewise; w' <= 0 returns the voxel to unseen.  Exact up to the int16
-// sdf and uint8 colour rounding, except where the weight saturated at 255.
-// Not in the reference (deleteBlock, map_struct.cu:327-363, has no callers).
-// kMixed: FP16 sdf and 8-bit weight codes (exact up to their rounding).
 template <bool kColour, bool kPacked, bool kMixed = false>
 __global__ __launch_bounds__(256) void k_deintegrate(MapDev m, const float *__restrict__ depth,
                                                      const float *__restrict__ nmap,
                                                      const unsigned char *__restrict__ rgb, int cols, int rows,
                                                      const float *__restrict__ pose24, lf_intrinsics K,
                                                      const float4 *__restrict__ samples) {
-    float Tcw[12];
-#pragma unroll
-    for (int i = 0; i < 12; ++i) Tcw[i] = pose24[12 + i];
-    const int nvis = (int)m.counters[LF_CNT_VISIBLE];
-    const unsigned int pass = kMixed ? m.counters[LF_CNT_FUSE_PASSES] : 0u;
-    const float vs = m.voxel_size, trunc = m.truncation, inv_trunc = m.inv_truncation;
-    const float zmin = m.zmin_update, zmax = m.zmax_update;
-    const int t = threadIdx.x;
-    const int lx = t & 7, ly = (t >> 3) & 7, lz0 = t >> 6;
-    for (int i = blockIdx.x; i < nvis; i += gridDim.x) {
-        const int4 p = reinterpret_cast<const int4 *>(m.visible_pos)[i];  // x, y, z, pool block
-        const int b = p.w;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int lz = lz0 + 4 * h;
-            const float wx = (float)(p.x * 8 + lx) * vs, wy = (float)(p.y * 8 + ly) * vs, wz = (float)(p.z * 8 + lz) * vs;
-            const f3 pt = xform(Tcw, f3{wx, wy, wz});
-            const int u = proj_floor(K.fx * pt.x / pt.z + K.cx + 0.5f);
-            const int v = proj_floor(K.fy * pt.y / pt.z + K.cy + 0.5f);
-            if (u < 0 || v < 0 || u > cols - 1 || v > rows - 1) continue;
-            const size_t pix = (size_t)v * cols + u;
-            float dist, wt;
-            unsigned char cin[3] = {0, 0, 0};
-            if (kPacked) {
-                const float4 smp = samples[pix];
-                dist = smp.x;
-                wt = smp.y;
-                const unsigned int c = __float_as_uint(smp.z);
-                cin[0] = (unsigned char)c; cin[1] = (unsigned char)(c >> 8); cin[2] = (unsigned char)(c >> 16);
-                if (isnan(dist) || dist > zmax || dist < zmin) continue;
-            } else {
-                dist = depth[pix];
-                const float nx = nmap[4 * pix], nz = nmap[4 * pix + 2];
-                if (isnan(dist) || isnan(nx) || dist > zmax || dist < zmin) continue;
-                wt = fabsf(sinf(nz)) / (dist * dist);
-                if (kColour) { cin[0] = rgb[3 * pix]; cin[1] = rgb[3 * pix + 1]; cin[2] = rgb[3 * pix + 2]; }
-            }
-            float sdf = dist - pt.z;
-            if (sdf < -trunc) continue;
-            sdf = fminf(1.0f, sdf * inv_trunc);
-            const size_t vi = (size_t)b * LF_BLOCK3 + (size_t)(t + 256 * h);
-            unsigned short *sdf16 = reinterpret_cast<unsigned short *>(m.sdf);
-            unsigned int *wd = reinterpret_cast<unsigned int *>(m.weight);  // mixed: voxel words
-            const unsigned int word = kMixed ? wd[vi] : 0u;
-            const float w0 = kMixed ? weight_value(word_code(word)) : m.weight[vi];
-            if (w0 == 0.0f) continue;  // nothing fused here
-            unsigned char *c = kMixed ? nullptr : m.rgb + (size_t)b * (3 * LF_BLOCK3) + (size_t)(t + 256 * h);
-            const float wr = w0 - wt;
-            // mixed: the stored w0 is within one code step (at most 1/16 of
-            // it) of the exact sum, so a remainder below that is the rounding
-            // of the fused weights and the voxel returns to unseen; a larger
-            // one is rounded stochastically, as fusion stores it
-            const bool keep = kMixed ? wr > w0 * (1.0f / 16.0f) : wr > 0.0f;
-            const unsigned int wr_code =
-                kMixed && keep ? max(1u, weight_code_sr(wr, voxel_rand(p.x, p.y, p.z, (unsigned int)(t + 256 * h), pass)))
-                               : 0u;
-            if (!keep) {
-                if (kMixed) {
-                    sdf16[vi] = kHalfUnseen;
-                    wd[vi] = kColour ? 0u : word & ~0xFFu;  // weight 0; colour cleared with colour fusion
-                } else {
-                    m.sdf[vi] = kSdfUnseen;
-                    m.weight[vi] = 0.0f;
-                    if (kColour) { c[0] = 0; c[LF_BLOCK3] = 0; c[2 * LF_BLOCK3] = 0; }
-                }
-                continue;
-            }
-            if (kMixed) {
-                const float sr = (half_bits_to_float(sdf16[vi]) * w0 - sdf * wt) / wr;
-                sdf16[vi] = float_to_half_bits(fmaxf(-1.0f, fminf(1.0f, sr)));
-                unsigned int colour = word & ~0xFFu;
-                if (kColour) {
-                    unsigned int ch[3];
-#pragma unroll
-                    for (int k = 0; k < 3; ++k) {
-                        const float cr = ((float)word_channel(word, k) * w0 - (float)cin[k] * wt) / wr;
-                        ch[k] = (unsigned int)(int)fmaxf(0.0f, fminf(255.0f, cr));
-                    }
-                    colour = word_colour_bits(ch[0], ch[1], ch[2]);
-                }
-                wd[vi] = wr_code | colour;
-            } else {
-                const float sr = (unpack_sdf(m.sdf[vi]) * w0 - sdf * wt) / wr;
-                m.sdf[vi] = pack_sdf(fmaxf(-1.0f, fminf(1.0f, sr)));
-                m.weight[vi] = wr;
-                if (kColour) {
-#pragma unroll
-                    for (int k = 0; k < 3; ++k) {
-                        const float cr = ((float)c[k * LF_BLOCK3] * w0 - (float)cin[k] * wt) / wr;
-                        c[k * LF_BLOCK3] = (unsigned char)(int)fmaxf(0.0f, fminf(255.0f, cr));
-                    }
-                }
-            }
-        }
-    }
+    __shared__ float s_wv[kMixed ? 256 : 1];
+    integrate_wg<true, kColour, kPacked, kMixed, kMixed, true>(m, depth, nmap, rgb, cols, rows, pose24, K, samples,
+                                                               blockIdx.x, gridDim.x, s_wv);
 }
 
 // ------------------------------------------------------------ keyframe re-fusion
@@ -966,20 +979,6 @@ struct RefuseVoxel {
     float w, sdf, col[3];
     bool changed;
 };
-
-// The means' numerators over the new weight, each rounded as by a division; a
-// weight outside the range that recip() holds for takes divisions.
-template <int kN>
-LF_DEV void over_weight(float *n, float w) {
-    if (__builtin_expect(w >= 0x1p-60f && w <= 0x1p60f, 1)) {
-        const Recip d = recip(w);
-#pragma unroll
-        for (int k = 0; k < kN; ++k) n[k] = quotient(n[k], d);
-    } else {
-#pragma unroll 1
-        for (int k = 0; k < kN; ++k) n[k] /= w;
-    }
-}
 
 // k_deintegrate's step.
 template <bool kColour, bool kMixed>

@@ -345,3 +345,94 @@ def test_allocation_of_scattered_requests(precision, width, height, band):
     m.deintegrate_weighted(dev(depth), dev(nmap), dev(rgb), pose, K)
     assert key(m.visible_blocks()) == seen and int(m.counters()[capi.CNT_ALLOCATED]) == n
     assert not m.t["slot_flag"].any()
+
+
+# images of 1 to 2 pixels, of odd sizes, and of more blocks than the launch's workgroups
+@pytest.mark.parametrize("width,height,dist", [(1, 1, 1.0), (2, 1, 1.0), (33, 7, 0.7), (161, 121, 1.5)])
+def test_separate_planes_fuse_and_take_out(width, height, dist):
+    """A frame fused and taken out from depth, normal and colour planes, against the updates restated in numpy.
+
+    The projections are the same float32 operations, so both pick the same pixels; a weight differs by sin's last
+    bits (1e-6 of it), a code or a colour by one where that moves a quotient past a whole number."""
+    rng = np.random.default_rng(11)
+    f32 = np.float32
+    f = 525.0 * max(width, 16) / 640
+    K = capi.intrinsics(width, height, f, f, (width - 1) / 2, (height - 1) / 2)
+    T = np.eye(4)
+    T[:3, 3] = (0.013, -0.007, 0.011)
+    a = 0.05
+    T[:3, :3] = [[np.cos(a), 0, np.sin(a)], [0, 1, 0], [-np.sin(a), 0, np.cos(a)]]
+    p24 = capi.pose24(T)
+    vs, trunc = f32(0.01), f32(0.03)
+    p = capi.map_params(1 << 14, 1 << 14, float(vs), float(trunc))
+    m = capi.Map(p, max(width, 8), max(height, 8))
+
+    def frame(lo, hi):
+        depth = (dist + rng.uniform(-0.02, 0.02, (height, width))).astype(f32)
+        nmap = rng.uniform(lo, hi, (height, width, 4)).astype(f32)
+        if width * height > 4:
+            depth[rng.random(depth.shape) < 0.05] = np.nan
+            nmap[rng.random(depth.shape) < 0.05, 0] = np.nan
+        return depth, nmap, rng.integers(0, 256, (height, width, 3)).astype(np.uint8)
+
+    def observe(blocks, fr):
+        depth, nmap, rgb = fr
+        q = np.arange(512)
+        w = [(blocks[:, k, None] * 8 + (q >> (3 * k) & 7)).astype(f32) * vs for k in range(3)]
+        M = p24[12:].reshape(3, 4)
+        c = [M[k, 0] * w[0] + M[k, 1] * w[1] + M[k, 2] * w[2] + M[k, 3] for k in range(3)]
+        with np.errstate(all="ignore"):
+            tu = f32(K.fx) * c[0] / c[2] + f32(K.cx) + f32(0.5)
+            tv = f32(K.fy) * c[1] / c[2] + f32(K.cy) + f32(0.5)
+        ok = (tu >= 0) & (tu < width) & (tv >= 0) & (tv < height)
+        u, v = np.where(ok, tu, 0).astype(int), np.where(ok, tv, 0).astype(int)
+        d, n = depth[v, u], nmap[v, u]
+        s = d - c[2]
+        with np.errstate(invalid="ignore"):
+            ok &= (d <= f32(p.zmax_update)) & (d >= f32(p.zmin_update)) & ~np.isnan(n[..., 0]) & ~(s < -trunc)
+        s = np.minimum(f32(1), s * f32(f32(1) / trunc))
+        return ok, s, np.abs(np.sin(n[..., 2])) / (d * d), rgb[v, u].transpose(0, 2, 1).astype(f32)
+
+    def step(fr, take_out):
+        planes = [dev(x) for x in fr]
+        before = {tuple(b): i for i, b in enumerate(m.blocks().tolist())}
+        _, s0, w0, c0 = m.voxels()
+        (m.deintegrate_weighted if take_out else m.update_weighted)(*planes, dev(p24), K)
+        torch.cuda.synchronize()
+        blocks, s1, w1, c1 = m.voxels()
+        n = len(blocks)
+        assert n > 0 and [before.get(tuple(b), i) for i, b in enumerate(blocks.tolist())] == list(range(n))
+        grow = lambda x: np.concatenate([x, np.zeros((n - len(x),) + x.shape[1:], x.dtype)])  # noqa: E731
+        codes, w0, c0 = grow(s0), grow(w0), grow(c0).astype(f32)
+        seen = {tuple(b) for b in m.visible_blocks().tolist()}
+        ok, s, w, col = observe(blocks, fr)
+        ok &= np.array([tuple(b) in seen for b in blocks.tolist()])[:, None]
+        s0 = codes.astype(f32) / f32(32767)
+        with np.errstate(all="ignore"):
+            if take_out:
+                ok &= w0 != 0
+                wn = w0 - w
+                sn = np.clip((s0 * w0 - s * w) / wn, -1, 1)
+                cn = np.clip((c0 * w0[:, None] - col * w[:, None]) / wn[:, None], 0, 255)
+                gone = ok & (wn <= 0)
+                sn, wn, cn = (np.where(g, 0, x) for g, x in ((gone, sn), (gone, wn), (gone[:, None], cn)))
+            else:
+                wn = w0 + w
+                sn = np.where(w0 == 0, s, (s0 * w0 + s * w) / wn)
+                cn = np.where(w0[:, None] == 0, col, (c0 * w0[:, None] + col * w[:, None]) / wn[:, None])
+        assert ok.any()
+        sn, cn = np.trunc(np.where(ok, sn, s0) * f32(32767)), np.trunc(np.where(ok[:, None], cn, c0))
+        wn = np.where(ok, wn, w0)
+        assert np.all(np.abs(w1 - wn) <= 4e-6 * np.maximum(w0, wn))
+        sure = np.abs(wn) > 1e-3 * w0  # the rest of a weight that all but cancels is rounding
+        ratio = np.maximum(1, w0 / np.maximum(wn, 1e-30))
+        assert np.all((np.abs(s1 - sn) <= 1 + 0.1 * ratio)[sure & (wn > 0)])
+        assert np.all((np.abs(c1 - cn) <= (1 + 1e-3 * ratio)[:, None]).transpose(0, 2, 1)[sure & (wn > 0)])
+        assert np.array_equal(s1[~ok], codes[~ok]) and np.array_equal(w1[~ok], w0[~ok])
+
+    first, second, third = frame(0.1, 0.3), frame(0.4, 1.0), frame(0.4, 1.0)
+    step(first, False)
+    step(second, False)
+    step(second, True)
+    step(third, True)  # heavier than what is left: the voxels return to unseen
+    assert (m.voxels()[2] == 0).any()
