@@ -126,12 +126,11 @@ LF_DEV float4 nmap_at(const V &vert, int w, int h, int x, int y) {
 // (depth_fusion.cu:356-428) in its operation order; z = colour r | g << 8 |
 // b << 16 as bits.
 template <bool kFast = false>
-LF_DEV float4 integration_sample(float dist, float4 n, const unsigned char *c) {
+LF_DEV float4 integration_sample(float dist, float4 n, unsigned int colour) {
     const float qnan = __int_as_float(0x7fc00000);
     // kFast (mixed precision): hardware sine and reciprocal
     const float wt = kFast ? fabsf(__sinf(n.z)) * __builtin_amdgcn_rcpf(dist * dist) : fabsf(sinf(n.z)) / (dist * dist);
-    const unsigned int rgba = (unsigned int)c[0] | ((unsigned int)c[1] << 8) | ((unsigned int)c[2] << 16);
-    return make_float4(isnan(n.x) ? qnan : dist, wt, __uint_as_float(rgba), 0.0f);
+    return make_float4(isnan(n.x) ? qnan : dist, wt, __uint_as_float(colour), 0.0f);
 }
 
 struct FloatAt {
@@ -237,14 +236,14 @@ __global__ void k_nmap(const float *__restrict__ vm, float *__restrict__ nm, int
 // its own image with 16x16 workgroups, one lane per output pixel, and the
 // workgroups of the parts follow each other in the 1-D grid.
 
-constexpr int kMaxParts = 4;
-enum PartKind { kFrameIn, kPyramid, kLevelMaps, kNmap };
+constexpr int kMaxParts = 3;
+enum PartKind { kFrameIn, kPyramidMaps, kLevelMaps, kVertexPyramid };
 
 struct Part {
     int kind, w, h, wg_begin;  // w, h: the part's output size
     int half;                  // FP16 intensity / gradient / vertex / normal planes
     const void *in0, *in1, *in2, *in3;
-    void *out0, *out1, *out2, *out3, *out4;
+    void *out0, *out1, *out2, *out3, *out4, *out5;
     lf_intrinsics K;
     float scale;
 };
@@ -254,22 +253,48 @@ struct Pass {
     int total_wg;  // workgroups of all parts
 };
 
-// The windowed parts (frame, pyramid, level maps, normal maps) of a 16x16
-// output tile with their windows staged in LDS: each source pixel of the tile
-// and its apron is read (and converted or back-projected) once instead of by
-// every lane whose window holds it, and the window taps need no border
-// arithmetic.  The values and the operation order are those of the per-pixel
-// functions (bilateral_at, pyr_down_at, back_project_at, nmap_at), so the
-// outputs are the same.
+// The parts of a 16x16 output tile have their windows staged in LDS: each source
+// pixel of the tile and its apron is read (and converted, reduced or
+// back-projected) once instead of by every lane whose window holds it, and the
+// window taps need no border arithmetic.  The values and the operation order are
+// those of the per-pixel functions (bilateral_at, pyr_down_at, resize_at,
+// back_project_at, nmap_at), so the outputs are the same.
 constexpr int kTile = 16;
-constexpr int kBilApron = 2, kBilSide = kTile + 2 * kBilApron;  // 5x5 bilateral window
+constexpr int kBilApron = 2, kBilSide = kTile + 2 * kBilApron;  // 5x5 bilateral window, and pyrDown's
 constexpr int kNrmApron = 1, kNrmSide = kTile + 2 * kNrmApron;  // 3x3 (cross) normal window
-constexpr int kPyrSide = 2 * kTile + 4;  // the 2x source rows / columns of a pyrDown tile, 5-tap apron
+constexpr int kPyrSide = 2 * kNrmSide + 3;  // the source rows / columns of an aproned tile's pyrDown
+constexpr int kVtxApron = 4, kVtxSide = kTile + 2 * kVtxApron;  // a quarter-size pixel around the tile
+constexpr int kHalfSide = kTile / 2 + 2, kQuarterSide = kTile / 4 + 2;
 union TileLds {
-    float depth[kBilSide * kBilSide];
-    float4 vert[kNrmSide * kNrmSide];
-    float src[kPyrSide * kPyrSide];
+    struct {
+        float depth[kBilSide * kBilSide], grey[kBilSide * kBilSide], filtered[kTile * kTile];
+    } frame;
+    struct {
+        float4 vert[kNrmSide * kNrmSide];
+        float grey[kNrmSide * kNrmSide], src[kPyrSide * kPyrSide];
+    } maps;
+    struct {
+        float4 full[kVtxSide * kVtxSide], half[kHalfSide * kHalfSide], quarter[kQuarterSide * kQuarterSide];
+    } vtx;
 };
+
+// The value that a later read of a stored plane gives.
+template <bool kHalf>
+LF_DEV float as_stored(float v) {
+    if constexpr (kHalf) return half_bits_to_float((unsigned short)float_to_half_bits(v));
+    else return v;
+}
+
+// pyr_down_at over a staged window: the tap of row j, column k is s[j * side + k].
+LF_DEV float pyr_down_window(const float *s, int side) {
+    float rs[5];
+#pragma unroll
+    for (int j = 0; j < 5; ++j) {
+        const float *r = s + j * side;
+        rs[j] = (r[0] + r[4]) + 4.0f * (r[1] + r[3]) + 6.0f * r[2];
+    }
+    return ((rs[0] + rs[4]) + 4.0f * (rs[1] + rs[3]) + 6.0f * rs[2]) * (1.0f / 256.0f);
+}
 
 // bilateral_at over the staged depths: the window of tile pixel (cx, cy) in
 // the apron's coordinates, reflect-101 already applied when staging.
@@ -292,129 +317,255 @@ LF_DEV float bilateral_tile(const float *s, int cx, int cy) {
     return s1 / s2;
 }
 
-// kFrameIn for the tile at (x0, y0).
+// kFrameIn for the tile at (x0, y0): raw and filtered depth, intensity and colour
+// of its pixels and (out4, out5) the 8x8 depths and intensities of the next level,
+// whose windows the tile's aprons hold.
+// Bound by the filter's 25 exponentials a pixel, about 20 vector instructions each
+// (5 us at 640x480).  A 640x480 upload of three levels: 24.3 us in four launches,
+// 16.8 in two.
 template <bool kHalf>
-LF_DEV void frame_in_tile(const Part &p, int x0, int y0, TileLds &lds) {
-    const int w = p.w, h = p.h;
+LF_DEV void frame_in_tile(const Part &p, int x0, int y0, TileLds &lds_all) {
+    auto &lds = lds_all.frame;
+    const int w = p.w, h = p.h, t = threadIdx.x;
     const uint16_t *d16 = static_cast<const uint16_t *>(p.in0);
-    for (int k = threadIdx.x; k < kBilSide * kBilSide; k += blockDim.x) {
-        const int sx = reflect101(x0 - kBilApron + k % kBilSide, w), sy = reflect101(y0 - kBilApron + k / kBilSide, h);
-        lds.depth[k] = depth_value(d16[(size_t)sy * w + sx], p.scale);
-    }
-    __syncthreads();
-    const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4, x = x0 + lx, y = y0 + ly;
-    if (x >= w || y >= h) return;
-    const size_t i = (size_t)y * w + x;
     const unsigned char *rgb = static_cast<const unsigned char *>(p.in1);
-    static_cast<float *>(p.out0)[i] = lds.depth[(ly + kBilApron) * kBilSide + lx + kBilApron];
-    static_cast<float *>(p.out1)[i] = bilateral_tile<kHalf>(lds.depth, lx + kBilApron, ly + kBilApron);
-    const unsigned char r = rgb[3 * i], g = rgb[3 * i + 1], b = rgb[3 * i + 2];
-    store1<kHalf>(p.out2, i, grey_of(r, g, b));
-    unsigned char *c = static_cast<unsigned char *>(p.out3) + 3 * i;
-    c[0] = r; c[1] = g; c[2] = b;
-}
-
-// kPyramid for the tile at (x0, y0): the depth resize (resize_at), the
-// intensity pyrDown from the tile's staged source window (reflect-101 applied
-// when staging), in pyr_down_at's operation order.
-template <bool kHalf>
-LF_DEV void pyramid_tile(const Part &p, int x0, int y0, TileLds &lds) {
-    const int w = p.w, h = p.h, sw = 2 * w, sh = 2 * h;
-    const PlaneAt<kHalf> in{p.in1, sw};
-    for (int k = threadIdx.x; k < kPyrSide * kPyrSide; k += blockDim.x) {
-        const int sx = reflect101(2 * x0 - 2 + k % kPyrSide, sw), sy = reflect101(2 * y0 - 2 + k / kPyrSide, sh);
-        lds.src[k] = in(sx, sy);
+    constexpr int kRounds = (kBilSide * kBilSide + 255) / 256;
+    uint16_t d[kRounds];
+    unsigned int c[kRounds];
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+        const int k = min(t + 256 * r, kBilSide * kBilSide - 1);
+        const int sx = reflect101(x0 - kBilApron + k % kBilSide, w), sy = reflect101(y0 - kBilApron + k / kBilSide, h);
+        const size_t i = (size_t)sy * w + sx;
+        d[r] = d16[i];
+        c[r] = rgb_at(rgb, i, w * h == 1);
+    }
+    const int rows = min(kTile, h - y0);
+    const bool full = x0 + kTile <= w;
+    unsigned int words = 0;  // the colour rows of a full tile, four bytes a lane
+    const size_t at_word = 3 * ((size_t)(y0 + t / 12) * w + x0) + 4 * (t % 12);
+    if (full && t < 12 * rows) __builtin_memcpy(&words, rgb + at_word, 4);
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+        const int k = t + 256 * r;
+        if (k >= kBilSide * kBilSide) break;
+        lds.depth[k] = depth_value(d[r], p.scale);
+        lds.grey[k] = grey_of((unsigned char)c[r], (unsigned char)(c[r] >> 8), (unsigned char)(c[r] >> 16));
     }
     __syncthreads();
-    const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4, x = x0 + lx, y = y0 + ly;
-    if (x >= w || y >= h) return;
+    const int lx = t & 15, ly = t >> 4, x = x0 + lx, y = y0 + ly;
     const size_t i = (size_t)y * w + x;
-    static_cast<float *>(p.out0)[i] = resize_at(static_cast<const float *>(p.in0), sw, x, y);
-    const float *s = lds.src + (2 * ly) * kPyrSide + 2 * lx;  // tap (j, k): s[j * kPyrSide + k]
-    float rs[5];
-#pragma unroll
-    for (int j = 0; j < 5; ++j) {
-        const float *r = s + j * kPyrSide;
-        rs[j] = (r[0] + r[4]) + 4.0f * (r[1] + r[3]) + 6.0f * r[2];
+    const int at = (ly + kBilApron) * kBilSide + lx + kBilApron;
+    unsigned char *col = static_cast<unsigned char *>(p.out3);
+    if (full && t < 12 * rows) __builtin_memcpy(col + at_word, &words, 4);
+    if (x < w && y < h) {
+        static_cast<float *>(p.out0)[i] = lds.depth[at];
+        store1<kHalf>(p.out2, i, lds.grey[at]);
+        if (!full)
+            for (int k = 0; k < 3; ++k) col[3 * i + k] = rgb[3 * i + k];
+        const float f = bilateral_tile<kHalf>(lds.depth, lx + kBilApron, ly + kBilApron);
+        static_cast<float *>(p.out1)[i] = f;
+        lds.filtered[t] = f;
     }
-    store1<kHalf>(p.out1, i, ((rs[0] + rs[4]) + 4.0f * (rs[1] + rs[3]) + 6.0f * rs[2]) * (1.0f / 256.0f));
+    if (!p.out4) return;
+    __syncthreads();
+    const int hx = t & 7, hy = (t >> 3) & 7, hw = w / 2;
+    const size_t o = (size_t)(y0 / 2 + hy) * hw + x0 / 2 + hx;
+    if (t >= 128 || x0 / 2 + hx >= hw || y0 / 2 + hy >= h / 2) return;
+    if (t < 64) {
+        const float *f = lds.filtered + 2 * hy * kTile + 2 * hx;
+        static_cast<float *>(p.out4)[o] = mean4(f[0], f[1], f[kTile], f[kTile + 1]);
+    } else {
+        float taps[5 * 5];
+#pragma unroll
+        for (int j = 0; j < 25; ++j) taps[j] = as_stored<kHalf>(lds.grey[(2 * hy + j / 5) * kBilSide + 2 * hx + j % 5]);
+        store1<kHalf>(p.out5, o, pyr_down_window(taps, 5));
+    }
 }
 
-// nmap_at of pixel (x, y), tile pixel (lx, ly), from the staged vertices:
-// its neighbours (min(x+1, w), y), (max(x-1, 0), y), (x, min(y+1, h)),
-// (x, max(y-1, 0)) are the tile's, staged with their coordinates clamped
-// into the image.
+// nmap_at of pixel (x, y), staged at v in rows of `side` vertices: its neighbours
+// (min(x+1, w), y), (max(x-1, 0), y), (x, min(y+1, h)), (x, max(y-1, 0)) are the
+// tile's, staged with their coordinates clamped into the image.
 template <bool kFast>
-LF_DEV float4 normal_tile(const float4 *v, int lx, int ly, int x, int y, int w, int h) {
+LF_DEV float4 normal_tile(const float4 *v, int side, int x, int y, int w, int h) {
     const float qnan = __int_as_float(0x7fc00000);
     if (x >= w - 1 || y >= h - 1) return make_float4(qnan, qnan, qnan, qnan);
-    const int cx = lx + kNrmApron, cy = ly + kNrmApron;
-    const float4 a = v[cy * kNrmSide + cx + 1], b = v[cy * kNrmSide + cx - 1], c = v[(cy + 1) * kNrmSide + cx],
-                 e = v[(cy - 1) * kNrmSide + cx];
+    const float4 a = v[1], b = v[-1], c = v[side], e = v[-side];
     const f3 cr = cross(f3{a.x - b.x, a.y - b.y, a.z - b.z}, f3{c.x - e.x, c.y - e.y, c.z - e.z});
     const f3 n = kFast ? mul(cr, __builtin_amdgcn_rsqf(dot(cr, cr))) : normalised(cr);
     return make_float4(n.x, n.y, n.z, 1.0f);
 }
 
-// kNmap for the tile at (x0, y0): the stored vertices of the tile and a
-// one-pixel apron staged once.  out1 / out2 (when set): the tile's 8x8
-// half-size and 4x4 quarter-size vertices (kVmapDown's and kVmapDown2's
-// values) from the same staged vertices, so the vertex map is read once.
+// kVertexPyramid for the tile at (x0, y0) of a vertex map: its normals (out0), its
+// 8x8 half-size and 4x4 quarter-size vertices (out1, out2, as stored
+// resizes give them) and their normals (out3, out4), all from one staged window
+// with a quarter-size pixel around the tile; a neighbour outside a level's image
+// is its border pixel.  7.5 us at 640x480 and two coarser levels; with the coarser
+// normals in a launch of their own, from the stored vertices, 6.1 + 4.6.
 template <bool kHalf>
-LF_DEV void nmap_tile(const Part &p, int x0, int y0, TileLds &lds) {
-    const int w = p.w, h = p.h;
+LF_DEV void vertex_pyramid_tile(const Part &p, int x0, int y0, TileLds &lds_all) {
+    auto &lds = lds_all.vtx;
+    const int w = p.w, h = p.h, t = threadIdx.x;
     const float4 *vm = static_cast<const float4 *>(p.in0);
-    for (int k = threadIdx.x; k < kNrmSide * kNrmSide; k += blockDim.x) {
-        const int sx = min(max(x0 - kNrmApron + k % kNrmSide, 0), w - 1),
-                  sy = min(max(y0 - kNrmApron + k / kNrmSide, 0), h - 1);
-        lds.vert[k] = vm[(size_t)sy * w + sx];
+    constexpr int kRounds = (kVtxSide * kVtxSide + 255) / 256;
+    float4 v[kRounds];
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+        const int k = min(t + 256 * r, kVtxSide * kVtxSide - 1);
+        const int sx = min(max(x0 - kVtxApron + k % kVtxSide, 0), w - 1),
+                  sy = min(max(y0 - kVtxApron + k / kVtxSide, 0), h - 1);
+        v[r] = vm[(size_t)sy * w + sx];
     }
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r)
+        if (t + 256 * r < kVtxSide * kVtxSide) lds.full[t + 256 * r] = v[r];
     __syncthreads();
-    // tile pixel (tx, ty) of the staged vertices (in-range pixels only)
-    const auto at = [&](int tx, int ty) { return lds.vert[(ty + kNrmApron) * kNrmSide + tx + kNrmApron]; };
-    const int t = threadIdx.x;
-    if (p.out1 && t < 64) {  // half-size pixel (x0 / 2 + i, y0 / 2 + j)
-        const int i = t & 7, j = t >> 3, hx = x0 / 2 + i, hy = y0 / 2 + j, hw = w / 2, hh = h / 2;
-        if (hx < hw && hy < hh)
-            store4<false>(p.out1, (size_t)hy * hw + hx, resize4_at(at, i, j));
-    } else if (p.out2 && t >= 64 && t < 80) {  // quarter-size pixel (x0 / 4 + i, y0 / 4 + j)
-        const int i = (t - 64) & 3, j = (t - 64) >> 2, qx = x0 / 4 + i, qy = y0 / 4 + j, qw = w / 4, qh = h / 4;
-        if (qx < qw && qy < qh)
-            store4<false>(p.out2, (size_t)qy * qw + qx, resize4_quarter_at(at, i, j));
+    // the map's pixel (x, y)
+    const auto full = [&](int x, int y) { return lds.full[(y - y0 + kVtxApron) * kVtxSide + x - x0 + kVtxApron]; };
+    const int hw = w / 2, hh = h / 2, qw = w / 4, qh = h / 4;
+    if (p.out1 && t < kHalfSide * kHalfSide) {
+        const int hx = min(max(x0 / 2 - 1 + t % kHalfSide, 0), hw - 1),
+                  hy = min(max(y0 / 2 - 1 + t / kHalfSide, 0), hh - 1);
+        lds.half[t] = resize4_at(full, hx, hy);
+    }
+    if (p.out2 && t >= 128 && t < 128 + kQuarterSide * kQuarterSide) {
+        const int k = t - 128;
+        const int qx = min(max(x0 / 4 - 1 + k % kQuarterSide, 0), qw - 1),
+                  qy = min(max(y0 / 4 - 1 + k / kQuarterSide, 0), qh - 1);
+        lds.quarter[k] = resize4_quarter_at(full, qx, qy);
     }
     const int lx = t & 15, ly = t >> 4, x = x0 + lx, y = y0 + ly;
-    if (x >= w || y >= h) return;
-    store4<kHalf>(p.out0, (size_t)y * w + x, normal_tile<kHalf>(lds.vert, lx, ly, x, y, w, h));
+    if (p.out0 && x < w && y < h) {
+        const float4 *c = lds.full + (ly + kVtxApron) * kVtxSide + lx + kVtxApron;
+        store4<kHalf>(p.out0, (size_t)y * w + x, normal_tile<kHalf>(c, kVtxSide, x, y, w, h));
+    }
+    if (!p.out1) return;
+    __syncthreads();
+    if (t < 64) {  // half-size pixel (x0 / 2 + i, y0 / 2 + j)
+        const int i = t & 7, j = t >> 3, hx = x0 / 2 + i, hy = y0 / 2 + j;
+        if (hx >= hw || hy >= hh) return;
+        const float4 *c = lds.half + (j + 1) * kHalfSide + i + 1;
+        store4<false>(p.out1, (size_t)hy * hw + hx, *c);
+        store4<kHalf>(p.out3, (size_t)hy * hw + hx, normal_tile<kHalf>(c, kHalfSide, hx, hy, hw, hh));
+    } else if (p.out2 && t < 80) {  // quarter-size pixel (x0 / 4 + i, y0 / 4 + j)
+        const int i = t & 3, j = (t - 64) >> 2, qx = x0 / 4 + i, qy = y0 / 4 + j;
+        if (qx >= qw || qy >= qh) return;
+        const float4 *c = lds.quarter + (j + 1) * kQuarterSide + i + 1;
+        store4<false>(p.out2, (size_t)qy * qw + qx, *c);
+        store4<kHalf>(p.out4, (size_t)qy * qw + qx, normal_tile<kHalf>(c, kQuarterSide, qx, qy, qw, qh));
+    }
+}
+
+// The vertex and normal of tile pixel (lx, ly) from the staged vertices.
+template <bool kHalf>
+LF_DEV float4 store_vertex_normal(const Part &p, const float4 *vert, int lx, int ly, int x, int y) {
+    const size_t i = (size_t)y * p.w + x;
+    const float4 *v = vert + (ly + kNrmApron) * kNrmSide + lx + kNrmApron;
+    store4<false>(p.out2, i, *v);  // vertices stay FP32
+    const float4 n = normal_tile<kHalf>(v, kNrmSide, x, y, p.w, p.h);
+    store4<kHalf>(p.out3, i, n);
+    return n;
 }
 
 // kLevelMaps for the tile at (x0, y0): the vertices of the tile and a
 // one-pixel apron (coordinates clamped into the image, as nmap_at's
-// neighbours are) back-projected once into LDS.
+// neighbours are) back-projected once into LDS.  Every load is issued ahead of
+// the barrier.
 template <bool kHalf>
-LF_DEV void level_maps_tile(const Part &p, int x0, int y0, TileLds &lds) {
-    const int w = p.w, h = p.h;
+LF_DEV void level_maps_tile(const Part &p, int x0, int y0, TileLds &lds_all) {
+    auto &lds = lds_all.maps;
+    const int w = p.w, h = p.h, t = threadIdx.x;
     const float *d = static_cast<const float *>(p.in0);
-    for (int k = threadIdx.x; k < kNrmSide * kNrmSide; k += blockDim.x) {
-        const int sx = min(max(x0 - kNrmApron + k % kNrmSide, 0), w - 1),
-                  sy = min(max(y0 - kNrmApron + k / kNrmSide, 0), h - 1);
-        lds.vert[k] = back_project_at(d[(size_t)sy * w + sx], sx, sy, p.K);
+    const int lx = t & 15, ly = t >> 4, x = x0 + lx, y = y0 + ly;
+    const int cx = min(x, w - 1), cy = min(y, h - 1);
+    constexpr int kRounds = (kNrmSide * kNrmSide + 255) / 256;
+    float z[kRounds];
+    int sx[kRounds], sy[kRounds];
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+        const int k = min(t + 256 * r, kNrmSide * kNrmSide - 1);
+        sx[r] = min(max(x0 - kNrmApron + k % kNrmSide, 0), w - 1);
+        sy[r] = min(max(y0 - kNrmApron + k / kNrmSide, 0), h - 1);
+        z[r] = d[(size_t)sy[r] * w + sx[r]];
     }
+    float gx, gy;
+    derivative_at(PlaneAt<kHalf>{p.in1, w}, w, h, cx, cy, gx, gy);
+    float dist = 0.0f;
+    unsigned int col = 0;
+    if (p.out4) {  // level 0: the pixel's integration sample
+        const size_t i = (size_t)cy * w + cx;
+        dist = static_cast<const float *>(p.in2)[i];
+        col = rgb_at(static_cast<const unsigned char *>(p.in3), i, w * h == 1);
+    }
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r)
+        if (t + 256 * r < kNrmSide * kNrmSide) lds.vert[t + 256 * r] = back_project_at(z[r], sx[r], sy[r], p.K);
     __syncthreads();
-    const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4, x = x0 + lx, y = y0 + ly;
     if (x >= w || y >= h) return;
     const size_t i = (size_t)y * w + x;
-    float gx, gy;
-    derivative_at(PlaneAt<kHalf>{p.in1, w}, w, h, x, y, gx, gy);
     store1<kHalf>(p.out0, i, gx);
     store1<kHalf>(p.out1, i, gy);
-    store4<false>(p.out2, i, lds.vert[(ly + kNrmApron) * kNrmSide + lx + kNrmApron]);  // vertices stay FP32
-    const float4 n = normal_tile<kHalf>(lds.vert, lx, ly, x, y, w, h);
-    store4<kHalf>(p.out3, i, n);
-    if (p.out4) {  // level 0: the pixel's integration sample
-        const float dist = static_cast<const float *>(p.in2)[i];
-        const unsigned char *col = static_cast<const unsigned char *>(p.in3) + 3 * i;
-        static_cast<float4 *>(p.out4)[i] = integration_sample<kHalf>(dist, n, col);
+    const float4 n = store_vertex_normal<kHalf>(p, lds.vert, lx, ly, x, y);
+    if (p.out4) static_cast<float4 *>(p.out4)[i] = integration_sample<kHalf>(dist, n, col);
+}
+
+// kPyramidMaps for the tile at (x0, y0) of a level: its depth and intensity
+// (out4, out5) from the finer level's, with a one-pixel apron that the neighbours'
+// workgroups compute too, and its maps from those in LDS.  The aprons cost a
+// quarter more of this small level and save a launch (4.5 us).
+template <bool kHalf>
+LF_DEV void pyramid_maps_tile(const Part &p, int x0, int y0, TileLds &lds_all) {
+    auto &lds = lds_all.maps;
+    const int w = p.w, h = p.h, sw = 2 * w, sh = 2 * h, t = threadIdx.x;
+    const PlaneAt<kHalf> in{p.in1, sw};
+    constexpr int kRounds = (kNrmSide * kNrmSide + 255) / 256, kSrcRounds = (kPyrSide * kPyrSide + 255) / 256;
+    const int bx = 2 * (x0 - kNrmApron) - 2, by = 2 * (y0 - kNrmApron) - 2;
+    float src[kSrcRounds];
+#pragma unroll
+    for (int r = 0; r < kSrcRounds; ++r) {
+        const int k = min(t + 256 * r, kPyrSide * kPyrSide - 1);
+        src[r] = in(reflect101(bx + k % kPyrSide, sw), reflect101(by + k / kPyrSide, sh));
     }
+    float z[kRounds];
+    int sx[kRounds], sy[kRounds];
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+        const int k = min(t + 256 * r, kNrmSide * kNrmSide - 1);
+        sx[r] = min(max(x0 - kNrmApron + k % kNrmSide, 0), w - 1);
+        sy[r] = min(max(y0 - kNrmApron + k / kNrmSide, 0), h - 1);
+        z[r] = resize_at(static_cast<const float *>(p.in0), sw, sx[r], sy[r]);
+    }
+#pragma unroll
+    for (int r = 0; r < kSrcRounds; ++r)
+        if (t + 256 * r < kPyrSide * kPyrSide) lds.src[t + 256 * r] = src[r];
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r)
+        if (t + 256 * r < kNrmSide * kNrmSide) lds.vert[t + 256 * r] = back_project_at(z[r], sx[r], sy[r], p.K);
+    const int lx = t & 15, ly = t >> 4, x = x0 + lx, y = y0 + ly;
+    const size_t i = (size_t)y * w + x;
+    const bool in_image = x < w && y < h;
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {  // the own pixel's depth is among the staged ones
+        const int k = t + 256 * r;
+        const int tx = k % kNrmSide - kNrmApron, ty = k / kNrmSide - kNrmApron;
+        if (k < kNrmSide * kNrmSide && tx >= 0 && tx < kTile && ty >= 0 && ty < kTile && x0 + tx < w && y0 + ty < h)
+            static_cast<float *>(p.out4)[(size_t)(y0 + ty) * w + x0 + tx] = z[r];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+        if (t + 256 * r >= kNrmSide * kNrmSide) break;
+        const float g = pyr_down_window(lds.src + (2 * sy[r] - 2 - by) * kPyrSide + 2 * sx[r] - 2 - bx, kPyrSide);
+        lds.grey[t + 256 * r] = as_stored<kHalf>(g);
+    }
+    __syncthreads();
+    if (!in_image) return;
+    const float *g = lds.grey + (ly + kNrmApron) * kNrmSide + lx + kNrmApron;
+    store1<kHalf>(p.out5, i, g[0]);
+    const bool last = x >= w - 1 || y >= h - 1;  // derivative_at's
+    store1<kHalf>(p.out0, i, last ? 0.0f : (g[1] - g[-1]) * 0.5f);
+    store1<kHalf>(p.out1, i, last ? 0.0f : (g[kNrmSide] - g[-kNrmSide]) * 0.5f);
+    store_vertex_normal<kHalf>(p, lds.vert, lx, ly, x, y);
 }
 
 // Part p's workgroup t (the tile it covers); every lane reaches the part's
@@ -435,14 +586,14 @@ LF_DEV void part_wg(const Part &p, int t, TileLds &lds) {
         else level_maps_tile<false>(p, x0, y0, lds);
         return;
     }
-    if (p.kind == kNmap) {
-        if (p.half) nmap_tile<true>(p, x0, y0, lds);
-        else nmap_tile<false>(p, x0, y0, lds);
+    if (p.kind == kVertexPyramid) {
+        if (p.half) vertex_pyramid_tile<true>(p, x0, y0, lds);
+        else vertex_pyramid_tile<false>(p, x0, y0, lds);
         return;
     }
-    if (p.kind == kPyramid) {
-        if (p.half) pyramid_tile<true>(p, x0, y0, lds);
-        else pyramid_tile<false>(p, x0, y0, lds);
+    if (p.kind == kPyramidMaps) {
+        if (p.half) pyramid_maps_tile<true>(p, x0, y0, lds);
+        else pyramid_maps_tile<false>(p, x0, y0, lds);
     }
 }
 
@@ -475,7 +626,7 @@ __global__ __launch_bounds__(256) void k_frame_pass_batch(const Pass *__restrict
     Part p = ps.part[pi];
     p.in0 = global_ptr(p.in0); p.in1 = global_ptr(p.in1); p.in2 = global_ptr(p.in2); p.in3 = global_ptr(p.in3);
     p.out0 = global_ptr(p.out0); p.out1 = global_ptr(p.out1); p.out2 = global_ptr(p.out2);
-    p.out3 = global_ptr(p.out3); p.out4 = global_ptr(p.out4);
+    p.out3 = global_ptr(p.out3); p.out4 = global_ptr(p.out4); p.out5 = global_ptr(p.out5);
     part_wg(p, wg - p.wg_begin, lds);
 }
 
@@ -524,34 +675,45 @@ int check_pyramid(int levels, const lf_intrinsics *K) {
     return LF_OK;
 }
 
-// DeviceImage::upload as levels + 1 passes: the frame pass (raw depth,
-// bilateral depth, intensity, colour copy), then per level its maps
-// (derivatives, vertices, normals) together with the next level's pyramids.
+// DeviceImage::upload: the frame pass (raw depth, bilateral depth, intensity,
+// colour copy; the next level's depth and intensity), then the maps (derivatives,
+// vertices, normals) of the first two levels with the third level's depth,
+// intensity and maps, then a pass a level from the fourth on.  The coarser level
+// goes first: its workgroups take the longest.
 int plan_upload(const uint16_t *depth_u16, const unsigned char *rgb, float depth_scale, int levels,
                 const lf_intrinsics *K, const LfImageLevels &m, std::vector<Pass> &out) {
     if (int rc = check_pyramid(levels, K)) return rc;
     if (!depth_u16 || !rgb) return lf_set_error(LF_ERR_ARG, "null frame input");
+    const auto maps = [&](int kind, int l) {
+        Part p = make_part(kind, K[l].width, K[l].height);
+        const int from = kind == kPyramidMaps ? l - 1 : l;
+        p.in0 = m.depth[from]; p.in1 = m.intensity[from]; p.K = K[l];
+        p.out0 = m.dx[l]; p.out1 = m.dy[l]; p.out2 = m.vmap[l]; p.out3 = m.nmap[l];
+        if (kind == kPyramidMaps) {
+            p.out4 = m.depth[l]; p.out5 = m.intensity[l];
+        } else if (l == 0 && m.samples) {
+            p.in2 = m.depth_raw; p.in3 = m.rgb; p.out4 = m.samples;
+        }
+        return p;
+    };
     Pass ps = {};
     Part f = make_part(kFrameIn, K[0].width, K[0].height);
     f.in0 = depth_u16; f.in1 = rgb; f.scale = depth_scale;
     f.out0 = m.depth_raw; f.out1 = m.depth[0]; f.out2 = m.intensity[0]; f.out3 = m.rgb;
+    if (levels > 1) {
+        f.out4 = m.depth[1]; f.out5 = m.intensity[1];
+    }
     ps.part[ps.nparts++] = f;
     seal_pass(ps, m.half_maps);
     out.push_back(ps);
-    for (int l = 0; l < levels; ++l) {
+    ps = Pass{};
+    if (levels > 2) ps.part[ps.nparts++] = maps(kPyramidMaps, 2);
+    for (int l = 0; l < std::min(levels, 2); ++l) ps.part[ps.nparts++] = maps(kLevelMaps, l);
+    seal_pass(ps, m.half_maps);
+    out.push_back(ps);
+    for (int l = 3; l < levels; ++l) {
         ps = Pass{};
-        Part p = make_part(kLevelMaps, K[l].width, K[l].height);
-        p.in0 = m.depth[l]; p.in1 = m.intensity[l]; p.K = K[l];
-        p.out0 = m.dx[l]; p.out1 = m.dy[l]; p.out2 = m.vmap[l]; p.out3 = m.nmap[l];
-        if (l == 0 && m.samples) {
-            p.in2 = m.depth_raw; p.in3 = m.rgb; p.out4 = m.samples;
-        }
-        ps.part[ps.nparts++] = p;
-        if (l + 1 < levels) {
-            Part q = make_part(kPyramid, K[l + 1].width, K[l + 1].height);
-            q.in0 = m.depth[l]; q.in1 = m.intensity[l]; q.out0 = m.depth[l + 1]; q.out1 = m.intensity[l + 1];
-            ps.part[ps.nparts++] = q;
-        }
+        ps.part[ps.nparts++] = maps(kPyramidMaps, l);
         seal_pass(ps, m.half_maps);
         out.push_back(ps);
     }
@@ -559,24 +721,22 @@ int plan_upload(const uint16_t *depth_u16, const unsigned char *rgb, float depth
 }
 
 // DeviceImage::resize_device_map: the vertex pyramid of a raycast level-0 map
-// and every level's normals, two levels per pass (a pass with base level b
-// writes the normals still missing below b + 1 and, from the base level's
-// staged tiles, the vertices of levels b + 1 and b + 2, the latter resized
-// twice).
+// and every level's normals, three levels in the first pass, two in each after it
+// (base level b is the coarsest that the pass before wrote).
 int plan_refresh(int levels, const lf_intrinsics *K, const LfImageLevels &m, std::vector<Pass> &out) {
     if (int rc = check_pyramid(levels, K)) return rc;
-    int nmap_done = 0;
-    for (int b = 0; nmap_done < levels; b += 2) {
+    for (int b = 0; b == 0 || b + 1 < levels; b += 2) {
         Pass ps = {};
-        for (; nmap_done <= b && nmap_done < levels; ++nmap_done) {
-            Part p = make_part(kNmap, K[nmap_done].width, K[nmap_done].height);
-            p.in0 = m.vmap[nmap_done]; p.out0 = m.nmap[nmap_done];
-            if (nmap_done == b) {  // the base level's tiles also write levels b + 1 and b + 2
-                if (b + 1 < levels) p.out1 = m.vmap[b + 1];
-                if (b + 2 < levels) p.out2 = m.vmap[b + 2];
-            }
-            ps.part[ps.nparts++] = p;
+        Part p = make_part(kVertexPyramid, K[b].width, K[b].height);
+        p.in0 = m.vmap[b];
+        if (b == 0) p.out0 = m.nmap[b];
+        if (b + 1 < levels) {
+            p.out1 = m.vmap[b + 1]; p.out3 = m.nmap[b + 1];
         }
+        if (b + 2 < levels) {
+            p.out2 = m.vmap[b + 2]; p.out4 = m.nmap[b + 2];
+        }
+        ps.part[ps.nparts++] = p;
         seal_pass(ps, m.half_maps);
         out.push_back(ps);
     }

@@ -184,6 +184,16 @@ template <class T> LF_DEV T &at_byte(T *base, unsigned int off) {
     return *reinterpret_cast<T *>(reinterpret_cast<C *>(base) + off);
 }
 
+// Pixel pix of a packed 3-byte image as r | g << 8 | b << 16 in one load: the
+// four bytes that end with it, or for pixel 0 the first four.  (An image of one
+// pixel has three.)
+LF_DEV unsigned int rgb_at(const unsigned char *__restrict__ rgb, size_t pix, bool one_pixel) {
+    if (__builtin_expect(one_pixel, 0)) return rgb[0] | (unsigned int)rgb[1] << 8 | (unsigned int)rgb[2] << 16;
+    unsigned int w;
+    __builtin_memcpy(&w, rgb + (pix ? 3 * pix - 1 : 0), 4);
+    return pix ? w >> 8 : w & 0xFFFFFFu;
+}
+
 // A 32-bit byte offset held in a vector register at this point of the code
 // (an empty asm statement, no instruction): the compiler can neither hoist it
 // out of a loop nor widen it to 64 bits early, so a load or store at_byte(p,

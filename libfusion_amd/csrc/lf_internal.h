@@ -44,12 +44,12 @@ struct LfImageLevels {
     int half_maps;                       // intensity / dx / dy are FP16, nmap 4 x FP16 (vmap stays float4)
 };
 
-// DeviceImage::upload (device_image.cpp:146-181) in levels + 1 launches.  Every
+// DeviceImage::upload (device_image.cpp:146-181) in max(2, levels - 1) launches.  Every
 // level must be exactly half of the one above (K[l] of each level).
 int lf_pyramid_upload(const uint16_t *depth_u16, const unsigned char *rgb, float depth_scale, int levels,
                     const lf_intrinsics *K, const LfImageLevels &m, hipStream_t st);
 // DeviceImage::resize_device_map (device_image.cpp:188-199): vertex pyramid of
-// vmap[0] and the normals of every level, in (levels + 1) / 2 launches.
+// vmap[0] and the normals of every level, in max(1, levels / 2) launches.
 int lf_pyramid_refresh(int levels, const lf_intrinsics *K, const LfImageLevels &m, hipStream_t st);
 
 // The same passes planned instead of launched, for a batch of images: each

@@ -396,15 +396,6 @@ LF_DEV void over_weight(float *n, float w) {
 struct PackedNormal {
     float x, y, z;
 };
-// Pixel pix of a packed 3-byte image as r | g << 8 | b << 16 in one load: the
-// four bytes that end with it, or for pixel 0 the first four.  (An image of one
-// pixel has three.)
-LF_DEV unsigned int rgb_at(const unsigned char *__restrict__ rgb, unsigned int pix, bool one_pixel) {
-    if (__builtin_expect(one_pixel, 0)) return rgb[0] | (unsigned int)rgb[1] << 8 | (unsigned int)rgb[2] << 16;
-    unsigned int w;
-    __builtin_memcpy(&w, rgb + (pix ? 3u * pix - 1u : 0u), 4);
-    return pix ? w >> 8 : w & 0xFFFFFFu;
-}
 
 // The de-integration of voxel o of a block: its weight w0 (kMixed: of its word),
 // sdf code and colours (FP32) as loaded, the frame's observation (sdf in

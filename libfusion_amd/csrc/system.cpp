@@ -198,7 +198,7 @@ LfImageLevels DeviceImage::levels_view() {
 
 // upload (device_image.cpp:146-181): depth to metres, colour copy, intensity,
 // bilateral filter, depth / intensity pyramids, then per level derivatives,
-// vertices and normals — fused into levels + 1 launches.
+// vertices and normals — fused into two launches up to three levels.
 int DeviceImage::upload(const uint16_t *depth_u16, const unsigned char *rgb, float depth_scale) {
     std::vector<lf_intrinsics> K(K_.begin(), K_.end());
     return lf_pyramid_upload(depth_u16, rgb, depth_scale, levels(), K.data(), levels_view(), stream_);

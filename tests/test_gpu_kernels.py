@@ -436,3 +436,61 @@ def test_separate_planes_fuse_and_take_out(width, height, dist):
     step(second, True)
     step(third, True)  # heavier than what is left: the voxels return to unseen
     assert (m.voxels()[2] == 0).any()
+
+
+# one level of odd size and of one pixel; levels of one pixel; partial tiles on every level; more levels than the
+# first passes hold
+@pytest.mark.parametrize("width,height,levels", [(1, 1, 1), (37, 5, 1), (2, 2, 2), (46, 18, 2), (4, 4, 3),
+                                                 (72, 40, 3), (72, 40, 4), (160, 96, 6)])
+def test_image_passes(width, height, levels):
+    """upload and resize_device_map store what the operations one at a time give, bit for bit, from a colour image
+    at an odd address too."""
+    rng = np.random.default_rng(3)
+    lib, st, P = capi.load(), capi.stream_ptr(), capi.ptr
+    f = 525.0 * width / 640
+    K = capi.intrinsics(width, height, f, f, (width - 1) / 2, (height - 1) / 2)
+    img = capi.Image(K, levels)
+    d16 = rng.integers(0, 6000, (height, width)).astype(np.uint16)
+    scale = float(np.float32(1e-3))
+    colours = dev(rng.integers(0, 256, 3 * width * height + 1).astype(np.uint8))
+    d16_t, rgb_t = dev(d16), colours[1:]
+    img.upload(d16_t, rgb_t, scale)
+    like = lambda l, *c: torch.empty((img.K[l].height, img.K[l].width) + c, device="cuda")  # noqa: E731
+
+    def same(l, plane, ref):
+        assert np.array_equal(img.plane(l, plane).cpu().numpy(), ref.cpu().numpy(), equal_nan=True), (l, plane)
+
+    def normals(vm, l):
+        n = like(l, 4)
+        capi.check(lib.lf_compute_nmap(P(vm), P(n), img.K[l].width, img.K[l].height, st))
+        return n
+
+    raw, depth, grey = like(0), [like(l) for l in range(levels)], [like(l) for l in range(levels)]
+    capi.check(lib.lf_depth_to_float(P(d16_t), P(raw), width, height, scale, st))
+    capi.check(lib.lf_bilateral_filter(P(raw), P(depth[0]), width, height, st))
+    capi.check(lib.lf_rgb_to_intensity(P(rgb_t), P(grey[0]), width, height, st))
+    same(0, capi.PLANE_RAW_DEPTH, raw)
+    same(0, capi.PLANE_RGB, rgb_t.view(height, width, 3))
+    for l in range(levels):
+        w, h = img.K[l].width, img.K[l].height
+        if l:
+            capi.check(lib.lf_pyr_down_depth(P(depth[l - 1]), P(depth[l]), 2 * w, 2 * h, st))
+            capi.check(lib.lf_pyr_down_image(P(grey[l - 1]), P(grey[l]), 2 * w, 2 * h, st))
+        dx, dy, vm = like(l), like(l), like(l, 4)
+        capi.check(lib.lf_compute_derivative(P(grey[l]), P(dx), P(dy), w, h, st))
+        capi.check(lib.lf_back_project_depth(P(depth[l]), P(vm), w, h, ctypes.byref(img.K[l]), st))
+        for plane, ref in ((capi.PLANE_DEPTH, depth[l]), (capi.PLANE_INTENSITY, grey[l]), (capi.PLANE_DX, dx),
+                           (capi.PLANE_DY, dy), (capi.PLANE_VMAP, vm), (capi.PLANE_NMAP, normals(vm, l))):
+            same(l, plane, ref)
+    v = dev(rng.uniform(-1, 4, (height, width, 4)).astype(np.float32))
+    torch.cuda.synchronize()
+    capi.copy_device_to(img.plane_ptr(0, capi.PLANE_VMAP), v)
+    img.resize_device_map()
+    for l in range(levels):
+        if l:
+            half = like(l, 4)
+            capi.check(lib.lf_pyr_down_vmap(P(v), P(half), img.K[l - 1].width, img.K[l - 1].height, st))
+            v = half
+        same(l, capi.PLANE_VMAP, v)
+        same(l, capi.PLANE_NMAP, normals(v, l))
+    img.close()
