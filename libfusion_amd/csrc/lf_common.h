@@ -227,6 +227,14 @@ LF_HD int dir_cell(int bx, int by, int bz) {
     return (int)((brick << 6) | ((z & 3u) << 4) | ((y & 3u) << 2) | (x & 3u));
 }
 
+// Axis kAxis's term of dir_cell: a block's cell is the sum of its three terms.
+template <int kAxis>
+LF_HD int dir_term(int b) {
+    constexpr unsigned int nb = LF_DIR_DIM / 4, brick = kAxis == 0 ? 64u : kAxis == 1 ? 64u * nb : 64u * nb * nb;
+    const unsigned int u = (unsigned int)(b + LF_DIR_DIM / 2);
+    return (int)((u >> 2) * brick + ((u & 3u) << (2 * kAxis)));
+}
+
 // Linear-probing lookup from the computeHash home bucket; returns the pool
 // block of (bx, by, bz) or -1.  The probe is bounded by the table size.  A
 // slot's key and block index are loaded together (one memory round trip per

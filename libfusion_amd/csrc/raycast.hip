@@ -273,8 +273,6 @@ LF_DEV int ray_floor(float v) {
     asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(v));
     return r;
 }
-// 1 when v's sign bit is clear, else 0 (for a v neither NaN nor zero: v > 0)
-LF_DEV unsigned int positive(float v) { return ~__float_as_uint(v) >> 31; }
 
 // The pool block of a block outside the block directory: the workgroup's LDS
 // cache of lookups, then the hash table.  (Inside the directory its load is
@@ -364,19 +362,19 @@ LF_DEV float read_sdf(const RayDev &r, BlockCache &bc, f3 p, bool &valid, int *v
 // read_sdf_interped (ray_tracing.cu:307-339).  Corner k is the voxel of
 // p + offset_k with offsets 0 or 1 per axis, so each axis has only two
 // coordinates, floor(p) and floor(p + 1), computed once, and the corners lie
-// in at most two blocks per axis.  Corner k's block is B[k & m], where m has
-// a bit for each axis whose two coordinates lie in different blocks and B[e]
-// is the block one step across the faces of e: B[0] is p's own block (the
-// lane's cache), and the others are looked up in one loop over the nonzero
-// subsets of m (one code path whatever faces a lane's corners straddle; none
-// in the common case).  Then all 8 sdf loads are issued in one round trip
+// in at most two blocks per axis.  Where they lie in one block (the common case)
+// that is the lane's cached block; otherwise all corners' blocks are loaded from
+// the directory in one round (a corner's cell is the sum of one term an axis), or,
+// beside or outside the directory, looked up one after the other over the nonzero
+// subsets of the axes whose two coordinates lie in different blocks.  Then all 8
+// sdf loads are issued in one round trip
 // (a corner in an unallocated block reads voxel 0 of pool block 0, and NaN
 // replaces corner 0's value).  An invalid corner is NaN and the corner values are
 // finite otherwise, so the result is valid exactly when it is not NaN.  The
 // arithmetic is the reference's order.
 // f0: floor(p) when the caller has it from the sample read at p, whose
 // block the lane's cache then holds; else computed and resolved here.
-template <bool kMixed>
+template <bool kMixed, bool kDir = false>
 LF_DEV float read_interp(const RayDev &r, BlockCache &bc, f3 p, bool &valid, const i3 *f0 = nullptr) {
     // floor(p) as int and as float (exact: an int from a float converts back
     // to that float)
@@ -390,35 +388,61 @@ LF_DEV float read_interp(const RayDev &r, BlockCache &bc, f3 p, bool &valid, con
               bz1 = cz[1] >> 3;
     const int m = (bx1 != bx0 ? 1 : 0) | (by1 != by0 ? 2 : 0) | (bz1 != bz0 ? 4 : 0);
     int bb[8];
-    bb[0] = f0 ? bc.b : resolve(r, bc, bx0, by0, bz0);
 #pragma unroll
-    for (int k = 1; k < 8; ++k) bb[k] = bb[0];
-    for (int e = m & -m; e != 0; e = (e - m) & m) {  // the nonzero subsets of m, increasing
-        const int b = corner_block(r, bc, (e & 1) ? bx1 : bx0, (e & 2) ? by1 : by0, (e & 4) ? bz1 : bz0);
+    for (int k = 0; k < 8; ++k) bb[k] = bc.b;
+    const bool cached = f0 || (bx0 == bc.bx && by0 == bc.by && bz0 == bc.bz);
+    if (m != 0 || !cached) {
+        constexpr int h = LF_DIR_DIM / 2;
+        constexpr unsigned int side = LF_DIR_DIM - 1;  // the block one step up lies in the directory too
+        const bool inside = (unsigned int)(bx0 + h) < side && (unsigned int)(by0 + h) < side &&
+                            (unsigned int)(bz0 + h) < side;
+        if (kDir || inside) {
+            const int c0[3] = {dir_term<0>(bx0), dir_term<1>(by0), dir_term<2>(bz0)},
+                      c1[3] = {dir_term<0>(bx1), dir_term<1>(by1), dir_term<2>(bz1)};
 #pragma unroll
-        for (int k = 1; k < 8; ++k)
-            if ((k & m) == e) bb[k] = b;
+            for (int k = f0 ? 1 : 0; k < 8; ++k)
+                bb[k] = at_byte(r.block_dir, 4u * (unsigned int)(((k & 1) ? c1[0] : c0[0]) + ((k & 2) ? c1[1] : c0[1]) +
+                                                                 ((k & 4) ? c1[2] : c0[2])));
+        } else {
+            bb[0] = f0 ? bc.b : resolve(r, bc, bx0, by0, bz0);
+#pragma unroll
+            for (int k = 1; k < 8; ++k) bb[k] = bb[0];
+            for (int e = m & -m; e != 0; e = (e - m) & m) {  // the nonzero subsets of m, increasing
+                const int b = corner_block(r, bc, (e & 1) ? bx1 : bx0, (e & 2) ? by1 : by0, (e & 4) ? bz1 : bz0);
+#pragma unroll
+                for (int k = 1; k < 8; ++k)
+                    if ((k & m) == e) bb[k] = b;
+            }
+        }
+        if (!f0) {
+            bc.bx = bx0; bc.by = by0; bc.bz = bz0; bc.b = bb[0];
+        }
     }
     // byte offsets of the corners' sdf: block << 10 | 2 * lidx
     const unsigned int ox[2] = {(unsigned int)(cx[0] & 7) << 1, (unsigned int)(cx[1] & 7) << 1},
                        oy[2] = {(unsigned int)(cy[0] & 7) << 4, (unsigned int)(cy[1] & 7) << 4},
                        oz[2] = {(unsigned int)(cz[0] & 7) << 7, (unsigned int)(cz[1] & 7) << 7};
-    const unsigned short *sdf16 = reinterpret_cast<const unsigned short *>(r.sdf);
-    unsigned short c[8];
+    using Code = typename std::conditional<kMixed, unsigned short, short>::type;
+    const Code *codes = reinterpret_cast<const Code *>(r.sdf);
+    Code c[8];
     int bmin = bb[0];
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
-        c[k] = at_byte(sdf16, ((unsigned int)max(bb[k], 0) << 10) | ox[k & 1] | oy[(k >> 1) & 1] | oz[k >> 2]);
+        c[k] = at_byte(codes, ((unsigned int)max(bb[k], 0) << 10) | ox[k & 1] | oy[(k >> 1) & 1] | oz[k >> 2]);
         bmin = min(bmin, bb[k]);
     }
-    const float qnan = __int_as_float(0x7fc00000);
     float s[8];
+    bool unknown = bmin < 0;  // a corner in an unallocated block
+    if constexpr (!kMixed) {  // or an unseen one, the lowest code (kHalfUnseen is a NaN already)
+        static_assert(kSdfUnseen == -32768, "the unseen code is the lowest");
+        int lowest = c[0];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        if constexpr (kMixed) s[k] = half_bits_to_float(c[k]);  // kHalfUnseen is a NaN already
-        else s[k] = (short)c[k] == kSdfUnseen ? qnan : unpack_sdf((short)c[k]);
+        for (int k = 1; k < 8; ++k) lowest = min(lowest, (int)c[k]);
+        unknown = unknown || lowest == kSdfUnseen;
     }
-    if (bmin < 0) s[0] = qnan;  // a corner in an unallocated block
+#pragma unroll
+    for (int k = 0; k < 8; ++k) s[k] = kMixed ? half_bits_to_float((unsigned short)c[k]) : unpack_sdf((short)c[k]);
+    if (unknown) s[0] = __int_as_float(0x7fc00000);
     float r0 = (1.0f - xyz.x) * s[0] + xyz.x * s[1];
     float r1 = (1.0f - xyz.x) * s[2] + xyz.x * s[3];
     const float r2 = (1.0f - xyz.y) * r0 + xyz.y * r1;
@@ -428,6 +452,117 @@ LF_DEV float read_interp(const RayDev &r, BlockCache &bc, f3 p, bool &valid, con
     const float v = (1.0f - xyz.z) * r2 + xyz.z * r3;
     valid = !isnan(v);
     return v;
+}
+
+// The march of a ray from res until its sample is on the surface (sdf <= 0), behind
+// one (back_face) or past the end.  kDir: every sample and its trilinear corners lie
+// in the block directory (by the caller's check), so that a block coordinate is 24
+// bits, one comparison tells a new block, its cell and its region's occupancy bit
+// are parts of one word, and the hash table is not in the loop.
+// Bound by an iteration's instructions, branches included (a wavefront passes
+// through nearly every path in each: its 64 rays differ), then by its two dependent
+// loads; the longest wavefront (90 iterations beside a mean of 21) is most of a
+// single map's time.  So steps through empty boxes are four at a time without a test,
+// and the general loop, 526 vector instructions long where this one has 290, is left
+// to wavefronts near the directory's end: 640x480, 5 mm, FP32 128.6 -> 89.6 us;
+// 1280x960, 4 mm, mixed 275 -> 183; 16 maps of 640x480, mixed 686 -> 521.  Slower:
+// passing several empty boxes in an inner loop (2 to 3 times: the rays fall out of
+// step), loading the next block's cell ahead (1.05 to 1.25 times).
+template <bool kMixed, bool kDir>
+LF_DEV void march(const RayDev &r, BlockCache &bc, f3 &res, const f3 dir2, float dist_s, const float dist_e, float &sdf,
+                  bool &back_face) {
+    const float qnan = __int_as_float(0x7fc00000);
+    // A sample in an unallocated block (or empty 4x4x4-block region) is
+    // followed by the reference's 2-voxel steps for as long as they stay
+    // inside that box, where every read finds nothing: those steps are
+    // taken without the reads, by the same float operations.  The count
+    // stops 0.05 voxels short of where the ray leaves the box, so that no
+    // sample the box does not surely hold is passed over.
+    const f3 half_inv = {__builtin_amdgcn_rcpf(dir2.x), __builtin_amdgcn_rcpf(dir2.y), __builtin_amdgcn_rcpf(dir2.z)};
+    // all ones where the ray runs towards + along the axis (the reciprocal's sign
+    // bit clear, +inf included): a box's exit face there is its far side
+    const int fwd_x = ~(__float_as_int(half_inv.x) >> 31), fwd_y = ~(__float_as_int(half_inv.y) >> 31),
+              fwd_z = ~(__float_as_int(half_inv.z) >> 31);
+    const float half_scale = r.half_step_scale;
+    int blk = -1, box_mask = 7;  // kDir: the cached block's packed coordinate; the box of a block without voxels
+    bool valid = false;
+    sdf = 1.0f;
+    back_face = false;
+    while (dist_s < dist_e) {
+        const float last_sdf = sdf;
+        const i3 fl = {ray_floor(res.x), ray_floor(res.y), ray_floor(res.z)};
+        if constexpr (kDir) {
+            constexpr int h = LF_DIR_DIM / 2;
+            static_assert(LF_DIR_DIM == 256, "8 bits an axis");
+            const unsigned int p = (unsigned int)((fl.x >> 3) + ((fl.y >> 3) << 8) + ((fl.z >> 3) << 16) +
+                                                  (h | h << 8 | h << 16));
+            if ((int)p != blk) {
+                blk = (int)p;
+                const unsigned int brick = ((p >> 2) & 63u) | ((p >> 4) & (63u << 6)) | ((p >> 6) & (63u << 12));
+                const unsigned int bit = brick ^ 0x820u;  // occupancy_bit's: the biased coordinates' top bits flipped
+                bc.b = -1;
+                box_mask = 31;
+                if ((bc.occ[(bit >> 5) & (LF_OCC_WORDS - 1)] >> (bit & 31u)) & 1u) {
+                    box_mask = 7;
+                    bc.b = at_byte(r.block_dir,
+                                   4u * (brick << 6 | (p & 3u) | ((p >> 6) & 12u) | ((p >> 12) & 48u)));  // dir_cell's
+                }
+            }
+        } else {
+            resolve(r, bc, fl.x >> 3, fl.y >> 3, fl.z >> 3);
+            box_mask = bc.box ? 31 : 7;  // region: 32 voxels a side; block: 8
+        }
+        if (bc.b < 0) {
+            sdf = qnan;
+            const float tx = ((float)(((fl.x & ~box_mask) | (fwd_x & box_mask)) - fwd_x) - res.x) * half_inv.x;
+            const float ty = ((float)(((fl.y & ~box_mask) | (fwd_y & box_mask)) - fwd_y) - res.y) * half_inv.y;
+            const float tz = ((float)(((fl.z & ~box_mask) | (fwd_z & box_mask)) - fwd_z) - res.z) * half_inv.z;
+            // steps to the exit (NaN / inf terms drop out); samples k >= 1 lie inside for 2k < exit - 0.05
+            const int quiet = (int)(fminf(tx, fminf(ty, tz)) - 0.025f);
+            res = add(res, dir2);
+            dist_s += 2.0f;
+            // as far as they surely end short of the ray's end too (a step not taken here is a read that finds nothing)
+            int n = min(quiet, (int)((dist_e - dist_s) * 0.4999f) - 1);
+            for (; n >= 4; n -= 4) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    res = add(res, dir2);
+                    dist_s += 2.0f;
+                }
+            }
+            if (n >= 2) {
+                res = add(add(res, dir2), dir2);
+                dist_s = (dist_s + 2.0f) + 2.0f;
+            }
+            if (n > 0 && (n & 1)) {
+                res = add(res, dir2);
+                dist_s += 2.0f;
+            }
+            continue;
+        }
+        const unsigned int off = (unsigned int)bc.b << 10 | (unsigned int)lidx(fl.x, fl.y, fl.z) << 1;
+        if constexpr (kMixed) {
+            sdf = half_bits_to_float(at_byte(reinterpret_cast<const unsigned short *>(r.sdf), off));
+            valid = !isnan(sdf);
+        } else {
+            const short code = at_byte(r.sdf, off);
+            valid = code != kSdfUnseen;
+            sdf = valid ? unpack_sdf(code) : qnan;
+        }
+        if (sdf <= 0.5f && sdf >= -0.5f) sdf = read_interp<kMixed, kDir>(r, bc, res, valid, &fl);
+        if (sdf <= 0.0f) {
+            if constexpr (kDir) {  // the cached block's coordinates, for the reads that follow
+                bc.bx = fl.x >> 3; bc.by = fl.y >> 3; bc.bz = fl.z >> 3;
+            }
+            break;
+        }
+        if (sdf >= 0.0f && last_sdf < 0.0f) { back_face = true; break; }
+        // half the reference's step max(sdf * step_scale, 1) (or 2), exactly; the
+        // march adds 2 dir (exact) times it, the same float as dir times the step
+        const float half_step = valid ? fmaxf(sdf * half_scale, 0.5f) : 1.0f;
+        res = add(res, mul(dir2, half_step));
+        dist_s = __builtin_fmaf(2.0f, half_step, dist_s);  // dist_s + step, one rounding
+    }
 }
 
 // MapRenderingDelegate::operator() (check_colour == false) and
@@ -441,12 +576,8 @@ LF_DEV void raycast_wg(const RayDev &r, float *__restrict__ vmap, unsigned char 
                        unsigned long long *s_cache, uint4 *s_occ) {
     // DenseMapping::raycast leaves the map untouched when nothing is visible
     // (voxel_hashing.cpp:92-93) or no rendering block was made (:105).
-    if (r.counters[LF_CNT_VISIBLE] == 0u || r.counters[LF_CNT_RENDER_BLOCKS] == 0u) return;
-    for (int i = threadIdx.x; i < kLdsCache; i += blockDim.x) s_cache[i] = 0ull;
-    const uint4 *occ4 = reinterpret_cast<const uint4 *>(r.occupancy);
-    for (int i = threadIdx.x; i < LF_OCC_WORDS / 4; i += blockDim.x) s_occ[i] = occ4[i];
-    __syncthreads();
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    // (The loads of the start are issued together, ahead of the test.)
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     // XCD-aware placement: workgroups are dealt to the 8 XCDs in turn, so
     // workgroup g (XCD g % 8) takes the (g / 8)-th workgroup tile of band g % 8:
     // each XCD marches a contiguous band of the image, and the blocks its rays
@@ -455,16 +586,27 @@ LF_DEV void raycast_wg(const RayDev &r, float *__restrict__ vmap, unsigned char 
     const int L = (wg % kXcds) * per_xcd + wg / kXcds;
     if (L >= nwg) return;
     const int tile_x = (L % wg_x) * 2 + (wave & 1), tile_y = (L / wg_x) * 2 + (wave >> 1);
+    const bool has_range = tile_x < r.tiles_x && tile_y < r.tiles_y;
+    const int tile = has_range ? tile_y * r.tiles_x + tile_x : 0;
+    const float z0 = r.zx[tile], z1 = r.zy[tile];
+    const uint4 *occ4 = reinterpret_cast<const uint4 *>(r.occupancy);
+    constexpr int kOccRounds = LF_OCC_WORDS / 4 / 256;
+    static_assert(kOccRounds * 256 * 4 == LF_OCC_WORDS, "whole rounds of the workgroup's 256 threads");
+    uint4 occ[kOccRounds];
+#pragma unroll
+    for (int i = 0; i < kOccRounds; ++i) occ[i] = occ4[threadIdx.x + 256 * i];
+    if (r.counters[LF_CNT_VISIBLE] == 0u || r.counters[LF_CNT_RENDER_BLOCKS] == 0u) return;
+    for (int i = threadIdx.x; i < kLdsCache; i += 256) s_cache[i] = 0ull;
+#pragma unroll
+    for (int i = 0; i < kOccRounds; ++i) s_occ[threadIdx.x + 256 * i] = occ[i];
+    __syncthreads();
     const int x = tile_x * 8 + (lane & 7), y = tile_y * 8 + (lane >> 3);
     if (x >= cols || y >= rows) return;
-    const size_t px = (size_t)y * cols + x;
     const float qnan = __int_as_float(0x7fc00000);
     float4 res4 = make_float4(qnan, qnan, qnan, qnan);
     unsigned char col[3] = {255, 255, 255};
     do {
-        if (tile_x >= r.tiles_x || tile_y >= r.tiles_y) break;
-        const int t = tile_y * r.tiles_x + tile_x;
-        const float z0 = r.zx[t], z1 = r.zy[t];
+        if (!has_range) break;
         if (z1 < 1e-3f || z0 < 1e-3f || isnan(z0) || isnan(z1)) break;
         const float *Twc = pose24;
         const float inv_vs = r.inv_voxel_size;  // the map's (scalar registers)
@@ -484,49 +626,20 @@ LF_DEV void raycast_wg(const RayDev &r, float *__restrict__ vmap, unsigned char 
         f3 res = bs;
         BlockCache bc = {kBad, kBad, kBad, -1, r.pool_fits_lds ? s_cache : nullptr,
                          reinterpret_cast<const unsigned int *>(s_occ), 0};
-        // A sample in an unallocated block (or empty 4x4x4-block region) is
-        // followed by the reference's 2-voxel steps for as long as they stay
-        // inside that box, where every read finds nothing: those steps are
-        // taken without the reads, by the same float operations.  The count
-        // stops 0.05 voxels short of where the ray leaves the box, so that no
-        // sample the box does not surely hold is passed over.
-        const f3 inv_dir = {__builtin_amdgcn_rcpf(dir.x), __builtin_amdgcn_rcpf(dir.y), __builtin_amdgcn_rcpf(dir.z)};
-        // bit a set: the ray runs towards + along axis a (inv_dir's sign bit
-        // clear, +inf included), so a box's exit face on that axis is its far side
-        const unsigned int fwd = positive(inv_dir.x) | positive(inv_dir.y) << 1 | positive(inv_dir.z) << 2;
-        // The march keeps 2 dir (exact), which a quiet step adds as it is; a
-        // step of s voxels adds 2 dir * (s / 2), the same float as dir * s
-        // (both factors are exact power-of-two scalings of the reference's).
-        const f3 dir2 = mul(dir, 2.0f);
+        const f3 dir2 = mul(dir, 2.0f);  // exact
         const float half_scale = r.half_step_scale;
-        float sdf = 1.0f, last_sdf, step;
-        bool valid = false, back_face = false;
-        while (dist_s < dist_e) {
-            last_sdf = sdf;
-            i3 fl;
-            sdf = read_sdf<kMixed>(r, bc, res, valid, nullptr, &fl);
-            int quiet = 0;  // further samples surely inside the same unallocated box
-            if (bc.b < 0) {
-                const int k = bc.box, sh = k + 3;  // region: 32 voxels a side; block: 8
-                const float tx = ((float)(((bc.bx >> k) + (int)(fwd & 1u)) << sh) - res.x) * inv_dir.x;
-                const float ty = ((float)(((bc.by >> k) + (int)((fwd >> 1) & 1u)) << sh) - res.y) * inv_dir.y;
-                const float tz = ((float)(((bc.bz >> k) + (int)(fwd >> 2)) << sh) - res.z) * inv_dir.z;
-                const float texit = fminf(tx, fminf(ty, tz));  // NaN / inf terms drop out
-                // samples at 2k (k >= 1) with 2k < texit - 0.05
-                if (texit < 1e4f) quiet = max(0, (int)ceilf(0.5f * (texit - 0.05f)) - 1);
-            }
-            if (sdf <= 0.5f && sdf >= -0.5f) sdf = read_interp<kMixed>(r, bc, res, valid, &fl);
-            if (sdf <= 0.0f) break;
-            if (sdf >= 0.0f && last_sdf < 0.0f) { back_face = true; break; }
-            // half the reference's step max(sdf * step_scale, 1) (or 2), exactly
-            const float half_step = valid ? fmaxf(sdf * half_scale, 0.5f) : 1.0f;
-            res = add(res, mul(dir2, half_step));
-            dist_s = __builtin_fmaf(2.0f, half_step, dist_s);  // dist_s + step, one rounding
-            for (int k = 0; k < quiet && dist_s < dist_e; ++k) {  // each: a read that finds nothing, a 2-voxel step
-                res = add(res, dir2);
-                dist_s += 2.0f;
-            }
-        }
+        float sdf, step;
+        bool valid = false, back_face;
+        // Where every sample of the wavefront's rays lies in the directory, with 4
+        // voxels for the trilinear corners and the rounding of the steps.
+        const float len = dist_e - dist_s;
+        const float far = fmaxf(fmaxf(fabsf(bs.x), fabsf(bs.x + dir.x * len)),
+                                fmaxf(fmaxf(fabsf(bs.y), fabsf(bs.y + dir.y * len)),
+                                      fmaxf(fabsf(bs.z), fabsf(bs.z + dir.z * len))));
+        if (__all(far < 4.0f * LF_DIR_DIM - 4.0f))
+            march<kMixed, true>(r, bc, res, dir2, dist_s, dist_e, sdf, back_face);
+        else
+            march<kMixed, false>(r, bc, res, dir2, dist_s, dist_e, sdf, back_face);
         if (back_face || !(sdf <= 0.0f)) break;
         const f3 dir1 = mul(dir2, 0.5f);  // dir again, exactly
         const float step_scale = 2.0f * half_scale;
@@ -556,15 +669,18 @@ LF_DEV void raycast_wg(const RayDev &r, float *__restrict__ vmap, unsigned char 
         const f3 q = xform(Tcw, mul(res, r.voxel_size));
         res4 = make_float4(q.x, q.y, q.z, 1.0f);
     } while (false);
+    const size_t px = (size_t)y * cols + x;
     reinterpret_cast<float4 *>(vmap)[px] = res4;
     if (rgb_out) {
-        unsigned char *o = rgb_out + 3 * ((size_t)y * cols + x);
+        unsigned char *o = rgb_out + 3 * px;
         o[0] = col[0]; o[1] = col[1]; o[2] = col[2];
     }
 }
 
+// Held to 64 VGPRs for 8 waves per SIMD (68 and 7 without: 1280x960 196 us, not 183;
+// 640x480, 5 waves per SIMD in all, within 1 us).
 template <bool kCheckColour, bool kMixed>
-__global__ __launch_bounds__(256) void k_raycast(RayDev r, float *__restrict__ vmap, unsigned char *__restrict__ rgb_out,
+__global__ __launch_bounds__(256, 8) void k_raycast(RayDev r, float *__restrict__ vmap, unsigned char *__restrict__ rgb_out,
                                                  int cols, int rows, const float *__restrict__ pose24,
                                                  lf_intrinsics K, int wg_x, int wg_y) {
     __shared__ unsigned long long s_cache[kLdsCache];
@@ -572,9 +688,7 @@ __global__ __launch_bounds__(256) void k_raycast(RayDev r, float *__restrict__ v
     raycast_wg<kCheckColour, kMixed>(r, vmap, rgb_out, cols, rows, pose24, K, wg_x, wg_y, blockIdx.x, s_cache, s_occ);
 }
 
-// Many maps' rays fill the chip many times over, so this kernel is held to 64
-// VGPRs for 8 waves per SIMD; the single-map kernel (about 5 waves per SIMD
-// in all) keeps the compiler's own allocation, whose sample chain is shorter.
+// As k_raycast for many maps, row y of the grid the map of jobs[y].
 template <bool kCheckColour, bool kMixed>
 __global__ __launch_bounds__(256, 8) void k_raycast_batch(const RayJob *__restrict__ jobs) {
     __shared__ unsigned long long s_cache[kLdsCache];

@@ -494,3 +494,47 @@ def test_image_passes(width, height, levels):
         same(l, capi.PLANE_VMAP, v)
         same(l, capi.PLANE_NMAP, normals(v, l))
     img.close()
+
+
+# the block directory ends 5.12 m from the origin on each axis: views inside it, across its faces, its corner, outside;
+# a step of 1.5 and of 25 voxels
+@pytest.mark.parametrize("band", [3, 50])
+@pytest.mark.parametrize("at", [(0.0, 0.0, 0.0), (5.0, 0.2, -0.5), (-5.1, 0.0, 1.0), (0.1, 5.08, 0.0), (0.0, 0.0, 4.2),
+                                (-4.95, -5.05, 4.3), (7.0, -6.5, 6.0)])
+def test_raycast_around_the_directory(at, band):
+    """Vertices and colours of a rough surface with holes, bit for bit the oracle's on the same volume."""
+    from oracle import oracle as O
+    rng = np.random.default_rng(17)
+    width, height = 72, 41
+    f = 525.0 * width / 640
+    K = capi.intrinsics(width, height, f, f, (width - 1) / 2, (height - 1) / 2)
+    u, v = np.meshgrid(np.linspace(0, 7, width), np.linspace(0, 4, height))
+    depth = (0.9 + 0.2 * np.sin(u) * np.cos(v) + 0.01 * rng.random((height, width))).astype(np.float32)
+    depth[rng.random(depth.shape) < 0.1] = 0.0
+    depth[10:20, 30:40] += 0.5
+    nmap = np.zeros((height, width, 4), np.float32)
+    nmap[..., 2] = 1.0
+    rgb = rng.integers(0, 256, (height, width, 3)).astype(np.uint8)
+    a, b = 0.3, -0.2
+    T = np.eye(4)
+    T[:3, :3] = (np.array([[np.cos(a), 0, np.sin(a)], [0, 1, 0], [-np.sin(a), 0, np.cos(a)]])
+                 @ np.array([[1, 0, 0], [0, np.cos(b), -np.sin(b)], [0, np.sin(b), np.cos(b)]]))
+    T[:3, 3] = at
+    p = capi.map_params(1 << 16, 1 << 15, 0.005, 0.005 * band)
+    m = capi.Map(p, width, height)
+    pose = dev(capi.pose24(T))
+    m.update_weighted(dev(depth), dev(nmap), dev(rgb), pose, K)
+    vm = torch.full((height, width, 4), float("nan"), device="cuda")
+    col = torch.zeros((height, width, 3), dtype=torch.uint8, device="cuda")
+    m.raycast(vm, pose, K, check_colour=True, rgb_out=col)
+    torch.cuda.synchronize()
+    om = O.Map(O.Params(p.num_buckets, p.num_entries, p.num_blocks, p.max_triangles, p.zmin_raycast, p.zmax_raycast,
+                        p.zmin_update, p.zmax_update, p.voxel_size, p.truncation), np.float32)
+    oK = O.make_intr(K.width, K.height, K.fx, K.fy, K.cx, K.cy)
+    om.update_weighted(depth, nmap, rgb, T, oK)
+    om.set_blocks(*m.voxels())
+    ovm, ocol = om.raycast(T, oK, width, height, check_colour=True, want_rgb=True)
+    hit = ~np.isnan(ovm[..., 0])
+    assert hit.mean() > 0.4
+    assert np.array_equal(vm.cpu().numpy()[hit], ovm[hit]) and np.isnan(vm.cpu().numpy()[~hit]).all()
+    assert np.array_equal(col.cpu().numpy(), ocol)
