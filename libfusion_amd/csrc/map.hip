@@ -220,16 +220,40 @@ struct AllocLds {
     unsigned short list[kDedup];  // positions in the set, in the order of insertion
     unsigned int n;
 };
-template <bool kInsert, bool kFast = false>
+constexpr int kFarTile = 8;
+LF_HD int far_tiles(int pixels) { return (pixels + kFarTile - 1) / kFarTile; }
+// A depth that the update accepts as an integer of the same order, above 0 (one
+// below zero as zero's); 0: a depth it does not.
+LF_DEV int far_code(float d, float zmin, float zmax) {
+    return isnan(d) || d > zmax || d < zmin ? 0 : __float_as_int(fmaxf(d, 0.0f)) + 1;
+}
+// The largest far_code of each 8x8-pixel tile of the workgroup's 16x16 pixels into far
+// (zero before): a wavefront's four rows of 16 by DPP and permlane swaps, then one
+// atomic per tile.
+LF_DEV void far_tiles_max(int code, int cols, int rows, int tx, int ty, int *far) {
+    code = max(code, __builtin_amdgcn_mov_dpp(code, 0xB1, 0xF, 0xF, false));   // quad_perm 1,0,3,2
+    code = max(code, __builtin_amdgcn_mov_dpp(code, 0x4E, 0xF, 0xF, false));   // quad_perm 2,3,0,1
+    code = max(code, __builtin_amdgcn_mov_dpp(code, 0x141, 0xF, 0xF, false));  // row_half_mirror
+    const auto a = __builtin_amdgcn_permlane16_swap(code, code, false, false);
+    code = max((int)a[0], (int)a[1]);
+    const auto b = __builtin_amdgcn_permlane32_swap(code, code, false, false);
+    code = max((int)b[0], (int)b[1]);
+    const int t = threadIdx.x, lane = t & 63, x = tx * 2 + (lane >> 3), y = ty * 2 + (t >> 7);
+    if ((lane & 7) == 0 && lane < 16 && x < far_tiles(cols) && y < far_tiles(rows) && code > 0)
+        atomicMax(&far[y * far_tiles(cols) + x], code);
+}
+
+template <bool kInsert, bool kFast, bool kFar = false>
 LF_DEV void alloc_wg(const MapDev &m, const float *__restrict__ depth, int cols, int rows,
                      const float *__restrict__ pose24, const lf_intrinsics &K, int tx, int ty, AllocLds &s,
-                     unsigned long long *slot_mask = nullptr, unsigned long long bit = 0ull) {
+                     unsigned long long *slot_mask = nullptr, unsigned long long bit = 0ull, int *far = nullptr) {
     const int tid = threadIdx.x;
     const int x = tx * 16 + (tid & 15), y = ty * 16 + (tid >> 4);
     const bool inside = x < cols && y < rows;
     // the pixel's depth is in flight while the request set is cleared
     const float z = inside ? depth[(size_t)y * cols + x] : 0.0f;
     for (int i = tid; i < kDedup; i += 256) s.set[i] = kEmptyKey;
+    if constexpr (kFar) far_tiles_max(inside ? far_code(z, m.zmin_update, m.zmax_update) : 0, cols, rows, tx, ty, far);
     if (tid == 0) s.n = 0u;
     if (tx == 0 && ty == 0 && tid == 0) {
         m.counters[LF_CNT_VISIBLE] = 0u;
@@ -380,14 +404,19 @@ int visible_grid(const lf_map_params *p) {
 // The means' numerators over the new weight, each rounded as by a division; a
 // weight outside the range that recip() holds for takes divisions.
 template <int kN>
+LF_DEV void divide_all(float *n, float w) {
+#pragma unroll 1
+    for (int k = 0; k < kN; ++k) n[k] /= w;
+}
+LF_DEV bool recip_holds(float w) { return (w >= 0x1p-60f) & (w <= 0x1p60f); }
+template <int kN>
 LF_DEV void over_weight(float *n, float w) {
-    if (__builtin_expect(w >= 0x1p-60f && w <= 0x1p60f, 1)) {
+    if (__builtin_expect(recip_holds(w), 1)) {
         const Recip d = recip(w);
 #pragma unroll
         for (int k = 0; k < kN; ++k) n[k] = quotient(n[k], d);
     } else {
-#pragma unroll 1
-        for (int k = 0; k < kN; ++k) n[k] /= w;
+        divide_all<kN>(n, w);
     }
 }
 
@@ -810,6 +839,7 @@ struct RefuseArgs {
     MapDev m;
     unsigned long long *slot_mask;  // per hash slot: bit k old pose k, bit n + k new pose k
     unsigned long long *list_mask;  // per visible-list entry: the poses whose steps it takes, the same bits
+    int *tile_far;                  // per keyframe and kFarTile^2 pixels: far_code of the largest depth in range
     const float *depth[kMaxRefuse];
     const float4 *samples[kMaxRefuse];
     const float *old24[kMaxRefuse];
@@ -824,15 +854,16 @@ __global__ void k_fill_u64(unsigned long long *p, size_t n) {
 }
 
 // Row y < n of the grid: keyframe y's band walk at its old pose (existing
-// blocks only); row n + k: keyframe k's at its new pose, allocating.
+// blocks only) and its tile_far; row n + k: keyframe k's at its new pose, allocating.
 template <bool kFast>
 __global__ __launch_bounds__(256) void k_refuse_alloc(RefuseArgs a) {
     __shared__ AllocLds s;
     const int tiles_x = (a.cols + 15) / 16;
     const int y = blockIdx.y, t = blockIdx.x;
     if (y < a.n)
-        alloc_wg<false, kFast>(a.m, a.depth[y], a.cols, a.rows, a.old24[y], a.K, t % tiles_x, t / tiles_x, s,
-                               a.slot_mask, 1ull << y);
+        alloc_wg<false, kFast, true>(a.m, a.depth[y], a.cols, a.rows, a.old24[y], a.K, t % tiles_x, t / tiles_x, s,
+                                     a.slot_mask, 1ull << y,
+                                     a.tile_far + (size_t)y * far_tiles(a.cols) * far_tiles(a.rows));
     else
         alloc_wg<true, kFast>(a.m, a.depth[y - a.n], a.cols, a.rows, a.new24[y - a.n], a.K, t % tiles_x,
                               t / tiles_x, s, a.slot_mask, 1ull << y);
@@ -858,22 +889,67 @@ LF_DEV bool surely_unseen(f3 c, float r, const lf_intrinsics &K, int cols, int r
     return gu < -ru || hu > ru || gv < -rv || hv > rv;
 }
 
+// A pose's camera-aligned box around a block's voxels: half sizes, and its centre
+// relative to the block's, with a hundredth of a block to spare.
+struct RefuseBox {
+    f3 half, shift;
+};
+LF_DEV RefuseBox refuse_box(const float *Tcw, float vs) {
+    RefuseBox b;
+    float *h = &b.half.x, *c = &b.shift.x;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const float x = Tcw[4 * i], y = Tcw[4 * i + 1], z = Tcw[4 * i + 2];
+        h[i] = 3.5f * vs * (fabsf(x) + fabsf(y) + fabsf(z)) + 0.08f * vs;
+        c[i] = -0.5f * vs * (x + y + z);  // voxels 0..7 around 3.5
+    }
+    return b;
+}
+
+// Whether keyframe k changes no voxel of the block whose box at this pose is
+// c +- half: every voxel that projects into the image lies more than the truncation
+// behind the largest depth of the tiles around it (or the tiles hold no depth).
+// The box's pixels are widened by one for the rounding of the voxels' projections.
+LF_DEV bool surely_behind(const RefuseArgs &a, int k, f3 c, f3 half) {
+    const float zn = c.z - half.z, zf = c.z + half.z;
+    if (!(zn > 0.0f) || !(a.K.fx > 0.0f) || !(a.K.fy > 0.0f)) return false;
+    const float in = __builtin_amdgcn_rcpf(zn), fn = __builtin_amdgcn_rcpf(zf);
+    const float x0 = c.x - half.x, x1 = c.x + half.x, y0 = c.y - half.y, y1 = c.y + half.y;
+    const float u0 = a.K.fx * x0 * (x0 < 0.0f ? in : fn) + a.K.cx - 0.5f,
+                u1 = a.K.fx * x1 * (x1 > 0.0f ? in : fn) + a.K.cx + 1.5f,
+                v0 = a.K.fy * y0 * (y0 < 0.0f ? in : fn) + a.K.cy - 0.5f,
+                v1 = a.K.fy * y1 * (y1 > 0.0f ? in : fn) + a.K.cy + 1.5f;
+    if (!(u1 - u0 < 4.0f * kFarTile) || !(v1 - v0 < 4.0f * kFarTile)) return false;  // at most 5x5 tiles; NaN
+    const int w = far_tiles(a.cols), h = far_tiles(a.rows);
+    const int tx0 = (int)fmaxf(u0, 0.0f) / kFarTile, tx1 = (int)fminf(u1, (float)(a.cols - 1)) / kFarTile;
+    const int ty0 = (int)fmaxf(v0, 0.0f) / kFarTile, ty1 = (int)fminf(v1, (float)(a.rows - 1)) / kFarTile;
+    const int *far = a.tile_far + (size_t)k * w * h;
+    int most = 0;
+    if (u1 >= 0.0f && v1 >= 0.0f)
+        for (int y = ty0; y <= ty1; ++y)
+            for (int x = tx0; x <= tx1; ++x) most = max(most, far[y * w + x]);
+    return most == 0 || __int_as_float(most - 1) - zn < -a.m.truncation * 1.0001f;
+}
+
 // The visible list becomes every allocated block that a keyframe's old or new
 // pose sees or whose slot the band walks marked (the slot flags are cleared),
-// each with the mask of the poses whose steps it takes.  Four lanes test a
-// block, every fourth pose each, and only the poses that a bounding sphere
-// leaves open corner by corner.  (Tested by each of a block's wavefronts in
-// k_refuse, the 2n poses' 8 corners were a quarter of that kernel's
-// instructions; one lane per block without the sphere took 104 us for 40
-// poses of 165k blocks, this 39 us.)
+// each with the mask of the poses whose steps it takes, less those whose depths all
+// lie in front of the block.  Four lanes test a block, every fourth pose each, and
+// only the poses that a bounding sphere leaves open corner by corner.  40 poses of
+// 165k blocks: 104 us with one lane per block and no sphere; 39 without the depths'
+// test, 54 with it, which takes 160 us off k_refuse (tiles of 4 pixels, as good a
+// test: 70).
 template <bool kFast>
 __global__ __launch_bounds__(kVisThreads) void k_refuse_visible(RefuseArgs a) {
     __shared__ unsigned int s_cnt[kVisThreads / kWave];
     __shared__ unsigned int s_base;
     __shared__ float s_pose[2 * kMaxRefuse][12];
+    __shared__ RefuseBox s_box[2 * kMaxRefuse];
     const MapDev &m = a.m;
     for (int i = threadIdx.x; i < 2 * a.n * 12; i += kVisThreads)
         s_pose[i / 12][i % 12] = refuse_pose(a, i / 12)[i % 12];
+    __syncthreads();
+    for (int i = threadIdx.x; i < 2 * a.n; i += kVisThreads) s_box[i] = refuse_box(s_pose[i], m.voxel_size);
     __syncthreads();
     const unsigned int nb = min(m.counters[LF_CNT_ALLOCATED], (unsigned int)m.num_blocks);
     // the half diagonal of a block with a hundredth of it to spare (coordinates
@@ -887,21 +963,32 @@ __global__ __launch_bounds__(kVisThreads) void k_refuse_visible(RefuseArgs a) {
         const unsigned int b = b0 + threadIdx.x / 4;
         bool vis = false;
         int4 p = make_int4(0, 0, 0, 0);
-        unsigned long long steps = 0ull, seen = 0ull, marks = 0ull;
+        unsigned long long steps = 0ull, seen = 0ull, idle = 0ull, marks = 0ull;
         bool flagged = false;
         if (b < nb) {
             p = reinterpret_cast<const int4 *>(m.block_pos)[b];
             marks = a.slot_mask[p.w];
             flagged = m.slot_flag[p.w] != 0;
             const f3 centre = {((float)p.x + 0.5f) * scale, ((float)p.y + 0.5f) * scale, ((float)p.z + 0.5f) * scale};
-            for (int j = sub; j < 2 * a.n; j += 4)
-                if (!surely_unseen(xform(s_pose[j], centre), radius, a.K, a.cols, a.rows, m.zmin_update, m.zmax_update) &&
-                    block_visible<kFast>(p.x, p.y, p.z, s_pose[j], a.K, a.cols, a.rows, m.zmin_update, m.zmax_update,
-                                         scale))
-                    seen |= 1ull << j;
+            unsigned int open = 0u;  // bit i: pose sub + 4 i
+            for (int i = 0, j = sub; j < 2 * a.n; ++i, j += 4)
+                if (!surely_unseen(xform(s_pose[j], centre), radius, a.K, a.cols, a.rows, m.zmin_update, m.zmax_update))
+                    open |= 1u << i;
+            for (; open; open &= open - 1u) {
+                const int j = sub + 4 * __builtin_ctz(open);
+                if (!block_visible<kFast>(p.x, p.y, p.z, s_pose[j], a.K, a.cols, a.rows, m.zmin_update, m.zmax_update,
+                                          scale))
+                    continue;
+                seen |= 1ull << j;
+                const f3 c = add(xform(s_pose[j], centre), s_box[j].shift);
+                if (surely_behind(a, j < a.n ? j : j - a.n, c, s_box[j].half))
+                    idle |= 1ull << j;
+            }
         }
         seen |= __shfl_xor(seen, 1);
         seen |= __shfl_xor(seen, 2);
+        idle |= __shfl_xor(idle, 1);
+        idle |= __shfl_xor(idle, 2);
         if (b < nb && sub == 0) {
             if (flagged) m.slot_flag[p.w] = 0;
             seen |= marks & ~kRefuseFresh;
@@ -913,7 +1000,7 @@ __global__ __launch_bounds__(kVisThreads) void k_refuse_visible(RefuseArgs a) {
                 old_mask = 0ull;
                 new_mask &= ~((walks & (0ull - walks)) - 1ull);
             }
-            steps = old_mask | new_mask << a.n;
+            steps = (old_mask | new_mask << a.n) & ~idle;
         }
         const unsigned long long ballot = __ballot(vis);
         if (lane == 0) s_cnt[wave] = (unsigned int)__popcll(ballot);
@@ -961,8 +1048,9 @@ LF_DEV RefuseProj refuse_project(const RefuseArgs &a, const float *Tcw, float wx
     }
     // the pixel (floor(tu), floor(tv)), in the image exactly when 0 <= tu < cols
     // and 0 <= tv < rows (NaN fails), where the floor is the truncating conversion
-    const bool in = tu >= 0.0f && tu < (float)a.cols && tv >= 0.0f && tv < (float)a.rows;
-    return {pt.z, in ? (unsigned int)(int)tv * (unsigned int)a.cols + (unsigned int)(int)tu : 0u, in};
+    const bool in = (tu >= 0.0f) & (tu < (float)a.cols) & (tv >= 0.0f) & (tv < (float)a.rows);
+    const unsigned int pix = __umul24((unsigned int)(int)tv, (unsigned int)a.cols) + (unsigned int)(int)tu;
+    return {pt.z, in ? pix : 0u, in};
 }
 
 // A voxel's running mean (sdf, colour) and weight.
@@ -971,7 +1059,7 @@ struct RefuseVoxel {
     bool changed;
 };
 
-// k_deintegrate's step.
+// take_out_voxel's arithmetic on a running mean.
 template <bool kColour, bool kMixed>
 LF_DEV void refuse_take_out(RefuseVoxel &v, float s, float wt, unsigned int rgb) {
     v.changed = true;
@@ -988,7 +1076,7 @@ LF_DEV void refuse_take_out(RefuseVoxel &v, float s, float wt, unsigned int rgb)
 #pragma unroll
         for (int q = 0; q < 3; ++q) n[1 + q] = v.col[q] * v.w - (float)((rgb >> (8 * q)) & 0xFFu) * wt;
     }
-    over_weight<kColour ? 4 : 1>(n, wr);
+    divide_all<kColour ? 4 : 1>(n, wr);
     v.sdf = fmaxf(-1.0f, fminf(1.0f, n[0]));
     if (kColour) {
 #pragma unroll
@@ -997,7 +1085,7 @@ LF_DEV void refuse_take_out(RefuseVoxel &v, float s, float wt, unsigned int rgb)
     v.w = wr;
 }
 
-// The weighted update's step.
+// The weighted update's.
 template <bool kColour>
 LF_DEV void refuse_put_in(RefuseVoxel &v, float s, float wt, unsigned int rgb) {
     v.changed = true;
@@ -1016,7 +1104,7 @@ LF_DEV void refuse_put_in(RefuseVoxel &v, float s, float wt, unsigned int rgb) {
 #pragma unroll
         for (int q = 0; q < 3; ++q) n[1 + q] = v.col[q] * v.w + (float)((rgb >> (8 * q)) & 0xFFu) * wt;
     }
-    over_weight<kColour ? 4 : 1>(n, wn);
+    divide_all<kColour ? 4 : 1>(n, wn);
     v.sdf = n[0];
     if (kColour) {
 #pragma unroll
@@ -1025,15 +1113,46 @@ LF_DEV void refuse_put_in(RefuseVoxel &v, float s, float wt, unsigned int rgb) {
     v.w = fminf(wn, 255.0f);
 }
 
+// One step of a voxel, de-integration or update (the same for a whole wavefront):
+// with the frame's weight signed, both are the mean of the two over w + ws, the
+// de-integration's clamped.  A first observation, a voxel that returns to unseen and
+// a weight outside recip()'s range take the functions above.
+template <bool kColour, bool kMixed>
+LF_DEV void refuse_step(RefuseVoxel &v, float s, float wt, unsigned int rgb, bool put_in) {
+    const float inf = __builtin_inff();
+    const float ws = put_in ? wt : -wt, wn = v.w + ws;
+    const bool plain = put_in ? v.w != 0.0f : (kMixed ? wn > v.w * (1.0f / 16.0f) : wn > 0.0f);
+    if (plain & recip_holds(wn)) {
+        const Recip d = recip(wn);
+        v.changed = true;
+        v.sdf = __builtin_amdgcn_fmed3f(quotient(v.sdf * v.w + s * ws, d), put_in ? -inf : -1.0f, put_in ? inf : 1.0f);
+        if (kColour) {
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+                v.col[q] = __builtin_amdgcn_fmed3f(quotient(v.col[q] * v.w + (float)((rgb >> (8 * q)) & 0xFFu) * ws, d),
+                                                   put_in ? -inf : 0.0f, put_in ? inf : 255.0f);
+        }
+        v.w = fminf(wn, 255.0f);
+    } else if (put_in) {
+        refuse_put_in<kColour>(v, s, wt, rgb);
+    } else if (v.w != 0.0f) {
+        refuse_take_out<kColour, kMixed>(v, s, wt, rgb);
+    }
+}
+
 // One lane per voxel (two voxels per lane, 256 lanes per block) of the visible
 // list: the steps of its mask in order, de-integrations (bits below n) first.
 // kMixed: FP16 sdf and the packed weight-code / colour word, the weights
 // rounded stochastically once at the end (as the update stores them).
 // Each step gathers 16 bytes per voxel: both voxels' samples of the next step
 // are loaded while the present one is applied, and the poses are in LDS.
-// 20 keyframes of 640x480 on 165k blocks (FP32, 4 mm): 1797 -> 936 us.
+// Bound by its vector instructions (the arithmetic of a projection and of four
+// weighted means a voxel and step).  20 keyframes of 640x480 on 165k blocks (FP32,
+// 4 mm): 1797 us at one voxel and one load after the other, 966 with divisions'
+// branches for either direction, 775 now with the steps that change nothing left out.
+// 64 VGPRs keep 8 waves a SIMD (66: 1018 us where 64 took 934).
 template <bool kColour, bool kMixed>
-__global__ __launch_bounds__(256) void k_refuse(RefuseArgs a) {
+__global__ __launch_bounds__(256, 8) void k_refuse(RefuseArgs a) {
     __shared__ float s_pose[2 * kMaxRefuse][12];
     const MapDev &m = a.m;
     const int t = threadIdx.x;
@@ -1089,33 +1208,40 @@ __global__ __launch_bounds__(256) void k_refuse(RefuseArgs a) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 pr[h] = refuse_project<kMixed>(a, T, wx, wy, wz[h]);
-                smp[h] = samples[pr[h].pix];
+                smp[h] = at_byte(samples, vgpr_offset(16u * pr[h].pix));
             }
+        };
+        bool use[2];
+        float sd[2], wt[2];
+        unsigned int rgb[2];
+        // the update's selection: in the image, depth within the range, sdf >= -truncation
+        auto arrive = [&]() {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const float d = smp[h].x;
+                sd[h] = d - pr[h].z;
+                use[h] = pr[h].in & !(d > zmax) & !(d < zmin) & (sd[h] >= -m.truncation);  // NaN fails the last
+                wt[h] = smp[h].y;
+                rgb[h] = __float_as_uint(smp[h].z);
+            }
+        };
+        auto apply = [&](bool put_in) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                if (use[h])
+                    refuse_step<kColour, kMixed>(v[h], fminf(1.0f, sd[h] * m.inv_truncation), wt[h], rgb[h], put_in);
         };
         int j = __builtin_ctzll(steps);
         look(j);
-        while (true) {
-            const RefuseProj pc[2] = {pr[0], pr[1]};
-            const float4 sc[2] = {smp[0], smp[1]};
-            const bool put_in = j >= a.n;
-            steps &= steps - 1ull;
-            const bool more = steps != 0ull;
-            if (more) {
-                j = __builtin_ctzll(steps);
-                look(j);
-            }
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                // the update's selection: in the image, depth within the range, sdf >= -truncation
-                const float d = sc[h].x, s = d - pc[h].z;
-                if (!pc[h].in || isnan(d) || d > zmax || d < zmin || s < -m.truncation) continue;
-                const float sn = fminf(1.0f, s * m.inv_truncation);
-                const unsigned int rgb = __float_as_uint(sc[h].z);
-                if (put_in) refuse_put_in<kColour>(v[h], sn, sc[h].y, rgb);
-                else if (v[h].w != 0.0f) refuse_take_out<kColour, kMixed>(v[h], sn, sc[h].y, rgb);
-            }
-            if (!more) break;
+        arrive();
+        while ((steps &= steps - 1ull) != 0ull) {
+            const int next = __builtin_ctzll(steps);
+            look(next);
+            apply(j >= a.n);
+            j = next;
+            arrive();
         }
+        apply(j >= a.n);
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             if (!v[h].changed) continue;
@@ -1351,13 +1477,15 @@ int lf_refuse_ev(const lf_map_params *p, const lf_map_storage *s, const float *c
     a.cols = cols;
     a.rows = rows;
     a.K = *K;
-    // the masks per slot and per listed block: stream-ordered device memory for the call's length
+    // the masks per slot and per listed block, the tiles' depths: stream-ordered device memory for the call's length
     const size_t E = (size_t)p->num_entries, B = (size_t)p->num_blocks;
     void *mask = nullptr;
-    LF_HIP_CHECK(hipMallocAsync(&mask, (E + B) * sizeof(unsigned long long), st));
+    const size_t F2 = ((size_t)n * far_tiles(cols) * far_tiles(rows) + 1) / 2;  // two to a word
+    LF_HIP_CHECK(hipMallocAsync(&mask, (E + F2 + B) * sizeof(unsigned long long), st));
     a.slot_mask = static_cast<unsigned long long *>(mask);
-    a.list_mask = a.slot_mask + E;
-    k_fill_u64<<<(int)std::min<size_t>(4096, (E + 255) / 256), 256, 0, st>>>(a.slot_mask, E);
+    a.list_mask = a.slot_mask + E + F2;
+    a.tile_far = reinterpret_cast<int *>(a.slot_mask + E);
+    k_fill_u64<<<(int)std::min<size_t>(4096, (E + F2 + 255) / 256), 256, 0, st>>>(a.slot_mask, E + F2);
     const int rc = refuse_launch(p, a, colour, st);
     const hipError_t ef = hipFreeAsync(mask, st);
     if (rc) return rc;

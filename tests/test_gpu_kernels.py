@@ -538,3 +538,52 @@ def test_raycast_around_the_directory(at, band):
     assert hit.mean() > 0.4
     assert np.array_equal(vm.cpu().numpy()[hit], ovm[hit]) and np.isnan(vm.cpu().numpy()[~hit]).all()
     assert np.array_equal(col.cpu().numpy(), ocol)
+
+
+# an image inside one tile, partial tiles, and blocks that span more tiles than the depth test looks at
+@pytest.mark.parametrize("width,height,voxel", [(7, 5, 0.01), (61, 43, 0.01), (64, 48, 0.01), (160, 120, 0.02)])
+def test_refusion_with_occlusions(width, height, voxel):
+    """Keyframes of patches at depths that hide each other, none and out of range among them: re-fusion leaves the
+    voxels seen, and their weights, that one keyframe after the other does (the same float weight arithmetic)."""
+    rng = np.random.default_rng(23)
+    f = 525.0 * max(width, 32) / 640
+    K = capi.intrinsics(width, height, f, f, (width - 1) / 2, (height - 1) / 2)
+    p = capi.map_params(1 << 17, 1 << 16, voxel, 3 * voxel)
+    n = 6
+    imgs, old, new = [], [], []
+
+    def pose():
+        T = np.eye(4)
+        a = rng.uniform(-0.3, 0.3)
+        T[:3, :3] = [[np.cos(a), 0, np.sin(a)], [0, 1, 0], [-np.sin(a), 0, np.cos(a)]]
+        T[:3, 3] = rng.uniform(-0.2, 0.2, 3)
+        return T
+
+    for _ in range(n):
+        patches = rng.choice([0, 500, 800, 1200, 1900, 2600, 9000], (height // 6 + 1, width // 9 + 1))
+        d16 = np.kron(patches, np.ones((6, 9), int))[:height, :width] + rng.integers(0, 4, (height, width))
+        img = capi.Image(K, 1)
+        img.upload(dev(d16.astype(np.uint16)), dev(rng.integers(0, 256, (height, width, 3)).astype(np.uint8)), 1e-3)
+        T = pose()
+        imgs.append(img)
+        old.append(dev(capi.pose24(T)))
+        T[:3, 3] += rng.uniform(-0.02, 0.02, 3)
+        new.append(dev(capi.pose24(T)))
+    base, seq, one = (capi.Map(p, max(width, 8), max(height, 8)) for _ in range(3))
+    for img, T in zip(imgs, old):
+        base.update_image(img, T)
+    base.copy_to(seq)
+    base.copy_to(one)
+    one.refuse_keyframes(imgs, old, new)
+    for img, T in zip(imgs, old):
+        seq.deintegrate_image(img, T)
+    for img, T in zip(imgs, new):
+        seq.update_image(img, T)
+    torch.cuda.synchronize()
+    bo, _, wo, _ = one.voxels()
+    bs, _, ws, _ = seq.voxels()
+    at = {tuple(b): i for i, b in enumerate(bo.tolist())}
+    assert set(map(tuple, bs.tolist())) == set(at) and (ws > 0).sum() > 50
+    assert np.array_equal(wo[[at[tuple(b)] for b in bs.tolist()]], ws)
+    for img in imgs:
+        img.close()
