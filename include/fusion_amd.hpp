@@ -112,7 +112,6 @@ private:
     LfImageLevels levels_view();
     std::vector<IntrinsicMatrix> K_;
     hipStream_t stream_;
-    int intensity_pyramid();
     GpuImage depth_raw_, image_, samples_, rendered_;
     std::vector<GpuImage> depth_, intensity_, dx_, dy_, vmap_, nmap_;
     bool half_maps_ = false;

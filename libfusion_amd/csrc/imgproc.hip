@@ -9,6 +9,7 @@
 //
 // All kernels are one lane per output pixel on 16x16 workgroups (4 wavefronts of
 // 16x4 pixels): every row segment a wavefront reads or writes is contiguous.
+#include <initializer_list>
 #include <vector>
 
 #include "lf_common.h"
@@ -237,7 +238,7 @@ __global__ void k_nmap(const float *__restrict__ vm, float *__restrict__ nm, int
 // workgroups of the parts follow each other in the 1-D grid.
 
 constexpr int kMaxParts = 3;
-enum PartKind { kFrameIn, kPyramidMaps, kLevelMaps, kVertexPyramid };
+enum PartKind { kFrameIn, kPyramidMaps, kLevelMaps, kVertexPyramid, kIntensityIn };
 
 struct Part {
     int kind, w, h, wg_begin;  // w, h: the part's output size
@@ -269,6 +270,7 @@ union TileLds {
     struct {
         float depth[kBilSide * kBilSide], grey[kBilSide * kBilSide], filtered[kTile * kTile];
     } frame;
+    float intensity[kBilSide * kBilSide];
     struct {
         float4 vert[kNrmSide * kNrmSide];
         float grey[kNrmSide * kNrmSide], src[kPyrSide * kPyrSide];
@@ -396,7 +398,7 @@ LF_DEV float4 normal_tile(const float4 *v, int side, int x, int y, int w, int h)
     return make_float4(n.x, n.y, n.z, 1.0f);
 }
 
-// kVertexPyramid for the tile at (x0, y0) of a vertex map: its normals (out0), its
+// kVertexPyramid for the tile at (x0, y0) of a vertex map: its copy (out5), its normals (out0), its
 // 8x8 half-size and 4x4 quarter-size vertices (out1, out2, as stored
 // resizes give them) and their normals (out3, out4), all from one staged window
 // with a quarter-size pixel around the tile; a neighbour outside a level's image
@@ -435,6 +437,7 @@ LF_DEV void vertex_pyramid_tile(const Part &p, int x0, int y0, TileLds &lds_all)
         lds.quarter[k] = resize4_quarter_at(full, qx, qy);
     }
     const int lx = t & 15, ly = t >> 4, x = x0 + lx, y = y0 + ly;
+    if (p.out5 && x < w && y < h) store4<false>(p.out5, (size_t)y * w + x, full(x, y));
     if (p.out0 && x < w && y < h) {
         const float4 *c = lds.full + (ly + kVtxApron) * kVtxSide + lx + kVtxApron;
         store4<kHalf>(p.out0, (size_t)y * w + x, normal_tile<kHalf>(c, kVtxSide, x, y, w, h));
@@ -470,7 +473,7 @@ LF_DEV float4 store_vertex_normal(const Part &p, const float4 *vert, int lx, int
 // kLevelMaps for the tile at (x0, y0): the vertices of the tile and a
 // one-pixel apron (coordinates clamped into the image, as nmap_at's
 // neighbours are) back-projected once into LDS.  Every load is issued ahead of
-// the barrier.
+// the barrier.  Without in0: the derivatives alone.
 template <bool kHalf>
 LF_DEV void level_maps_tile(const Part &p, int x0, int y0, TileLds &lds_all) {
     auto &lds = lds_all.maps;
@@ -486,7 +489,7 @@ LF_DEV void level_maps_tile(const Part &p, int x0, int y0, TileLds &lds_all) {
         const int k = min(t + 256 * r, kNrmSide * kNrmSide - 1);
         sx[r] = min(max(x0 - kNrmApron + k % kNrmSide, 0), w - 1);
         sy[r] = min(max(y0 - kNrmApron + k / kNrmSide, 0), h - 1);
-        z[r] = d[(size_t)sy[r] * w + sx[r]];
+        z[r] = d ? d[(size_t)sy[r] * w + sx[r]] : 0.0f;
     }
     float gx, gy;
     derivative_at(PlaneAt<kHalf>{p.in1, w}, w, h, cx, cy, gx, gy);
@@ -505,6 +508,7 @@ LF_DEV void level_maps_tile(const Part &p, int x0, int y0, TileLds &lds_all) {
     const size_t i = (size_t)y * w + x;
     store1<kHalf>(p.out0, i, gx);
     store1<kHalf>(p.out1, i, gy);
+    if (!d) return;
     const float4 n = store_vertex_normal<kHalf>(p, lds.vert, lx, ly, x, y);
     if (p.out4) static_cast<float4 *>(p.out4)[i] = integration_sample<kHalf>(dist, n, col);
 }
@@ -533,7 +537,7 @@ LF_DEV void pyramid_maps_tile(const Part &p, int x0, int y0, TileLds &lds_all) {
         const int k = min(t + 256 * r, kNrmSide * kNrmSide - 1);
         sx[r] = min(max(x0 - kNrmApron + k % kNrmSide, 0), w - 1);
         sy[r] = min(max(y0 - kNrmApron + k / kNrmSide, 0), h - 1);
-        z[r] = resize_at(static_cast<const float *>(p.in0), sw, sx[r], sy[r]);
+        z[r] = p.in0 ? resize_at(static_cast<const float *>(p.in0), sw, sx[r], sy[r]) : 0.0f;
     }
 #pragma unroll
     for (int r = 0; r < kSrcRounds; ++r)
@@ -548,7 +552,8 @@ LF_DEV void pyramid_maps_tile(const Part &p, int x0, int y0, TileLds &lds_all) {
     for (int r = 0; r < kRounds; ++r) {  // the own pixel's depth is among the staged ones
         const int k = t + 256 * r;
         const int tx = k % kNrmSide - kNrmApron, ty = k / kNrmSide - kNrmApron;
-        if (k < kNrmSide * kNrmSide && tx >= 0 && tx < kTile && ty >= 0 && ty < kTile && x0 + tx < w && y0 + ty < h)
+        if (p.in0 && k < kNrmSide * kNrmSide && tx >= 0 && tx < kTile && ty >= 0 && ty < kTile && x0 + tx < w &&
+            y0 + ty < h)
             static_cast<float *>(p.out4)[(size_t)(y0 + ty) * w + x0 + tx] = z[r];
     }
     __syncthreads();
@@ -565,7 +570,45 @@ LF_DEV void pyramid_maps_tile(const Part &p, int x0, int y0, TileLds &lds_all) {
     const bool last = x >= w - 1 || y >= h - 1;  // derivative_at's
     store1<kHalf>(p.out0, i, last ? 0.0f : (g[1] - g[-1]) * 0.5f);
     store1<kHalf>(p.out1, i, last ? 0.0f : (g[kNrmSide] - g[-kNrmSide]) * 0.5f);
-    store_vertex_normal<kHalf>(p, lds.vert, lx, ly, x, y);
+    if (p.in0) store_vertex_normal<kHalf>(p, lds.vert, lx, ly, x, y);
+}
+
+// kIntensityIn for the tile at (x0, y0): the intensity (of a colour image in0, or in1
+// itself), its derivatives and (out3) the 8x8 intensities of the next level.  FP32
+// planes.
+LF_DEV void intensity_in_tile(const Part &p, int x0, int y0, TileLds &lds) {
+    const int w = p.w, h = p.h, t = threadIdx.x;
+    const unsigned char *rgb = static_cast<const unsigned char *>(p.in0);
+    const float *grey = static_cast<const float *>(p.in1);
+#pragma unroll
+    for (int r = 0; r < (kBilSide * kBilSide + 255) / 256; ++r) {
+        const int k = t + 256 * r;
+        if (k >= kBilSide * kBilSide) break;
+        const int sx = reflect101(x0 - kBilApron + k % kBilSide, w), sy = reflect101(y0 - kBilApron + k / kBilSide, h);
+        const size_t i = (size_t)sy * w + sx;
+        float v;
+        if (rgb) {
+            const unsigned int c = rgb_at(rgb, i, w * h == 1);
+            v = grey_of((unsigned char)c, (unsigned char)(c >> 8), (unsigned char)(c >> 16));
+        } else {
+            v = grey[i];
+        }
+        lds.intensity[k] = v;
+    }
+    __syncthreads();
+    const int lx = t & 15, ly = t >> 4, x = x0 + lx, y = y0 + ly;
+    if (x < w && y < h) {
+        const size_t i = (size_t)y * w + x;
+        const float *g = lds.intensity + (ly + kBilApron) * kBilSide + lx + kBilApron;
+        static_cast<float *>(p.out0)[i] = g[0];
+        const bool last = x >= w - 1 || y >= h - 1;  // derivative_at's borders, not the staged reflection
+        static_cast<float *>(p.out1)[i] = last ? 0.0f : (g[1] - g[x > 0 ? -1 : 0]) * 0.5f;
+        static_cast<float *>(p.out2)[i] = last ? 0.0f : (g[kBilSide] - g[y > 0 ? -kBilSide : 0]) * 0.5f;
+    }
+    const int hx = t & 7, hy = t >> 3;
+    if (!p.out3 || t >= 64 || x0 / 2 + hx >= w / 2 || y0 / 2 + hy >= h / 2) return;
+    static_cast<float *>(p.out3)[(size_t)(y0 / 2 + hy) * (w / 2) + x0 / 2 + hx] =
+        pyr_down_window(lds.intensity + 2 * hy * kBilSide + 2 * hx, kBilSide);
 }
 
 // Part p's workgroup t (the tile it covers); every lane reaches the part's
@@ -589,6 +632,10 @@ LF_DEV void part_wg(const Part &p, int t, TileLds &lds) {
     if (p.kind == kVertexPyramid) {
         if (p.half) vertex_pyramid_tile<true>(p, x0, y0, lds);
         else vertex_pyramid_tile<false>(p, x0, y0, lds);
+        return;
+    }
+    if (p.kind == kIntensityIn) {
+        intensity_in_tile(p, x0, y0, lds);
         return;
     }
     if (p.kind == kPyramidMaps) {
@@ -723,13 +770,21 @@ int plan_upload(const uint16_t *depth_u16, const unsigned char *rgb, float depth
 // DeviceImage::resize_device_map: the vertex pyramid of a raycast level-0 map
 // and every level's normals, three levels in the first pass, two in each after it
 // (base level b is the coarsest that the pass before wrote).
-int plan_refresh(int levels, const lf_intrinsics *K, const LfImageLevels &m, std::vector<Pass> &out) {
+// vmap: the level-0 map where it isn't m.vmap[0] already, copied there.
+int plan_refresh(int levels, const lf_intrinsics *K, const LfImageLevels &m, std::vector<Pass> &out,
+                 const float *vmap = nullptr) {
     if (int rc = check_pyramid(levels, K)) return rc;
     for (int b = 0; b == 0 || b + 1 < levels; b += 2) {
         Pass ps = {};
         Part p = make_part(kVertexPyramid, K[b].width, K[b].height);
         p.in0 = m.vmap[b];
-        if (b == 0) p.out0 = m.nmap[b];
+        if (b == 0) {
+            p.out0 = m.nmap[b];
+            if (vmap && vmap != m.vmap[b]) {
+                p.in0 = vmap;
+                p.out5 = m.vmap[b];
+            }
+        }
         if (b + 1 < levels) {
             p.out1 = m.vmap[b + 1]; p.out3 = m.nmap[b + 1];
         }
@@ -740,6 +795,36 @@ int plan_refresh(int levels, const lf_intrinsics *K, const LfImageLevels &m, std
         seal_pass(ps, m.half_maps);
         out.push_back(ps);
     }
+    return LF_OK;
+}
+
+// The intensity pyramid of a colour image or an intensity plane with its derivatives:
+// two levels' intensities and the first's derivatives in one pass, the second's
+// derivatives and the third level in the next, then a pass a level.
+int plan_intensity(const unsigned char *rgb, const float *intensity, int levels, const lf_intrinsics *K,
+                   const LfImageLevels &m, std::vector<Pass> &out) {
+    if (int rc = check_pyramid(levels, K)) return rc;
+    const auto add_pass = [&](std::initializer_list<Part> parts) {
+        Pass ps = {};
+        for (const Part &p : parts) ps.part[ps.nparts++] = p;
+        seal_pass(ps, 0);
+        out.push_back(ps);
+    };
+    const auto derivatives = [&](int kind, int l) {
+        Part p = make_part(kind, K[l].width, K[l].height);
+        p.in1 = m.intensity[kind == kPyramidMaps ? l - 1 : l];
+        p.out0 = m.dx[l]; p.out1 = m.dy[l];
+        if (kind == kPyramidMaps) p.out5 = m.intensity[l];
+        return p;
+    };
+    Part f = make_part(kIntensityIn, K[0].width, K[0].height);
+    f.in0 = rgb; f.in1 = intensity;
+    f.out0 = m.intensity[0]; f.out1 = m.dx[0]; f.out2 = m.dy[0];
+    if (levels > 1) f.out3 = m.intensity[1];
+    add_pass({f});
+    if (levels == 2) add_pass({derivatives(kLevelMaps, 1)});
+    if (levels > 2) add_pass({derivatives(kPyramidMaps, 2), derivatives(kLevelMaps, 1)});
+    for (int l = 3; l < levels; ++l) add_pass({derivatives(kPyramidMaps, l)});
     return LF_OK;
 }
 
@@ -763,9 +848,17 @@ int lf_pyramid_upload(const uint16_t *depth_u16, const unsigned char *rgb, float
     return launch_all(passes, st);
 }
 
-int lf_pyramid_refresh(int levels, const lf_intrinsics *K, const LfImageLevels &m, hipStream_t st) {
+int lf_pyramid_refresh(int levels, const lf_intrinsics *K, const LfImageLevels &m, hipStream_t st, const float *vmap) {
     std::vector<Pass> passes;
-    if (int rc = plan_refresh(levels, K, m, passes)) return rc;
+    if (int rc = plan_refresh(levels, K, m, passes, vmap)) return rc;
+    return launch_all(passes, st);
+}
+
+int lf_pyramid_intensity(const unsigned char *rgb, const float *intensity, int levels, const lf_intrinsics *K,
+                         const LfImageLevels &m, hipStream_t st) {
+    if (!rgb && !intensity) return lf_set_error(LF_ERR_ARG, "null intensity");
+    std::vector<Pass> passes;
+    if (int rc = plan_intensity(rgb, intensity, levels, K, m, passes)) return rc;
     return launch_all(passes, st);
 }
 

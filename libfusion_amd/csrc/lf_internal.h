@@ -49,8 +49,14 @@ struct LfImageLevels {
 int lf_pyramid_upload(const uint16_t *depth_u16, const unsigned char *rgb, float depth_scale, int levels,
                     const lf_intrinsics *K, const LfImageLevels &m, hipStream_t st);
 // DeviceImage::resize_device_map (device_image.cpp:188-199): vertex pyramid of
-// vmap[0] and the normals of every level, in max(1, levels / 2) launches.
-int lf_pyramid_refresh(int levels, const lf_intrinsics *K, const LfImageLevels &m, hipStream_t st);
+// vmap[0] and the normals of every level, in max(1, levels / 2) launches.  vmap
+// (or null): a level-0 map to take for vmap[0], copied there.
+int lf_pyramid_refresh(int levels, const lf_intrinsics *K, const LfImageLevels &m, hipStream_t st,
+                       const float *vmap = nullptr);
+// The intensity pyramid of a colour image (rgb), or of an intensity plane, and
+// its derivatives in max(1, levels - 1) launches; FP32 planes.
+int lf_pyramid_intensity(const unsigned char *rgb, const float *intensity, int levels, const lf_intrinsics *K,
+                         const LfImageLevels &m, hipStream_t st);
 
 // The same passes planned instead of launched, for a batch of images: each
 // pass is an lf_pass_bytes() device descriptor appended to out, and pass p of

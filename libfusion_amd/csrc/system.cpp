@@ -237,35 +237,27 @@ const GpuImage &DeviceImage::get_rendered_scene_textured() {
 int DeviceImage::set_vmap(const float *vmap) {
     if (!vmap) return lf_set_error(LF_ERR_ARG, "null vertex map");
     if (half_maps_) return lf_set_error(LF_ERR_ARG, "set_vmap takes FP32 images only");
-    const size_t n = (size_t)K_[0].width * K_[0].height;
-    LF_HIP_CHECK(hipMemcpyAsync(vmap_[0].ptr<float>(), vmap, n * 16, hipMemcpyDeviceToDevice, stream_));
-    return resize_device_map();
-}
-
-int DeviceImage::intensity_pyramid() {
-    void *st = stream_;
-    for (int l = 1; l < levels(); ++l)
-        LF_RC(lf_pyr_down_image(intensity_[l - 1].ptr<float>(), intensity_[l].ptr<float>(), K_[l - 1].width,
-                                K_[l - 1].height, st));
-    for (int l = 0; l < levels(); ++l)
-        LF_RC(lf_compute_derivative(intensity_[l].ptr<float>(), dx_[l].ptr<float>(), dy_[l].ptr<float>(),
-                                    K_[l].width, K_[l].height, st));
-    return LF_OK;
+    if (reinterpret_cast<uintptr_t>(vmap) % 16 != 0) {  // the passes read whole vertices
+        const size_t n = (size_t)K_[0].width * K_[0].height;
+        LF_HIP_CHECK(hipMemcpyAsync(vmap_[0].ptr<float>(), vmap, n * 16, hipMemcpyDeviceToDevice, stream_));
+        return resize_device_map();
+    }
+    std::vector<lf_intrinsics> K(K_.begin(), K_.end());
+    return lf_pyramid_refresh(levels(), K.data(), levels_view(), stream_, vmap);
 }
 
 int DeviceImage::set_intensity(const float *intensity) {
     if (!intensity) return lf_set_error(LF_ERR_ARG, "null intensity");
     if (half_maps_) return lf_set_error(LF_ERR_ARG, "set_intensity takes FP32 images only");
-    const size_t n = (size_t)K_[0].width * K_[0].height;
-    LF_HIP_CHECK(hipMemcpyAsync(intensity_[0].ptr<float>(), intensity, n * 4, hipMemcpyDeviceToDevice, stream_));
-    return intensity_pyramid();
+    std::vector<lf_intrinsics> K(K_.begin(), K_.end());
+    return lf_pyramid_intensity(nullptr, intensity, levels(), K.data(), levels_view(), stream_);
 }
 
 int DeviceImage::set_image(const unsigned char *rgb) {
     if (!rgb) return lf_set_error(LF_ERR_ARG, "null image");
     if (half_maps_) return lf_set_error(LF_ERR_ARG, "set_image takes FP32 images only");
-    LF_RC(lf_rgb_to_intensity(rgb, intensity_[0].ptr<float>(), K_[0].width, K_[0].height, stream_));
-    return intensity_pyramid();
+    std::vector<lf_intrinsics> K(K_.begin(), K_.end());
+    return lf_pyramid_intensity(rgb, nullptr, levels(), K.data(), levels_view(), stream_);
 }
 
 int DeviceImage::set_depth(const float *depth) {

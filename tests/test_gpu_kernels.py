@@ -587,3 +587,56 @@ def test_refusion_with_occlusions(width, height, voxel):
     assert np.array_equal(wo[[at[tuple(b)] for b in bs.tolist()]], ws)
     for img in imgs:
         img.close()
+
+
+@pytest.mark.parametrize("width,height,levels", [(1, 1, 1), (37, 5, 1), (2, 2, 2), (46, 18, 2), (4, 4, 3),
+                                                 (72, 40, 3), (160, 96, 6)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_tracker_planes(width, height, levels, offset):
+    """set_*_image, set_*_intensity and set_*_vmap store what the operations one at a time give, bit for bit, from
+    planes at unaligned addresses too (offset floats, or bytes, into their buffer)."""
+    rng = np.random.default_rng(7)
+    lib, st, P = capi.load(), capi.stream_ptr(), capi.ptr
+    f = 525.0 * width / 640
+    tr = capi.Tracker(capi.intrinsics(width, height, f, f, (width - 1) / 2, (height - 1) / 2), levels)
+    n = width * height
+    rgb = dev(rng.integers(0, 256, 3 * n + offset).astype(np.uint8))[offset:]
+    grey = dev(rng.uniform(0, 255, n + offset).astype(np.float32))[offset:]
+    vmap = dev(rng.uniform(-1, 4, 4 * n + offset).astype(np.float32))[offset:]
+
+    def same(source, l, which, ref):
+        out = ctypes.c_void_p()
+        capi.check(lib.lf_tracker_plane(tr.h, source, l, which, ctypes.byref(out)))
+        t = torch.empty_like(ref)
+        capi.copy_device(t, out.value, t.numel() * t.element_size())
+        assert np.array_equal(t.cpu().numpy(), ref.cpu().numpy(), equal_nan=True), (source, l, which)
+
+    tr.set("set_source_image", rgb)
+    tr.set("set_reference_intensity", grey)
+    tr.set("set_reference_vmap", vmap)
+    first = torch.empty(height, width, device="cuda")
+    capi.check(lib.lf_rgb_to_intensity(P(rgb), P(first), width, height, st))
+    for source, plane in ((1, first), (0, grey.view(height, width).clone())):
+        for l in range(levels):
+            w, h = tr.K[l].width, tr.K[l].height
+            if l:
+                half = torch.empty(h, w, device="cuda")
+                capi.check(lib.lf_pyr_down_image(P(plane), P(half), 2 * w, 2 * h, st))
+                plane = half
+            dx, dy = torch.empty_like(plane), torch.empty_like(plane)
+            capi.check(lib.lf_compute_derivative(P(plane), P(dx), P(dy), w, h, st))
+            for which, ref in ((capi.PLANE_INTENSITY, plane), (capi.PLANE_DX, dx), (capi.PLANE_DY, dy)):
+                if source or which == capi.PLANE_INTENSITY:
+                    same(source, l, which, ref)
+    v = vmap.view(height, width, 4).clone()
+    for l in range(levels):
+        w, h = tr.K[l].width, tr.K[l].height
+        if l:
+            half = torch.empty(h, w, 4, device="cuda")
+            capi.check(lib.lf_pyr_down_vmap(P(v), P(half), 2 * w, 2 * h, st))
+            v = half
+        nm = torch.empty_like(v)
+        capi.check(lib.lf_compute_nmap(P(v), P(nm), w, h, st))
+        same(0, l, capi.PLANE_VMAP, v)
+        same(0, l, capi.PLANE_NMAP, nm)
+    tr.close()
