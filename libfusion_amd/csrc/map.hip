@@ -509,12 +509,14 @@ LF_DEV void fill_weight_table(float *s) {
 // this function fills (every thread of the workgroup calls it).
 // Workgroup wg of nwg (grid-stride over the visible list).
 // Bound by the voxels' bytes with packed samples (a 640x480 frame, 5 mm, FP32:
-// 238 MB in 53 us; mixed at 848x480, 4 mm: 215 MB in 48 us).  With separate
+// 238 MB in 53 us; mixed at 848x480, 4 mm: 215 MB in 46 us).  With separate
 // planes by the gathers (three a voxel) and the arithmetic: the projection's two
 // quotients share one refined reciprocal, the update's four another, a colour and
 // a normal are one load each (645x483, 5 mm: 74.6 us with divisions and scalar
-// loads, 71.0 now; take-out, a voxel at a time with its loads in sequence before,
-// 89.8, now 71.5).
+// loads, 68.3 now; take-out, a voxel at a time with its loads in sequence before,
+// 89.8, now 70.2).  Many mixed maps by the vector instructions: 16 of 640x480, 5 mm,
+// 539 us with the low weight codes and the colours' clamps computed for all, 524 now
+// (one of 848x480, 4 mm, 48.3 -> 46.1).
 template <bool kWeighted, bool kColour, bool kPacked, bool kMixed, bool kTable = false, bool kTakeOut = false>
 LF_DEV void integrate_wg(const MapDev &m, const float *__restrict__ depth, const float *__restrict__ nmap,
                          const unsigned char *__restrict__ rgb, int cols, int rows, const float *__restrict__ pose24,
@@ -597,8 +599,17 @@ LF_DEV void integrate_wg(const MapDev &m, const float *__restrict__ depth, const
                 tu = quotient(K.fx * pt.x, iz) + K.cx + 0.5f;
                 tv = quotient(K.fy * pt.y, iz) + K.cy + 0.5f;
             }
-            ok[h] = tu >= 0.0f && tu < fcols && tv >= 0.0f && tv < frows;
-            pix[h] = ok[h] ? __umul24((unsigned int)tv, (unsigned int)cols) + (unsigned int)tu : 0u;
+            // The tests are one mask in FP32 and short-circuited in mixed
+            // precision, here and below: the other way round, 645x483 FP32
+            // takes 71.0 us, not 68.3, 16 mixed maps 567, not 524.
+            if constexpr (kMixed) {
+                ok[h] = tu >= 0.0f && tu < fcols && tv >= 0.0f && tv < frows;
+                pix[h] = ok[h] ? __umul24((unsigned int)tv, (unsigned int)cols) + (unsigned int)tu : 0u;
+            } else {
+                ok[h] = (tu >= 0.0f) & (tu < fcols) & (tv >= 0.0f) & (tv < frows);
+                const unsigned int at = __umul24((unsigned int)tv, (unsigned int)cols) + (unsigned int)tu;
+                pix[h] = ok[h] ? at : 0u;
+            }
             ptz[h] = pt.z;
             dist[h] = 0.0f; nz[h] = 0.0f; wpk[h] = 0.0f; cpk[h] = 0u;
         }
@@ -643,11 +654,18 @@ LF_DEV void integrate_wg(const MapDev &m, const float *__restrict__ depth, const
         for (int h = 0; h < 2; ++h) {
             const float d = dist[h];
             bool in = ok[h];
-            if (kPacked) in = in && !(isnan(d) || d > zmax || d < zmin);
-            else if (kWeighted) in = in && !(isnan(d) || isnan(nx[h]) || d > zmax || d < zmin);
-            else in = in && !(isnan(d) || (double)d < 1e-2 || d > zmax || d < zmin);
-            sdf[h] = d - ptz[h];
-            in = in && !(sdf[h] < -trunc);
+            if constexpr (kMixed) {
+                if (kPacked) in = in && !(isnan(d) || d > zmax || d < zmin);
+                else if (kWeighted) in = in && !(isnan(d) || isnan(nx[h]) || d > zmax || d < zmin);
+                else in = in && !(isnan(d) || (double)d < 1e-2 || d > zmax || d < zmin);
+                sdf[h] = d - ptz[h];
+                in = in && !(sdf[h] < -trunc);
+            } else {
+                sdf[h] = d - ptz[h];
+                in = in & !(d > zmax) & !(d < zmin) & (sdf[h] >= -trunc);  // a NaN depth fails the last
+                if (!kPacked && kWeighted) in = in & !isnan(nx[h]);
+                if (!kWeighted) in = in & !((double)d < 1e-2);
+            }
             ok[h] = in;
             if constexpr (!kMixed) {
                 const unsigned int o = in ? vo[h] : 0u;
@@ -691,7 +709,8 @@ LF_DEV void integrate_wg(const MapDev &m, const float *__restrict__ depth, const
                     // a first observation with a positive weight is seen, as in
                     // the reference (the smallest code stands for weights below
                     // it); a zero weight leaves the voxel unseen
-                    const unsigned int code = wt > 0.0f ? max(1u, weight_code_sr(fminf(wt, 255.0f), rnd)) : 0u;
+                    const unsigned int code =
+                        wt > 0.0f ? max(1u, weight_code_sr_in_range(fminf(wt, 255.0f), rnd)) : 0u;
                     at_byte(sdf16, vgpr_offset(2u * o)) = code == 0u ? kHalfUnseen : float_to_half_bits(sdf_h);
                     if (kColour) colour = word_colour_bits(cin[0], cin[1], cin[2]);
                     at_byte(wd_b, vgpr_offset(4u * o)) = code | colour;
@@ -700,15 +719,13 @@ LF_DEV void integrate_wg(const MapDev &m, const float *__restrict__ depth, const
                 const float inv = __builtin_amdgcn_rcpf(wp[h] + wt);
                 const float spf = half_bits_to_float((unsigned short)sp[h]);
                 at_byte(sdf16, vgpr_offset(2u * o)) = float_to_half_bits((spf * wp[h] + sdf_h * wt) * inv);
-                const unsigned int code = weight_code_sr(fminf(wp[h] + wt, 255.0f), rnd);
+                const unsigned int code = weight_code_sr_in_range(fminf(wp[h] + wt, 255.0f), rnd);
                 if (kColour) {
-                    unsigned int ch[3];
+                    float mc[3];
 #pragma unroll
-                    for (int k = 0; k < 3; ++k) {
-                        const float mc = ((float)word_channel(word[h], k) * wp[h] + (float)cin[k] * wt) * inv;
-                        ch[k] = (unsigned int)(int)fminf(mc, 255.0f);
-                    }
-                    colour = word_colour_bits(ch[0], ch[1], ch[2]);
+                    for (int k = 0; k < 3; ++k)
+                        mc[k] = ((float)word_channel(word[h], k) * wp[h] + (float)cin[k] * wt) * inv;
+                    colour = word_colour_of(mc[0], mc[1], mc[2]);
                 }
                 at_byte(wd_b, vgpr_offset(4u * o)) = code | colour;
                 continue;

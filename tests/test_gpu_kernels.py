@@ -640,3 +640,67 @@ def test_tracker_planes(width, height, levels, offset):
         same(0, l, capi.PLANE_VMAP, v)
         same(0, l, capi.PLANE_NMAP, nm)
     tr.close()
+
+
+# none, far below the first normal code's 2^-6, on both sides of it, ordinary, large
+@pytest.mark.parametrize("weight", [0.0, 3e-4, 0.0155, 0.0157, 0.5, 6.0])
+def test_mixed_weights_and_colours(weight):
+    """A mixed map's words after two frames of one depth, weight and colour each: the weight codes are
+    lf_weight_code_dither of the summed weights with the voxel's random bits (but for the sum's last bit: one code at a
+    few voxels), the colours the truncated means (one level either side, by the mean's rounding)."""
+    rng = np.random.default_rng(2)
+    width, height, d = 40, 30, np.float32(0.4)
+    K = capi.intrinsics(width, height, 40.0, 40.0, (width - 1) / 2, (height - 1) / 2)
+    p = capi.map_params(1 << 12, 1 << 12, 0.01, 0.03, precision=MIXED)
+    m = capi.Map(p, width, height)
+    pose = dev(capi.pose24(np.eye(4)))
+    lib = capi.load()
+    value = lambda c: c / 1024 if c < 16 else (1 + (c & 15) / 16) * 2.0 ** ((c >> 4) - 7)  # noqa: E731
+    values = np.array([value(c) for c in range(256)], np.float32)
+
+    def words():
+        n = int(m.counters()[capi.CNT_ALLOCATED])
+        w = m.t["weight"][: 512 * n].view(n, 512).cpu().numpy().view(np.uint32)
+        return m.blocks().astype(np.int64), w & 0xFF, np.stack([w >> (8 + 8 * k) & 0xFF for k in range(3)], -1)
+
+    def fuse(wt, rgb):
+        nmap = np.zeros((height, width, 4), np.float32)
+        nmap[..., 2] = np.arcsin(np.float64(wt) * np.float64(d) ** 2)
+        m.update_weighted(dev(np.full((height, width), d)), dev(nmap),
+                          dev(np.full((height, width, 3), rgb, np.uint8)), pose, K)
+        torch.cuda.synchronize()
+
+    def random_bits(blocks, i, l):
+        x, y, z = (blocks[i, k] * c & 0xFFFFFFFF for k, c in enumerate((0x9E3779B1, 0x85EBCA77, 0xC2B2AE3D)))
+        r = x ^ y ^ z ^ ((l + (int(m.counters()[8]) << 9)) * 0x27D4EB2F & 0xFFFFFFFF)
+        r ^= r >> 16
+        r = r * 0x7FEB352D & 0xFFFFFFFF
+        r ^= r >> 15
+        r = r * 0x846CA68B & 0xFFFFFFFF
+        return r ^ r >> 16
+
+    def check(at, codes, sums):
+        blocks, i, l = at
+        want = np.array([lib.lf_weight_code_dither(float(s), int(r))
+                         for s, r in zip(sums, random_bits(blocks, i, l))])
+        off = np.abs(codes[i, l].astype(int) - np.maximum(want, 1))
+        assert off.max() <= 1 and (off > 0).mean() < 0.01, (off.max(), (off > 0).mean())
+
+    first, second, wt2 = rng.integers(0, 256, 3), rng.integers(0, 256, 3), np.float32(0.3)
+    fuse(weight, first)
+    blocks, c1, col1 = words()
+    if weight == 0.0:
+        assert not c1.any()
+        fuse(wt2, second)
+        blocks, c1, col1 = words()
+        first, weight = second, wt2
+    i, l = np.nonzero(c1)
+    assert len(i) > 5000 and (col1[i, l] == first).all()
+    check((blocks, i, l), c1, np.full(len(i), np.float32(weight)))
+    fuse(wt2, second)
+    again, c2, col2 = words()
+    assert np.array_equal(again[: len(blocks)], blocks)
+    w1 = values[c1[i, l]]
+    check((again, i, l), c2, np.minimum(w1 + wt2, np.float32(255)))
+    mean = (w1[:, None].astype(np.float64) * first + np.float64(wt2) * second) / (w1[:, None].astype(np.float64) + wt2)
+    assert np.all(np.abs(col2[i, l] - np.floor(mean)) <= 1)
