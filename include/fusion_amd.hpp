@@ -15,6 +15,7 @@
 #include <hip/hip_runtime.h>
 
 #include <memory>
+#include <mutex>
 #include <string>
 #include <utility>
 #include <vector>
@@ -210,6 +211,12 @@ public:
     LfTrackState *state() const { return state_; }
     // Synchronising read of the last result (update = estimate^-1).
     TrackingResult result();
+    TrackingResult result_of(const LfTrackState &state) const;
+    // The state after the work enqueued on this tracker's stream (synchronising;
+    // several threads may read).  copy_state: by a copy beside the kernels of other
+    // streams, which does not wait for those (a Batch's steps: synchronise it first).
+    int read_state(LfTrackState &out);
+    int copy_state(LfTrackState &out) const;
     // Synchronising read of the last Gauss-Newton step's FP64 sums (31 values).
     int read_sums(double *sums31);
     float icp_weight = 1e6f;  // icp_tracker.cpp:89-90
@@ -219,6 +226,8 @@ private:
                 std::vector<unsigned char> *jobs = nullptr, std::vector<int> *grids = nullptr);
     hipStream_t stream_;
     LfTrackState *state_ = nullptr;
+    LfTrackState *state_host_ = nullptr;  // pinned: read_state's kernel writes it
+    std::mutex read_;
     float *scratch_ = nullptr;
     bool context_mode_ = false;
     int batch_share_ = 1;

@@ -639,8 +639,9 @@ int lf_batch_tuning(lf_batch *b);
 /* Read tuned choices from path (lines "<shape> <values>", later lines win) and
  * append new ones to it; null or "" stops using a file. */
 int lf_batch_tune_file(const char *path);
-/* System i's camera pose (4x4 row-major doubles; synchronising), last
- * tracking result and map counters. */
+/* System i's camera pose (4x4 row-major doubles), last tracking result and map
+ * counters: those of the steps done so far, so lf_batch_synchronize first for
+ * those of the steps processed. */
 int lf_batch_get_pose(lf_batch *b, int i, double *out16);
 int lf_batch_get_tracking(lf_batch *b, int i, int *success, float *icp_error);
 int lf_batch_read_counters(lf_batch *b, int i, unsigned int *out16);

@@ -77,6 +77,8 @@ int lf_track_begin(LfTrackState *st, const double *T12, hipStream_t stream);
 int lf_track_finish(LfTrackState *st, hipStream_t stream);
 // Set the odometry pose directly (first frame / restart): T given as 3x4 doubles (host).
 int lf_track_set_pose(LfTrackState *st, const double *T12, hipStream_t stream);
+// The state into pinned host memory (there once the stream has come this far).
+int lf_track_read(const LfTrackState *st, LfTrackState *host, hipStream_t stream);
 
 // Batched tracking: one step of several systems in one launch.  A job is
 // the launch arguments of one system's step (lf_track_job_bytes each);

@@ -339,6 +339,9 @@ size_t DenseMapping::fetch_mesh_with_colour(float *vertex, unsigned char *colour
 DenseTracking::DenseTracking(hipStream_t stream) : stream_(stream) {
     if (hipMalloc(&state_, sizeof(LfTrackState)) != hipSuccess) throw std::bad_alloc();
     if (hipMalloc(&scratch_, lf_track_scratch_floats() * sizeof(float)) != hipSuccess) throw std::bad_alloc();
+    void *pinned = nullptr;
+    if (hipHostMalloc(&pinned, sizeof(LfTrackState), hipHostMallocDefault) != hipSuccess) throw std::bad_alloc();
+    state_host_ = static_cast<LfTrackState *>(pinned);
     // every field defined before the first frame (errors 0, success 0, counts 0)
     if (hipMemsetAsync(state_, 0, sizeof(LfTrackState), stream_) != hipSuccess)
         throw std::runtime_error("hipMemsetAsync failed");
@@ -365,6 +368,7 @@ int DenseTracking::compute_transform(const TrackingContext &c) {
 DenseTracking::~DenseTracking() {
     (void)hipFree(state_);
     (void)hipFree(scratch_);
+    (void)hipHostFree(state_host_);
 }
 
 // compute_transform(ref, cur, ctx) (icp_tracker.cpp:23-156): levels coarse to
@@ -433,16 +437,32 @@ int DenseTracking::enqueue(DeviceImage &ref, DeviceImage &cur, const TrackingCon
     return LF_OK;
 }
 
-TrackingResult DenseTracking::result() {
-    LfTrackState h;
+int DenseTracking::read_state(LfTrackState &out) {
+    std::lock_guard<std::mutex> lock(read_);
+    LF_RC(lf_track_read(state_, state_host_, stream_));
+    LF_HIP_CHECK(hipStreamSynchronize(stream_));
+    out = *state_host_;
+    return LF_OK;
+}
+
+int DenseTracking::copy_state(LfTrackState &out) const {
+    LF_HIP_CHECK(hipMemcpyAsync(&out, state_, sizeof(out), hipMemcpyDeviceToHost, stream_));
+    LF_HIP_CHECK(hipStreamSynchronize(stream_));
+    return LF_OK;
+}
+
+TrackingResult DenseTracking::result_of(const LfTrackState &h) const {
     TrackingResult r;
-    if (hipMemcpyAsync(&h, state_, sizeof(h), hipMemcpyDeviceToHost, stream_) != hipSuccess) return r;
-    if (hipStreamSynchronize(stream_) != hipSuccess) return r;
     r.sucess = h.success != 0;
     // compute_transform(ctx) reports last_icp_error (icp_tracker.cpp:310)
     r.icp_error = context_mode_ ? h.gn.last_icp_error : h.gn.icp_error;
     r.update = r.sucess ? SE3d::from3x4(h.gn.est).inverse() : SE3d();
     return r;
+}
+
+TrackingResult DenseTracking::result() {
+    LfTrackState h;
+    return read_state(h) == LF_OK ? result_of(h) : TrackingResult();
 }
 
 int DenseTracking::read_sums(double *sums31) {
@@ -1290,6 +1310,12 @@ int System::writeMapToDisk(const std::string &file_name) { return mapping_->writ
 
 int System::readMapFromDisk(const std::string &file_name) { return mapping_->readMapFromDisk(file_name); }
 
+static void pose_of(const LfTrackState &state, double *out16) {
+    for (int i = 0; i < 12; ++i) out16[i] = state.pose[i];
+    out16[12] = out16[13] = out16[14] = 0;
+    out16[15] = 1;
+}
+
 int System::restart() {  // system.cpp:148-157
     double T[16];
     LF_RC(get_camera_pose(T));
@@ -1311,11 +1337,8 @@ size_t System::fetch_mesh_with_colour(float *v, unsigned char *c, int max_tri) {
 
 int System::get_camera_pose(double *out16) {
     LfTrackState h;
-    LF_HIP_CHECK(hipMemcpyAsync(&h, odometry_->tracker().state(), sizeof(h), hipMemcpyDeviceToHost, stream_));
-    LF_HIP_CHECK(hipStreamSynchronize(stream_));
-    for (int i = 0; i < 12; ++i) out16[i] = h.pose[i];
-    out16[12] = out16[13] = out16[14] = 0;
-    out16[15] = 1;
+    LF_RC(odometry_->tracker().read_state(h));
+    pose_of(h, out16);
     return LF_OK;
 }
 
@@ -1742,12 +1765,17 @@ static int batch_index(lf_batch *b, int i) {
 extern "C" int lf_batch_get_pose(lf_batch *b, int i, double *out16) {
     if (int rc = batch_index(b, i)) return rc;
     if (!out16) return lf_set_error(LF_ERR_ARG, "null pose output");
-    return b->b->system(i).get_camera_pose(out16);
+    LfTrackState h;
+    LF_RC(b->b->system(i).odometry().tracker().copy_state(h));
+    fusion::pose_of(h, out16);
+    return LF_OK;
 }
 
 extern "C" int lf_batch_get_tracking(lf_batch *b, int i, int *success, float *icp_error) {
     if (int rc = batch_index(b, i)) return rc;
-    fusion::TrackingResult r = b->b->system(i).odometry().tracker().result();
+    const fusion::DenseTracking &t = b->b->system(i).odometry().tracker();
+    LfTrackState h;
+    const fusion::TrackingResult r = t.copy_state(h) == LF_OK ? t.result_of(h) : fusion::TrackingResult();
     if (success) *success = r.sucess ? 1 : 0;
     if (icp_error) *icp_error = r.icp_error;
     return LF_OK;

@@ -704,3 +704,20 @@ def test_mixed_weights_and_colours(weight):
     check((again, i, l), c2, np.minimum(w1 + wt2, np.float32(255)))
     mean = (w1[:, None].astype(np.float64) * first + np.float64(wt2) * second) / (w1[:, None].astype(np.float64) + wt2)
     assert np.all(np.abs(col2[i, l] - np.floor(mean)) <= 1)
+
+
+def test_state_reads_from_several_threads():
+    """A System's pose and tracking result, read by threads at once beside the frames enqueued, are the serial reads'."""
+    from concurrent.futures import ThreadPoolExecutor
+    rng = np.random.default_rng(1)
+    K = capi.intrinsics(64, 48, 52.5, 52.5, 31.5, 23.5)
+    s = capi.System(K, capi.map_params(1 << 12, 1 << 12, 0.02, 0.06), 2, (3, 2), 1e-3)
+    u, v = np.meshgrid(np.linspace(0, 6, 64), np.linspace(0, 4, 48))
+    for f in range(3):
+        d16 = (1000 + 150 * np.sin(u + 0.01 * f) * np.cos(v)).astype(np.uint16)
+        s.process(dev(d16), dev(rng.integers(0, 256, (48, 64, 3)).astype(np.uint8)))
+        with ThreadPoolExecutor(4) as pool:
+            poses = list(pool.map(lambda _: s.pose(), range(8)))
+            results = list(pool.map(lambda _: s.tracking(), range(8)))
+        assert all(np.array_equal(p, s.pose()) for p in poses)
+        assert all(r == s.tracking() for r in results)
