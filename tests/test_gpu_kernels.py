@@ -720,4 +720,4 @@ def test_state_reads_from_several_threads():
             poses = list(pool.map(lambda _: s.pose(), range(8)))
             results = list(pool.map(lambda _: s.tracking(), range(8)))
         assert all(np.array_equal(p, s.pose()) for p in poses)
-        assert all(r == s.tracking() for r in results)
+        assert all(np.array_equal(r, s.tracking(), equal_nan=True) for r in results)  # a lost frame has no error
