@@ -357,7 +357,7 @@ private:
 // system's frame, pass p of all systems in one launch, on an upload stream
 // that overlaps the previous step's fusion and raycast; runs the Gauss-Newton
 // steps of all systems on the batch's stream, step s of every system in one
-// launch pair; fuses each map on its own stream; runs one batched z-range +
+// launch; fuses each map on its own stream; runs one batched z-range +
 // raycast launch per stage for all maps; then the re-pyramids, again one
 // launch per pass for all systems.  The batched launches replace 2 x 18 tracking
 // launches and 6 pyramid launches per system and pack the raycasts' long-ray

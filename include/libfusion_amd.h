@@ -558,7 +558,7 @@ int lf_system_read_timing(lf_system *sys, int stage, int *launches, double *tota
  * sizes may differ).  lf_batch_process takes one frame per system (device
  * pointers, uint16 depth and uint8 RGB of system i's size): pass p of every
  * system's image pyramid runs in one launch, Gauss-Newton step s of every
- * system in one launch pair, each map is fused on its own stream, then one
+ * system in one launch, each map is fused on its own stream, then one
  * batched z-range + raycast launch per stage covers every map, then the
  * re-pyramids.  All systems share one precision (LF_ERR_ARG otherwise).  The
  * tracking reductions of n systems take 1/n of a lone system's grid each, so
