@@ -565,6 +565,18 @@ LF_DEV void march(const RayDev &r, BlockCache &bc, f3 &res, const f3 dir2, float
     }
 }
 
+// Workgroup tiles in a row that one XCD takes: an eighth of the image where all its
+// workgroups are resident at once (8 of 4 wavefronts on each of 256 CUs), as each
+// L2 then holds a band of the volume; above that, as the bands' unequal work adds up,
+// 4 in turn.  640x480 (1200 workgroups): 86.3 us by bands, 89.5 in turn; 1280x960
+// (4800): 182.5 and 170.0.
+LF_HD int xcd_chunk(int nwg) { return nwg > 2048 ? 4 : (nwg + kXcds - 1) / kXcds; }
+// Workgroups to launch for nwg: whole rounds of chunks.
+LF_HD int xcd_grid(int nwg) {
+    const int round = kXcds * xcd_chunk(nwg);
+    return (nwg + round - 1) / round * round;
+}
+
 // MapRenderingDelegate::operator() (check_colour == false) and
 // ::raycast_with_colour (check_colour == true): ray_tracing.cu:346-425,478-564.
 // Workgroup wg (its index within this raycast's grid; the grid's x extent is
@@ -579,11 +591,10 @@ LF_DEV void raycast_wg(const RayDev &r, float *__restrict__ vmap, unsigned char 
     // (The loads of the start are issued together, ahead of the test.)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     // XCD-aware placement: workgroups are dealt to the 8 XCDs in turn, so
-    // workgroup g (XCD g % 8) takes the (g / 8)-th workgroup tile of band g % 8:
-    // each XCD marches a contiguous band of the image, and the blocks its rays
-    // read stay in that XCD's L2.
-    const int nwg = wg_x * wg_y, per_xcd = (nwg + kXcds - 1) / kXcds;
-    const int L = (wg % kXcds) * per_xcd + wg / kXcds;
+    // workgroup g (XCD g % 8) takes the (g / 8)-th workgroup tile of its XCD's
+    // chunks, and the blocks its rays read stay in that XCD's L2.
+    const int nwg = wg_x * wg_y, chunk = xcd_chunk(nwg), in_xcd = wg / kXcds;
+    const int L = (in_xcd / chunk * kXcds + wg % kXcds) * chunk + in_xcd % chunk;
     if (L >= nwg) return;
     const int tile_x = (L % wg_x) * 2 + (wave & 1), tile_y = (L / wg_x) * 2 + (wave >> 1);
     const bool has_range = tile_x < r.tiles_x && tile_y < r.tiles_y;
@@ -699,7 +710,7 @@ __global__ __launch_bounds__(256, 8) void k_raycast_batch(const RayJob *__restri
     __shared__ unsigned long long s_cache[kLdsCache];
     __shared__ uint4 s_occ[LF_OCC_WORDS / 4];
     const RayJob &j = jobs[blockIdx.y];
-    const int g = kXcds * ((j.wg_x * j.wg_y + kXcds - 1) / kXcds);
+    const int g = xcd_grid(j.wg_x * j.wg_y);
     if ((int)blockIdx.x >= g) return;  // this raycast's grid is smaller than the batch's
     raycast_wg<kCheckColour, kMixed>(global_ray(j.r), global_ptr(j.vmap), global_ptr(j.rgb_out), j.cols, j.rows,
                                      global_ptr(j.pose24), j.K, j.wg_x, j.wg_y, blockIdx.x, s_cache, s_occ);
@@ -767,7 +778,7 @@ int lf_raycast_ev(const lf_map_params *p, const lf_map_storage *s, float *vmap, 
     LF_LAUNCH_CHECK();
     const int tx = (cols + 7) / 8, ty = (rows + 7) / 8;
     const int wg_x = (tx + 1) / 2, wg_y = (ty + 1) / 2;  // 2x2 tiles per workgroup
-    const int g = kXcds * ((wg_x * wg_y + kXcds - 1) / kXcds);
+    const int g = xcd_grid(wg_x * wg_y);
     if (e0) LF_HIP_CHECK(hipEventRecord(e0, st));
     if (p->precision == LF_PRECISION_MIXED) {  // FP16 voxels
         if (check_colour) k_raycast<true, true><<<g, 256, 0, st>>>(r, vmap, rgb_out, cols, rows, pose24, *K, wg_x, wg_y);
@@ -819,7 +830,7 @@ int lf_raycast_batch_make(const LfRayItem *items, int n, void *jobs_host, LfRayB
         const int T = it.s->tiles_x * it.s->tiles_y;
         d.tiles_max = std::max(d.tiles_max, T);
         d.zgrid_max = std::max(d.zgrid_max, zrange_grid(it.p));
-        d.grid_max = std::max(d.grid_max, kXcds * ((J[i].wg_x * J[i].wg_y + kXcds - 1) / kXcds));
+        d.grid_max = std::max(d.grid_max, xcd_grid(J[i].wg_x * J[i].wg_y));
         lds_max = std::max(lds_max, 2 * (size_t)T * sizeof(int));
     }
     d.zrange_lds = lds_max;

@@ -721,3 +721,33 @@ def test_state_reads_from_several_threads():
             results = list(pool.map(lambda _: s.tracking(), range(8)))
         assert all(np.array_equal(p, s.pose()) for p in poses)
         assert all(np.array_equal(r, s.tracking(), equal_nan=True) for r in results)  # a lost frame has no error
+
+
+# one workgroup, one per XCD and one more, the last grid whose workgroups are resident at once and the first that isn't
+@pytest.mark.parametrize("width,height", [(16, 8), (128, 16), (144, 16), (1024, 512), (1040, 512)])
+def test_raycast_grids(width, height):
+    """Every pixel of a raycast is the oracle's, bit for bit, whichever XCD takes its tile."""
+    from oracle import oracle as O
+    f = 0.8 * width
+    K = capi.intrinsics(width, height, f, f, (width - 1) / 2, (height - 1) / 2)
+    u, v = np.meshgrid(np.linspace(0, 9, width), np.linspace(0, 5, height))
+    depth = (0.8 + 0.1 * np.sin(u) * np.cos(v)).astype(np.float32)
+    nmap = np.zeros((height, width, 4), np.float32)
+    nmap[..., 2] = 1.0
+    rgb = np.full((height, width, 3), 77, np.uint8)
+    T = np.eye(4)
+    p = capi.map_params(1 << 16, 1 << 15, 0.01, 0.03)
+    m = capi.Map(p, width, height)
+    pose = dev(capi.pose24(T))
+    m.update_weighted(dev(depth), dev(nmap), dev(rgb), pose, K)
+    vm = torch.full((height, width, 4), -1.0, device="cuda")
+    m.raycast(vm, pose, K)
+    torch.cuda.synchronize()
+    om = O.Map(O.Params(p.num_buckets, p.num_entries, p.num_blocks, p.max_triangles, p.zmin_raycast, p.zmax_raycast,
+                        p.zmin_update, p.zmax_update, p.voxel_size, p.truncation), np.float32)
+    oK = O.make_intr(K.width, K.height, K.fx, K.fy, K.cx, K.cy)
+    om.update_weighted(depth, nmap, rgb, T, oK)
+    om.set_blocks(*m.voxels())
+    ovm = om.raycast(T, oK, width, height)
+    assert (~np.isnan(ovm[..., 0])).mean() > 0.5
+    assert np.array_equal(vm.cpu().numpy(), ovm, equal_nan=True)
