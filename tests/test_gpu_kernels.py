@@ -751,3 +751,34 @@ def test_raycast_grids(width, height):
     ovm = om.raycast(T, oK, width, height)
     assert (~np.isnan(ovm[..., 0])).mean() > 0.5
     assert np.array_equal(vm.cpu().numpy(), ovm, equal_nan=True)
+
+
+# one tile; a workgroup's box one narrower, as wide and one wider than the 32 lanes of its rows; the grid that just fits
+# LDS; one that doesn't
+@pytest.mark.parametrize("width,height", [(8, 8), (248, 120), (256, 256), (264, 272), (1280, 960), (1600, 1040)])
+def test_zrange_tiles(width, height):
+    """Each tile's depth range is the oracle's, bit for bit, however many workgroups and passes share it."""
+    from oracle import oracle as O
+    f = 0.8 * width
+    K = capi.intrinsics(width, height, f, f, (width - 1) / 2, (height - 1) / 2)
+    u, v = np.meshgrid(np.linspace(0, 9, width), np.linspace(0, 5, height))
+    depth = (0.8 + 0.1 * np.sin(u) * np.cos(v)).astype(np.float32)
+    nmap = np.zeros((height, width, 4), np.float32)
+    nmap[..., 2] = 1.0
+    rgb = np.full((height, width, 3), 77, np.uint8)
+    T = np.eye(4)
+    p = capi.map_params(1 << 16, 1 << 15, 0.005, 0.015)
+    m = capi.Map(p, width, height)
+    pose = dev(capi.pose24(T))
+    m.update_weighted(dev(depth), dev(nmap), dev(rgb), pose, K)
+    m.raycast(torch.empty((height, width, 4), device="cuda"), pose, K)
+    torch.cuda.synchronize()
+    om = O.Map(O.Params(p.num_buckets, p.num_entries, p.num_blocks, p.max_triangles, p.zmin_raycast, p.zmax_raycast,
+                        p.zmin_update, p.zmax_update, p.voxel_size, p.truncation), np.float32)
+    oK = O.make_intr(K.width, K.height, K.fx, K.fy, K.cx, K.cy)
+    om.update_weighted(depth, nmap, rgb, T, oK)
+    near, far = om.zrange(T, oK, width, height)
+    tiles = (width // 8) * (height // 8)
+    got = m.t["zrange"].cpu().numpy()
+    assert (near < 100).mean() > 0.9
+    assert np.array_equal(got[:tiles], near.ravel()) and np.array_equal(got[tiles : 2 * tiles], far.ravel())
