@@ -936,8 +936,10 @@ LF_DEV bool surely_behind(const RefuseArgs &a, int k, f3 c, f3 half) {
     const int *far = a.tile_far + (size_t)k * w * h;
     int most = 0;
     if (u1 >= 0.0f && v1 >= 0.0f)
-        for (int y = ty0; y <= ty1; ++y)
-            for (int x = tx0; x <= tx1; ++x) most = max(most, far[y * w + x]);
+        for (int y = ty0; y <= ty1; y += 3)  // nine tiles' loads in flight, the last row and column repeated
+            for (int x = tx0; x <= tx1; x += 3)
+#pragma unroll
+                for (int i = 0; i < 9; ++i) most = max(most, far[min(y + i / 3, ty1) * w + min(x + i % 3, tx1)]);
     return most == 0 || __int_as_float(most - 1) - zn < -a.m.truncation * 1.0001f;
 }
 
@@ -948,24 +950,27 @@ LF_DEV bool surely_behind(const RefuseArgs &a, int k, f3 c, f3 half) {
 // only the poses that a bounding sphere leaves open corner by corner.  40 poses of
 // 165k blocks: 104 us with one lane per block and no sphere; 39 without the depths'
 // test, 54 with it, which takes 160 us off k_refuse (tiles of 4 pixels, as good a
-// test: 70).
+// test: 70).  Bound by the latency of a lane's chain of poses: 60 -> 44 us (under the
+// profiler) with nine tiles' loads in flight and three workgroups of 512 lanes on a CU
+// for one of 1024 (77 VGPRs; 57 at 64 VGPRs and 1024 lanes, 50 with 256 lanes).
+constexpr int kRefuseVisThreads = 512;
 template <bool kFast>
-__global__ __launch_bounds__(kVisThreads) void k_refuse_visible(RefuseArgs a) {
-    __shared__ unsigned int s_cnt[kVisThreads / kWave];
+__global__ __launch_bounds__(kRefuseVisThreads) void k_refuse_visible(RefuseArgs a) {
+    __shared__ unsigned int s_cnt[kRefuseVisThreads / kWave];
     __shared__ unsigned int s_base;
     __shared__ float s_pose[2 * kMaxRefuse][12];
     __shared__ RefuseBox s_box[2 * kMaxRefuse];
     const MapDev &m = a.m;
-    for (int i = threadIdx.x; i < 2 * a.n * 12; i += kVisThreads)
+    for (int i = threadIdx.x; i < 2 * a.n * 12; i += kRefuseVisThreads)
         s_pose[i / 12][i % 12] = refuse_pose(a, i / 12)[i % 12];
     __syncthreads();
-    for (int i = threadIdx.x; i < 2 * a.n; i += kVisThreads) s_box[i] = refuse_box(s_pose[i], m.voxel_size);
+    for (int i = threadIdx.x; i < 2 * a.n; i += kRefuseVisThreads) s_box[i] = refuse_box(s_pose[i], m.voxel_size);
     __syncthreads();
     const unsigned int nb = min(m.counters[LF_CNT_ALLOCATED], (unsigned int)m.num_blocks);
     // the half diagonal of a block with a hundredth of it to spare (coordinates
     // are rounded to 2^-24 of at most a few thousand blocks)
     const float scale = 8.0f * m.voxel_size, radius = 0.875f * scale;
-    constexpr unsigned int kPerWg = kVisThreads / 4;
+    constexpr unsigned int kPerWg = kRefuseVisThreads / 4;
     const unsigned int stride = gridDim.x * kPerWg;
     const int lane = lane_id(), wave = threadIdx.x / kWave, sub = threadIdx.x & 3;
     const unsigned long long all = (1ull << a.n) - 1ull;
@@ -1017,7 +1022,7 @@ __global__ __launch_bounds__(kVisThreads) void k_refuse_visible(RefuseArgs a) {
         __syncthreads();
         if (threadIdx.x == 0) {
             unsigned int total = 0;
-            for (int w = 0; w < kVisThreads / kWave; ++w) {
+            for (int w = 0; w < kRefuseVisThreads / kWave; ++w) {
                 const unsigned int c = s_cnt[w];
                 s_cnt[w] = total;
                 total += c;
@@ -1452,9 +1457,9 @@ static int refuse_launch(const lf_map_params *p, const RefuseArgs &a, int colour
     if (mixed) k_refuse_alloc<true><<<g, 256, 0, st>>>(a);
     else k_refuse_alloc<false><<<g, 256, 0, st>>>(a);
     LF_LAUNCH_CHECK();
-    const int V = std::min(4 * kVisGrid, std::max(1, (p->num_blocks + kVisThreads / 4 - 1) / (kVisThreads / 4)));
-    if (mixed) k_refuse_visible<true><<<V, kVisThreads, 0, st>>>(a);
-    else k_refuse_visible<false><<<V, kVisThreads, 0, st>>>(a);
+    const int V = std::min(8 * kVisGrid, std::max(1, (p->num_blocks + kRefuseVisThreads / 4 - 1) / (kRefuseVisThreads / 4)));
+    if (mixed) k_refuse_visible<true><<<V, kRefuseVisThreads, 0, st>>>(a);
+    else k_refuse_visible<false><<<V, kRefuseVisThreads, 0, st>>>(a);
     LF_LAUNCH_CHECK();
     const int G = integrate_grid();
     if (mixed) {
