@@ -71,7 +71,7 @@ struct RayJob {
     unsigned char *rgb_out;
     const float *pose24;
     lf_intrinsics K;
-    int cols, rows, wg_x, wg_y;
+    int cols, rows, wg_x, wg_y, chunk;
 };
 
 // Workgroup wg of nwg: the z-range tiles back to k_zrange_clear's values.
@@ -574,15 +574,16 @@ LF_DEV void march(const RayDev &r, BlockCache &bc, f3 &res, const f3 dir2, float
     }
 }
 
-// Workgroup tiles in a row that one XCD takes: an eighth of the image where all its
-// workgroups are resident at once (8 of 4 wavefronts on each of 256 CUs), as each
-// L2 then holds a band of the volume; above that, as the bands' unequal work adds up,
-// 4 in turn.  640x480 (1200 workgroups): 86.3 us by bands, 89.5 in turn; 1280x960
-// (4800): 182.5 and 170.0.
-LF_HD int xcd_chunk(int nwg) { return nwg > 2048 ? 4 : (nwg + kXcds - 1) / kXcds; }
+// Workgroup tiles in a row that one XCD takes: an eighth of the image where all the
+// launch's workgroups are resident at once (8 of 4 wavefronts on each of 256 CUs), as
+// each L2 then holds a band of the volume; above that, as the bands' unequal work adds
+// up, 4 in turn.  640x480 (1200 workgroups): 86.3 us by bands, 89.5 in turn; 1280x960
+// (4800): 182.5 and 170.0; 16 maps of 640x480 (19200): four batched steps 7903 and
+// 7832 (tiles one at a time 7811 to 7955).
+LF_HD int xcd_chunk(int nwg, int launch) { return launch > 2048 ? 4 : (nwg + kXcds - 1) / kXcds; }
 // Workgroups to launch for nwg: whole rounds of chunks.
-LF_HD int xcd_grid(int nwg) {
-    const int round = kXcds * xcd_chunk(nwg);
+LF_HD int xcd_grid(int nwg, int chunk) {
+    const int round = kXcds * chunk;
     return (nwg + round - 1) / round * round;
 }
 
@@ -593,8 +594,8 @@ LF_HD int xcd_grid(int nwg) {
 // voxels in (the vertices out are float4 in both precisions).
 template <bool kCheckColour, bool kMixed>
 LF_DEV void raycast_wg(const RayDev &r, float *__restrict__ vmap, unsigned char *__restrict__ rgb_out, int cols,
-                       int rows, const float *__restrict__ pose24, const lf_intrinsics &K, int wg_x, int wg_y, int wg,
-                       unsigned long long *s_cache, uint4 *s_occ) {
+                       int rows, const float *__restrict__ pose24, const lf_intrinsics &K, int wg_x, int wg_y, int chunk,
+                       int wg, unsigned long long *s_cache, uint4 *s_occ) {
     // DenseMapping::raycast leaves the map untouched when nothing is visible
     // (voxel_hashing.cpp:92-93) or no rendering block was made (:105).
     // (The loads of the start are issued together, ahead of the test.)
@@ -602,7 +603,7 @@ LF_DEV void raycast_wg(const RayDev &r, float *__restrict__ vmap, unsigned char 
     // XCD-aware placement: workgroups are dealt to the 8 XCDs in turn, so
     // workgroup g (XCD g % 8) takes the (g / 8)-th workgroup tile of its XCD's
     // chunks, and the blocks its rays read stay in that XCD's L2.
-    const int nwg = wg_x * wg_y, chunk = xcd_chunk(nwg), in_xcd = wg / kXcds;
+    const int nwg = wg_x * wg_y, in_xcd = wg / kXcds;
     const int L = (in_xcd / chunk * kXcds + wg % kXcds) * chunk + in_xcd % chunk;
     if (L >= nwg) return;
     const int tile_x = (L % wg_x) * 2 + (wave & 1), tile_y = (L / wg_x) * 2 + (wave >> 1);
@@ -710,7 +711,8 @@ __global__ __launch_bounds__(256, 8) void k_raycast(RayDev r, float *__restrict_
                                                  lf_intrinsics K, int wg_x, int wg_y) {
     __shared__ unsigned long long s_cache[kLdsCache];
     __shared__ uint4 s_occ[LF_OCC_WORDS / 4];
-    raycast_wg<kCheckColour, kMixed>(r, vmap, rgb_out, cols, rows, pose24, K, wg_x, wg_y, blockIdx.x, s_cache, s_occ);
+    raycast_wg<kCheckColour, kMixed>(r, vmap, rgb_out, cols, rows, pose24, K, wg_x, wg_y,
+                                     xcd_chunk(wg_x * wg_y, wg_x * wg_y), blockIdx.x, s_cache, s_occ);
 }
 
 // As k_raycast for many maps, row y of the grid the map of jobs[y].
@@ -719,10 +721,10 @@ __global__ __launch_bounds__(256, 8) void k_raycast_batch(const RayJob *__restri
     __shared__ unsigned long long s_cache[kLdsCache];
     __shared__ uint4 s_occ[LF_OCC_WORDS / 4];
     const RayJob &j = jobs[blockIdx.y];
-    const int g = xcd_grid(j.wg_x * j.wg_y);
+    const int g = xcd_grid(j.wg_x * j.wg_y, j.chunk);
     if ((int)blockIdx.x >= g) return;  // this raycast's grid is smaller than the batch's
     raycast_wg<kCheckColour, kMixed>(global_ray(j.r), global_ptr(j.vmap), global_ptr(j.rgb_out), j.cols, j.rows,
-                                     global_ptr(j.pose24), j.K, j.wg_x, j.wg_y, blockIdx.x, s_cache, s_occ);
+                                     global_ptr(j.pose24), j.K, j.wg_x, j.wg_y, j.chunk, blockIdx.x, s_cache, s_occ);
 }
 
 // Dynamic LDS available to one workgroup on this device (less the static use).
@@ -787,7 +789,7 @@ int lf_raycast_ev(const lf_map_params *p, const lf_map_storage *s, float *vmap, 
     LF_LAUNCH_CHECK();
     const int tx = (cols + 7) / 8, ty = (rows + 7) / 8;
     const int wg_x = (tx + 1) / 2, wg_y = (ty + 1) / 2;  // 2x2 tiles per workgroup
-    const int g = xcd_grid(wg_x * wg_y);
+    const int g = xcd_grid(wg_x * wg_y, xcd_chunk(wg_x * wg_y, wg_x * wg_y));
     if (e0) LF_HIP_CHECK(hipEventRecord(e0, st));
     if (p->precision == LF_PRECISION_MIXED) {  // FP16 voxels
         if (check_colour) k_raycast<true, true><<<g, 256, 0, st>>>(r, vmap, rgb_out, cols, rows, pose24, *K, wg_x, wg_y);
@@ -816,6 +818,7 @@ int lf_raycast_batch_make(const LfRayItem *items, int n, void *jobs_host, LfRayB
     d.n = n;
     d.mixed = items[0].p && items[0].p->precision == LF_PRECISION_MIXED;
     size_t lds_max = 0;
+    long long total = 0;
     for (int i = 0; i < n; ++i) {
         const LfRayItem &it = items[i];
         if (!it.p || !it.s || !it.vmap || !it.pose24 || !it.K)
@@ -839,10 +842,15 @@ int lf_raycast_batch_make(const LfRayItem *items, int n, void *jobs_host, LfRayB
         const int T = it.s->tiles_x * it.s->tiles_y;
         d.tiles_max = std::max(d.tiles_max, T);
         d.zgrid_max = std::max(d.zgrid_max, zrange_grid(it.p));
-        d.grid_max = std::max(d.grid_max, xcd_grid(J[i].wg_x * J[i].wg_y));
+        total += J[i].wg_x * J[i].wg_y;
         lds_max = std::max(lds_max, 2 * (size_t)T * sizeof(int));
     }
     d.zrange_lds = lds_max;
+    for (int i = 0; i < n; ++i) {
+        const int nwg = J[i].wg_x * J[i].wg_y;
+        J[i].chunk = xcd_chunk(nwg, (int)std::min<long long>(total, INT_MAX));
+        d.grid_max = std::max(d.grid_max, xcd_grid(nwg, J[i].chunk));
+    }
     // n maps share the z-range launch: each takes 1/n of a lone map's grid
     // (at least 64 workgroups), so that a workgroup's LDS tile grid, cleared
     // and flushed once, collects several passes of blocks

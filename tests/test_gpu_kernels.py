@@ -782,3 +782,37 @@ def test_zrange_tiles(width, height):
     got = m.t["zrange"].cpu().numpy()
     assert (near < 100).mean() > 0.9
     assert np.array_equal(got[:tiles], near.ravel()) and np.array_equal(got[tiles : 2 * tiles], far.ravel())
+
+
+@pytest.mark.parametrize("precision", [FP32, MIXED])
+@pytest.mark.parametrize("n", [1, 2])
+def test_batch_raycast_grids(n, precision):
+    """Maps dealt to the XCDs by bands where few (1500 workgroups) and a few tiles at a time where many (2700): the
+    poses tracked against their raycasts are those of each map alone."""
+    from libfusion_amd.synth import Scene
+    cfgs, frames = [], []
+    for div in [1] * n + [2]:
+        sc = Scene(1, 7)
+        K = capi.intrinsics(sc.width // div, sc.height // div, sc.fx / div, sc.fy / div, (sc.cx + 0.5) / div - 0.5,
+                            (sc.cy + 0.5) / div - 0.5)
+        p = capi.map_params(1 << 18, 1 << 15, 0.01, 0.03, precision=precision)
+        cfgs.append(capi.system_config(K, p, 2, (4, 3), sc.depth_scale))
+        shots = [sc.render(sc.pose(i), K.width, K.height, K.fx, K.fy, K.cx, K.cy, noise=True, frame_id=i)
+                 for i in range(3)]
+        frames.append([(dev(d.view(np.int16)), dev(c)) for d, c in shots])
+    torch.cuda.synchronize()
+
+    def run(which):
+        b = capi.Batch([cfgs[i] for i in which])
+        for t in range(3):
+            b.process([frames[i][t][0] for i in which], [frames[i][t][1] for i in which])
+        b.synchronize()
+        assert all(b.tracking(k)[0] for k in range(len(which)))
+        poses = [b.pose(k) for k in range(len(which))]
+        b.close()
+        return poses
+
+    together = run(range(n + 1))
+    for i in (0, n):
+        # the tracking sums of 1 / n of the workgroups in another order: see test_batch_tracking_workgroups
+        assert np.allclose(together[i], run([i])[0], rtol=0, atol=3e-7), i
