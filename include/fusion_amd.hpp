@@ -188,7 +188,10 @@ public:
              std::vector<unsigned char> &jobs, std::vector<int> &grids);
     // Planned steps of a tracker that shares its launches with share - 1
     // others take 1/share of the reduction grid (a Batch sets it).
-    void set_batch_share(int share) { batch_share_ = share < 1 ? 1 : share; }
+    void set_batch_share(int share) {
+        batch_share_ = share < 1 ? 1 : share;
+        in_batch_ = true;
+    }
     // wgs > 0: planned steps take exactly that many workgroups (at most a
     // lone system's grid) instead of 1/share of it.
     void set_batch_workgroups(int wgs) { batch_wgs_ = wgs < 0 ? 0 : wgs; }
@@ -209,12 +212,14 @@ public:
     DeviceImage *source() { return src_.get(); }
     DeviceImage *reference() { return ref_.get(); }
     LfTrackState *state() const { return state_; }
+    // The odometry pose (3x4, row-major), as a first frame or a restart sets it.
+    int set_pose(const double *T12);
     // Synchronising read of the last result (update = estimate^-1).
     TrackingResult result();
     TrackingResult result_of(const LfTrackState &state) const;
     // The state after the work enqueued on this tracker's stream (synchronising;
     // several threads may read).  copy_state: by a copy beside the kernels of other
-    // streams, which does not wait for those (a Batch's steps: synchronise it first).
+    // streams, which does not wait for those (a Batch's steps: Batch::read_state does).
     int read_state(LfTrackState &out);
     int copy_state(LfTrackState &out) const;
     // Synchronising read of the last Gauss-Newton step's FP64 sums (31 values).
@@ -231,6 +236,8 @@ private:
     float *scratch_ = nullptr;
     bool context_mode_ = false;
     int batch_share_ = 1;
+    bool in_batch_ = false;
+    unsigned long long records_ = 0;  // pose records written so far
     int batch_wgs_ = 0;
     std::unique_ptr<DeviceImage> src_, ref_;
 };
@@ -373,7 +380,15 @@ public:
     // raycast; pinned host buffers make the copies asynchronous.
     int process_host(const uint16_t *const *depth, const unsigned char *const *rgb);
     int synchronize();
+    // System i's tracking state and map counters after the steps processed so far
+    // (synchronising; one thread may read while another processes: a read and the
+    // enqueueing of a step exclude each other).
+    int read_state(int i, LfTrackState &out);
+    int read_counters(int i, unsigned int *out16);
+    // System i's pose after the last step tracked so far, without waiting (from any thread).
+    int latest_pose(int i, double *out16);
     int size() const { return (int)sys_.size(); }
+    // Work on a system's own stream does not wait for the steps: synchronize() first.
     System &system(int i) { return *sys_[i]; }
     hipStream_t stream() const { return stream_; }
     // Event timing on the batch stream (LF_BATCH_TIMING_* bits; 0: off) and
@@ -433,6 +448,9 @@ private:
     std::vector<hipEvent_t> ready_;  // per system: its tracking and fusion are enqueued
     hipStream_t aux_ = nullptr;      // the step's descriptor table and uploads
     hipEvent_t uploaded_ = nullptr;  // the step's uploads
+    // held while a step is enqueued and while a state is read; the turn to take it
+    std::mutex step_mutex_, turn_mutex_;
+    std::unique_lock<std::mutex> lock_steps();
     bool half_maps_ = false;  // the systems are mixed precision
     int parity_ = 0;
     // the step's descriptors (frame passes, tracking jobs, raycast jobs),

@@ -640,11 +640,14 @@ int lf_batch_tuning(lf_batch *b);
  * append new ones to it; null or "" stops using a file. */
 int lf_batch_tune_file(const char *path);
 /* System i's camera pose (4x4 row-major doubles), last tracking result and map
- * counters: those of the steps done so far, so lf_batch_synchronize first for
- * those of the steps processed. */
+ * counters after the steps processed so far (synchronising). */
 int lf_batch_get_pose(lf_batch *b, int i, double *out16);
 int lf_batch_get_tracking(lf_batch *b, int i, int *success, float *icp_error);
 int lf_batch_read_counters(lf_batch *b, int i, unsigned int *out16);
+/* System i's pose without waiting for the steps: that of the last one whose
+ * tracking has ended when the read arrives, one or two before the last
+ * processed while those run.  From any thread, beside lf_batch_process. */
+int lf_batch_latest_pose(lf_batch *b, int i, double *out16);
 /* System i's map (the arrays of its volume, as lf_system_map). */
 int lf_batch_map(lf_batch *b, int i, lf_map_params *p, lf_map_storage *s);
 

@@ -169,6 +169,7 @@ SIGNATURES = [
     ("lf_batch_get_option", I, [P, I, P]),
     ("lf_batch_read_timing", I, [P, I, P, P]),
     ("lf_batch_get_pose", I, [P, I, P]),
+    ("lf_batch_latest_pose", I, [P, I, P]),
     ("lf_batch_get_tracking", I, [P, I, P, P]),
     ("lf_batch_read_counters", I, [P, I, P]),
 ]
@@ -683,9 +684,13 @@ class Batch:
         check(load().lf_batch_get_option(self.h, int(option), ctypes.byref(v)))
         return v.value
 
-    def pose(self, i):
+    def pose(self, i, wait=False):
+        """System i's pose: after the steps processed (wait, lf_batch_get_pose), or without
+        waiting after the last one tracked so far (lf_batch_latest_pose), which is the same
+        once the batch is synchronised."""
         T = np.zeros((4, 4))
-        check(load().lf_batch_get_pose(self.h, int(i), T.ctypes.data_as(P)))
+        read = load().lf_batch_get_pose if wait else load().lf_batch_latest_pose
+        check(read(self.h, int(i), T.ctypes.data_as(P)))
         return T
 
     def tracking(self, i):

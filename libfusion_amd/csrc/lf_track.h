@@ -18,6 +18,23 @@ struct LfGnState {
     int pad;
 };
 
+// A frame's pose for a reader that waits for nothing: record n is the state's record[n & 1],
+// and a copy of one caught between its stores does not match its check.
+struct LfPoseRecord {
+    double pose[12];
+    unsigned long long number;  // in the order of the frames (0: empty)
+    unsigned long long check;
+};
+__host__ __device__ inline unsigned long long lf_pose_check(const LfPoseRecord &r) {
+    unsigned long long h = 0;  // an empty record's
+    for (int k = 0; k < 12; ++k) {
+        h = (h ^ __builtin_bit_cast(unsigned long long, r.pose[k])) * 0x9E3779B97F4A7C15ull;
+        h ^= h >> 29;
+    }
+    h = (h ^ r.number) * 0x9E3779B97F4A7C15ull;
+    return h ^ h >> 32;
+}
+
 // One tracker's state in device memory.  Poses are 3x4 row-major doubles.
 struct LfTrackState {
     LfGnState gn;        // after the last step that was taken
@@ -29,6 +46,7 @@ struct LfTrackState {
     // odometry chain (DenseOdometry::trackFrame, rgbd_odometry.cpp:18-48)
     double pose[12];     // T_world_camera of the current frame
     float pose24[24];    // float T_world_camera and T_camera_world for the mapping kernels
+    LfPoseRecord record[2];  // pose after the last frame and the one before it (of a batch's systems)
     // the last Gauss-Newton step's FP64 sums: A = w H_icp + H_rgb and b in
     // create_jtjjtr<6,7> order (0-26), ICP r^2 / count (27 / 28), RGB r^2 /
     // count (29 / 30)
@@ -59,6 +77,7 @@ struct LfStepFlags {
     int prev_grid;            // its workgroups
     int context_mode;         // compute_transform(ctx) (icp_tracker.cpp:210-314): NaN errors are not
                               // flagged and the finish always succeeds with update = estimate^-1
+    unsigned long long record;  // number of the frame's pose record (0: none is written)
     double init[12];          // initial estimate, 3x4 row-major (step 0)
 };
 
@@ -74,9 +93,9 @@ int lf_track_step(const LfTrackLevel &lv, float *scratch, LfTrackState *st, cons
 int lf_track_begin(LfTrackState *st, const double *T12, hipStream_t stream);
 // End of a tracked frame: success test, update = est^-1 (or identity), chain the
 // odometry pose and refresh pose24.  Only needed when a frame schedules no step.
-int lf_track_finish(LfTrackState *st, hipStream_t stream);
+int lf_track_finish(LfTrackState *st, unsigned long long record, hipStream_t stream);
 // Set the odometry pose directly (first frame / restart): T given as 3x4 doubles (host).
-int lf_track_set_pose(LfTrackState *st, const double *T12, hipStream_t stream);
+int lf_track_set_pose(LfTrackState *st, const double *T12, unsigned long long record, hipStream_t stream);
 // The state into pinned host memory (there once the stream has come this far).
 int lf_track_read(const LfTrackState *st, LfTrackState *host, hipStream_t stream);
 

@@ -60,6 +60,7 @@ struct ReduceArgs {
     int prev_first_iter;   // the previous step's first_iter,
     int prev_grid;         // and its workgroups (partial rows)
     int context_mode;      // compute_transform(ctx) semantics
+    unsigned long long record;  // number of the end's pose among the state's records (0: not recorded)
     float icp_weight;
     double init[12];       // initial estimate (step 0)
     float init_f[12];      // the same in FP32 (the first step's pose, uniform across the grid)
@@ -720,11 +721,22 @@ __global__ __launch_bounds__(kThreads) void k_reduce(ReduceArgs a, float *__rest
     for (int g = tid; g < G; g += kThreads) store_agent(&flags[g], 0ull);
 }
 
+// The pose as record `number` (0: none).
+LF_DEV void record_pose(LfTrackState &st, const double *pose, unsigned long long number) {
+    if (number == 0ull) return;
+    LfPoseRecord r;
+    for (int k = 0; k < 12; ++k) r.pose[k] = pose[k];
+    r.number = number;
+    r.check = lf_pose_check(r);
+    st.record[number & 1ull] = r;
+}
+
 // End of DenseTracking::compute_transform (icp_tracker.cpp:143-155) and the
 // odometry chain of DenseOdometry::trackFrame (rgbd_odometry.cpp:39): success
 // test, update = est^-1 (or identity), pose = pose * update, pose24 refreshed.
 // est and invalid are the frame's final estimate and flag (already in st).
-LF_DEV void track_finish(LfTrackState &st, const double *est, int invalid, bool context_mode) {
+LF_DEV void track_finish(LfTrackState &st, const double *est, int invalid, bool context_mode,
+                         unsigned long long record) {
     double inv_est[12], D[12];
     m34_inv(est, inv_est);
     m34_mul(inv_est, st.init, D);
@@ -743,6 +755,7 @@ LF_DEV void track_finish(LfTrackState &st, const double *est, int invalid, bool 
         st.pose24[k] = (float)P[k];
         st.pose24[12 + k] = (float)Pi[k];
     }
+    record_pose(st, P, record);
 }
 
 // LDS of a tracking step's workgroup: the wavefronts' partial sums, and what
@@ -861,7 +874,7 @@ __global__ __launch_bounds__(kThreads, 4) void k_track_step(ReduceArgs a) {
 // its loop) left the estimate as it was then.
 LF_DEV void track_end_wg(const ReduceArgs &a, StepLds &s) {
     const LfGnState g = solve_previous(a, 0, s);
-    if (threadIdx.x == 0) track_finish(*a.st, g.est, g.invalid, a.context_mode != 0);
+    if (threadIdx.x == 0) track_finish(*a.st, g.est, g.invalid, a.context_mode != 0, a.record);
 }
 
 __global__ __launch_bounds__(kThreads) void k_track_end(ReduceArgs a) {
@@ -908,12 +921,12 @@ __global__ __launch_bounds__(kThreads) void k_track_end_batch(const TrackJob *__
     track_end_wg(global_args(j.a), s);
 }
 
-__global__ void k_track_finish(LfTrackState *st) {
+__global__ void k_track_finish(LfTrackState *st, unsigned long long record) {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
     LfTrackState &s = *st;
     double est[12];
     for (int k = 0; k < 12; ++k) est[k] = s.gn.est[k];
-    track_finish(s, est, s.gn.invalid, false);
+    track_finish(s, est, s.gn.invalid, false, record);
 }
 
 __global__ void k_track_begin(LfTrackState *st, double t0, double t1, double t2, double t3, double t4, double t5,
@@ -929,8 +942,8 @@ __global__ void k_track_begin(LfTrackState *st, double t0, double t1, double t2,
     st->gn.iterations = 0;
 }
 
-__global__ void k_track_set_pose(LfTrackState *st, double t0, double t1, double t2, double t3, double t4, double t5,
-                                 double t6, double t7, double t8, double t9, double t10, double t11) {
+__global__ void k_track_set_pose(LfTrackState *st, unsigned long long record, double t0, double t1, double t2,
+                                 double t3, double t4, double t5, double t6, double t7, double t8, double t9, double t10, double t11) {
     const double T[12] = {t0, t1, t2, t3, t4, t5, t6, t7, t8, t9, t10, t11};
     double Ti[12];
     m34_inv(T, Ti);
@@ -940,6 +953,7 @@ __global__ void k_track_set_pose(LfTrackState *st, double t0, double t1, double 
         st->pose24[12 + k] = (float)Ti[k];
     }
     st->success = 1;
+    record_pose(*st, T, record);
 }
 
 // The state to pinned host memory: a launch and a wait take about 20 us less than a
@@ -995,6 +1009,7 @@ static ReduceArgs step_args(const LfTrackLevel &lv, float *scratch, LfTrackState
     a.prev_grid = f.prev_grid;
     a.icp_weight = icp_weight;
     a.context_mode = f.context_mode;
+    a.record = f.record;
     for (int k = 0; k < 12; ++k) {
         a.init[k] = f.init[k];
         a.init_f[k] = (float)f.init[k];
@@ -1066,14 +1081,15 @@ int lf_track_batch_end(const void *jobs, int n, hipStream_t stream) {
     return LF_OK;
 }
 
-int lf_track_finish(LfTrackState *st, hipStream_t stream) {
-    k_track_finish<<<1, 64, 0, stream>>>(st);
+int lf_track_finish(LfTrackState *st, unsigned long long record, hipStream_t stream) {
+    k_track_finish<<<1, 64, 0, stream>>>(st, record);
     LF_LAUNCH_CHECK();
     return LF_OK;
 }
 
-int lf_track_set_pose(LfTrackState *st, const double *T, hipStream_t stream) {
-    k_track_set_pose<<<1, 1, 0, stream>>>(st, T[0], T[1], T[2], T[3], T[4], T[5], T[6], T[7], T[8], T[9], T[10], T[11]);
+int lf_track_set_pose(LfTrackState *st, const double *T, unsigned long long record, hipStream_t stream) {
+    k_track_set_pose<<<1, 1, 0, stream>>>(st, record, T[0], T[1], T[2], T[3], T[4], T[5], T[6], T[7], T[8], T[9], T[10],
+                                          T[11]);
     LF_LAUNCH_CHECK();
     return LF_OK;
 }

@@ -346,7 +346,7 @@ DenseTracking::DenseTracking(hipStream_t stream) : stream_(stream) {
     if (hipMemsetAsync(state_, 0, sizeof(LfTrackState), stream_) != hipSuccess)
         throw std::runtime_error("hipMemsetAsync failed");
     const double I[12] = {1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1, 0};
-    lf_track_set_pose(state_, I, stream_);
+    lf_track_set_pose(state_, I, ++records_, stream_);
 }
 
 DenseTracking::DenseTracking(const IntrinsicMatrix &K, int num_pyr, hipStream_t stream) : DenseTracking(stream) {
@@ -390,6 +390,7 @@ int DenseTracking::enqueue(DeviceImage &ref, DeviceImage &cur, const TrackingCon
     context_mode_ = context_mode;
     LfStepFlags f = {};
     f.context_mode = context_mode ? 1 : 0;
+    f.record = in_batch_ ? ++records_ : 0;  // only a batch's systems are read while they are tracked
     (c.use_initial_guess_ ? c.initial_estimate_ : SE3d()).matrix3x4(f.init);
     struct Step { int level, it; };
     std::vector<Step> plan;
@@ -399,7 +400,7 @@ int DenseTracking::enqueue(DeviceImage &ref, DeviceImage &cur, const TrackingCon
     }
     if (plan.empty()) {
         LF_RC(lf_track_begin(state_, f.init, stream_));
-        return lf_track_finish(state_, stream_);
+        return lf_track_finish(state_, f.record, stream_);
     }
     // a launch per step and one that ends the frame (the last step's level, of which it reads nothing)
     for (size_t s = 0; s <= plan.size(); ++s) {
@@ -436,6 +437,8 @@ int DenseTracking::enqueue(DeviceImage &ref, DeviceImage &cur, const TrackingCon
     }
     return LF_OK;
 }
+
+int DenseTracking::set_pose(const double *T12) { return lf_track_set_pose(state_, T12, ++records_, stream_); }
 
 int DenseTracking::read_state(LfTrackState &out) {
     std::lock_guard<std::mutex> lock(read_);
@@ -492,7 +495,7 @@ int DenseOdometry::trackFrame(const uint16_t *depth, const unsigned char *rgb, f
     if (!initialized_) {
         double T[12];
         initial_pose.matrix3x4(T);
-        LF_RC(lf_track_set_pose(tracker_.state(), T, stream_));
+        LF_RC(tracker_.set_pose(T));
         advance();
         initialized_ = true;
         return LF_OK;
@@ -519,7 +522,7 @@ int DenseOdometry::planFrame(const uint16_t *depth, const unsigned char *rgb, fl
     if (!initialized_) {
         double T[12];
         initial_pose.matrix3x4(T);
-        LF_RC(lf_track_set_pose(tracker_.state(), T, stream_));
+        LF_RC(tracker_.set_pose(T));
         advance();
         initialized_ = true;
         return LF_OK;
@@ -974,13 +977,22 @@ int Batch::read_timing(int stage, int *launches, double *total_ms) {
     return LF_OK;
 }
 
+// The step lock, taken in turn: a thread that waits for it holds the turn, so one that
+// takes it again and again (reading poses in a loop) cannot keep another from it.
+std::unique_lock<std::mutex> Batch::lock_steps() {
+    std::lock_guard<std::mutex> turn(turn_mutex_);
+    return std::unique_lock<std::mutex>(step_mutex_);
+}
+
 int Batch::process(const uint16_t *const *depth, const unsigned char *const *rgb) {
+    const auto lock = lock_steps();
     tune_begin_step();
     LF_RC(step(depth, rgb, false));
     return tune_end_step();
 }
 
 int Batch::process_host(const uint16_t *const *depth, const unsigned char *const *rgb) {
+    const auto lock = lock_steps();
     tune_begin_step();
     LF_RC(step(depth, rgb, true));
     return tune_end_step();
@@ -1230,6 +1242,43 @@ int Batch::synchronize() {
     return LF_OK;
 }
 
+static void pose_of(const double *pose12, double *out16) {
+    for (int i = 0; i < 12; ++i) out16[i] = pose12[i];
+    out16[12] = out16[13] = out16[14] = 0;
+    out16[15] = 1;
+}
+
+// The steps write a system's state and map on the batch's stream; a first frame's pose is
+// set on the system's own, where the copy runs.
+int Batch::read_state(int i, LfTrackState &out) {
+    const auto lock = lock_steps();
+    LF_HIP_CHECK(hipStreamSynchronize(stream_));
+    return sys_[i]->odometry().tracker().copy_state(out);
+}
+
+// The newer of the two records that the copy holds whole.  A frame rewrites the older, so
+// both can be missed only where frames end during the copy: then it is taken again.
+int Batch::latest_pose(int i, double *out16) {
+    for (int attempt = 0; attempt < 64; ++attempt) {
+        LfTrackState h;
+        LF_RC(sys_[i]->odometry().tracker().copy_state(h));
+        const LfPoseRecord *best = nullptr;
+        for (const LfPoseRecord &r : h.record)
+            if (lf_pose_check(r) == r.check && (!best || r.number > best->number)) best = &r;
+        if (best) {
+            pose_of(best->pose, out16);
+            return LF_OK;
+        }
+    }
+    return lf_set_error(LF_ERR_NOT_READY, "batch system %d's pose changed during every read", i);
+}
+
+int Batch::read_counters(int i, unsigned int *out16) {
+    const auto lock = lock_steps();
+    LF_HIP_CHECK(hipStreamSynchronize(stream_));
+    return lf_map_read_counters(&sys_[i]->mapping().storage(), out16, sys_[i]->stream());
+}
+
 int System::process_images(const uint16_t *depth, const unsigned char *rgb) {
     DenseOdometry &od = *odometry_;
     if (graphs_ && timing_ == 0 && mapping_enabled && od.initialized() && !od.trackingLost) {
@@ -1310,12 +1359,6 @@ int System::writeMapToDisk(const std::string &file_name) { return mapping_->writ
 
 int System::readMapFromDisk(const std::string &file_name) { return mapping_->readMapFromDisk(file_name); }
 
-static void pose_of(const LfTrackState &state, double *out16) {
-    for (int i = 0; i < 12; ++i) out16[i] = state.pose[i];
-    out16[12] = out16[13] = out16[14] = 0;
-    out16[15] = 1;
-}
-
 int System::restart() {  // system.cpp:148-157
     double T[16];
     LF_RC(get_camera_pose(T));
@@ -1338,7 +1381,7 @@ size_t System::fetch_mesh_with_colour(float *v, unsigned char *c, int max_tri) {
 int System::get_camera_pose(double *out16) {
     LfTrackState h;
     LF_RC(odometry_->tracker().read_state(h));
-    pose_of(h, out16);
+    pose_of(h.pose, out16);
     return LF_OK;
 }
 
@@ -1766,16 +1809,22 @@ extern "C" int lf_batch_get_pose(lf_batch *b, int i, double *out16) {
     if (int rc = batch_index(b, i)) return rc;
     if (!out16) return lf_set_error(LF_ERR_ARG, "null pose output");
     LfTrackState h;
-    LF_RC(b->b->system(i).odometry().tracker().copy_state(h));
-    fusion::pose_of(h, out16);
+    LF_RC(b->b->read_state(i, h));
+    fusion::pose_of(h.pose, out16);
     return LF_OK;
+}
+
+extern "C" int lf_batch_latest_pose(lf_batch *b, int i, double *out16) {
+    if (int rc = batch_index(b, i)) return rc;
+    if (!out16) return lf_set_error(LF_ERR_ARG, "null pose output");
+    return b->b->latest_pose(i, out16);
 }
 
 extern "C" int lf_batch_get_tracking(lf_batch *b, int i, int *success, float *icp_error) {
     if (int rc = batch_index(b, i)) return rc;
     const fusion::DenseTracking &t = b->b->system(i).odometry().tracker();
     LfTrackState h;
-    const fusion::TrackingResult r = t.copy_state(h) == LF_OK ? t.result_of(h) : fusion::TrackingResult();
+    const fusion::TrackingResult r = b->b->read_state(i, h) == LF_OK ? t.result_of(h) : fusion::TrackingResult();
     if (success) *success = r.sucess ? 1 : 0;
     if (icp_error) *icp_error = r.icp_error;
     return LF_OK;
@@ -1791,6 +1840,5 @@ extern "C" int lf_batch_map(lf_batch *b, int i, lf_map_params *p, lf_map_storage
 
 extern "C" int lf_batch_read_counters(lf_batch *b, int i, unsigned int *out16) {
     if (int rc = batch_index(b, i)) return rc;
-    fusion::System &s = b->b->system(i);
-    return lf_map_read_counters(&s.mapping().storage(), out16, s.stream());
+    return b->b->read_counters(i, out16);
 }
