@@ -241,8 +241,9 @@ LF_DEV void alloc_wg(const MapDev &m, const float *__restrict__ depth, int cols,
     if (tx == 0 && ty == 0 && tid == 0) {
         m.counters[LF_CNT_VISIBLE] = 0u;
         // one more fusion pass: read by the integration / de-integration that
-        // follows this kernel (the seed of the mixed weights' dither)
-        m.counters[LF_CNT_FUSE_PASSES] = m.counters[LF_CNT_FUSE_PASSES] + 1u;
+        // follows this kernel (the seed of the mixed weights' dither).  Atomic, as
+        // the 2 n walks of a re-fusion count side by side
+        atomicAdd(&m.counters[LF_CNT_FUSE_PASSES], 1u);
     }
     float Twc[12];
 #pragma unroll

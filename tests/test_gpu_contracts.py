@@ -17,6 +17,65 @@ def dev(a):
     return torch.from_numpy(np.ascontiguousarray(a)).cuda()
 
 
+def room_images(K, n, seed):
+    """n frames of patches at several depths around the origin, as images with poses (device pose24)."""
+    rng = np.random.default_rng(seed)
+    imgs, poses = [], []
+    for _ in range(n):
+        patches = rng.choice([0, 700, 900, 1300, 2100], (K.height // 8 + 1, K.width // 8 + 1))
+        d16 = np.kron(patches, np.ones((8, 8), int))[:K.height, :K.width] + rng.integers(0, 4, (K.height, K.width))
+        img = capi.Image(K, 1)
+        img.upload(dev(d16.astype(np.uint16)), dev(rng.integers(0, 256, (K.height, K.width, 3)).astype(np.uint8)), 1e-3)
+        imgs.append(img)
+        T = np.eye(4)
+        a = rng.uniform(-0.3, 0.3)
+        T[:3, :3] = [[np.cos(a), 0, np.sin(a)], [0, 1, 0], [-np.sin(a), 0, np.cos(a)]]
+        T[:3, 3] = rng.uniform(-0.2, 0.2, 3)
+        poses.append(T)
+    return imgs, poses
+
+
+def by_block(m):
+    """A map's sdf codes, weights (words of a mixed map) and colours by block coordinate."""
+    n = int(m.counters()[capi.CNT_ALLOCATED])
+    b = m.blocks()
+    order = np.lexsort(b.T)
+    rgb = m.t["rgb"][: 1536 * n].view(n, -1).cpu().numpy()[order] if m.params.precision == FP32 else None
+    return [b[order], m.t["sdf"][: 512 * n].view(n, 512).cpu().numpy()[order],
+            m.t["weight"][: 512 * n].view(n, 512).cpu().numpy()[order]] + ([rgb] if rgb is not None else [])
+
+
+@pytest.mark.parametrize("n", [1, 12])
+def test_mixed_refusion_gives_the_same_twice(n):
+    """A mixed re-fusion counts 2 n passes, whatever the order of its walks, and so rounds the weights (by their
+    stochastic rounding, seeded by the count) the same in two runs from one map."""
+    K = capi.intrinsics(96, 64, 80.0, 80.0, 47.5, 31.5)
+    p = capi.map_params(1 << 16, 1 << 15, 0.01, 0.03, precision=MIXED)
+    imgs, poses = room_images(K, n, 5)
+    old = [dev(capi.pose24(T)) for T in poses]
+    new = []
+    for T in poses:
+        T[:3, 3] += 0.015
+        new.append(dev(capi.pose24(T)))
+    base = capi.Map(p, K.width, K.height)
+    for img, T in zip(imgs, old):
+        base.update_image(img, T)
+    before = int(base.counters()[capi.CNT_FUSE_PASSES])
+    assert before == n
+    runs = []
+    for _ in range(4):
+        m = capi.Map(p, K.width, K.height)
+        base.copy_to(m)
+        m.refuse_keyframes(imgs, old, new)
+        torch.cuda.synchronize()
+        assert int(m.counters()[capi.CNT_FUSE_PASSES]) == before + 2 * n
+        runs.append(by_block(m))
+    for r in runs[1:]:
+        assert all(np.array_equal(x, y) for x, y in zip(r, runs[0]))
+    for img in imgs:
+        img.close()
+
+
 def batch_of(n, precision, graphs):
     """A batch of n 640x480 cameras of one moving scene each, and six frames of them."""
     from libfusion_amd.synth import Scene
