@@ -886,10 +886,22 @@ LF_DEV const float *refuse_pose(const RefuseArgs &a, int j) {
     return (j < a.n ? a.old24[j] : a.new24[j - a.n]) + 12;
 }
 
+// The largest of a wavefront's 64 values, in every lane.
+LF_DEV int wave_max(int v) {
+    v = max(v, __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, false));   // quad_perm 1,0,3,2
+    v = max(v, __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, false));   // quad_perm 2,3,0,1
+    v = max(v, __builtin_amdgcn_mov_dpp(v, 0x141, 0xF, 0xF, false));  // row_half_mirror
+    v = max(v, __builtin_amdgcn_mov_dpp(v, 0x128, 0xF, 0xF, false));  // row_ror:8
+    const auto a = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    v = max((int)a[0], (int)a[1]);
+    const auto b = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return max((int)b[0], (int)b[1]);
+}
+
 // Whether a pose surely sees no corner of the block around the camera point c
-// (every corner within r of it): behind or beyond the update range, or outside
-// one of the image's four planes.  Slack for the rounding of c and of the
-// projections of block_visible.
+// (every corner within r of it, the rounding of c and of block_visible's
+// projections included): behind or beyond the update range, or outside one of the
+// image's four planes.
 LF_DEV bool surely_unseen(f3 c, float r, const lf_intrinsics &K, int cols, int rows, float zmin, float zmax) {
     if (c.z + r < zmin || c.z - r > zmax) return true;
     if (!(c.z - r > 0.0f)) return false;  // a corner may lie behind the camera: its projection flips
@@ -900,26 +912,47 @@ LF_DEV bool surely_unseen(f3 c, float r, const lf_intrinsics &K, int cols, int r
     return gu < -ru || hu > ru || gv < -rv || hv > rv;
 }
 
-// A pose's camera-aligned box around a block's voxels: half sizes, and its centre
-// relative to the block's, with a hundredth of a block to spare.
+// What a pose T_cw makes of a block: radius, around its centre, of its corners; half and
+// shift, the camera-aligned box around its voxels (half sizes, centre relative to the
+// block's).  Each with a hundredth of a block to spare, and for any linear part, not
+// rotations alone.
+// A block at P (its largest coordinate) is transformed with a rounding of at most 2^-20 M,
+// M = row sum of |T_cw| times P plus the translation: 14 roundings of 2^-24 for a point and
+// the centre.  The same again covers block_visible's projections: a slack of
+// scale P + offset.
 struct RefuseBox {
     f3 half, shift;
 };
-LF_DEV RefuseBox refuse_box(const float *Tcw, float vs) {
+struct RefuseSlack {
+    float radius, scale, offset;
+};
+LF_DEV RefuseBox refuse_box(const float *Tcw, float vs, RefuseSlack &s) {
     RefuseBox b;
     float *h = &b.half.x, *c = &b.shift.x;
+    float rows = 0.0f, offset = 0.0f, gram = 0.0f;
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
-        const float x = Tcw[4 * i], y = Tcw[4 * i + 1], z = Tcw[4 * i + 2];
-        h[i] = 3.5f * vs * (fabsf(x) + fabsf(y) + fabsf(z)) + 0.08f * vs;
+        const float x = Tcw[4 * i], y = Tcw[4 * i + 1], z = Tcw[4 * i + 2], row = fabsf(x) + fabsf(y) + fabsf(z);
+        h[i] = 3.5f * vs * row + 0.08f * vs;
         c[i] = -0.5f * vs * (x + y + z);  // voxels 0..7 around 3.5
+        rows = fmaxf(rows, row);
+        offset = fmaxf(offset, fabsf(Tcw[4 * i + 3]));
+        float sum = 0.0f;  // row i of T^t T, whose largest bounds the square of T's norm (1 for a rotation)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) sum += fabsf(Tcw[i] * Tcw[j] + Tcw[4 + i] * Tcw[4 + j] + Tcw[8 + i] * Tcw[8 + j]);
+        gram = fmaxf(gram, sum);
     }
+    // half a block's diagonal is 0.8660 of its side
+    s.radius = (8.0f * vs) * fmaf(0.867f, __builtin_amdgcn_sqrtf(gram), 0.008f);
+    s.scale = 0x1p-19f * rows;
+    s.offset = 0x1p-19f * offset;
     return b;
 }
 
 // Whether keyframe k changes no voxel of the block whose box at this pose is
-// c +- half: every voxel that projects into the image lies more than the truncation
-// behind the largest depth of the tiles around it (or the tiles hold no depth).
+// c +- half (their rounding included): every voxel that projects into the image lies more
+// than the truncation behind the largest depth of the tiles around it (or the tiles hold
+// no depth).
 // The box's pixels are widened by one for the rounding of the voxels' projections.
 LF_DEV bool surely_behind(const RefuseArgs &a, int k, f3 c, f3 half) {
     const float zn = c.z - half.z, zf = c.z + half.z;
@@ -956,21 +989,35 @@ LF_DEV bool surely_behind(const RefuseArgs &a, int k, f3 c, f3 half) {
 // for one of 1024 (77 VGPRs; 57 at 64 VGPRs and 1024 lanes, 50 with 256 lanes).
 constexpr int kRefuseVisThreads = 512;
 template <bool kFast>
-__global__ __launch_bounds__(kRefuseVisThreads) void k_refuse_visible(RefuseArgs a) {
+__global__ __launch_bounds__(kRefuseVisThreads, 6) void k_refuse_visible(RefuseArgs a) {
     __shared__ unsigned int s_cnt[kRefuseVisThreads / kWave];
     __shared__ unsigned int s_base;
     __shared__ float s_pose[2 * kMaxRefuse][12];
     __shared__ RefuseBox s_box[2 * kMaxRefuse];
+    __shared__ int s_most[3];  // the largest radius, slack scale and offset of all poses, as bits
     const MapDev &m = a.m;
     for (int i = threadIdx.x; i < 2 * a.n * 12; i += kRefuseVisThreads)
         s_pose[i / 12][i % 12] = refuse_pose(a, i / 12)[i % 12];
     __syncthreads();
-    for (int i = threadIdx.x; i < 2 * a.n; i += kRefuseVisThreads) s_box[i] = refuse_box(s_pose[i], m.voxel_size);
+    if (threadIdx.x < kWave) {  // a lane a pose
+        const int i = threadIdx.x;
+        RefuseSlack s = {0.0f, 0.0f, 0.0f};
+        if (i < 2 * a.n) s_box[i] = refuse_box(s_pose[i], m.voxel_size, s);
+        // (the bits of a NaN, from a pose that is not finite, are the largest: no test below says unseen then)
+        int most[3] = {__float_as_int(s.radius), __float_as_int(s.scale), __float_as_int(s.offset)};
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            most[k] = wave_max(most[k] & 0x7FFFFFFF);
+            if (i == 0) s_most[k] = most[k];
+        }
+    }
     __syncthreads();
+    // One bound for all poses, the same in every lane.  (20 keyframes: 39.0 us without the
+    // slack, 40.1 with it; a radius and slack per pose 45, the maxima by LDS atomics 59.)
+    const auto uniform = [&](int i) { return __int_as_float(__builtin_amdgcn_readfirstlane(s_most[i])); };
+    const RefuseSlack most = {uniform(0), uniform(1), uniform(2)};
     const unsigned int nb = min(m.counters[LF_CNT_ALLOCATED], (unsigned int)m.num_blocks);
-    // the half diagonal of a block with a hundredth of it to spare (coordinates
-    // are rounded to 2^-24 of at most a few thousand blocks)
-    const float scale = 8.0f * m.voxel_size, radius = 0.875f * scale;
+    const float scale = 8.0f * m.voxel_size;
     constexpr unsigned int kPerWg = kRefuseVisThreads / 4;
     const unsigned int stride = gridDim.x * kPerWg;
     const int lane = lane_id(), wave = threadIdx.x / kWave, sub = threadIdx.x & 3;
@@ -986,9 +1033,12 @@ __global__ __launch_bounds__(kRefuseVisThreads) void k_refuse_visible(RefuseArgs
             marks = a.slot_mask[p.w];
             flagged = m.slot_flag[p.w] != 0;
             const f3 centre = {((float)p.x + 0.5f) * scale, ((float)p.y + 0.5f) * scale, ((float)p.z + 0.5f) * scale};
+            const float P = fmaxf(fmaxf(fabsf(centre.x), fabsf(centre.y)), fabsf(centre.z)) + scale;
+            const float e = fmaf(most.scale, P, most.offset);
             unsigned int open = 0u;  // bit i: pose sub + 4 i
             for (int i = 0, j = sub; j < 2 * a.n; ++i, j += 4)
-                if (!surely_unseen(xform(s_pose[j], centre), radius, a.K, a.cols, a.rows, m.zmin_update, m.zmax_update))
+                if (!surely_unseen(xform(s_pose[j], centre), most.radius + e, a.K, a.cols, a.rows, m.zmin_update,
+                                   m.zmax_update))
                     open |= 1u << i;
             for (; open; open &= open - 1u) {
                 const int j = sub + 4 * __builtin_ctz(open);
@@ -997,7 +1047,7 @@ __global__ __launch_bounds__(kRefuseVisThreads) void k_refuse_visible(RefuseArgs
                     continue;
                 seen |= 1ull << j;
                 const f3 c = add(xform(s_pose[j], centre), s_box[j].shift);
-                if (surely_behind(a, j < a.n ? j : j - a.n, c, s_box[j].half))
+                if (surely_behind(a, j < a.n ? j : j - a.n, c, add(s_box[j].half, f3{e, e, e})))
                     idle |= 1ull << j;
             }
         }

@@ -76,6 +76,48 @@ def test_mixed_refusion_gives_the_same_twice(n):
         img.close()
 
 
+# at the origin; tens of kilometres from it, where a float coordinate is good to a fifth or to half a voxel; a camera
+# whose unit is a quarter of the map's, and four of them
+@pytest.mark.parametrize("offset,unit", [((0, 0, 0), 1.0), ((30000, -9000, 17000), 1.0), ((-61000, 0, 3000), 1.0),
+                                         ((0, 0, 0), 0.25), ((100, 50, -20), 4.0)])
+def test_refusion_at_any_pose(offset, unit):
+    """Re-fusion leaves the voxels seen, and their weights, that de-integrating and fusing one keyframe after the
+    other does (the same float arithmetic per voxel), wherever the cameras are and whatever their unit."""
+    K = capi.intrinsics(160, 96, 130.0, 130.0, 79.5, 47.5)
+    voxel = 0.01 * max(unit, 0.5)
+    p = capi.map_params(1 << 17, 1 << 16, voxel, 3 * voxel)
+    imgs, poses = room_images(K, 5, 9)
+
+    def pose24(T):  # T_wc = unit R, t and its inverse
+        R, t = T[:3, :3], T[:3, 3] * unit + np.asarray(offset, float)
+        wc = np.concatenate([unit * R, t[:, None]], 1)
+        cw = np.concatenate([R.T / unit, -(R.T @ t / unit)[:, None]], 1)
+        return dev(np.concatenate([wc.ravel(), cw.ravel()]).astype(np.float32))
+
+    old = [pose24(T) for T in poses]
+    new = []
+    for k, T in enumerate(poses):
+        T[:3, 3] += (0.02, -0.01, 0.013 * (k - 2))
+        new.append(pose24(T))
+    base, seq, one = (capi.Map(p, K.width, K.height) for _ in range(3))
+    for img, T in zip(imgs, old):
+        base.update_image(img, T)
+    base.copy_to(seq)
+    base.copy_to(one)
+    one.refuse_keyframes(imgs, old, new)
+    for img, T in zip(imgs, old):
+        seq.deintegrate_image(img, T)
+    for img, T in zip(imgs, new):
+        seq.update_image(img, T)
+    torch.cuda.synchronize()
+    (bo, _, wo, _), (bs, _, ws, _) = by_block(one), by_block(seq)
+    assert int(seq.counters()[capi.CNT_OVERFLOW]) == 0 and (ws > 0).sum() > 5000
+    assert np.array_equal(bo, bs)
+    assert np.array_equal(wo, ws), int((wo != ws).sum())
+    for img in imgs:
+        img.close()
+
+
 def batch_of(n, precision, graphs):
     """A batch of n 640x480 cameras of one moving scene each, and six frames of them."""
     from libfusion_amd.synth import Scene
