@@ -153,10 +153,14 @@ LF_HD unsigned int weight_code_sr(float w, unsigned int rnd) {
     return !(w > 0.0f) ? 0u : w < 0.015625f ? small : big;
 }
 
-// weight_code_sr of a w in (0, 255], whose code needs no clamp; the codes below 2^-6,
-// which few weights have, are computed only in a wavefront that has one.
+// weight_code_sr of a w in [2^-6, 255], whose code needs no clamp.
+LF_DEV unsigned int weight_code_sr_normal(float w, unsigned int rnd) {
+    return (__float_as_uint(w) - (120u << 23) + (rnd & 0x7FFFFu)) >> 19;
+}
+// weight_code_sr of a w in (0, 255]; the codes below 2^-6, which few weights have, are
+// computed only in a wavefront that has one.
 LF_DEV unsigned int weight_code_sr_in_range(float w, unsigned int rnd) {
-    unsigned int c = (__float_as_uint(w) - (120u << 23) + (rnd & 0x7FFFFu)) >> 19;
+    unsigned int c = weight_code_sr_normal(w, rnd);
     if (__builtin_expect(__any(w < 0.015625f), 0)) c = w < 0.015625f ? weight_code_sr(w, rnd) : c;
     return c;
 }
@@ -203,7 +207,7 @@ LF_DEV unsigned int rgb_at(const unsigned char *__restrict__ rgb, size_t pix, bo
 }
 
 // The colour bits of a mixed voxel's word from three means in [0, 256) (above by
-// rounding only): each truncated, at most 255.
+// rounding only): each truncated, at most 255.  A NaN becomes 0 here.
 LF_DEV unsigned int word_colour_of(float r, float g, float b) {
     // the conversion rounds and clamps; of a whole number it takes that number
     unsigned int c = __builtin_amdgcn_cvt_pk_u8_f32(floorf(r), 1, 0u);

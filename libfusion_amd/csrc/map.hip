@@ -710,16 +710,23 @@ LF_DEV void integrate_wg(const MapDev &m, const float *__restrict__ depth, const
                     at_byte(wd_b, vgpr_offset(4u * o)) = code | colour;
                     continue;
                 }
-                const float inv = __builtin_amdgcn_rcpf(wp[h] + wt);
+                const float wn = wp[h] + wt, inv = __builtin_amdgcn_rcpf(wn);
                 const float spf = half_bits_to_float((unsigned short)sp[h]);
                 at_byte(sdf16, vgpr_offset(2u * o)) = float_to_half_bits((spf * wp[h] + sdf_h * wt) * inv);
-                const unsigned int code = weight_code_sr_in_range(fminf(wp[h] + wt, 255.0f), rnd);
+                unsigned int code = weight_code_sr_normal(fminf(wn, 255.0f), rnd);
+                float mc[3];
                 if (kColour) {
-                    float mc[3];
 #pragma unroll
                     for (int k = 0; k < 3; ++k)
                         mc[k] = ((float)word_channel(word[h], k) * wp[h] + (float)cin[k] * wt) * inv;
                     colour = word_colour_of(mc[0], mc[1], mc[2]);
+                }
+                // Few wavefronts hold a weight below 2^-6 or one that makes the means NaN (not
+                // finite, or past 2^60 here): their codes and clamps, with one test for both
+                // (a clamp for all: 526.5 us for the 16 maps' 523.4).
+                if (__builtin_expect(__any(__float_as_uint(wn) - (121u << 23) > (187u - 121u) << 23), 0)) {
+                    code = weight_code_sr(fminf(wn, 255.0f), rnd);
+                    if (kColour) colour = word_colour_of(fminf(mc[0], 255.0f), fminf(mc[1], 255.0f), fminf(mc[2], 255.0f));
                 }
                 at_byte(wd_b, vgpr_offset(4u * o)) = code | colour;
                 continue;
