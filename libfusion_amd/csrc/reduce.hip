@@ -1100,11 +1100,17 @@ int lf_track_read(const LfTrackState *st, LfTrackState *host, hipStream_t stream
     return LF_OK;
 }
 
+// A tag that no other call of either reduction in this process has (they may share a
+// scratch) and that no float pair is likely to hold.
+static unsigned long long next_tag() {
+    static std::atomic<unsigned long long> calls{0};
+    return 0x9E3779B97F4A7C15ull * (calls.fetch_add(1, std::memory_order_relaxed) + 1);
+}
+
 // The launch of a stand-alone reduction: rows and flags share the scratch of
 // `capacity` floats.
 template <int kMode>
 static int launch_reduce(ReduceArgs &a, float *scratch, size_t capacity, float *sum29, hipStream_t st) {
-    static std::atomic<unsigned long long> calls{0};
     const int G = grid_for(a.lv);
     a.partials = scratch;
     // the flags behind the most rows, on an 8-byte boundary
@@ -1112,9 +1118,7 @@ static int launch_reduce(ReduceArgs &a, float *scratch, size_t capacity, float *
     auto *flags = reinterpret_cast<unsigned long long *>((end + 7) & ~(uintptr_t)7);
     if (reinterpret_cast<uintptr_t>(flags + G) > reinterpret_cast<uintptr_t>(scratch + capacity))
         return lf_set_error(LF_ERR_CAPACITY, "a reduction of %d workgroups does not fit %zu scratch floats", G, capacity);
-    // a tag no other call has and no float pair is likely to hold
-    const unsigned long long tag = 0x9E3779B97F4A7C15ull * (calls.fetch_add(1, std::memory_order_relaxed) + 1);
-    k_reduce<kMode><<<G, kThreads, 0, st>>>(a, sum29, flags, tag);
+    k_reduce<kMode><<<G, kThreads, 0, st>>>(a, sum29, flags, next_tag());
     LF_LAUNCH_CHECK();
     return LF_OK;
 }
