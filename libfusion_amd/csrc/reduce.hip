@@ -29,6 +29,7 @@
 #include <atomic>
 #include <cfloat>
 #include <climits>
+#include <functional>
 #include <mutex>
 
 #include "lf_common.h"
@@ -1107,11 +1108,24 @@ static unsigned long long next_tag() {
     return 0x9E3779B97F4A7C15ull * (calls.fetch_add(1, std::memory_order_relaxed) + 1);
 }
 
+// Floats of the most rows and the flags behind them on an 8-byte boundary.
+constexpr size_t kRowsAndFlags = (size_t)kGrid * kVals + 2 * kGrid + 1;
+// A caller's scratch holds them twice with room for the sums between.
+static_assert((size_t)kGrid * 62 + 64 >= 2 * kRowsAndFlags + kVals, "sums inside the scratch overlap one place only");
+
 // The launch of a stand-alone reduction: rows and flags share the scratch of
-// `capacity` floats.
+// `capacity` floats.  They lie at its start, or at its end where the caller has the
+// sums written into the start: one workgroup may store them while another still
+// reads the rows.
 template <int kMode>
 static int launch_reduce(ReduceArgs &a, float *scratch, size_t capacity, float *sum29, hipStream_t st) {
     const int G = grid_for(a.lv);
+    const auto overlap = [](const float *x, size_t nx, const float *y, size_t ny) {
+        return std::less<const float *>()(x, y + ny) && std::less<const float *>()(y, x + nx);
+    };
+    const size_t shift = capacity > kRowsAndFlags && overlap(sum29, kVals, scratch, kRowsAndFlags) ? capacity - kRowsAndFlags : 0;
+    capacity -= shift;
+    scratch += shift;
     a.partials = scratch;
     // the flags behind the most rows, on an 8-byte boundary
     const uintptr_t end = reinterpret_cast<uintptr_t>(scratch + (size_t)kGrid * kVals);

@@ -1,5 +1,6 @@
 """GPU: what the entry points promise beside their values: which work a read waits for, what a call's scratch may
 hold, that a call gives the same twice, inputs at the end of the ranges that they take."""
+import ctypes
 import threading
 
 import numpy as np
@@ -116,6 +117,42 @@ def test_refusion_at_any_pose(offset, unit):
     assert np.array_equal(wo, ws), int((wo != ws).sum())
     for img in imgs:
         img.close()
+
+
+# a single workgroup, 45 of them, the capped grid
+@pytest.mark.parametrize("width,height", [(20, 15), (160, 144), (640, 480)])
+def test_reduction_sums_inside_the_scratch(width, height):
+    """sum29 anywhere in the scratch: the rows, the flags, its middle, its end.  The same sums as beside it."""
+    rng = np.random.default_rng(4)
+    K = capi.intrinsics(width, height, 1.2 * width, 1.2 * width, (width - 1) / 2, (height - 1) / 2)
+    d = (1.0 + 0.1 * rng.random((height, width))).astype(np.float32)
+    x, y = np.meshgrid(np.arange(width), np.arange(height))
+    v = np.stack([d * (x - K.cx) / K.fx, d * (y - K.cy) / K.fy, d, np.ones_like(d)], -1).astype(np.float32)
+    n = rng.normal(size=(height, width, 4)).astype(np.float32)
+    n[..., :3] /= np.linalg.norm(n[..., :3], axis=-1, keepdims=True)
+    I, g = (rng.random((height, width)).astype(np.float32) * s for s in (200, 20))
+    t = [dev(a) for a in (v, n, v + np.float32(0.001), n, I, I + 1, g, g)]
+    lib, P, pose = capi.load(), capi.ptr, dev(np.eye(4, dtype=np.float32)[:3].ravel())
+    size = lib.lf_reduce_scratch_floats()
+    scratch = torch.zeros(size + 64, device="cuda")
+
+    def both(at):
+        out = []
+        st = capi.stream_ptr()
+        s = scratch[at: at + 29]
+        for _ in range(3):
+            capi.check(lib.lf_icp_reduce(P(t[0]), P(t[1]), P(t[2]), P(t[3]), width, height, P(pose), ctypes.byref(K),
+                                         P(scratch), P(s), st))
+            out.append(s.cpu().numpy().copy())
+            capi.check(lib.lf_rgb_step(P(t[4]), P(t[5]), P(t[2]), P(t[6]), P(t[7]), width, height, 5.0, P(pose),
+                                       ctypes.byref(K), P(scratch), P(s), st))
+            out.append(s.cpu().numpy().copy())
+        return out
+
+    want = both(size)  # behind the scratch
+    assert want[0][28] > 100 and want[1][28] > 100
+    for at in (0, 1, 512 * 14, 512 * 29 - 15, 512 * 29 + 3, 512 * 31 - 29, 512 * 31, 512 * 31 + 17, size // 2, size - 29):
+        assert all(np.array_equal(a, b) for a, b in zip(both(at), want)), at
 
 
 # a normal whose z is NaN, and a depth of 0 accepted by the range: frame weights of NaN and of infinity
