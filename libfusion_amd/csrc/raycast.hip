@@ -345,27 +345,17 @@ LF_DEV unsigned short sdf_bits(const RayDev &r, int vi) { return at_byte(reinter
 // findVoxel + read_sdf (ray_tracing.cu:291-305) at a sample of an in-range
 // ray.  A voxel is valid when its weight is non-zero, which the sdf plane
 // encodes (kSdfUnseen; kHalfUnseen, a NaN, in mixed precision), so one 2-byte
-// load per sample decides both validity and value.
-// floor_out (or null) receives floor(p).
+// load per sample decides both validity and value.  (The march reads its samples
+// itself; this is the voxel whose colour is taken, -1 where it is not valid.)
 template <bool kMixed>
-LF_DEV float read_sdf(const RayDev &r, BlockCache &bc, f3 p, bool &valid, int *voxel_out = nullptr,
-                      i3 *floor_out = nullptr) {
+LF_DEV int valid_voxel(const RayDev &r, BlockCache &bc, f3 p) {
     const int vx = ray_floor(p.x), vy = ray_floor(p.y), vz = ray_floor(p.z);
-    if (floor_out) *floor_out = i3{vx, vy, vz};
     const int b = resolve(r, bc, vx >> 3, vy >> 3, vz >> 3);
-    valid = false;
-    if (b < 0) return __int_as_float(0x7fc00000);
+    if (b < 0) return -1;
     const int vi = b * LF_BLOCK3 + lidx(vx, vy, vz);
-    if (voxel_out) *voxel_out = vi;
-    if constexpr (kMixed) {
-        const float sv = half_bits_to_float(sdf_bits(r, vi));
-        valid = !isnan(sv);
-        return sv;
-    }
-    const short sd = (short)sdf_bits(r, vi);
-    if (sd == kSdfUnseen) return __int_as_float(0x7fc00000);
-    valid = true;
-    return unpack_sdf(sd);
+    const unsigned short code = sdf_bits(r, vi);
+    const bool valid = kMixed ? !isnan(half_bits_to_float(code)) : (short)code != kSdfUnseen;
+    return valid ? vi : -1;
 }
 
 // read_sdf_interped (ray_tracing.cu:307-339).  Corner k is the voxel of
@@ -676,10 +666,8 @@ LF_DEV void raycast_wg(const RayDev &r, float *__restrict__ vmap, unsigned char 
         res = add(res, mul(dir1, step));
         if (!valid) break;
         if (kCheckColour) {  // read_colour (ray_tracing.cu:427-441)
-            bool cv;
-            int vi = -1;
-            read_sdf<kMixed>(r, bc, res, cv, &vi);
-            if (!cv) break;
+            const int vi = valid_voxel<kMixed>(r, bc, res);
+            if (vi < 0) break;
             if constexpr (kMixed) {  // colour packed beside the weight code
                 const unsigned int word = reinterpret_cast<const unsigned int *>(r.weight)[vi];
                 col[0] = (unsigned char)word_channel(word, 0);

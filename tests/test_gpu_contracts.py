@@ -155,6 +155,45 @@ def test_reduction_sums_inside_the_scratch(width, height):
         assert all(np.array_equal(a, b) for a, b in zip(both(at), want)), at
 
 
+# inside the block directory, across its upper and its lower end, beside it, far outside it
+@pytest.mark.parametrize("centre", [(0, 0, 3), (126, 1, 4), (-127, -126, 2), (2, 0, 127), (3, 131, 2), (-200, 150, 260)])
+def test_mixed_raycast_around_the_directory(centre):
+    """A mixed map's raycast of a rough surface with holes, vertex for vertex and colour for colour that of an FP32 map
+    of the same values: sdfs of -1 and 1, which both storages hold exactly."""
+    from tests.test_gpu_kernels import map_of_blocks
+    rng = np.random.default_rng(31)
+    width, height, voxel = 72, 48, 0.01
+    pos = np.array([(x, y, z) for x in range(-4, 4) for y in range(-4, 4) for z in range(-1, 2)]) + centre
+    pos = pos[rng.random(len(pos)) < 0.85]
+    z, y, x = np.meshgrid(*[np.arange(8)] * 3, indexing="ij")
+    at = pos[:, :, None] * 8 + np.stack([x.ravel(), y.ravel(), z.ravel()])[None]
+    surface = centre[2] * 8 + 4 + 3 * np.sin(0.3 * at[:, 0]) * np.cos(0.2 * at[:, 1]) + rng.random((len(pos), 512))
+    inside = at[:, 2] > surface
+    seen = rng.random((len(pos), 512)) < 0.93
+    rgb = rng.integers(0, 256, (len(pos), 3, 512)).astype(np.uint8)
+    one, minus = np.float16(1).view(np.int16), np.float16(-1).view(np.int16)
+    codes = {FP32: np.where(seen, np.where(inside, -32767, 32767), capi.SDF_UNSEEN).astype(np.int16),
+             MIXED: np.where(seen, np.where(inside, minus, one), -1).astype(np.int16)}
+    weight = {FP32: seen.astype(np.float32), MIXED: (0x70 * seen).astype(np.uint8)}
+    K = capi.intrinsics(width, height, 60.0, 60.0, (width - 1) / 2, (height - 1) / 2)
+    for turn in (0.0, 0.4, -0.7):
+        T = np.eye(4)
+        T[:3, :3] = [[np.cos(turn), 0, np.sin(turn)], [0, 1, 0], [-np.sin(turn), 0, np.cos(turn)]]
+        T[:3, 3] = (np.array(centre) + 0.5) * 0.08 - 0.7 * T[:3, 2]
+        got = []
+        for precision in (FP32, MIXED):
+            m = map_of_blocks(precision, pos, codes[precision], weight[precision], rgb, voxel, size=(width, height))
+            vm = torch.zeros((height, width, 4), device="cuda")
+            col = torch.zeros((height, width, 3), dtype=torch.uint8, device="cuda")
+            m.raycast_check_visibility(vm, dev(capi.pose24(T)), K, rgb_out=col)
+            torch.cuda.synchronize()
+            got.append((vm.cpu().numpy(), col.cpu().numpy()))
+        hit = ~np.isnan(got[0][0][..., 0])
+        assert hit.mean() > 0.2
+        assert np.array_equal(got[0][0][hit], got[1][0][hit]) and np.isnan(got[1][0][~hit]).all()
+        assert np.array_equal(got[0][1], got[1][1])
+
+
 # a normal whose z is NaN, and a depth of 0 accepted by the range: frame weights of NaN and of infinity
 @pytest.mark.parametrize("depth,normal", [(0.04, float("nan")), (0.0, 1.0)])
 def test_mixed_colours_of_frames_without_a_finite_weight(depth, normal):
