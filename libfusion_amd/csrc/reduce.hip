@@ -672,6 +672,19 @@ LF_DEV double block_sums_d(CombinedSums &sums, double (*s_wave)[32]) {
     return t;
 }
 
+// Whether this lane's share of G <= 64 kChunks flags all hold the tag, every load in
+// flight at once (a loop that ends at the first other flag takes 64 of them a memory
+// round: 0.7 us more a launch at 512 workgroups).
+template <int kChunks>
+LF_DEV bool all_set(const unsigned long long *flags, int G, unsigned long long tag) {
+    unsigned long long f[kChunks], differ = 0ull;
+#pragma unroll
+    for (int c = 0; c < kChunks; ++c) f[c] = load_agent(&flags[min(c * 64 + (int)threadIdx.x, G - 1)]);
+#pragma unroll
+    for (int c = 0; c < kChunks; ++c) differ |= f[c] ^ tag;
+    return differ == 0ull;
+}
+
 // Stand-alone reductions (lf_icp_reduce, lf_rgb_step) in one launch.  kMode 1:
 // ICP rows, 2: RGB rows.  Each workgroup writes its kVals partials value-major
 // (value v of workgroup g at v * G + g), then its flag, and reads every flag: the
@@ -683,9 +696,11 @@ LF_DEV double block_sums_d(CombinedSums &sums, double (*s_wave)[32]) {
 // waits for its rows' stores before its flag's, and for its flag's before it
 // reads the others, so the one whose flag arrives last sees them all.  Another
 // may too: both store the same sums.
-// A call's time is its launches on the host (19.6 us for an ICP and a
-// photometric reduction of 160x120 in two launches each): 5.0 + 2.8 us of
-// kernels became 6.3, and the call 13.8 us.
+// A small call's time is its launches on the host, a large one's the rows.  An ICP and
+// a photometric reduction, in two launches each and now, us among others (waited for
+// alone): 160x120 17.6 and 13.9 (31.5 and 27.9), 320x240 17.6 and 14.2 (31.8 and 29.9),
+// 640x480 20.4 and 19.6 (36.2 and 35.7), 848x480 21.9 and 22.1 (38.3 and 38.4), 1280x960
+// 36.5 and 36.5 (52.6 and 52.6).
 template <int kMode>
 __global__ __launch_bounds__(kThreads) void k_reduce(ReduceArgs a, float *__restrict__ out29, unsigned long long *flags,
                                                      unsigned long long tag) {
@@ -709,8 +724,8 @@ __global__ __launch_bounds__(kThreads) void k_reduce(ReduceArgs a, float *__rest
         wait_stores();
         if (tid == 0) store_agent(&flags[blockIdx.x], tag);
         wait_stores();
-        bool all = true;
-        for (int g = tid; g < G; g += 64) all = all && load_agent(&flags[g]) == tag;
+        const bool all = G <= 64 ? all_set<1>(flags, G, tag) : G <= 256 ? all_set<4>(flags, G, tag)
+                                                                        : all_set<kGrid / 64>(flags, G, tag);
         if (__ballot(all) == ~0ull && tid == 0) s_all = 1;
         else if (tid == 0) s_all = 0;
     }
