@@ -8,10 +8,12 @@
 // (compute_transform :23-156).
 //
 // MI355X design:
-//  * One kernel evaluates both the ICP row and the RGB row of every reference
-//    pixel (they share the projected vertex), accumulating 2 x 29 sums per lane.
-//  * Wavefront reduction uses 64-lane shuffles, then 4 wavefront partials meet
-//    in LDS; each workgroup writes one partial row.
+//  * A tracking step evaluates both the ICP row and the RGB row of every reference
+//    pixel (they share the projected vertex) and accumulates their combined normal
+//    equations, 31 FP64 sums per lane; a stand-alone reduction has one kind of row
+//    and 29 FP32 sums.
+//  * A wavefront's sums are a transpose butterfly by DPP and permlane swaps, then the
+//    8 wavefronts' partials meet in LDS; each workgroup writes one partial row.
 //  * One lane per reference pixel, so a whole pyramid level is in flight at
 //    once (the pass is bound by memory latency, not bandwidth); each pixel's
 //    loads are issued in two rounds.
@@ -25,7 +27,7 @@
 //    round trip (the reference downloads the sums and solves on the host twice
 //    per iteration).
 //  * The stand-alone reductions of the C-ABI (lf_icp_reduce, lf_rgb_step) are
-//    one launch, whose last workgroup sums the rows.
+//    one launch, in which a workgroup that finds every row written sums them.
 #include <atomic>
 #include <cfloat>
 #include <climits>
@@ -61,7 +63,6 @@ struct ReduceArgs {
     int prev_first_iter;   // the previous step's first_iter,
     int prev_grid;         // and its workgroups (partial rows)
     int context_mode;      // compute_transform(ctx) semantics
-    unsigned long long record;  // number of the end's pose among the state's records (0: not recorded)
     float icp_weight;
     double init[12];       // initial estimate (step 0)
     float init_f[12];      // the same in FP32 (the first step's pose, uniform across the grid)
@@ -888,14 +889,14 @@ __global__ __launch_bounds__(kThreads, 4) void k_track_step(ReduceArgs a) {
 // After the frame's last step (one workgroup): its solve, then the finish.  A
 // frame that ended before (an error became NaN, the finest level broke out of
 // its loop) left the estimate as it was then.
-LF_DEV void track_end_wg(const ReduceArgs &a, StepLds &s) {
+LF_DEV void track_end_wg(const ReduceArgs &a, StepLds &s, unsigned long long record) {
     const LfGnState g = solve_previous(a, 0, s);
-    if (threadIdx.x == 0) track_finish(*a.st, g.est, g.invalid, a.context_mode != 0, a.record);
+    if (threadIdx.x == 0) track_finish(*a.st, g.est, g.invalid, a.context_mode != 0, record);
 }
 
-__global__ __launch_bounds__(kThreads) void k_track_end(ReduceArgs a) {
+__global__ __launch_bounds__(kThreads) void k_track_end(ReduceArgs a, unsigned long long record) {
     __shared__ StepLds s;
-    track_end_wg(a, s);
+    track_end_wg(a, s, record);
 }
 
 // Launch arguments read from a descriptor table, their pointers asserted global.
@@ -916,6 +917,7 @@ LF_DEV ReduceArgs global_args(const ReduceArgs &d) {
 struct TrackJob {
     ReduceArgs a;
     int G;
+    unsigned long long record;  // number of the end's pose record (0: none)
 };
 
 // Step s of several systems (each its own tracker state, scratch and
@@ -934,7 +936,7 @@ __global__ __launch_bounds__(kThreads) void k_track_end_batch(const TrackJob *__
     __shared__ StepLds s;
     const TrackJob &j = jobs[blockIdx.x];
     if (j.G <= 0) return;
-    track_end_wg(global_args(j.a), s);
+    track_end_wg(global_args(j.a), s, j.record);
 }
 
 __global__ void k_track_finish(LfTrackState *st, unsigned long long record) {
@@ -1025,7 +1027,6 @@ static ReduceArgs step_args(const LfTrackLevel &lv, float *scratch, LfTrackState
     a.prev_grid = f.prev_grid;
     a.icp_weight = icp_weight;
     a.context_mode = f.context_mode;
-    a.record = f.record;
     for (int k = 0; k < 12; ++k) {
         a.init[k] = f.init[k];
         a.init_f[k] = (float)f.init[k];
@@ -1048,7 +1049,7 @@ int lf_track_step(const LfTrackLevel &lv, float *scratch, LfTrackState *st, cons
     if (int rc = check_level(lv)) return rc;
     const ReduceArgs a = step_args(lv, scratch, st, f, icp_weight);
     const int G = step_grid(lv, 1, 0, f.end);
-    if (f.end) k_track_end<<<1, kThreads, 0, stream>>>(a);
+    if (f.end) k_track_end<<<1, kThreads, 0, stream>>>(a, f.record);
     else if (lv.half_maps) k_track_step<true><<<G, kThreads, 0, stream>>>(a);
     else k_track_step<false><<<G, kThreads, 0, stream>>>(a);
     LF_LAUNCH_CHECK();
@@ -1070,6 +1071,7 @@ int lf_track_job_make(const LfTrackLevel &lv, float *scratch, LfTrackState *st, 
     // aggregate in mixed precision.  16 and 64 workgroups each measured
     // slower than 32 (5.46k and 5.61k against 5.74k).
     j.G = step_grid(lv, share, wgs, f.end);
+    j.record = f.record;
     if (grid) *grid = j.G;
     return LF_OK;
 }
