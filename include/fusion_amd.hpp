@@ -187,13 +187,14 @@ public:
     int plan(DeviceImage &reference, DeviceImage &current, const TrackingContext &c,
              std::vector<unsigned char> &jobs, std::vector<int> &grids);
     // Planned steps of a tracker that shares its launches with share - 1
-    // others take 1/share of the reduction grid (a Batch sets it).
+    // others take 1/share of the resident workgroups (512) and at most a lone
+    // system's 256 (a Batch sets it).
     void set_batch_share(int share) {
         batch_share_ = share < 1 ? 1 : share;
         in_batch_ = true;
     }
-    // wgs > 0: planned steps take exactly that many workgroups (at most a
-    // lone system's grid) instead of 1/share of it.
+    // wgs > 0: planned steps take that many workgroups (at most 512 and one per 512
+    // pixels of the level) instead of a share.
     void set_batch_workgroups(int wgs) { batch_wgs_ = wgs < 0 ? 0 : wgs; }
     // compute_transform(ctx) (icp_tracker.cpp:210-314) on the set_* pyramids
     // (source = current frame, reference = last); success is unconditional.
@@ -362,13 +363,12 @@ private:
 // Several independent systems stepped together (no counterpart in the
 // reference, which runs one System per process).  A step uploads every
 // system's frame, pass p of all systems in one launch, on an upload stream
-// that overlaps the previous step's fusion and raycast; runs the Gauss-Newton
-// steps of all systems on the batch's stream, step s of every system in one
-// launch; fuses each map on its own stream; runs one batched z-range +
-// raycast launch per stage for all maps; then the re-pyramids, again one
-// launch per pass for all systems.  The batched launches replace 2 x 18 tracking
-// launches and 6 pyramid launches per system and pack the raycasts' long-ray
-// tails onto one grid.
+// that overlaps the previous step's tracking, fusion and raycast; then, on the
+// batch's stream and each in one launch for all systems, the Gauss-Newton steps
+// and the frames' ends, the maps' allocation, visible lists and integration, the
+// z-ranges and raycasts, and the re-pyramids, pass by pass.  With three levels and
+// 18 steps that is 28 launches, where each system alone takes as many, and the
+// raycasts' long-ray tails share one grid.
 class Batch {
 public:
     Batch(const lf_system_config *cfgs, int n);

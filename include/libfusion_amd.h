@@ -558,10 +558,11 @@ int lf_system_read_timing(lf_system *sys, int stage, int *launches, double *tota
  * sizes may differ).  lf_batch_process takes one frame per system (device
  * pointers, uint16 depth and uint8 RGB of system i's size): pass p of every
  * system's image pyramid runs in one launch, Gauss-Newton step s of every
- * system in one launch, each map is fused on its own stream, then one
- * batched z-range + raycast launch per stage covers every map, then the
- * re-pyramids.  All systems share one precision (LF_ERR_ARG otherwise).  The
- * tracking reductions of n systems take 1/n of a lone system's grid each, so
+ * system in one launch, every map's allocation, visible list and integration in
+ * one launch each, then one batched z-range + raycast launch per stage covers
+ * every map, then the re-pyramids.  All systems share one precision (LF_ERR_ARG
+ * otherwise).  The tracking reductions of n systems take 512 / n workgroups each
+ * (at most a lone system's 256), so
  * each system's poses, tracking results and volume equal those of the same
  * system run alone up to FP64 summation order in the tracking sums (exactly
  * when n is 1).
@@ -599,7 +600,8 @@ int lf_batch_read_timing(lf_batch *b, int stage, int *launches, double *total_ms
  *     upload stream beside the previous step's fusion and raycast; 0 on the
  *     batch stream ahead of the step's tracking.
  *   LF_BATCH_OPT_TRACK_WORKGROUPS: workgroups per system of each Gauss-Newton
- *     step, 1..512 (0, the default: 512 / n, at most the level's pixels / 512).
+ *     step, 1..512 (0, the default: 512 / n and at most 256; never more than the
+ *     level's pixels / 512).
  *   LF_BATCH_OPT_INTEGRATE_WORKGROUPS: workgroups per map of the batched
  *     integration, 1..65535 (0, the default: max(2048, 8192 / n)).
  *   LF_BATCH_OPT_ZRANGE_WORKGROUPS: workgroups per map of the batched z-range

@@ -19,7 +19,8 @@
 //  * A 16x16-pixel workgroup first deduplicates its requests in an LDS hash set
 //    (ds_cmpst_b64): neighbouring pixels request the same few blocks, so only
 //    unique keys reach HBM.
-//  * The visible list is appended with one atomic per wavefront (ballot + popc).
+//  * The visible list is appended with one atomic per workgroup (ballots, the
+//    wavefronts' counts prefixed in LDS).
 //  * Integration walks the visible list with a fixed grid (grid-stride), one
 //    256-thread workgroup per 8^3 block: each lane owns two voxels of the
 //    block's contiguous 512-voxel run, so every voxel plane is read and written

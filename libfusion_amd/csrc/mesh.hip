@@ -21,8 +21,10 @@
 //  * One atomic reserves the output of the workgroup's eight blocks: the
 //    appends to one counter serialise.
 //  Measured on 18k blocks / 2.43 M triangles with normals (8 mm, mixed, 175 MB
-//  out): 406 -> 95 us.  Half of that is the chain block -> neighbours ->
-//  lattice -> reservation (49 us with the emission left out), so the kernel is
+//  out): 406 -> 95 us.  Whole calls, the count read: vertices 238 -> 96 us (FP32 88),
+//  normals 365 -> 109 (FP32 364 -> 105), colours, each vertex's gathered where it is
+//  emitted, 320 -> 109 (FP32 354 -> 108).  Half of the kernel is the chain block ->
+//  neighbours -> lattice -> reservation (49 us with the emission left out), so it is
 //  held to 64 VGPRs for 8 wavefronts per SIMD; stores through LDS, contiguous
 //  over the wavefront, cost that occupancy and took 114 us, and the eight
 //  wavefronts sharing one triangle list 138 us.
