@@ -136,8 +136,8 @@ LF_DEV void stage_block(const MeshDev &m, MeshWave &s, int blk_i, int4 P, int la
     const size_t own = (size_t)blk_i * LF_BLOCK3 + 8 * lane;
     unsigned short row[8];
     {
-        const uint4 r = *reinterpret_cast<const uint4 *>(sdf16 + own);
-        const unsigned int q[4] = {r.x, r.y, r.z, r.w};
+        unsigned int q[4];  // one 16-byte load; a caller's plane need only be aligned to its codes
+        __builtin_memcpy(q, sdf16 + own, 16);
 #pragma unroll
         for (int k = 0; k < 8; ++k) row[k] = (unsigned short)(q[k >> 1] >> (16 * (k & 1)));
         if constexpr (kMode == 2) {

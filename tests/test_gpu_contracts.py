@@ -8,6 +8,7 @@ import pytest
 import torch
 
 from libfusion_amd import capi
+from tests.helpers import triangles_in_hash_order
 
 pytestmark = pytest.mark.gpu
 
@@ -153,6 +154,27 @@ def test_reduction_sums_inside_the_scratch(width, height):
     assert want[0][28] > 100 and want[1][28] > 100
     for at in (0, 1, 512 * 14, 512 * 29 - 15, 512 * 29 + 3, 512 * 31 - 29, 512 * 31, 512 * 31 + 17, size // 2, size - 29):
         assert all(np.array_equal(a, b) for a, b in zip(both(at), want)), at
+
+
+@pytest.mark.parametrize("precision", [FP32, MIXED])
+def test_mesh_of_an_sdf_plane_between_other_data(precision):
+    """A caller's sdf plane that starts on no 4-byte boundary: the same triangles as from one that does."""
+    from tests.test_gpu_kernels import map_of_blocks
+    rng = np.random.default_rng(8)
+    pos = np.array([(x, y, z) for x in range(3) for y in range(2) for z in range(2)])
+    value = rng.choice([-1.0, 1.0], (len(pos), 512))
+    sdf = (value.astype(np.float16).view(np.int16) if precision == MIXED else (value * 32767).astype(np.int16))
+    weight = np.full((len(pos), 512), 0x70, np.uint8) if precision == MIXED else np.ones((len(pos), 512), np.float32)
+    m = map_of_blocks(precision, pos, sdf, weight, rng.integers(0, 256, (len(pos), 3, 512)).astype(np.uint8))
+    want, _, n = m.mesh(0, 100000)
+    aside = torch.zeros(m.t["sdf"].numel() + 8, dtype=torch.int16, device="cuda")
+    for at in (1, 3, 5):
+        plane = aside[at: at + m.t["sdf"].numel()]
+        plane.copy_(m.t["sdf"])
+        m.storage.sdf = plane.data_ptr()
+        got, _, k = m.mesh(0, 100000)
+        assert k == n > 1000
+        assert np.array_equal(*(triangles_in_hash_order(t.cpu().numpy()) for t in (got, want)))
 
 
 # inside the block directory, across its upper and its lower end, beside it, far outside it
