@@ -509,7 +509,7 @@ LF_DEV void fill_weight_table(float *s) {
 // a normal are one load each (645x483, 5 mm: 74.6 us with divisions and scalar
 // loads, 68.3 now; take-out, a voxel at a time with its loads in sequence before,
 // 89.8, now 70.2).  16 mixed maps of 640x480, 5 mm, by both: 2.56 GB, at 4.9 TB/s
-// the rate of a large copy, and 414 us of vector instructions: 539 us with the low
+// the rate of a large copy, and 421 us of vector instructions: 539 us with the low
 // weight codes and the colours' clamps computed for all, 524 now (one map of 848x480,
 // 4 mm, 48.3 -> 46.1).
 template <bool kWeighted, bool kColour, bool kPacked, bool kMixed, bool kTable = false, bool kTakeOut = false>
